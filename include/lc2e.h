@@ -81,7 +81,11 @@ const char* lc2e_last_error(void);
  * (interpolator.cuh:27-41 global __constant__ mappers). */
 int lc2e_create(int device, size_t hbm_budget_bytes, lc2e_engine** out);
 void lc2e_destroy(lc2e_engine* e);
-/* Bytes currently allocated by the engine and its budget. */
+/* Bytes currently charged to the engine's budget, and the budget. An engine without a budget
+ * also keeps, with each 3D pair whose moving image is the high-resolution one (radius up to
+ * 4), a workspace of 8 bytes per grid voxel and pose of its largest batch, at most 1 GiB or
+ * one pose; it is not counted here. Under a budget such pairs are evaluated without it, by a
+ * slower kernel (LC2 agrees to rounding), so what a budget admits does not depend on it. */
 int lc2e_memory(lc2e_engine* e, size_t* used, size_t* budget);
 
 /* Upload a resident fixed or moving image. Replaces Interpolator*'s thrust copies of the

@@ -145,6 +145,10 @@ struct lc2e_pair {
     int* mi_ext = nullptr;
     unsigned* mi_hist = nullptr;
     double* mi_out = nullptr;
+    // two-kernel path: the warped moving image of ws_poses poses, 8 bytes per voxel and pose
+    // (kept with the pair; see grow_workspace)
+    float2* ws = nullptr;
+    int ws_poses = 0;
     int resident_per_cu = 0;  // fused work-groups one CU holds at once (0: not queried yet)
     // separable path (radius beyond the fused kernels): grids and box-sum buffers, made at
     // pair creation
@@ -188,6 +192,20 @@ lc2e::FusedArgs make_args(lc2e_pair* p, const float* d_mats, double* d_partials,
 // The pair's evaluation kernels for n poses: the fused kernel, or the separable path for
 // radii beyond it.
 hipError_t launch_eval(lc2e_pair* p, const lc2e::FusedArgs& a, int n, hipStream_t st) {
+    if (p->ws) {
+        // as many poses at a time as the workspace holds, in equal parts
+        const int parts = (n + p->ws_poses - 1) / p->ws_poses, step = (n + parts - 1) / parts;
+        for (int b = 0; b < n; b += step) {
+            const int m = std::min(step, n - b);
+            lc2e::FusedArgs s = a;
+            s.mats = a.mats + (size_t)b * a.mats_per_pose * 12;
+            s.partials = a.partials + (size_t)b * a.blocks_per_pose * 2;
+            hipError_t err = lc2e::launch_warp_grad3(s, m, st);
+            if (err == hipSuccess) err = lc2e::launch_moments3(s, m, st);
+            if (err != hipSuccess) return err;
+        }
+        return hipSuccess;
+    }
     if (p->sep)
         return lc2e::launch_sep(a, p->info.grid_ndim, p->info.src_ndim, p->info.high_res_is_moving, n,
                                 st);
@@ -201,9 +219,11 @@ int resident_per_cu(lc2e_pair* p) {
     if (p->resident_per_cu <= 0) {
         const lc2e::FusedArgs a = make_args(p, nullptr, nullptr, Tiling{});
         int per_cu = 0;
-        if (lc2e::fused_resident_per_cu(a, p->info.grid_ndim, p->info.src_ndim,
-                                        p->info.high_res_is_moving, &per_cu) != hipSuccess ||
-            per_cu <= 0)
+        const hipError_t err =
+            p->ws ? lc2e::moments_resident_per_cu(a, &per_cu)
+                  : lc2e::fused_resident_per_cu(a, p->info.grid_ndim, p->info.src_ndim,
+                                                p->info.high_res_is_moving, &per_cu);
+        if (err != hipSuccess || per_cu <= 0)
             per_cu = 1;
         p->resident_per_cu = per_cu;
     }
@@ -231,7 +251,8 @@ int model_zchunk(lc2e_pair* p, int n) {
     const int cus = p->e->cus > 0 ? p->e->cus : 256;
     const int per_xcd = std::max(1, cus / lc2e::kXcds * resident_per_cu(p));
     const int cmax = round_zchunk(ez);
-    constexpr double kOverhead = 2.0;  // per work-group, in plane steps (fitted)
+    // per work-group, in plane steps (fitted): the two-kernel path only fills its pipeline
+    const double extra = p->ws ? 8.0 : 2 * r + 2 + 2.0;
     int best = cmax;
     double best_cost = -1.0;
     std::vector<double> heap;
@@ -242,13 +263,13 @@ int model_zchunk(lc2e_pair* p, int n) {
         const long long rounds = (tiles8 / lc2e::kXcds * n + per_xcd - 1) / per_xcd;
         double cost = 0.0;
         if (rounds > 32) {
-            cost = (double)rounds * (c + 2 * r + 2 + kOverhead);
+            cost = (double)rounds * (c + extra);
         } else {
             for (int x = 0; x < lc2e::kXcds; ++x) {
                 heap.assign(per_xcd, 0.0);  // a min-heap of slot finishing times
                 for (long long t = x; t < tiles8; t += lc2e::kXcds) {
                     const double len = t >= tiles ? 0.5
-                        : (double)std::min<long long>(c, ez - (t / cols) * c) + 2 * r + 2 + kOverhead;
+                        : (double)std::min<long long>(c, ez - (t / cols) * c) + extra;
                     for (int k = 0; k < n; ++k) {
                         std::pop_heap(heap.begin(), heap.end(), std::greater<double>());
                         heap.back() += len;
@@ -279,7 +300,7 @@ Tiling tiling_for(lc2e_pair* p, int n) {
         t.zchunk = round_zchunk(p->zchunk_forced > 0 ? p->zchunk_forced
                                 : it != p->tuned.end() ? it->second : model_zchunk(p, n));
         t.tiles = lc2e::fused_blocks_3d(p->v, r, t.zchunk, &t.ntx, &t.nty, &t.nzc);
-        t.bpp = lc2e::fused_partials_3d(p->v, r);
+        t.bpp = p->ws ? lc2e::moments_partials_3d(p->v, r) : lc2e::fused_partials_3d(p->v, r);
         p->last_zchunk = t.zchunk;
     } else {
         // one work-group and one partial per tile and run of kFrameRun frames (fixed, so
@@ -321,9 +342,34 @@ void free_mi(lc2e_pair* p) {
     p->mi_bins = 0;
 }
 
+// The two-kernel path's workspace for n poses, up to kWorkspaceBytes (at least one pose).
+// Only an engine without an HBM budget keeps one: under a budget the fused kernel, which
+// needs none, evaluates the same values, so what a budget admits does not depend on it.
+// Returns false if there is none (nothing is lost: the fused kernel runs).
+constexpr size_t kWorkspaceBytes = size_t(1) << 30;
+bool grow_workspace(lc2e_pair* p, int n) {
+    const size_t per = (p->vbytes / sizeof(float)) * sizeof(float2);
+    const int want = (int)std::min<size_t>((size_t)std::max(n, 1), std::max<size_t>(1, kWorkspaceBytes / per));
+    if (want <= p->ws_poses) return true;
+    void* d = nullptr;
+    if (hipSetDevice(p->e->device) != hipSuccess || hipMalloc(&d, (size_t)want * per) != hipSuccess) {
+        (void)hipGetLastError();
+        return p->ws != nullptr;
+    }
+    if (p->ws) {
+        drop_graphs(p);
+        (void)hipFree(p->ws);  // waits for launches that use it
+    }
+    p->ws = static_cast<float2*>(d);
+    p->ws_poses = want;
+    p->model_cache.clear();
+    return true;
+}
+
 // Batch buffers for n poses whose launches use up to bpp work-groups per pose.
 int ensure_capacity(lc2e_pair* p, int n, int bpp) {
     if (bpp < 1) bpp = 1;
+    if (p->ws) (void)grow_workspace(p, n);
     if (n <= p->cap && bpp <= p->part_bpp) return LC2E_OK;
     int cap = p->cap > 1 ? p->cap : 1;
     while (cap < n) cap *= 2;
@@ -390,6 +436,7 @@ lc2e::FusedArgs make_args(lc2e_pair* p, const float* d_mats, double* d_partials,
     a.blocks_per_pose = t.bpp;
     a.tiles = t.tiles;
     a.mats_per_pose = p->mats_per_pose();
+    a.warp2 = p->ws;
     if (p->sep) {
         const size_t V = p->vbytes / sizeof(float);
         a.sep_img = p->sep_grids;
@@ -729,6 +776,7 @@ int lc2e_pair_create(lc2e_engine* e, lc2e_volume* fixed, lc2e_volume* moving,
         }
         err = lc2e::launch_sobel(p->stat_img, p->v, dim, p->stat_grad, e->stream);
     }
+    if (err == hipSuccess && dim == 3 && high_res_is_moving && !sep && !e->budget) (void)grow_workspace(p, 1);
     if (err == hipSuccess) err = hipStreamSynchronize(e->stream);
     if (err != hipSuccess) {
         lc2e_pair_destroy(p);
@@ -751,6 +799,7 @@ void lc2e_pair_destroy(lc2e_pair* p) {
     if (p->ustat) p->e->release(p->ustat, 2 * (p->vbytes / sizeof(float)) * sizeof(double));
     if (p->sep_grids) p->e->release(p->sep_grids, p->sep_grid_bytes);
     if (p->sep_sums) p->e->release(p->sep_sums, p->sep_sum_bytes);
+    if (p->ws) (void)hipFree(p->ws);
     delete p;
 }
 
@@ -1050,10 +1099,9 @@ int lc2e_pair_autotune(lc2e_pair* p, int n, const float* mats, int iters, int* b
         HIP_TRY(hipMemcpy(p->d_mats, mats, (size_t)n * p->mats_per_pose() * 12 * sizeof(float),
                           hipMemcpyHostToDevice));
         lc2e::FusedArgs a = make_args(p, p->d_mats, p->d_partials, t);
-        HIP_TRY(lc2e::launch_fused(a, 3, p->info.src_ndim, p->info.high_res_is_moving, n, st));
+        HIP_TRY(launch_eval(p, a, n, st));
         HIP_TRY(hipEventRecord(e0, st));
-        for (int it = 0; it < iters; ++it)
-            HIP_TRY(lc2e::launch_fused(a, 3, p->info.src_ndim, p->info.high_res_is_moving, n, st));
+        for (int it = 0; it < iters; ++it) HIP_TRY(launch_eval(p, a, n, st));
         HIP_TRY(hipEventRecord(e1, st));
         HIP_TRY(hipEventSynchronize(e1));
         float ms = 0.0f;

@@ -81,6 +81,7 @@ struct FusedArgs {
     float* sep_grad;
     double* sep_a;
     double* sep_b;
+    float2* warp2;  // two-kernel path: (I, |Sobel I|) of the moving image per pose and voxel
 };
 
 // Number of work-groups one pose needs (0 if the grid has no valid patch centre).
@@ -101,6 +102,13 @@ int pose_run(const VGeom& v, int grid_ndim, int src_ndim, int mats_per_pose, int
 // CU at once (hipOccupancyMaxActiveBlocksPerMultiprocessor).
 hipError_t fused_resident_per_cu(const FusedArgs& a, int grid_ndim, int src_ndim, int movi,
                                  int* per_cu);
+// Two-kernel 3D path (moving high-resolution image, r <= kMaxR3): k_warp_grad3 writes the
+// warped image and its |Sobel| into FusedArgs::warp2 (n poses), k_moments3d forms the patch
+// sums and the partials from it, bit for bit as the fused kernel.
+hipError_t launch_warp_grad3(const FusedArgs& a, int n_poses, hipStream_t st);
+hipError_t launch_moments3(const FusedArgs& a, int n_poses, hipStream_t st);
+int moments_partials_3d(const VGeom& v, int r);  // partial sums per pose
+hipError_t moments_resident_per_cu(const FusedArgs& a, int* per_cu);
 hipError_t launch_reduce(const double* partials, int blocks_per_pose, int n_poses, double* out,
                          hipStream_t st);
 // Separable path for radii beyond the fused kernels (3D r > kMaxR3, 2D r > kMaxR2): per

@@ -1,0 +1,453 @@
+// 3D LC2 with the moving image as the high-resolution one, in two kernels: k_warp_grad3 writes
+// the warped image and its |Sobel| for every voxel of the grid and pose (8 bytes), and
+// k_moments3d forms the patch moments from those grids and combines them.
+//
+// The fused kernel (k_fused3d) computes both per 16x16 tile, so it warps 2.25 and takes the
+// Sobel of 1.89 positions per output voxel, and its 238 VGPRs hold two waves per SIMD. Apart,
+// the first kernel's tile has 1.2 warped positions per voxel, and the second needs 84 VGPRs.
+// The grids cost 8 bytes written and about 10 read per voxel and pose, at 1 TB/s far from the
+// memory's rate. 192x192x160 grid, 7^3 patch, 32 poses: 3.40 -> 2.80 ms.
+#include <mutex>
+
+#include "lc2e_device.hpp"
+
+namespace lc2e {
+
+namespace {
+
+constexpr int kGradX = 32, kGradY = 16;  // output tile of k_warp_grad3
+
+// The moving high-resolution image I and its |Sobel| G at every grid voxel of a pose, as
+// float2, bit for bit as k_fused3d forms them. A work-group marches along z over a 32x16
+// column; the gathers of the next plane are in flight during the Sobel of this one, and the
+// two LDS planes take one barrier per step. Bound by VALU issue (102 instructions per voxel,
+// 73% of the issue slots): 365 us for 16 poses of 192x192x160, 2 TB/s written.
+template <typename T, bool P2>
+__global__ __launch_bounds__(256) void k_warp_grad3(FusedArgs a, int ntx, int nty, int zc, int tiles,
+                                                    int npose) {
+    constexpr int IXE = kGradX + 2, IYE = kGradY + 2, NI = IXE * IYE;
+    constexpr int SPT = (NI + 255) / 256;
+    __shared__ float s_in[2][NI];
+    int tile, pose;
+    if (!map_block(tiles, npose, tile, pose)) return;
+    const int tid = threadIdx.x;
+    const int tcol = tile % (ntx * nty), zci = tile / (ntx * nty);
+    const int x0 = (tcol % ntx) * kGradX, y0 = (tcol / ntx) * kGradY;
+    const int X = a.v.X, Y = a.v.Y, Z = a.v.Z;
+    const int z0 = zci * zc, z1 = min(z0 + zc, Z);
+    const T* __restrict__ src = static_cast<const T*>(a.src);
+    float m[12];
+    {
+        const float* mp = a.mats + (size_t)pose * 12;
+#pragma unroll
+        for (int k = 0; k < 12; ++k) m[k] = mp[k];
+    }
+    const int wbase = __builtin_amdgcn_readfirstlane(tid & ~63);
+    float cxy[SPT][3];
+    unsigned in_xy = 0;
+#pragma unroll
+    for (int j = 0; j < SPT; ++j) {
+        const int i = tid + j * 256;
+        const int lx = i % IXE, ly = i / IXE;
+        const int gx = x0 - 1 + lx, gy = y0 - 1 + ly;
+        if (i < NI && gx >= 0 && gx < X && gy >= 0 && gy < Y) in_xy |= 1u << j;
+        const float Lx = fmaf((float)gx, a.v.sx, a.v.ox), Ly = fmaf((float)gy, a.v.sy, a.v.oy);
+        cxy[j][0] = fmaf(m[1], Ly, m[0] * Lx);
+        cxy[j][1] = fmaf(m[5], Ly, m[4] * Lx);
+        cxy[j][2] = fmaf(m[9], Ly, m[8] * Lx);
+    }
+    Pending3<T> pend[SPT];
+    auto has = [&](int j) { return (j + 1) * 256 <= NI || j * 256 + wbase < NI; };
+    auto issue = [&](int z) {
+        const bool zin = z >= 0 && z < Z;
+        const float lz = fmaf((float)z, a.v.sz, a.v.oz);
+#pragma unroll
+        for (int j = 0; j < SPT; ++j)
+            if (has(j)) issue3c<P2>(src, a.s, m, cxy[j], lz, zin && ((in_xy >> j) & 1u), pend[j]);
+    };
+    auto finish = [&](float* dst) {
+#pragma unroll
+        for (int j = 0; j < SPT; ++j) {
+            if (!has(j)) continue;
+            const int i = tid + j * 256;
+            const float v = finish3(pend[j]);
+            if (i < NI) dst[i] = v;
+        }
+    };
+    const int lx = tid % kGradX, ly = 2 * (tid / kGradX);
+    const int gx = x0 + lx, gy = y0 + ly;
+    const bool ok0 = gx < X && gy < Y, ok1 = gx < X && gy + 1 < Y;
+    float2* __restrict__ out = a.warp2 + (size_t)pose * X * Y * Z;
+    const unsigned o0 = (unsigned)(gy * X + gx);
+    float tA[2][3], tBx[2][3], tBy[2][3], Ip[2], Ic[2];
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+#pragma unroll
+        for (int k = 0; k < 3; ++k) tA[e][k] = tBx[e][k] = tBy[e][k] = 0.f;
+        Ip[e] = Ic[e] = 0.f;
+    }
+    issue(z0 - 1);
+    int buf = 0;
+    for (int z = z0 - 1; z <= z1; ++z, buf ^= 1) {
+        finish(s_in[buf]);
+        __syncthreads();
+        if (z < z1) issue(z + 1);
+        const float* row = s_in[buf] + ly * IXE + lx;
+        float sm[4], df[4], cm[4];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const float l = row[r * IXE], c = row[r * IXE + 1], rr = row[r * IXE + 2];
+            sm[r] = fmaf(2.0f, c, l) + rr;  // (l + 2c) + r: 2c is exact
+            df[r] = rr - l;
+            cm[r] = c;
+        }
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+            tA[e][0] = tA[e][1]; tA[e][1] = tA[e][2];
+            tBx[e][0] = tBx[e][1]; tBx[e][1] = tBx[e][2];
+            tBy[e][0] = tBy[e][1]; tBy[e][1] = tBy[e][2];
+            tA[e][2] = fmaf(2.0f, sm[e + 1], sm[e]) + sm[e + 2];
+            tBx[e][2] = fmaf(2.0f, df[e + 1], df[e]) + df[e + 2];
+            tBy[e][2] = sm[e + 2] - sm[e];
+            Ip[e] = Ic[e];
+            Ic[e] = cm[e + 1];
+        }
+        if (z > z0) {
+            float2* o = out + (size_t)(z - 1) * X * Y;
+#pragma unroll
+            for (int e = 0; e < 2; ++e) {
+                const float gxv = fmaf(2.0f, tBx[e][1], tBx[e][0]) + tBx[e][2];
+                const float gyv = fmaf(2.0f, tBy[e][1], tBy[e][0]) + tBy[e][2];
+                const float gzv = tA[e][2] - tA[e][0];
+                const float G = sqrtf(fmaf(gzv, gzv, fmaf(gyv, gyv, gxv * gxv)));
+                if (e ? ok1 : ok0) o[o0 + (e ? X : 0)] = make_float2(Ip[e], G);
+            }
+        }
+    }
+}
+
+// A uniform base plus a 32-bit byte offset per lane (one saddr + voffset access). The empty
+// asm keeps the sum out of the loop optimiser's sight: it would carry a 64-bit pointer per
+// lane for every unrolled step (46 spilled VGPRs at R = 3).
+__device__ __forceinline__ const char* at_bytes(const void* base, unsigned ofs) {
+    asm volatile("" : "+v"(ofs));
+    return static_cast<const char*>(base) + ofs;
+}
+
+// ---------------------------------------------------------------------------
+// Patch moments and combine on the grids: a 16x16 column of output voxels over `zchunk`
+// planes of one pose, one work-group per CU, its waves in three roles that work on three LDS
+// buffers at once, with one barrier per step:
+//   z waves: z window sums of the 7 products channels of step s, two planes at a time (they
+//     share W - 1 planes; the ring of input planes is 3 floats per plane, where a ring of
+//     plane sums would be 14 VGPRs per plane), written to buffer s;
+//   x waves: x window sums of step s - 1 in place, a row of 16 outputs per lane;
+//   y waves: y window sums of two pixels per lane of step s - 2, and their combine.
+// The LDS and the VALU are both about two thirds busy at R = 3. LDS writes are what costs:
+// per wave a ds_write_b64 takes 6.2 cycles, a ds_write_b128 13, a ds_read_b64 2.2, a
+// ds_read_b128 4.1, but a ds_read2_b64 of two rows 8.0 (measured), so the y sums stay in
+// registers up to the combine (no second write) and are read row by row.
+// Measured at 192x192x160, R = 3, 16 poses: 1.03 ms; with every phase on all waves and a
+// barrier between phases 1.13 ms (512 threads, 80 VGPRs), with the z sums last in a VGPR ring
+// 1.13 ms (256 threads, 158 VGPRs); one plane per step, two work-groups per CU: 1.62 ms.
+// Raised priorities for the x or the y waves: 1 to 8% slower.
+// ---------------------------------------------------------------------------
+// Planes a pipeline step carries: two where three buffers of them fit the LDS.
+template <int R, int NC>
+struct Mom {
+    static constexpr int W = 2 * R + 1, PX = kTile3X + 2 * R, PY = kTile3Y + 2 * R, NP = PX * PY;
+    static constexpr int PS = lds_stride(PX), PL = PY * PS;  // LDS row stride, plane size
+    static constexpr int KP = 3 * 2 * NC * PL * 8 <= 160 * 1024 ? 2 : 1;
+    static constexpr int BUF = KP * NC * PL;                 // doubles per buffer
+    // waves per role; a z wave takes ZP positions per lane
+    static constexpr int ZP = 2;
+    static constexpr int ZW = (NP + ZP * 64 - 1) / (ZP * 64), YW = 2 * KP, XW = (KP * NC * PY + 63) / 64;
+    static constexpr int NW = ZW + YW + XW, NTHR = NW * 64;
+    static constexpr size_t lds = 3 * BUF * sizeof(double);
+    static_assert(NW <= 16 && lds <= 160 * 1024, "roles and buffers fit a CU");
+};
+
+// Two window sums of width W of in[0 .. W].
+template <int W>
+__device__ __forceinline__ void window2(const double (&in)[W + 1], double& o0, double& o1) {
+    double mid = in[1];
+#pragma unroll
+    for (int j = 2; j < W; ++j) mid += in[j];
+    o0 = in[0] + mid;
+    o1 = mid + in[W];
+}
+
+template <int R>
+__global__ __launch_bounds__((Mom<R, 7>::NTHR)) void k_moments3d(FusedArgs a) {
+    constexpr int NC = 7;
+    using M = Mom<R, NC>;
+    constexpr int TX = kTile3X, TY = kTile3Y, W = M::W, PX = M::PX, PY = M::PY, NP = M::NP, PS = M::PS,
+                  PL = M::PL, KP = M::KP, BUF = M::BUF, N3 = W * W * W;
+    extern __shared__ __align__(16) double s_buf[];
+
+    int tile, pose;
+    if (!map_block(a.tiles, a.npose, tile, pose)) return;  // whole work-group
+    const int rank = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    const int cols = a.ntx * a.nty;
+    const int tcol = tile % cols, zc = tile / cols;
+    const int x0 = R + (tcol % a.ntx) * TX, y0 = R + (tcol / a.ntx) * TY;
+    const int z0 = R + zc * a.zchunk;
+    const int zend = min(z0 + a.zchunk, a.v.Z - R);
+    const int X = a.v.X, Y = a.v.Y, Z = a.v.Z, XY = X * Y;
+    const int nout = zend - z0;
+    const int n = (nout + KP - 1) / KP;  // steps with products
+
+    if (rank >= M::YW && rank < M::YW + M::ZW) {
+        // z window sums of ZP positions per lane, two planes at a time
+        constexpr int ZP = M::ZP, K = W + 1;
+        const int i0 = (rank - M::YW) * 64 + lane;
+        int d_ofs[ZP];
+        unsigned g_ofs[ZP];  // bytes of one float per voxel
+#pragma unroll
+        for (int e = 0; e < ZP; ++e) {
+            const int i = min(i0 + e * M::ZW * 64, NP - 1);
+            const int lx = i % PX, ly = i / PX;
+            d_ofs[e] = ly * PS + lx;
+            g_ofs[e] = (unsigned)(min(y0 - R + ly, Y - 1) * X + min(x0 - R + lx, X - 1)) * 4u;
+        }
+        const float2* __restrict__ ig = a.warp2 + (size_t)pose * Z * XY;
+        float2 vi[K][ZP];
+        float vu[K][ZP];
+        auto load = [&](auto slot_c, int z) {
+            constexpr int k = decltype(slot_c)::value;
+            const size_t zo = (size_t)min(z, Z - 1) * XY;
+#pragma unroll
+            for (int e = 0; e < ZP; ++e) {
+                __builtin_memcpy(&vi[k][e], at_bytes(ig + zo, g_ofs[e] * 2u), 8);
+                __builtin_memcpy(&vu[k][e], at_bytes(a.stat_img + zo, g_ofs[e]), 4);
+            }
+        };
+        Unroll<0, K>::run([&](auto kc) { load(kc, z0 - R + decltype(kc)::value); });
+        int buf = 0;
+        for (int p0 = 0; p0 < nout; p0 += 2 * (R + 1)) {
+            Unroll<0, R + 1>::run([&](auto kc) {
+                constexpr int k = decltype(kc)::value;
+                const int p = p0 + 2 * k;
+                if (p >= nout) return;  // block-uniform
+                double s[ZP][NC];
+#pragma unroll
+                for (int e = 0; e < ZP; ++e) {
+                    auto add = [&](double (&t)[NC], int j) {
+                        const double I = vi[(2 * k + j) % K][e].x, G = vi[(2 * k + j) % K][e].y,
+                                     U = vu[(2 * k + j) % K][e];
+                        t[0] += I;
+                        t[1] += G;
+                        t[2] = fma(I, I, t[2]);  // products of two floats are exact in FP64
+                        t[3] = fma(G, G, t[3]);
+                        t[4] = fma(I, G, t[4]);
+                        t[5] = fma(U, I, t[5]);
+                        t[6] = fma(U, G, t[6]);
+                    };
+                    // the ring stays in floats: without this the compiler keeps each plane's
+                    // FP64 values from step to step as well, and spills
+#pragma unroll
+                    for (int j = 0; j < K; ++j) asm volatile("" : "+v"(vi[j][e].x), "+v"(vi[j][e].y), "+v"(vu[j][e]));
+                    {
+                        const double I = vi[(2 * k + 1) % K][e].x, G = vi[(2 * k + 1) % K][e].y,
+                                     U = vu[(2 * k + 1) % K][e];
+                        s[e][0] = I; s[e][1] = G; s[e][2] = I * I; s[e][3] = G * G; s[e][4] = I * G;
+                        s[e][5] = U * I; s[e][6] = U * G;
+                    }
+#pragma unroll
+                    for (int j = 2; j < W; ++j) add(s[e], j);
+                    double t[NC];
+#pragma unroll
+                    for (int c = 0; c < NC; ++c) t[c] = s[e][c];
+                    add(t, 0);
+                    add(s[e], W);
+                    // the positions past the region repeat the last one, with its values
+                    double* d = s_buf + buf * BUF + d_ofs[e];
+#pragma unroll
+                    for (int c = 0; c < NC; ++c) d[c * PL] = t[c];
+                    if (KP == 2)
+#pragma unroll
+                        for (int c = 0; c < NC; ++c) d[(NC + c) * PL] = s[e][c];
+                }
+                // the two oldest planes make room for the next two
+                load(std::integral_constant<int, (2 * k) % K>{}, z0 - R + p + W + 1);
+                load(std::integral_constant<int, (2 * k + 1) % K>{}, z0 - R + p + W + 2);
+                __syncthreads();
+                buf = buf == 2 ? 0 : buf + 1;
+                if (KP == 1 && p + 1 < nout) {
+#pragma unroll
+                    for (int e = 0; e < ZP; ++e)
+#pragma unroll
+                        for (int c = 0; c < NC; ++c) s_buf[buf * BUF + d_ofs[e] + c * PL] = s[e][c];
+                    __syncthreads();
+                    buf = buf == 2 ? 0 : buf + 1;
+                }
+            });
+        }
+        __syncthreads();
+        return;
+    }
+    if (rank >= M::YW + M::ZW) {
+        // x window sums in place
+        const int t0 = (rank - M::YW - M::ZW) * 64 + lane;
+        __syncthreads();
+        int buf = 0;
+        for (int s = 0; s < n; ++s) {
+            for (int t = t0; t < KP * NC * PY; t += M::XW * 64) {  // one round
+                double* r = s_buf + buf * BUF + (t / PY) * PL + (t % PY) * PS;
+                r = static_cast<double*>(__builtin_assume_aligned(r, 16));
+                window_run<W>(r, 1, r, 1);
+            }
+            buf = buf == 2 ? 0 : buf + 1;
+            __syncthreads();
+        }
+        return;
+    }
+    // y window sums of two pixels of a column and their combine. Lanes 16 apart take rows 8
+    // apart: their LDS reads then fall into distinct halves of the banks.
+    const int plane = rank >> 1;
+    const int ox = lane % TX, oy = 8 * (lane / TX & 1) + 2 * (lane / (2 * TX)) + 4 * (rank & 1);
+    const bool ok0 = x0 + ox < X - R && y0 + oy < Y - R, ok1 = ok0 && y0 + oy + 1 < Y - R;
+    const unsigned vo0 = ok0 ? (unsigned)((y0 + oy) * X + (x0 + ox)) * 8u : 0u;
+    const unsigned vo1 = ok1 ? vo0 + (unsigned)X * 8u : 0u;
+    double mu[2], cyy[2];
+    auto stats = [&](int zo) {
+        const size_t zp = (size_t)min(zo, zend - 1) * XY;
+        __builtin_memcpy(&mu[0], at_bytes(a.ustat_mean + zp, vo0), 8);
+        __builtin_memcpy(&cyy[0], at_bytes(a.ustat_cyy + zp, vo0), 8);
+        __builtin_memcpy(&mu[1], at_bytes(a.ustat_mean + zp, vo1), 8);
+        __builtin_memcpy(&cyy[1], at_bytes(a.ustat_cyy + zp, vo1), 8);
+    };
+    double acc_m = 0.0, acc_w = 0.0;
+    __syncthreads();
+    stats(z0 + plane);
+    __syncthreads();
+    int buf = 0;
+    for (int s = 0; s < n; ++s) {
+        const int zo = z0 + s * KP + plane;
+        const bool zok = zo < zend;
+        // one address per row, of unknown relation to the others: the compiler would pair two
+        // rows in a ds_read2_b64, which takes 8 cycles where two ds_read_b64 take 4.4 (measured)
+        const double* row[W + 1];
+#pragma unroll
+        for (int j = 0; j < W + 1; ++j) {
+            unsigned ofs = (unsigned)(buf * BUF + plane * NC * PL + (oy + j) * PS + ox);
+            asm volatile("" : "+v"(ofs));
+            row[j] = s_buf + ofs;
+        }
+        double S[2][NC];
+#pragma unroll
+        for (int c = 0; c < NC; ++c) {
+            double in[W + 1];
+#pragma unroll
+            for (int j = 0; j < W + 1; ++j) in[j] = row[j][c * PL];
+            window2<W>(in, S[0][c], S[1][c]);
+            // at most two channels in flight: all reads first would take 112 VGPRs
+            asm volatile("" : "+v"(S[0][c]), "+v"(S[1][c]));
+            if (c % 2 == 1) __builtin_amdgcn_sched_barrier(0);
+        }
+        const double m0[2] = {mu[0], mu[1]}, c0[2] = {ok0 && zok ? cyy[0] : -1.0, ok1 && zok ? cyy[1] : -1.0};
+        stats(zo + KP);
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+            double w, meas;
+            const bool ok = c0[j] >= 0.0;
+            combine_static_u_any(S[j], m0[j], ok ? c0[j] : 1.0, N3, w, meas);
+            acc_m += ok ? meas : 0.0;
+            acc_w += ok ? w : 0.0;
+            if (a.wmap && ok) {
+                const size_t vo = (size_t)zo * XY + (size_t)(y0 + oy + j) * X + (x0 + ox);
+                a.wmap[vo] = w;
+                a.mmap[vo] = meas;
+            }
+        }
+        // partials per block of kZBlock output planes, tile column and combining wave, at
+        // fixed positions in z
+        const int ze = z0 + (s + 1) * KP;
+        if ((ze - R) % kZBlock == 0 || ze >= zend) {
+            wave_reduce_store(acc_m, acc_w,
+                              a.partials + (((size_t)pose * a.blocks_per_pose +
+                                             ((size_t)((ze - 1 - R) / kZBlock) * cols + tcol) * M::YW + rank) * 2));
+            acc_m = 0.0;
+            acc_w = 0.0;
+        }
+        buf = buf == 2 ? 0 : buf + 1;
+        if (s + 1 < n) __syncthreads();
+    }
+}
+
+template <typename T, bool P2>
+void warp_grad3(const FusedArgs& a, int ntx, int nty, int zc, int tiles, int n, hipStream_t st) {
+    const int tiles8 = (tiles + kXcds - 1) / kXcds * kXcds;
+    hipLaunchKernelGGL((k_warp_grad3<T, P2>), dim3((unsigned)tiles8 * n), dim3(256), 0, st, a, ntx, nty,
+                       zc, tiles, n);
+}
+
+template <int R>
+hipError_t moments3(const FusedArgs& a, dim3 grid, hipStream_t st, int* occ) {
+    using M = Mom<R, 7>;
+    static std::once_flag once;
+    static hipError_t err = hipSuccess;
+    std::call_once(once, [] {
+        err = hipFuncSetAttribute(reinterpret_cast<const void*>(&k_moments3d<R>),
+                                  hipFuncAttributeMaxDynamicSharedMemorySize, (int)M::lds);
+    });
+    if (err != hipSuccess) return err;
+    if (occ) return hipOccupancyMaxActiveBlocksPerMultiprocessor(occ, k_moments3d<R>, M::NTHR, M::lds);
+    hipLaunchKernelGGL((k_moments3d<R>), grid, dim3(M::NTHR), M::lds, st, a);
+    return hipGetLastError();
+}
+
+hipError_t moments3r(const FusedArgs& a, dim3 grid, hipStream_t st, int* occ) {
+    switch (a.r) {
+        case 1: return moments3<1>(a, grid, st, occ);
+        case 2: return moments3<2>(a, grid, st, occ);
+        case 3: return moments3<3>(a, grid, st, occ);
+        case 4: return moments3<4>(a, grid, st, occ);
+        case 5: return moments3<5>(a, grid, st, occ);
+        case 6: return moments3<6>(a, grid, st, occ);
+        default: return hipErrorInvalidValue;
+    }
+}
+
+}  // namespace
+
+hipError_t launch_warp_grad3(const FusedArgs& a, int n, hipStream_t st) {
+    const int ntx = (a.v.X + kGradX - 1) / kGradX, nty = (a.v.Y + kGradY - 1) / kGradY;
+    // z-chunks: about 2048 work-groups (the CUs hold about that many), at least 8 planes each
+    // (two more are warped per chunk)
+    const int want = (int)std::max(1LL, 2048LL / ((long long)ntx * nty * n));
+    const int zc = std::max(8, (a.v.Z + want - 1) / want);
+    const int tiles = ntx * nty * ((a.v.Z + zc - 1) / zc);
+    if (a.s.pow2) {
+        if (a.src_f16) warp_grad3<__half, true>(a, ntx, nty, zc, tiles, n, st);
+        else warp_grad3<float, true>(a, ntx, nty, zc, tiles, n, st);
+    } else {
+        if (a.src_f16) warp_grad3<__half, false>(a, ntx, nty, zc, tiles, n, st);
+        else warp_grad3<float, false>(a, ntx, nty, zc, tiles, n, st);
+    }
+    return hipGetLastError();
+}
+
+int moments_partials_3d(const VGeom& v, int r) {
+    int ntx, nty, nzc;
+    if (fused_blocks_3d(v, r, kZBlock, &ntx, &nty, &nzc) <= 0) return 0;
+    const int yw = r == 1 ? Mom<1, 7>::YW : r == 2 ? Mom<2, 7>::YW : r == 3 ? Mom<3, 7>::YW : 2;
+    return ntx * nty * nzc * yw;
+}
+
+hipError_t launch_moments3(const FusedArgs& a, int n, hipStream_t st) {
+    if (a.tiles == 0 || n <= 0) return hipSuccess;
+    if (a.zchunk <= 0 || a.zchunk % kZBlock != 0) return hipErrorInvalidValue;
+    FusedArgs b = a;
+    b.npose = n;
+    const long long tiles8 = (a.tiles + kXcds - 1) / kXcds * (long long)kXcds;
+    if (tiles8 * n > 0x7fffffffLL) return hipErrorInvalidValue;
+    return moments3r(b, dim3((unsigned)(tiles8 * n)), st, nullptr);
+}
+
+hipError_t moments_resident_per_cu(const FusedArgs& a, int* per_cu) {
+    *per_cu = 0;
+    return moments3r(a, dim3(1), nullptr, per_cu);
+}
+
+}  // namespace lc2e

@@ -572,3 +572,36 @@ def test_sweep_with_partial_last_frame_run(engine):
     p.close()
     fv.close()
     mv.close()
+
+
+@pytest.mark.parametrize("r,dims", [(1, (18, 19, 5)), (2, (36, 20, 13)), (3, (39, 23, 18)),
+                                    (4, (25, 41, 9)), (4, (24, 24, 26))])
+def test_3d_two_kernel_path_equals_fused_and_oracle(engine, r, dims):
+    """An engine without a budget evaluates the moving high-resolution role with the warped
+    image in a workspace (two kernels), one with a budget with the fused kernel. At grids of
+    one and several tiles, partial tiles, an odd number of output planes and a single one:
+    both match the oracle, and each other to rounding."""
+    w = synth.config1(seed=3, mr_dims=(48, 44, 40), us_dims=dims, us_spacing=0.75, patch_radius=r)
+    budgeted = E.Engine(0, hbm_budget=1 << 30)
+    print(f"two-kernel path: r {r}, grid {dims}", flush=True)
+    rng = np.random.default_rng(r)
+    poses = [w.true_pose] + [synth.perturb(w.true_pose, rng, 3) for _ in range(4)]
+    got = []
+    for e in (engine, budgeted):
+        p = _pair_for(e, w)
+        mats = np.stack([p.pose_to_matrix(q) for q in poses])
+        b = p.eval_batch(mats)
+        for k in range(len(poses)):
+            assert p.eval(mats[k]) == b.lc2[k]
+        p.set_tuning(8)
+        assert np.array_equal(p.eval_batch(mats).lc2, b.lc2)
+        got.append(b)
+        p.close()
+    for k in (0, len(poses) - 1):
+        res, *_ = _oracle_eval(w, mats[k])
+        assert res.n_valid > 0
+        for b in got:
+            assert abs(b.lc2[k] - res.lc2) < LC2_TOL
+    assert np.allclose(got[0].lc2, got[1].lc2, rtol=1e-10, atol=0)
+    assert np.allclose(got[0].sum_w, got[1].sum_w, rtol=1e-10, atol=0)
+    budgeted.close()
