@@ -82,10 +82,12 @@ const char* lc2e_last_error(void);
 int lc2e_create(int device, size_t hbm_budget_bytes, lc2e_engine** out);
 void lc2e_destroy(lc2e_engine* e);
 /* Bytes currently charged to the engine's budget, and the budget. An engine without a budget
- * also keeps, with each 3D pair whose moving image is the high-resolution one (radius up to
- * 4), a workspace of 8 bytes per grid voxel and pose of its largest batch, at most 1 GiB or
- * one pose; it is not counted here. Under a budget such pairs are evaluated without it, by a
- * slower kernel (LC2 agrees to rounding), so what a budget admits does not depend on it. */
+ * also keeps, and does not count here: with a pair, its statistics of a static high-resolution
+ * image (40 bytes per grid voxel) or a workspace for the warped moving image (4 or 8 bytes per
+ * grid voxel and pose of its largest batch, at most 1 GiB or one pose); and up to 1 GiB of
+ * freed blocks for the next allocations of their size, given back with the engine. Under a
+ * budget a pair does without them, so what a budget admits does not depend on them: 2D values
+ * are the same bits, 3D values up to radius 4 come from another kernel and agree to rounding. */
 int lc2e_memory(lc2e_engine* e, size_t* used, size_t* budget);
 
 /* Upload a resident fixed or moving image. Replaces Interpolator*'s thrust copies of the
@@ -107,11 +109,12 @@ void lc2e_volume_destroy(lc2e_volume* v);
  *  dim: LC2 grid dimensionality; 2 with a 3D moving volume is the 2D->3D mode
  *       (Interpolator2DTo3D, interpolator.cu:1538-1786); a fixed image with dims[2] > 1 and
  *       dim 2 is a stack of independent 2D frames.
- *  patch_radius: 1..64. Radii up to 4 (3D) / 10 (2D) run the fused kernels; larger radii run
- *       a separable path (the reference's global-memory kernel for large patches,
+ *  patch_radius: 1..64. Radii up to 6 (3D) / 10 (2D) keep every patch sum on the chip; larger
+ *       radii run a separable path (the reference's global-memory kernel for large patches,
  *       cu_lc2_3d.cu:769-827), whose buffers -- the moving image and its |Sobel| on the grid
  *       and two f64 box-sum buffers of 7 (moving high-resolution image) or 10 channels -- are
- *       allocated here, against the budget. */
+ *       allocated here, against the budget. 3D radii 5 and 6 charge a workspace of one pose (4
+ *       or 8 bytes per voxel) and the image statistics instead, which is less. */
 int lc2e_pair_create(lc2e_engine* e, lc2e_volume* fixed, lc2e_volume* moving,
                      const float resampled_spacing[3], int high_res_is_moving,
                      int center_overlaid, int patch_radius, int dim, lc2e_pair** out);

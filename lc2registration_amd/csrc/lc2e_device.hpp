@@ -522,6 +522,130 @@ __device__ __forceinline__ bool combine_static_u(const double* S, double mu, dou
     return true;
 }
 
+// The part of the fit that a static high-resolution image decides, from its channels I, G, II,
+// GG, IG: patch means and the coefficients of e = A p^2 + B p q + C q^2, the explained part of
+// an ultrasound with the centred products p = C_UI, q = C_UG (explained_var with its rank rule).
+__device__ __forceinline__ void store_image_stats(const double* S, int N, double* out, long long stride) {
+    const double inv_n = 1.0 / (double)N;
+    const double si = S[0], sg = S[1], mi = si * inv_n, mg = sg * inv_n;
+    const double a = fma(-mi, si, S[2]), b = fma(-mg, sg, S[3]), c = fma(-mi, sg, S[4]);
+    const bool ikeep = a > kTauConst * S[2], gkeep = b > kTauConst * S[3];
+    const double ab = a * b, det = fma(-c, c, ab);
+    double A = 0.0, B = 0.0, C = 0.0;
+    if (ikeep && gkeep) {
+        if (det > kTauColl * ab) {
+            const double d = rcp64(det);
+            A = b * d;
+            B = -2.0 * c * d;
+            C = a * d;
+        } else {
+            const double ra = rsq64(a), rb = rsq64(b);
+            const double k = rcp64(2.0 + 2.0 * fabs(c) * ra * rb);
+            A = ra * ra * k;
+            B = (c < 0.0 ? -2.0 : 2.0) * ra * rb * k;
+            C = rb * rb * k;
+        }
+    } else if (ikeep) {
+        A = rcp64(a);
+    } else if (gkeep) {
+        C = rcp64(b);
+    }
+    out[0] = mi;
+    out[stride] = mg;
+    out[2 * stride] = A;
+    out[3 * stride] = B;
+    out[4 * stride] = C;
+}
+
+// Static high-resolution image: channels U, UU, UI, UG (NaN where a pixel of the patch is not
+// above the threshold) and the image's statistics st[k * stride]. false where w = 0.
+struct ImageStats {
+    double mi, mg, A, B, C;
+};
+__device__ __forceinline__ ImageStats load_image_stats(const double* st, long long stride) {
+    return {st[0], st[stride], st[2 * stride], st[3 * stride], st[4 * stride]};
+}
+__device__ __forceinline__ bool combine_static_image(const double* S, const ImageStats& t, int N,
+                                                     double& w_out, double& m_out) {
+    const double inv_n = 1.0 / (double)N, inv_n1 = 1.0 / (double)(N - 1);
+    const double su = S[0], my = su * inv_n;
+    const double cyy = fma(-my, su, S[1]);
+    const bool ok = cyy * inv_n1 > kZeroThreshold;
+    const double p = fma(-t.mi, su, S[2]), q = fma(-t.mg, su, S[3]);
+    const double e = fma(fma(t.B, q, t.A * p), p, (t.C * q) * q);
+    weight_measure(ok ? cyy : 1.0, e, inv_n1, w_out, m_out);
+    return ok;
+}
+
+// Patch statistics of a static ultrasound from its channels U, UU: mean and centred energy, or
+// 0 and -1 where w = 0.
+__device__ __forceinline__ void store_us_stats(const double* S, int N, double* mean, double* cyy) {
+    const double inv_n = 1.0 / (double)N, m = S[0] * inv_n, c = fma(-m, S[0], S[1]);
+    const bool ok = c * (1.0 / (double)(N - 1)) > kZeroThreshold;
+    *mean = ok ? m : 0.0;
+    *cyy = ok ? c : -1.0;
+}
+
+// Channels of a role and the products of one position added to their sums.
+// kRoleMovingImage: I, G, II, GG, IG, UI, UG; kRoleStaticImage: U, UU, UI, UG, followed in
+// kRoleStaticImageFull by I, G, II, GG, IG; kRoleImageStats: those five; kRoleUsStats: U, UU.
+template <int ROLE>
+struct Role {
+    static constexpr int NC = ROLE == kRoleMovingImage ? 7 : ROLE == kRoleStaticImage ? 4
+                            : ROLE == kRoleStaticImageFull ? 9 : ROLE == kRoleImageStats ? 5 : 2;
+    static constexpr bool HAS_I = ROLE != kRoleUsStats, HAS_U = ROLE != kRoleImageStats;
+    static constexpr bool SUMS = ROLE == kRoleMovingImage || ROLE == kRoleStaticImage || ROLE == kRoleStaticImageFull;
+    __device__ __forceinline__ static void add(double (&t)[NC], double I, double G, double U) {
+        constexpr bool STAT = ROLE == kRoleStaticImage || ROLE == kRoleStaticImageFull;
+        constexpr int c = ROLE == kRoleStaticImageFull ? 4 : 0;
+        if constexpr (STAT || ROLE == kRoleUsStats) {
+            t[0] += U;
+            t[1] = fma(U, U, t[1]);  // products of two floats are exact in FP64
+            if constexpr (STAT) {
+                t[2] = fma(U, I, t[2]);
+                t[3] = fma(U, G, t[3]);
+            }
+        }
+        if constexpr (HAS_I && ROLE != kRoleStaticImage) {
+            t[c] += I;
+            t[c + 1] += G;
+            t[c + 2] = fma(I, I, t[c + 2]);
+            t[c + 3] = fma(G, G, t[c + 3]);
+            t[c + 4] = fma(I, G, t[c + 4]);
+        }
+        if constexpr (ROLE == kRoleMovingImage) {
+            t[5] = fma(U, I, t[5]);
+            t[6] = fma(U, G, t[6]);
+        }
+    }
+};
+
+// A uniform base plus a 32-bit byte offset per lane (one saddr + voffset access). The empty
+// asm keeps the sum out of the loop optimiser's sight: it would carry a 64-bit pointer per
+// lane for every unrolled step.
+__device__ __forceinline__ const char* at_bytes(const void* base, unsigned ofs) {
+    asm volatile("" : "+v"(ofs));
+    return static_cast<const char*>(base) + ofs;
+}
+template <typename V>
+__device__ __forceinline__ V load_at(const V* base, unsigned ofs) {
+    V v;
+    __builtin_memcpy(&v, at_bytes(base, ofs), sizeof(V));
+    return v;
+}
+
+// Matrix i of the launch: from memory, or a single matrix from the kernel's arguments.
+__device__ __forceinline__ void load_matrix(const FusedArgs& a, size_t i, float (&m)[12]) {
+    if (a.inline_mat) {
+#pragma unroll
+        for (int k = 0; k < 12; ++k) m[k] = a.m0[k];
+    } else {
+        const float* mp = a.mats + i * 12;
+#pragma unroll
+        for (int k = 0; k < 12; ++k) m[k] = mp[k];
+    }
+}
+
 // Work-group -> (tile, pose) on a 1D grid of roundup(tiles, 8) x npose work-groups.
 // Work-groups go to the 8 XCDs round-robin by linear id; this mapping keeps all poses of
 // one tile on the same XCD and adjacent in time (32 poses fill that XCD's 32 CUs), so the
@@ -578,10 +702,6 @@ __device__ __forceinline__ void wave_reduce_store(double am, double aw, double* 
 // walk down consecutive rows cover 8 distinct groups of 4 banks. (Odd strides suit
 // single-double accesses and left 33% more conflict cycles here.)
 __host__ __device__ constexpr int lds_stride(int n) { return n + ((6 - n % 4) % 4); }
-// The 2D kernel's 16-wide tiles: odd strides. Its x pass has one run of 16 per row, and
-// there odd strides give 1.5% more throughput than 2 (mod 4), by measurement.
-__host__ __device__ constexpr int lds_stride_2d(int n) { return n | 1; }
-
 // Products of one position into the channel planes of the LDS buffer (plane size np,
 // position i). NC = 9 (+count): I, G, U, II, GG, IG, UU, UI, UG.
 // NC = 7: I, G, II, GG, IG, UI, UG.
@@ -618,7 +738,7 @@ __device__ __forceinline__ void store_products(double* s_prod, int* s_cnt, int n
 // window. (A sliding sum that adds the entering and subtracts the leaving value keeps the
 // rounding residue of every large value that passed through it, which swamps windows of
 // small variance further along the run.) Each input is read once.
-template <int W, typename V, int NO = 16, bool TIGHT = false>
+template <int W, typename V, int NO = 16>
 __device__ __forceinline__ void window_run(const V* in, int stride, V* out, int ostride) {
     constexpr int NB = (NO + W - 1) / W;  // blocks that hold outputs
     constexpr int NIN = NO - 1 + W;       // inputs of the run
@@ -642,12 +762,8 @@ __device__ __forceinline__ void window_run(const V* in, int stride, V* out, int 
                 pre = j == 0 ? raw[j] : pre + raw[j];
             }
         }
-        if (TIGHT) __builtin_amdgcn_sched_barrier(0);
     }
 }
-
-// Row of output oy of the in-place box sums (box_xy_inplace) in the products planes.
-__host__ __device__ constexpr int box_row(int oy, int w) { return oy < 8 ? oy : oy + w - 1; }
 
 }  // namespace
 

@@ -64,6 +64,93 @@ struct lc2e_engine {
     size_t used = 0;
     std::mutex mu;      // guards `used`: a serving loop allocates from its own thread
 
+    // Freed device and pinned host blocks kept for the next allocation of about their size,
+    // by an engine without a budget: a hipMalloc or hipFree of a volume takes 0.1 to 0.5 ms. At
+    // most kKeepDevice and kKeepHost bytes; given back when an allocation fails and with the
+    // engine. A block is kept only once the device is idle (as hipFree waits for it).
+    struct Block {
+        void* p;
+        size_t bytes;
+    };
+    static constexpr size_t kKeepDevice = size_t(1) << 30, kKeepHost = size_t(16) << 20;
+    std::vector<Block> kept_device, kept_host;  // guarded by mu
+
+    void* take(std::vector<Block>& kept, size_t bytes) {
+        if (budget) return nullptr;
+        std::lock_guard<std::mutex> lk(mu);
+        int best = -1;
+        for (int i = 0; i < (int)kept.size(); ++i)
+            if (kept[i].bytes >= bytes && kept[i].bytes <= bytes + bytes / 4 + 4096 &&
+                (best < 0 || kept[i].bytes < kept[best].bytes))
+                best = i;
+        if (best < 0) return nullptr;
+        void* p = kept[best].p;
+        sizes[p] = kept[best].bytes;
+        kept.erase(kept.begin() + best);
+        return p;
+    }
+    // true if the block is kept
+    bool keep(std::vector<Block>& kept, size_t limit, void* p, size_t bytes) {
+        if (budget || bytes > limit / 2) return false;
+        if (hipSetDevice(device) != hipSuccess || hipDeviceSynchronize() != hipSuccess) return false;
+        std::lock_guard<std::mutex> lk(mu);
+        auto it = sizes.find(p);
+        if (it != sizes.end()) {
+            bytes = it->second;  // the block's own size, if it had been reused
+            sizes.erase(it);
+        }
+        size_t total = bytes;
+        for (const Block& b : kept) total += b.bytes;
+        if (total > limit) return false;
+        kept.push_back({p, bytes});
+        return true;
+    }
+    std::map<void*, size_t> sizes;  // reused blocks in use that are larger than asked for
+    void give_back() {
+        std::vector<Block> d, h;
+        {
+            std::lock_guard<std::mutex> lk(mu);
+            d.swap(kept_device);
+            h.swap(kept_host);
+        }
+        for (const Block& b : d) (void)hipFree(b.p);
+        for (const Block& b : h) (void)hipHostFree(b.p);
+    }
+    // Device memory without a charge to the budget.
+    hipError_t raw_alloc(void** p, size_t bytes) {
+        if (!bytes) bytes = 1;
+        if ((*p = take(kept_device, bytes))) return hipSuccess;
+        hipError_t err = hipSetDevice(device);
+        if (err == hipSuccess) err = hipMalloc(p, bytes);
+        if (err != hipSuccess) {  // again without the kept blocks
+            (void)hipGetLastError();
+            give_back();
+            err = hipMalloc(p, bytes);
+        }
+        return err;
+    }
+    void raw_free(void* p, size_t bytes) {
+        if (p && !keep(kept_device, kKeepDevice, p, bytes ? bytes : 1)) {
+            forget(p);
+            (void)hipFree(p);
+        }
+    }
+    // Mapped, coherent pinned host memory.
+    hipError_t host_alloc(void** p, size_t bytes) {
+        if ((*p = take(kept_host, bytes))) return hipSuccess;
+        return hipHostMalloc(p, bytes, hipHostMallocMapped | hipHostMallocCoherent);
+    }
+    void host_free(void* p, size_t bytes) {
+        if (p && !keep(kept_host, kKeepHost, p, bytes)) {
+            forget(p);
+            (void)hipHostFree(p);
+        }
+    }
+    void forget(void* p) {
+        std::lock_guard<std::mutex> lk(mu);
+        sizes.erase(p);
+    }
+
     int alloc(void** p, size_t bytes) {
         {
             std::lock_guard<std::mutex> lk(mu);
@@ -72,8 +159,7 @@ struct lc2e_engine {
                             used, bytes, budget);
             used += bytes;  // reserved before the allocation, returned if it fails
         }
-        hipError_t err = hipSetDevice(device);
-        if (err == hipSuccess) err = hipMalloc(p, bytes ? bytes : 1);
+        const hipError_t err = raw_alloc(p, bytes);
         if (err != hipSuccess) {
             std::lock_guard<std::mutex> lk(mu);
             used -= bytes;
@@ -83,7 +169,7 @@ struct lc2e_engine {
     }
     void release(void* p, size_t bytes) {
         if (p) {
-            (void)hipFree(p);
+            raw_free(p, bytes);
             std::lock_guard<std::mutex> lk(mu);
             used -= bytes;
         }
@@ -129,6 +215,8 @@ struct lc2e_pair {
     double* h_out = nullptr;   // pinned, mapped and coherent
     float* h_mats_dev = nullptr;   // their device addresses
     double* h_out_dev = nullptr;
+    double* h_part = nullptr;      // pinned, mapped and coherent: kHostPartials partials
+    double* h_part_dev = nullptr;
     size_t cap_bytes = 0;
     bool use_graph = false;
     std::map<int, GraphEntry> graphs;
@@ -145,10 +233,15 @@ struct lc2e_pair {
     int* mi_ext = nullptr;
     unsigned* mi_hist = nullptr;
     double* mi_out = nullptr;
-    // two-kernel path: the warped moving image of ws_poses poses, 8 bytes per voxel and pose
-    // (kept with the pair; see grow_workspace)
-    float2* ws = nullptr;
+    // two-kernel path: the warped moving image of ws_poses poses (ws_bytes each) and, if the
+    // static image is the high-resolution one, its statistics; kept with the pair (see
+    // make_two_kernel)
+    bool two = false;
+    bool two_charged = false;  // the memory below counts against the engine's budget
+    void* ws = nullptr;
+    size_t ws_bytes = 0;
     int ws_poses = 0;
+    double* istat = nullptr;
     int resident_per_cu = 0;  // fused work-groups one CU holds at once (0: not queried yet)
     // separable path (radius beyond the fused kernels): grids and box-sum buffers, made at
     // pair creation
@@ -163,6 +256,11 @@ struct lc2e_pair {
     long long prof_launches = 0;
 
     int mats_per_pose() const { return info.per_frame_matrices ? info.n_frames : 1; }
+    int role() const {
+        return info.high_res_is_moving ? lc2e::kRoleMovingImage
+               : istat || info.grid_ndim == 3 ? lc2e::kRoleStaticImage : lc2e::kRoleStaticImageFull;
+    }
+    size_t voxels() const { return vbytes / sizeof(float); }
 };
 
 namespace {
@@ -189,10 +287,25 @@ int round_zchunk(int c) { return (c + lc2e::kZBlock - 1) / lc2e::kZBlock * lc2e:
 
 lc2e::FusedArgs make_args(lc2e_pair* p, const float* d_mats, double* d_partials, const Tiling& t);
 
+// 2D launches that warp in the moments kernel itself: all of a pair without a workspace, and
+// those too small to fill the device, where a second launch costs more than warping each
+// pixel of the moments' row halos again (static high-resolution image, 256x256, 64 poses: 42 us
+// in place, 58 us through the grid; moving, 128 frames 512x384, r = 6, 3 poses: 1.99 ms in
+// place, 1.59 ms through the grid). The same values either way, bit for bit.
+constexpr long long kInPlaceWaves = 2048;
+bool in_place(const lc2e_pair* p, int tiles, int n) {
+    return p->info.grid_ndim == 2 && (!p->ws || (long long)tiles * 4 * n < kInPlaceWaves);
+}
+
 // The pair's evaluation kernels for n poses: the fused kernel, or the separable path for
 // radii beyond it.
 hipError_t launch_eval(lc2e_pair* p, const lc2e::FusedArgs& a, int n, hipStream_t st) {
-    if (p->ws) {
+    if (p->two && in_place(p, a.tiles, n)) {
+        lc2e::FusedArgs s = a;
+        s.in_place = 1;
+        return lc2e::launch_moments(s, p->info.grid_ndim, p->role(), n, st);
+    }
+    if (p->two) {
         // as many poses at a time as the workspace holds, in equal parts
         const int parts = (n + p->ws_poses - 1) / p->ws_poses, step = (n + parts - 1) / parts;
         for (int b = 0; b < n; b += step) {
@@ -200,8 +313,9 @@ hipError_t launch_eval(lc2e_pair* p, const lc2e::FusedArgs& a, int n, hipStream_
             lc2e::FusedArgs s = a;
             s.mats = a.mats + (size_t)b * a.mats_per_pose * 12;
             s.partials = a.partials + (size_t)b * a.blocks_per_pose * 2;
-            hipError_t err = lc2e::launch_warp_grad3(s, m, st);
-            if (err == hipSuccess) err = lc2e::launch_moments3(s, m, st);
+            hipError_t err = lc2e::launch_warp_grid(s, p->info.grid_ndim, p->info.src_ndim,
+                                                    p->info.high_res_is_moving, m, st);
+            if (err == hipSuccess) err = lc2e::launch_moments(s, p->info.grid_ndim, p->role(), m, st);
             if (err != hipSuccess) return err;
         }
         return hipSuccess;
@@ -209,8 +323,8 @@ hipError_t launch_eval(lc2e_pair* p, const lc2e::FusedArgs& a, int n, hipStream_
     if (p->sep)
         return lc2e::launch_sep(a, p->info.grid_ndim, p->info.src_ndim, p->info.high_res_is_moving, n,
                                 st);
-    return lc2e::launch_fused(a, p->info.grid_ndim, p->info.src_ndim, p->info.high_res_is_moving, n,
-                              st);
+    if (p->info.grid_ndim == 2) return lc2e::launch_fused2(a, p->info.src_ndim, n, st);
+    return lc2e::launch_fused(a, p->info.high_res_is_moving, n, st);
 }
 
 // Fused work-groups one CU holds at once for this pair's kernel (queried once, then kept).
@@ -220,9 +334,9 @@ int resident_per_cu(lc2e_pair* p) {
         const lc2e::FusedArgs a = make_args(p, nullptr, nullptr, Tiling{});
         int per_cu = 0;
         const hipError_t err =
-            p->ws ? lc2e::moments_resident_per_cu(a, &per_cu)
-                  : lc2e::fused_resident_per_cu(a, p->info.grid_ndim, p->info.src_ndim,
-                                                p->info.high_res_is_moving, &per_cu);
+            p->two ? lc2e::moments_resident_per_cu(a, p->info.grid_ndim, p->role(), &per_cu)
+            : p->info.grid_ndim == 2 ? lc2e::fused2_resident_per_cu(a, p->info.src_ndim, &per_cu)
+                                     : lc2e::fused_resident_per_cu(a, p->info.high_res_is_moving, &per_cu);
         if (err != hipSuccess || per_cu <= 0)
             per_cu = 1;
         p->resident_per_cu = per_cu;
@@ -252,7 +366,7 @@ int model_zchunk(lc2e_pair* p, int n) {
     const int per_xcd = std::max(1, cus / lc2e::kXcds * resident_per_cu(p));
     const int cmax = round_zchunk(ez);
     // per work-group, in plane steps (fitted): the two-kernel path only fills its pipeline
-    const double extra = p->ws ? 8.0 : 2 * r + 2 + 2.0;
+    const double extra = p->two ? 8.0 : 2 * r + 2 + 2.0;
     int best = cmax;
     double best_cost = -1.0;
     std::vector<double> heap;
@@ -300,7 +414,7 @@ Tiling tiling_for(lc2e_pair* p, int n) {
         t.zchunk = round_zchunk(p->zchunk_forced > 0 ? p->zchunk_forced
                                 : it != p->tuned.end() ? it->second : model_zchunk(p, n));
         t.tiles = lc2e::fused_blocks_3d(p->v, r, t.zchunk, &t.ntx, &t.nty, &t.nzc);
-        t.bpp = p->ws ? lc2e::moments_partials_3d(p->v, r) : lc2e::fused_partials_3d(p->v, r);
+        t.bpp = lc2e::fused_partials_3d(p->v, r);
         p->last_zchunk = t.zchunk;
     } else {
         // one work-group and one partial per tile and run of kFrameRun frames (fixed, so
@@ -310,16 +424,38 @@ Tiling tiling_for(lc2e_pair* p, int n) {
         t.nzc = tf > 0 ? (p->v.Z + t.zchunk - 1) / t.zchunk : 0;
         t.tiles = t.bpp = t.ntx * t.nty * t.nzc;
     }
+    if (p->two) {
+        lc2e::FusedArgs a{};
+        a.v = p->v;
+        a.r = r;
+        a.zchunk = t.zchunk;
+        lc2e::moments_tiling(&a, p->info.grid_ndim, p->role());
+        t.zchunk = a.zchunk;
+        t.ntx = a.ntx;
+        t.nty = a.nty;
+        t.nzc = a.nzc;
+        t.tiles = a.tiles;
+        t.bpp = a.blocks_per_pose;
+    }
     return t;
 }
+
+// Launches of up to kDirectPoses poses with at most kHostPose partials each add them up on the
+// host (enqueue_batch).
+constexpr int kDirectPoses = 8;
+constexpr int kHostPose = 256;
+constexpr size_t kHostPartials = (size_t)kDirectPoses * kHostPose;
 
 void free_batch(lc2e_pair* p) {
     drop_graphs(p);
     lc2e_engine* e = p->e;
     if (p->d_mats) e->release(p->d_mats, (size_t)p->cap * p->mats_per_pose() * 12 * sizeof(float));
     if (p->d_partials) e->release(p->d_partials, (size_t)p->cap * p->part_bpp * 2 * sizeof(double));
-    if (p->h_mats) (void)hipHostFree(p->h_mats);
-    if (p->h_out) (void)hipHostFree(p->h_out);
+    e->host_free(p->h_mats, (size_t)p->cap * p->mats_per_pose() * 12 * sizeof(float));
+    e->host_free(p->h_out, (size_t)p->cap * 3 * sizeof(double));
+    e->host_free(p->h_part, kHostPartials * 2 * sizeof(double));
+    p->h_part = nullptr;
+    p->h_part_dev = nullptr;
     p->d_mats = nullptr;
     p->d_partials = nullptr;
     p->h_mats = nullptr;
@@ -342,28 +478,88 @@ void free_mi(lc2e_pair* p) {
     p->mi_bins = 0;
 }
 
-// The two-kernel path's workspace for n poses, up to kWorkspaceBytes (at least one pose).
-// Only an engine without an HBM budget keeps one: under a budget the fused kernel, which
-// needs none, evaluates the same values, so what a budget admits does not depend on it.
-// Returns false if there is none (nothing is lost: the fused kernel runs).
+// Memory of the two-kernel path beside the budgeted buffers.
+int two_alloc(lc2e_pair* p, void** d, size_t bytes) {
+    if (p->two_charged) return p->e->alloc(d, bytes);
+    if (p->e->raw_alloc(d, bytes) == hipSuccess) return LC2E_OK;
+    (void)hipGetLastError();
+    return fail(LC2E_ERR_HIP, "workspace of %zu bytes", bytes);
+}
+void two_free(lc2e_pair* p, void* d, size_t bytes) {
+    if (!d) return;
+    if (p->two_charged) p->e->release(d, bytes);
+    else p->e->raw_free(d, bytes);  // waits for launches that use it
+}
+
+// The workspace for n poses, up to kWorkspaceBytes (at least one pose); larger launches go
+// through it in parts. Only an engine without an HBM budget grows it past one pose.
 constexpr size_t kWorkspaceBytes = size_t(1) << 30;
-bool grow_workspace(lc2e_pair* p, int n) {
-    const size_t per = (p->vbytes / sizeof(float)) * sizeof(float2);
-    const int want = (int)std::min<size_t>((size_t)std::max(n, 1), std::max<size_t>(1, kWorkspaceBytes / per));
-    if (want <= p->ws_poses) return true;
-    void* d = nullptr;
-    if (hipSetDevice(p->e->device) != hipSuccess || hipMalloc(&d, (size_t)want * per) != hipSuccess) {
-        (void)hipGetLastError();
-        return p->ws != nullptr;
+int grow_workspace(lc2e_pair* p, int n) {
+    if (p->e->budget) {
+        if (!p->two_charged) return LC2E_OK;
+        n = 1;
     }
+    const size_t per = p->voxels() * (p->info.high_res_is_moving ? sizeof(float2) : sizeof(float));
+    const int want = (int)std::min<size_t>((size_t)std::max(n, 1), std::max<size_t>(1, kWorkspaceBytes / per));
+    if (want <= p->ws_poses) return LC2E_OK;
+    void* d = nullptr;
+    const int rc = two_alloc(p, &d, (size_t)want * per);
+    if (rc < 0) return p->ws ? LC2E_OK : rc;  // what is there still serves
     if (p->ws) {
         drop_graphs(p);
-        (void)hipFree(p->ws);  // waits for launches that use it
+        two_free(p, p->ws, (size_t)p->ws_poses * p->ws_bytes);
     }
-    p->ws = static_cast<float2*>(d);
+    p->ws = d;
+    p->ws_bytes = per;
     p->ws_poses = want;
     p->model_cache.clear();
-    return true;
+    return LC2E_OK;
+}
+
+void free_two(lc2e_pair* p) {
+    two_free(p, p->ws, (size_t)p->ws_poses * p->ws_bytes);
+    two_free(p, p->istat, lc2e::kImageStats * p->voxels() * sizeof(double));
+    p->ws = nullptr;
+    p->istat = nullptr;
+    p->ws_poses = 0;
+    p->two = false;
+}
+
+lc2e::FusedArgs make_args(lc2e_pair* p, const float* d_mats, double* d_partials, const Tiling& t);
+
+// A role of the two-kernel path's moments that writes statistics of a static image.
+hipError_t launch_stats(lc2e_pair* p, int role, hipStream_t st) {
+    lc2e::FusedArgs a = make_args(p, nullptr, nullptr, Tiling{});
+    a.zchunk = 32;  // planes per work-group (3D)
+    a.istat_out = p->istat;
+    a.ustat_mean_out = p->ustat;
+    a.ustat_cyy_out = p->ustat + p->voxels();
+    lc2e::moments_tiling(&a, p->info.grid_ndim, role);
+    return lc2e::launch_moments(a, p->info.grid_ndim, role, 1, st);
+}
+
+// Sets the moments path up. 2D pairs use it from the radii on at which it is faster than the
+// fused kernel (with a static high-resolution image always), and do without its memory where
+// there is none (in_place). 3D radii beyond the fused kernel need its memory, which is less than the
+// separable path's and charged to the budget. Other 3D radii use it on an engine without a
+// budget only: under one the fused kernel, which needs no workspace, evaluates the pair, so
+// what a budget admits is what it admitted without this path.
+int make_two_kernel(lc2e_pair* p, bool required) {
+    const bool two_d = p->info.grid_ndim == 2;
+    if (two_d && p->info.high_res_is_moving && p->info.patch_radius <= lc2e::kMaxRFused2) return LC2E_OK;
+    p->two_charged = required && p->e->budget;
+    p->two = two_d;
+    if (!required && p->e->budget) return LC2E_OK;
+    p->two = true;
+    const bool grid = !two_d || p->info.high_res_is_moving;  // else warped in place
+    int rc = grid ? grow_workspace(p, 1) : LC2E_OK;
+    if (rc >= 0 && !p->info.high_res_is_moving)
+        rc = two_alloc(p, (void**)&p->istat, lc2e::kImageStats * p->voxels() * sizeof(double));
+    if (rc < 0) {
+        free_two(p);
+        p->two = two_d;
+    }
+    return rc < 0 && required ? rc : LC2E_OK;
 }
 
 // Batch buffers for n poses whose launches use up to bpp work-groups per pose.
@@ -390,15 +586,22 @@ int ensure_capacity(lc2e_pair* p, int n, int bpp) {
     void* ho = nullptr;
     // mapped and coherent: small launches read their matrices from here and every launch's
     // reduction writes its results here, with no copy command (enqueue_batch)
-    const unsigned fl = hipHostMallocMapped | hipHostMallocCoherent;
-    hipError_t he = hipHostMalloc(&hm, (size_t)cap * mpp * 12 * sizeof(float), fl);
+    hipError_t he = e->host_alloc(&hm, (size_t)cap * mpp * 12 * sizeof(float));
     if (he == hipSuccess) {
         p->h_mats = (float*)hm;
-        he = hipHostMalloc(&ho, (size_t)cap * 3 * sizeof(double), fl);
+        he = e->host_alloc(&ho, (size_t)cap * 3 * sizeof(double));
         if (he == hipSuccess) p->h_out = (double*)ho;
+    }
+    void* hp = nullptr;
+    if (he == hipSuccess) {
+        he = e->host_alloc(&hp, kHostPartials * 2 * sizeof(double));
+        if (he == hipSuccess) p->h_part = (double*)hp;
     }
     void* dm = nullptr;
     void* dout = nullptr;
+    void* dpart = nullptr;
+    if (he == hipSuccess) he = hipHostGetDevicePointer(&dpart, hp, 0);
+    p->h_part_dev = (double*)dpart;
     if (he == hipSuccess) he = hipHostGetDevicePointer(&dm, hm, 0);
     if (he == hipSuccess) he = hipHostGetDevicePointer(&dout, ho, 0);
     if (he == hipSuccess) {
@@ -436,7 +639,12 @@ lc2e::FusedArgs make_args(lc2e_pair* p, const float* d_mats, double* d_partials,
     a.blocks_per_pose = t.bpp;
     a.tiles = t.tiles;
     a.mats_per_pose = p->mats_per_pose();
-    a.warp2 = p->ws;
+    a.warp2 = static_cast<float2*>(p->ws);
+    a.warp1 = static_cast<float*>(p->ws);
+    a.istat = p->istat;
+    a.src3 = p->info.src_ndim == 3 ? 1 : 0;
+    a.in_place = p->two && !p->ws && p->info.grid_ndim == 2 ? 1 : 0;
+    a.istat_stride = (long long)V;
     if (p->sep) {
         const size_t V = p->vbytes / sizeof(float);
         a.sep_img = p->sep_grids;
@@ -452,23 +660,31 @@ lc2e::FusedArgs make_args(lc2e_pair* p, const float* d_mats, double* d_partials,
 // (up to kDirectPoses poses of one matrix each, on a single volume or image: each
 // work-group reads its pose's 12 floats once) read the pinned matrices in place instead of
 // copying them, and the reduction always writes the results in place: one or two commands
-// per batch instead of four.
-constexpr int kDirectPoses = 8;
-int enqueue_batch(lc2e_pair* p, int n, const Tiling& t, hipStream_t st) {
+// per batch instead of four. Where a launch is not captured, a single matrix goes with the
+// kernel's arguments (a read from pinned memory takes 1.2 us at a kernel's start), and few
+// partials go straight to pinned memory for the host to add up (*host_sum; a launch less:
+// 2D 256x256 single pose 30.7 -> 24.5 us with both).
+int enqueue_batch(lc2e_pair* p, int n, const Tiling& t, hipStream_t st, bool captured, bool* host_sum) {
     const int mpp = p->mats_per_pose();
     const bool direct = !p->sep && mpp == 1 && n <= kDirectPoses &&
                         (p->info.grid_ndim == 3 || p->v.Z == 1);
+    const bool host = !captured && n <= kDirectPoses && t.tiles > 0 && t.bpp <= kHostPose;
+    *host_sum = host;
     if (!direct)
         HIP_TRY(hipMemcpyAsync(p->d_mats, p->h_mats, (size_t)n * mpp * 12 * sizeof(float),
                                hipMemcpyHostToDevice, st));
     if (t.tiles > 0) {
-        lc2e::FusedArgs a = make_args(p, direct ? p->h_mats_dev : p->d_mats, p->d_partials, t);
+        lc2e::FusedArgs a = make_args(p, direct ? p->h_mats_dev : p->d_mats, host ? p->h_part_dev : p->d_partials, t);
+        if (direct && n == 1 && !captured) {
+            a.inline_mat = 1;
+            std::memcpy(a.m0, p->h_mats, sizeof(a.m0));
+        }
         // timed launches are eager (run_batch), the events bracket the fused kernel
         const bool timed = p->profile;
         if (timed) HIP_TRY(hipEventRecord(p->ev0, st));
         HIP_TRY(launch_eval(p, a, n, st));
         if (timed) HIP_TRY(hipEventRecord(p->ev1, st));
-        HIP_TRY(lc2e::launch_reduce(p->d_partials, t.bpp, n, p->h_out_dev, st));
+        if (!host) HIP_TRY(lc2e::launch_reduce(p->d_partials, t.bpp, n, p->h_out_dev, st));
     } else {
         // no patch centre fits in the grid: every sum is zero
         HIP_TRY(lc2e::launch_reduce(p->d_partials, 0, n, p->h_out_dev, st));
@@ -476,15 +692,39 @@ int enqueue_batch(lc2e_pair* p, int n, const Tiling& t, hipStream_t st) {
     return LC2E_OK;
 }
 
+// The sums of k_reduce from the partials in h_part, added in its order: 256 running sums of
+// every 256th partial, then halves (here at most one partial each).
+void sum_partials(lc2e_pair* p, int n, int bpp) {
+    double m[kHostPose], w[kHostPose];
+    for (int i = 0; i < n; ++i) {
+        const double* s = p->h_part + (size_t)i * bpp * 2;
+        for (int k = 0; k < kHostPose; ++k) {
+            m[k] = k < bpp ? 0.0 + s[2 * k] : 0.0;
+            w[k] = k < bpp ? 0.0 + s[2 * k + 1] : 0.0;
+        }
+        for (int h = kHostPose / 2; h > 0; h >>= 1)
+            for (int k = 0; k < h; ++k) {
+                m[k] += m[k + h];
+                w[k] += w[k + h];
+            }
+        double l = m[0] / w[0];
+        if (!std::isfinite(l)) l = 0.0;
+        p->h_out[3 * i] = m[0];
+        p->h_out[3 * i + 1] = w[0];
+        p->h_out[3 * i + 2] = l;
+    }
+}
+
 // Runs a batch of n poses staged in h_mats; the buffers must already fit tiling t.
 int run_batch(lc2e_pair* p, int n, const Tiling& t) {
     hipStream_t st = p->e->stream;
+    bool host_sum = false;
     if (p->use_graph && !p->profile) {
         auto it = p->graphs.find(n);
         if (it == p->graphs.end()) {
             GraphEntry g;
             HIP_TRY(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal));
-            int rc = enqueue_batch(p, n, t, st);
+            int rc = enqueue_batch(p, n, t, st, true, &host_sum);
             hipGraph_t graph = nullptr;
             hipError_t ce = hipStreamEndCapture(st, &graph);
             if (rc >= 0 && ce == hipSuccess) ce = hipGraphInstantiate(&g.exec, graph, nullptr, nullptr, 0);
@@ -498,10 +738,11 @@ int run_batch(lc2e_pair* p, int n, const Tiling& t) {
         }
         HIP_TRY(hipGraphLaunch(it->second.exec, st));
     } else {
-        int rc = enqueue_batch(p, n, t, st);
+        int rc = enqueue_batch(p, n, t, st, false, &host_sum);
         if (rc < 0) return rc;
     }
     HIP_TRY(hipStreamSynchronize(st));
+    if (host_sum) sum_partials(p, n, t.bpp);
     if (p->profile && t.tiles > 0) {
         float ms = 0.0f;
         HIP_TRY(hipEventElapsedTime(&ms, p->ev0, p->ev1));
@@ -536,8 +777,8 @@ double launch_share(lc2e_pair* p, int n) {
     const Tiling t = tiling_for(p, n);
     if (t.tiles <= 0 || n <= 0) return 0.0;
     const int per_cu = resident_per_cu(p);
-    const int prun = p->sep ? 1 : pose_run(p->v, p->info.grid_ndim, p->info.src_ndim,
-                                           p->mats_per_pose(), t.tiles, n);
+    const bool fused2 = p->info.grid_ndim == 2 && !p->two && !p->sep;
+    const int prun = fused2 ? pose_run(p->v, p->info.src_ndim, p->mats_per_pose(), t.tiles, n) : 1;
     const double wgs = (double)((t.tiles + kXcds - 1) / kXcds * kXcds) * ((n + prun - 1) / prun);
     const int cus = p->e->cus > 0 ? p->e->cus : 256;
     return wgs / ((double)cus * per_cu);
@@ -581,6 +822,7 @@ void lc2e_destroy(lc2e_engine* e) {
     (void)hipSetDevice(e->device);
     (void)hipStreamSynchronize(e->stream);
     (void)hipStreamDestroy(e->stream);
+    e->give_back();
     delete e;
 }
 
@@ -606,21 +848,49 @@ int lc2e_volume_upload(lc2e_engine* e, const void* host, lc2e_dtype dtype, const
     }
     const long long n = (long long)geom->dims[0] * geom->dims[1] * geom->dims[2];
     if (n >= (1LL << 31)) return fail(LC2E_ERR_UNSUPPORTED, "volume exceeds 2^31 voxels");
+    if (storage != LC2E_STORE_AUTO && storage != LC2E_F16 && storage != LC2E_F32)
+        return fail(LC2E_ERR_INVALID, "storage must be F16, F32 or AUTO");
+    HIP_TRY(hipSetDevice(e->device));
+    // The raw voxels on the device (also its conversion's input) and a word that the kernels
+    // set where a voxel is out of range: the device reads them at the memory's rate, where a
+    // scan on the host took half of an upload.
+    struct Scope {
+        lc2e_engine* e;
+        void* staging = nullptr;
+        size_t bytes = 0;
+        int* flag = nullptr;
+        ~Scope() {
+            e->raw_free(staging, bytes);
+            e->host_free(flag, sizeof(int));
+        }
+    } tmp{e};
+    HIP_TRY(e->host_alloc((void**)&tmp.flag, sizeof(int)));
+    void* flag_dev = nullptr;
+    HIP_TRY(hipHostGetDevicePointer(&flag_dev, tmp.flag, 0));
+    *tmp.flag = 0;
+    auto stage = [&]() {
+        tmp.bytes = (size_t)n * dsz;
+        hipError_t err = e->raw_alloc(&tmp.staging, tmp.bytes);
+        if (err == hipSuccess)
+            err = hipMemcpyAsync(tmp.staging, host, tmp.bytes, hipMemcpyHostToDevice, e->stream);
+        return err;
+    };
     int f16;
     if (storage == LC2E_STORE_AUTO) {
         f16 = (dtype == LC2E_U8 || dtype == LC2E_F16) ? 1 : 0;
         if (dtype == LC2E_I16) {
             // every integer in [-2048, 2048] is exact in half precision (11-bit significand),
             // which covers CT in Hounsfield units: half storage is then lossless
-            const short* h = static_cast<const short*>(host);
-            f16 = 1;
-            for (long long i = 0; i < n && f16; ++i)
-                if (h[i] < -2048 || h[i] > 2048) f16 = 0;
+            hipError_t err = stage();
+            if (err == hipSuccess)
+                err = lc2e::launch_check(tmp.staging, dtype, n, 2048.0f, (int*)flag_dev, e->stream);
+            if (err == hipSuccess) err = hipStreamSynchronize(e->stream);
+            if (err != hipSuccess) return fail(LC2E_ERR_HIP, "volume upload failed: %s", hipGetErrorString(err));
+            f16 = *tmp.flag ? 0 : 1;
+            *tmp.flag = 0;
         }
     }
-    else if (storage == LC2E_F16) f16 = 1;
-    else if (storage == LC2E_F32) f16 = 0;
-    else return fail(LC2E_ERR_INVALID, "storage must be F16, F32 or AUTO");
+    else f16 = storage == LC2E_F16;
     // the samplers address a volume and its zeroed tail with 32-bit byte offsets
     const long long pad = lc2e::volume_pad_elems(geom->dims[0], geom->dims[1]);
     if ((n + pad) * (f16 ? 2 : 4) > 0xffffffffLL)
@@ -628,20 +898,25 @@ int lc2e_volume_upload(lc2e_engine* e, const void* host, lc2e_dtype dtype, const
                     "volume of %lld voxels (plus a %lld-voxel zeroed tail) exceeds the 4 GiB "
                     "that %s storage can address%s", n, pad, f16 ? "f16" : "f32",
                     f16 ? "" : "; store it as F16");
-    // The samplers rely on finite voxels (a zero-weight corner must contribute exactly 0).
-    if (dtype == LC2E_F32) {
-        const float lim = f16 ? 65504.0f : 3.4028235e38f;
-        const float* h = static_cast<const float*>(host);
-        for (long long i = 0; i < n; ++i)
-            if (!(std::fabs(h[i]) <= lim))
-                return fail(LC2E_ERR_INVALID, "value %g at %lld is not finite%s", h[i], i,
-                            f16 ? " in half storage" : "");
-    } else if (dtype == LC2E_F16) {
-        const unsigned short* h = static_cast<const unsigned short*>(host);
-        for (long long i = 0; i < n; ++i)
-            if ((h[i] & 0x7c00u) == 0x7c00u)
-                return fail(LC2E_ERR_INVALID, "half value 0x%04x at %lld is not finite", h[i], i);
-    }
+    // The samplers rely on finite voxels (a zero-weight corner must contribute exactly 0): the
+    // largest magnitude admitted, and the error that names the first voxel past it.
+    const float lim = dtype == LC2E_F32 && !f16 ? 3.4028235e38f : 65504.0f;
+    const bool check = dtype == LC2E_F32 || dtype == LC2E_F16;
+    auto bad_voxel = [&]() {
+        if (dtype == LC2E_F32) {
+            const float* h = static_cast<const float*>(host);
+            for (long long i = 0; i < n; ++i)
+                if (!(std::fabs(h[i]) <= lim))
+                    return fail(LC2E_ERR_INVALID, "value %g at %lld is not finite%s", h[i], i,
+                                f16 ? " in half storage" : "");
+        } else if (dtype == LC2E_F16) {
+            const unsigned short* h = static_cast<const unsigned short*>(host);
+            for (long long i = 0; i < n; ++i)
+                if ((h[i] & 0x7c00u) == 0x7c00u)
+                    return fail(LC2E_ERR_INVALID, "half value 0x%04x at %lld is not finite", h[i], i);
+        }
+        return LC2E_OK;
+    };
     auto* v = new lc2e_volume();
     v->e = e;
     v->g = *geom;
@@ -651,29 +926,29 @@ int lc2e_volume_upload(lc2e_engine* e, const void* host, lc2e_dtype dtype, const
     int rc = e->alloc(&v->d, v->bytes);
     if (rc < 0) {
         delete v;
-        return rc;
+        const std::string why = g_last_error;
+        const int bad = bad_voxel();  // an invalid volume is invalid whether it fits or not
+        if (bad >= 0) g_last_error = why;
+        return bad < 0 ? bad : rc;
     }
-    {
-        // zeroed tail (lc2e::volume_pad_elems): the samplers' reads past the last voxel
-        hipError_t pe = hipMemsetAsync(static_cast<char*>(v->d) + (size_t)n * esz, 0,
-                                       (size_t)pad * esz, e->stream);
-        if (pe != hipSuccess) {
-            e->release(v->d, v->bytes);
-            delete v;
-            return fail(LC2E_ERR_HIP, "volume padding failed: %s", hipGetErrorString(pe));
-        }
+    // zeroed tail (lc2e::volume_pad_elems): the samplers' reads past the last voxel
+    hipError_t err = hipMemsetAsync(static_cast<char*>(v->d) + (size_t)n * esz, 0, (size_t)pad * esz, e->stream);
+    if (dtype == (f16 ? LC2E_F16 : LC2E_F32)) {  // stored as it comes
+        if (err == hipSuccess)
+            err = hipMemcpyAsync(v->d, host, (size_t)n * dsz, hipMemcpyHostToDevice, e->stream);
+        if (err == hipSuccess) err = lc2e::launch_check(v->d, dtype, n, lim, (int*)flag_dev, e->stream);
+    } else {
+        if (err == hipSuccess && !tmp.staging) err = stage();
+        if (err == hipSuccess && check)
+            err = lc2e::launch_check(tmp.staging, dtype, n, lim, (int*)flag_dev, e->stream);
+        if (err == hipSuccess)
+            err = lc2e::launch_convert(tmp.staging, (int)dtype, v->d, f16, n, e->stream);
     }
-    // stage the raw bytes on the device, convert there
-    void* staging = nullptr;
-    hipError_t err = hipMalloc(&staging, (size_t)n * dsz);
-    if (err == hipSuccess)
-        err = hipMemcpyAsync(staging, host, (size_t)n * dsz, hipMemcpyHostToDevice, e->stream);
-    if (err == hipSuccess) err = lc2e::launch_convert(staging, (int)dtype, v->d, f16, n, e->stream);
     if (err == hipSuccess) err = hipStreamSynchronize(e->stream);
-    if (staging) (void)hipFree(staging);
-    if (err != hipSuccess) {
+    if (err != hipSuccess || *tmp.flag) {
         e->release(v->d, v->bytes);
         delete v;
+        if (err == hipSuccess && (rc = bad_voxel()) < 0) return rc;
         return fail(LC2E_ERR_HIP, "volume upload failed: %s", hipGetErrorString(err));
     }
     *out = v;
@@ -701,8 +976,8 @@ int lc2e_pair_create(lc2e_engine* e, lc2e_volume* fixed, lc2e_volume* moving,
     // (beyond the fused samplers' 24-bit offsets), take the separable path
     const bool big_slices = moving->g.dims[2] > 1 &&
                             (long long)moving->g.dims[0] * moving->g.dims[1] >= lc2e::kMaxFusedSlice;
-    const bool sep = (dim == 3 && patch_radius > lc2e::kMaxR3) ||
-                     (dim == 2 && patch_radius > lc2e::kMaxR2) || big_slices;
+    const bool small_r = patch_radius <= (dim == 3 ? lc2e::kMaxR3 : lc2e::kMaxR2);
+    const int two_max = dim == 3 ? lc2e::kMaxRMom3 : lc2e::kMaxR2;
     const int src_ndim = moving->g.dims[2] > 1 ? 3 : 2;
     if (dim == 3 && (src_ndim != 3 || fixed->g.dims[2] < 1))
         return fail(LC2E_ERR_INVALID, "3D LC2 needs a 3D moving volume");
@@ -714,6 +989,10 @@ int lc2e_pair_create(lc2e_engine* e, lc2e_volume* fixed, lc2e_volume* moving,
     const long long V = (long long)pg.virt.dims[0] * pg.virt.dims[1] * pg.virt.dims[2];
     if (V >= (1LL << 31)) return fail(LC2E_ERR_UNSUPPORTED, "virtual grid exceeds 2^31 voxels");
 
+    // (the 3D moments kernel addresses a plane of the grid with 32-bit byte offsets)
+    const bool big_plane = dim == 3 && (long long)pg.virt.dims[0] * pg.virt.dims[1] >= (1LL << 28);
+    const bool moments = patch_radius <= two_max && !big_plane;
+    const bool sep = big_slices || (!small_r && !moments);
     auto* p = new lc2e_pair();
     p->gen = g_generation.fetch_add(1);
     p->e = e;
@@ -757,6 +1036,10 @@ int lc2e_pair_create(lc2e_engine* e, lc2e_volume* fixed, lc2e_volume* moving,
     lc2e::SGeom fsg = lc2e::make_sgeom(fg.dims, fg.spacing, fg.origin);
     hipError_t err = lc2e::launch_warp_static(fixed->d, fixed->f16, fsg, p->v, dim, src_ndim,
                                               p->stat_img, e->stream);
+    if (err == hipSuccess && !sep && moments && (rc = make_two_kernel(p, !small_r)) < 0) {
+        lc2e_pair_destroy(p);
+        return rc;
+    }
     if (err == hipSuccess && high_res_is_moving) {
         // the fixed image is the ultrasound: its patch statistics are pose-independent
         rc = e->alloc((void**)&p->ustat, 2 * (size_t)V * sizeof(double));
@@ -764,8 +1047,9 @@ int lc2e_pair_create(lc2e_engine* e, lc2e_volume* fixed, lc2e_volume* moving,
             lc2e_pair_destroy(p);
             return rc;
         }
-        err = lc2e::launch_ustats(p->stat_img, p->v, dim, patch_radius, p->ustat, p->ustat + V,
-                                  e->stream);
+        err = moments ? launch_stats(p, lc2e::kRoleUsStats, e->stream)
+                    : lc2e::launch_ustats(p->stat_img, p->v, dim, patch_radius, p->ustat, p->ustat + V,
+                                          e->stream);
     }
     if (err == hipSuccess && !high_res_is_moving) {
         // the fixed image is the high-resolution one: its |Sobel| is pose-independent
@@ -775,8 +1059,8 @@ int lc2e_pair_create(lc2e_engine* e, lc2e_volume* fixed, lc2e_volume* moving,
             return rc;
         }
         err = lc2e::launch_sobel(p->stat_img, p->v, dim, p->stat_grad, e->stream);
+        if (err == hipSuccess && p->istat) err = launch_stats(p, lc2e::kRoleImageStats, e->stream);
     }
-    if (err == hipSuccess && dim == 3 && high_res_is_moving && !sep && !e->budget) (void)grow_workspace(p, 1);
     if (err == hipSuccess) err = hipStreamSynchronize(e->stream);
     if (err != hipSuccess) {
         lc2e_pair_destroy(p);
@@ -799,7 +1083,7 @@ void lc2e_pair_destroy(lc2e_pair* p) {
     if (p->ustat) p->e->release(p->ustat, 2 * (p->vbytes / sizeof(float)) * sizeof(double));
     if (p->sep_grids) p->e->release(p->sep_grids, p->sep_grid_bytes);
     if (p->sep_sums) p->e->release(p->sep_sums, p->sep_sum_bytes);
-    if (p->ws) (void)hipFree(p->ws);
+    free_two(p);
     delete p;
 }
 

@@ -15,6 +15,10 @@
 // FP32 values are exact in FP64), which removes the cancellation an FP32
 // sliding-window sum would suffer on intensities with small local variance.
 //
+// Pairs are evaluated by k_moments3d / k_moments2d (their files say how), by k_fused2d (2D, moving
+// high-resolution image, small patches), by k_fused3d (3D under an HBM budget: it needs no
+// workspace) or by the separable path (the remaining radii).
+//
 // 3D structure (k_fused3d): a 256-thread work-group (two per CU) owns a 16x16 column
 // of output voxels over `zchunk` planes and marches along z. Per input plane:
 // warp the plane (+ Sobel halo) into LDS, separable Sobel of each 3x3 neighbourhood
@@ -22,8 +26,7 @@
 // LDS (van Herk / Gil-Werman: no partial sum holds a value from outside its window), and
 // a (2R+1)-slot register ring of plane sums and pair sums of planes gives the z window
 // sum; complete patch sums are combined in FP64 and accumulated per thread. No
-// intermediate volume touches HBM. Patch radii beyond the fused kernels run the
-// separable path (k_sep_pass / k_sep_combine) through HBM.
+// intermediate volume touches HBM.
 #include <algorithm>
 #include <map>
 #include <mutex>
@@ -97,55 +100,6 @@ __device__ __forceinline__ void box_xy(const double* s_prod, const int* s_cnt, d
     __syncthreads();
 }
 
-// Box sums in place (the 2D kernel), for 16x16 outputs: the x pass writes each row's 16
-// outputs over the start of that row of s_prod, and the y pass writes each column run's 8
-// outputs over rows that no other run reads: run 0 over rows 0..7, run 1 over rows
-// W+7 .. W+14 (the last 8 of its own input rows). A task reads each of its inputs before it
-// overwrites it, so output (ox, oy) of channel c ends up at
-// s_prod[c * ps * py + box_row(oy, W) * ps + ox] with no second buffer: the LDS of the x
-// pass's output and of the sums is saved, which lets more work-groups share a CU.
-template <int NC, bool CNT, int NTHR, int W, bool PRIO_X = false, bool PRIO_Y = false>
-__device__ __forceinline__ void box_xy_inplace(double* s_prod, int* s_cnt, int ps, int py,
-                                               int tid) {
-    constexpr int NT = NC + (CNT ? 1 : 0);
-    const int np = ps * py;
-    if constexpr (PRIO_X) __builtin_amdgcn_s_setprio(2);
-    for (int t = tid; t < NT * py; t += NTHR) {
-        const int row = t % py, c = t / py;
-        if (c < NC) {
-            double* r = s_prod + c * np + row * ps;
-            window_run<W>(r, 1, r, 1);
-        } else {
-            int* r = s_cnt + row * ps;
-            window_run<W>(r, 1, r, 1);
-        }
-    }
-    if constexpr (PRIO_X) __builtin_amdgcn_s_setprio(0);
-    __syncthreads();
-    if constexpr (PRIO_Y) __builtin_amdgcn_s_setprio(2);
-    for (int t = tid; t < NT * 16 * 2; t += NTHR) {
-        const int col = t % 16, rest = t / 16;
-        const int seg = rest % 2, c = rest / 2;
-        const int in_ofs = seg * 8 * ps + col, out_ofs = box_row(seg * 8, W) * ps + col;
-        if (c < NC)
-            window_run<W, double, 8>(s_prod + c * np + in_ofs, ps, s_prod + c * np + out_ofs, ps);
-        else
-            window_run<W, int, 8>(s_cnt + in_ofs, ps, s_cnt + out_ofs, ps);
-    }
-    if constexpr (PRIO_Y) __builtin_amdgcn_s_setprio(0);
-    __syncthreads();
-}
-
-// box_xy_inplace for a patch radius known only at run time, 1 <= r <= RMAX.
-template <int NC, bool CNT, int NTHR, int RMAX = kMaxR2, int RR = 1>
-__device__ __forceinline__ void box_xy_inplace_r(int r, double* s_prod, int* s_cnt, int tid) {
-    if (r == RR)
-        box_xy_inplace<NC, CNT, NTHR, 2 * RR + 1, true, true>(s_prod, s_cnt,
-                                                             lds_stride_2d(16 + 2 * RR), 16 + 2 * RR, tid);
-    else if constexpr (RR < RMAX)
-        box_xy_inplace_r<NC, CNT, NTHR, RMAX, RR + 1>(r, s_prod, s_cnt, tid);
-}
-
 // ---------------------------------------------------------------------------
 // 3D fused kernel: a TX x TY column of output voxels over `zchunk` planes of one pose.
 // MOVI: the moving image is the high-resolution I (warped + Sobel here), the fixed
@@ -212,9 +166,7 @@ __global__ __launch_bounds__(TX * TY, 1) void k_fused3d(FusedArgs a) {
     const T* __restrict__ src = static_cast<const T*>(a.src);
     float m[12];
     {
-        const float* mp = a.mats + (size_t)pose * a.mats_per_pose * 12;
-#pragma unroll
-        for (int k = 0; k < 12; ++k) m[k] = mp[k];
+        load_matrix(a, (size_t)pose * a.mats_per_pose, m);
     }
     // warped plane of step s: MOVI -> zi = z0-R-1+s (Sobel input), else zp = z0-R+s
     const int zw0 = MOVI ? z0 - R - 1 : z0 - R;
@@ -584,252 +536,7 @@ __global__ __launch_bounds__(TX * TY, 1) void k_fused3d(FusedArgs a) {
 }
 
 // ---------------------------------------------------------------------------
-// 2D fused kernel: one 16x16 output tile of a run of `zchunk` (kFrameRun) consecutive
-// frames of one pose (a single image is one frame). Dynamic LDS sized for the runtime patch
-// radius. Frame f + 1's gathers (and its static image values and ultrasound statistics)
-// are issued while frame f's box sums and combine run, as in the 3D kernel's z-steps. Each
-// thread adds its pixel's measure and weight over the run's frames in frame order, and the
-// work-group reduces them once into the partial of (run, tile). The run length does not
-// depend on the batch, so neither do the results.
-// ---------------------------------------------------------------------------
-template <bool MOVI, bool SRC3D, typename T, int RMAX, bool P2>
-// MOVI at r <= 3: at most 128 VGPRs, four work-groups per CU (the f32-source variant
-// would take 129 and drop to three)
-__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(MOVI && RMAX <= 3 ? 4 : 1)))
-void k_fused2d(FusedArgs a) {
-    extern __shared__ double s_dyn[];
-    static_assert(kTile2X == 16 && kTile2Y == 16, "box_xy_inplace sums 16x16 tiles");
-    constexpr int NC = MOVI ? 7 : 9;
-    constexpr bool CNT = !MOVI;
-    // per-thread gathers / products positions at the largest radius of this variant
-    // (r <= RMAX): the pipelined gathers are held in registers
-    constexpr int SPT = ((kTile2X + 2 * RMAX + 2) * (kTile2Y + 2 * RMAX + 2) + kThreads - 1) / kThreads;
-    constexpr int PPT = ((kTile2X + 2 * RMAX) * (kTile2Y + 2 * RMAX) + kThreads - 1) / kThreads;
-    const int R = a.r, W = 2 * R + 1, PX = kTile2X + 2 * R, PY = kTile2Y + 2 * R, NP = PX * PY;
-    const int IXE = PX + 2, IYE = PY + 2;
-    // MOVI: warped rows 32 + PX/2 floats apart in LDS, so the paired Sobel reads of a wave
-    // (PX lanes per row group, groups two rows apart) fall into distinct banks
-    const int SIS = MOVI ? 32 + PX / 2 : IXE;
-    const int PS = lds_stride_2d(PX);                         // products row stride
-    const int wex = MOVI ? IXE : PX;                          // warped region edge
-    const int wofs = MOVI ? R + 1 : R;                        // it starts at x0 - wofs
-    const int NI = MOVI ? IXE * IYE : NP;
-    // The box sums run in place in the products planes (box_xy_inplace).
-    double* s_prod = s_dyn;                                   // NC*PY*PS
-    double* s_red = s_prod + NC * PY * PS;                    // 8
-    float* s_in = reinterpret_cast<float*>(s_red + 8);        // NI
-    int* s_cnt = reinterpret_cast<int*>(s_in + NI);           // PY*PS
-
-    // A work-group takes one tile of either a run of frames of one pose (frame stacks, 3D
-    // sources) or, with a.prun > 1 (single images of a 2D source), a run of a.prun poses:
-    // their gathers pipeline like a run's frames, and the tile's static values are loaded
-    // once. Each pose still gets one partial per tile, so the results do not depend on the
-    // run length. (With a 3D source prun is the constant 1: the frame stacks' code is not
-    // touched by the pose runs.)
-    const int prun = (!SRC3D && a.prun > 1) ? a.prun : 1;
-    int tile, prun_idx;
-    if (!map_block(a.tiles, (a.npose + prun - 1) / prun, tile, prun_idx)) return;  // whole work-group
-    const int p0 = prun_idx * prun, p1 = min(p0 + prun, a.npose);
-    const int tid = threadIdx.x;
-    const int cols = a.ntx * a.nty;
-    const int tcol = tile % cols, run = tile / cols;
-    const int f0 = run * a.zchunk, f1 = min(f0 + a.zchunk, a.v.Z);
-    const int nit = prun > 1 ? p1 - p0 : f1 - f0;  // iterations: poses or frames
-    const int tx = tcol % a.ntx, ty = tcol / a.ntx;
-    const int x0 = R + tx * kTile2X, y0 = R + ty * kTile2Y;
-    const int X = a.v.X, Y = a.v.Y;
-    const float lz = a.v.oz;
-    const T* __restrict__ src = static_cast<const T*>(a.src);
-
-    // Per-thread positions, the same for every frame (the radius is a run-time value, so
-    // the divisions are done once here, not per frame): virtual-grid coordinates of the
-    // warped positions, and the LDS / image offsets of the products positions.
-    float gLx[SPT], gLy[SPT];
-    int g_sin[SPT];     // LDS offset of warped position j in s_in
-    unsigned g_in = 0;  // bit j: warped position j lies in the grid
-#pragma unroll
-    for (int j = 0; j < SPT; ++j) {
-        const int i = tid + j * kThreads;
-        const int lx = i % wex, ly = i / wex;
-        g_sin[j] = MOVI ? ly * SIS + lx : i;
-        const int gx = x0 - wofs + lx, gy = y0 - wofs + ly;
-        if (i < NI && gx >= 0 && gx < X && gy >= 0 && gy < Y) g_in |= 1u << j;
-        gLx[j] = fmaf((float)gx, a.v.sx, a.v.ox);
-        gLy[j] = fmaf((float)gy, a.v.sy, a.v.oy);
-    }
-    // MOVI: slots 2k and 2k + 1 are the vertically adjacent products positions (lx, ly0)
-    // and (lx, ly0 + 1), ly0 even, of pair t = tid + k * kThreads: their 3x3 Sobel
-    // neighbourhoods share two rows, so 4 rows are read and smoothed instead of 6, with the
-    // same operations per position. (PPT is even at every RMAX; PY = 16 + 2R is even.)
-    static_assert(PPT % 2 == 0, "products slots come in pairs");
-    const int NPAIR = PX * (PY / 2);
-    int p_in_ofs[PPT], p_prod_ofs[PPT], p_img_ofs[PPT];  // s_in, s_prod, image (frame 0)
-    unsigned p_in = 0;  // bit j: products position j holds an image value
-#pragma unroll
-    for (int j = 0; j < PPT; ++j) {
-        const int t = tid + (j >> 1) * kThreads;
-        const int i = MOVI ? t : tid + j * kThreads;
-        const int lx = MOVI ? t % PX : i % PX;
-        const int ly = MOVI ? 2 * (t / PX) + (j & 1) : i / PX;
-        const int gx = x0 - R + lx, gy = y0 - R + ly;
-        if ((MOVI ? t < NPAIR : i < NP) && gx < X && gy < Y) p_in |= 1u << j;
-        p_in_ofs[j] = MOVI ? ly * SIS + lx : i;
-        p_prod_ofs[j] = ly * PS + lx;
-        p_img_ofs[j] = gy * X + gx;
-    }
-
-    using Pend = typename std::conditional<SRC3D, Pending3<T>, Pending2<T>>::type;
-    Pend pend[SPT];
-    // (No wave-uniform skip of empty slots here, unlike the 3D kernel: in this kernel it
-    // cost 6% on the tracked sweep, 29.09 -> 30.93 ms per launch, measured.)
-    // the matrix of iteration it: pose p0 + it (pose runs) or frame f0 + it of pose p0
-    auto issue_frame = [&](int it) {
-        float m[12];
-        const float* mp = prun > 1 ? a.mats + (size_t)(p0 + it) * a.mats_per_pose * 12
-                                   : a.mats + ((size_t)p0 * a.mats_per_pose +
-                                               (a.mats_per_pose > 1 ? f0 + it : 0)) * 12;
-#pragma unroll
-        for (int k = 0; k < 12; ++k) m[k] = mp[k];
-#pragma unroll
-        for (int j = 0; j < SPT; ++j) {
-            if (j * kThreads >= NI) break;  // uniform
-            const bool inside = (g_in >> j) & 1u;
-            if constexpr (SRC3D) issue3<P2>(src, a.s, m, gLx[j], gLy[j], lz, inside, pend[j]);
-            else issue2<P2>(src, a.s, m, gLx[j], gLy[j], inside, pend[j]);
-        }
-    };
-    // static image values of the products positions (U if MOVI, else I and |grad I|)
-    float pre0[PPT], pre1[PPT];
-    auto issue_static = [&](int frame) {
-        const int plane = frame * X * Y;
-#pragma unroll
-        for (int j = 0; j < PPT; ++j) {
-            // uniform: slot j holds pair j / 2 (MOVI) or position tid + j * kThreads
-            if (MOVI ? (j >> 1) * kThreads >= NPAIR : j * kThreads >= NP) break;
-            const bool in = (p_in >> j) & 1u;
-            const int vidx = plane + p_img_ofs[j];
-            pre0[j] = in ? a.stat_img[vidx] : 0.0f;
-            if (!MOVI) pre1[j] = in ? a.stat_grad[vidx] : 0.0f;
-        }
-    };
-    // static ultrasound statistics of this thread's output pixel
-    const int ox = tid % kTile2X, oy = tid / kTile2X;
-    const bool out_ok = (x0 + ox < X - R) && (y0 + oy < Y - R);
-    double mu_pre = 0.0, cyy_pre = -1.0;
-    auto issue_stats = [&](int frame) {
-        if (MOVI && out_ok) {
-            const int vo = frame * X * Y + (y0 + oy) * X + (x0 + ox);
-            mu_pre = a.ustat_mean[vo];
-            cyy_pre = a.ustat_cyy[vo];
-        }
-    };
-
-    double acc_m = 0.0, acc_w = 0.0;
-    issue_frame(0);
-    issue_static(f0);
-    issue_stats(f0);
-    for (int it = 0; it < nit; ++it) {
-        const int f = prun > 1 ? f0 : f0 + it;  // frame of this iteration
-        // 1. the warped tile of iteration it (raised wave priority, as in the 3D kernel)
-        __builtin_amdgcn_s_setprio(2);
-#pragma unroll
-        for (int j = 0; j < SPT; ++j) {
-            if (j * kThreads >= NI) break;  // uniform
-            const int i = tid + j * kThreads;
-            float v;
-            if constexpr (SRC3D) v = finish3(pend[j]);
-            else v = finish2(pend[j]);
-            if (i < NI) s_in[g_sin[j]] = v;
-        }
-        __builtin_amdgcn_s_setprio(0);
-        float cur0[PPT], cur1[PPT];
-#pragma unroll
-        for (int j = 0; j < PPT; ++j) {
-            cur0[j] = pre0[j];
-            cur1[j] = pre1[j];
-        }
-        const double mu = mu_pre, cyy = cyy_pre;
-        if (prun == 1 && f + 1 < f1) {  // the next frame's static values (pose runs: the same)
-            issue_static(f + 1);
-            issue_stats(f + 1);
-        }
-        __syncthreads();
-        // 2. |Sobel| and the products
-        if constexpr (MOVI) {
-#pragma unroll
-            for (int jp = 0; jp < PPT / 2; ++jp) {
-                if (jp * kThreads >= NPAIR) break;  // uniform
-                if (tid + jp * kThreads < NPAIR) {
-                    // 3x3 Sobel read from the warped tile: rows ly0 .. ly0 + 3, smooth
-                    // s = (l + 2c) + r and difference d = r - l along x
-                    float sv[4], dv[4], cv[4];
-#pragma unroll
-                    for (int k = 0; k < 4; ++k) {
-                        const float* row = s_in + p_in_ofs[2 * jp] + k * SIS;
-                        const float l = row[0], c = row[1], r = row[2];
-                        dv[k] = r - l;
-                        sv[k] = (l + 2.0f * c) + r;
-                        cv[k] = c;
-                    }
-#pragma unroll
-                    for (int e = 0; e < 2; ++e) {
-                        const float gxv = (dv[e] + 2.0f * dv[e + 1]) + dv[e + 2];
-                        const float gyv = sv[e + 2] - sv[e];
-                        const float G = sqrtf(fmaf(gyv, gyv, gxv * gxv));
-                        store_products<NC>(s_prod, s_cnt, PY * PS, p_prod_ofs[2 * jp + e],
-                                           cv[e + 1], G, cur0[2 * jp + e]);
-                    }
-                }
-            }
-        } else {
-#pragma unroll
-            for (int j = 0; j < PPT; ++j) {
-                if (j * kThreads >= NP) break;  // uniform
-                if (tid + j * kThreads < NP)
-                    store_products<NC>(s_prod, s_cnt, PY * PS, p_prod_ofs[j], cur0[j], cur1[j],
-                                       s_in[p_in_ofs[j]]);
-            }
-        }
-        __syncthreads();  // s_in reads done; products visible
-        // the next iteration's gathers fly during the box sums and the combine
-        if (it + 1 < nit) issue_frame(it + 1);
-        // 3. box sums
-        box_xy_inplace_r<NC, CNT, kThreads, RMAX>(R, s_prod, s_cnt, tid);
-        // 4. combine; each thread adds its pixel's values over the run's frames in order
-        if (out_ok) {
-            const int so = box_row(oy, W) * PS + ox;  // this pixel's sums
-            double S[NC];
-#pragma unroll
-            for (int c = 0; c < NC; ++c) S[c] = s_prod[c * PY * PS + so];
-            double w, meas;
-            bool ok;
-            if (MOVI) ok = combine_static_u(S, mu, cyy, W * W, w, meas);
-            else ok = combine(S, s_cnt[so], W * W, w, meas);
-            if (ok) {
-                acc_m += meas;
-                acc_w += w;
-                if (a.wmap) {
-                    const int vo = f * X * Y + (y0 + oy) * X + (x0 + ox);
-                    a.wmap[vo] = w;
-                    a.mmap[vo] = meas;
-                }
-            }
-        }
-        if (prun > 1) {  // block-uniform: this pose's partial of the tile
-            double* dst = a.partials + ((size_t)(p0 + it) * a.blocks_per_pose + (size_t)run * cols + tcol) * 2;
-            block_reduce_store<kThreads>(acc_m, acc_w, s_red, dst);
-            acc_m = 0.0;
-            acc_w = 0.0;
-        }
-    }
-    if (prun == 1) {
-        double* dst = a.partials + ((size_t)p0 * a.blocks_per_pose + (size_t)run * cols + tcol) * 2;
-        block_reduce_store<kThreads>(acc_m, acc_w, s_red, dst);
-    }
-}
-
-// ---------------------------------------------------------------------------
-// Separable path for patch radii beyond the fused kernels (3D r > kMaxR3, 2D r > kMaxR2):
+// Separable path for patch radii beyond the other kernels (3D r > kMaxRMom3, 2D r > kMaxR2):
 // the reference switches to a global-memory kernel there (cu_lc2_3d.cu:769-827, chosen at
 // :1133-1177). Here, per pose: the moving image is warped (and, if it is the high-resolution
 // one, its |Sobel| taken) into two f32 grids, then the patch sums of every moment channel are
@@ -1049,9 +756,8 @@ __global__ void k_warp_moving(FusedArgs a, int grid3, int src3, float* out) {
     for (long long i = blockIdx.x * (long long)blockDim.x + threadIdx.x; i < n;
          i += (long long)gridDim.x * blockDim.x) {
         const int x = (int)(i % v.X), y = (int)((i / v.X) % v.Y), z = (int)(i / ((long long)v.X * v.Y));
-        const float* mp = a.mats + (size_t)(grid3 ? 0 : (a.mats_per_pose > 1 ? z : 0)) * 12;
         float m[12];
-        for (int k = 0; k < 12; ++k) m[k] = mp[k];
+        load_matrix(a, grid3 ? 0 : (a.mats_per_pose > 1 ? z : 0), m);
         const float lx = fmaf((float)x, v.sx, v.ox), ly = fmaf((float)y, v.sy, v.oy);
         const float lz = grid3 ? fmaf((float)z, v.sz, v.oz) : v.oz;
         out[i] = src3 ? sample3(src, a.s, m, lx, ly, lz) : sample2(src, a.s, m, lx, ly);
@@ -1327,33 +1033,59 @@ __global__ void k_sobel(const float* img, VGeom v, int grid3, float* out) {
     }
 }
 
+__device__ __forceinline__ float raw_value(const void* in, int dtype, long long i) {
+    switch (dtype) {
+        case 0: return (float)static_cast<const unsigned char*>(in)[i];
+        case 1: return (float)static_cast<const short*>(in)[i];
+        case 2: return __half2float(static_cast<const __half*>(in)[i]);
+        default: return static_cast<const float*>(in)[i];
+    }
+}
+
+// 16 bytes of input per thread and step (blocks from hipMalloc are aligned to that); the last
+// elements one by one. Both kernels below read at the memory's rate: k_check 50 MB in 14 us.
+template <typename F>
+__device__ __forceinline__ void for_vectors(long long n, int per, F&& f) {
+    const long long nv = (n + per - 1) / per;
+    for (long long v = blockIdx.x * 256LL + threadIdx.x; v < nv; v += (long long)gridDim.x * 256) f(v * per, min((long long)per, n - v * per));
+}
+
+__global__ __launch_bounds__(256) void k_check(const void* in, int in_dtype, long long n, float lim, int* flag) {
+    bool bad = false;
+    const int per = in_dtype == 3 ? 4 : 8;
+    for_vectors(n, per, [&](long long i0, long long m) {
+        if (m == per) {
+            uint4 w = static_cast<const uint4*>(in)[i0 / per];
+            if (in_dtype == 3) {
+                float x[4];
+                __builtin_memcpy(x, &w, 16);
+#pragma unroll
+                for (int k = 0; k < 4; ++k) bad |= !(fabsf(x[k]) <= lim);
+            } else {
+                short x[8];
+                __builtin_memcpy(x, &w, 16);
+#pragma unroll
+                for (int k = 0; k < 8; ++k) {
+                    __half h;
+                    __builtin_memcpy(&h, &x[k], 2);
+                    bad |= !(fabsf(in_dtype == 1 ? (float)x[k] : __half2float(h)) <= lim);
+                }
+            }
+        } else {
+            for (long long i = i0; i < i0 + m; ++i) bad |= !(fabsf(raw_value(in, in_dtype, i)) <= lim);
+        }
+    });
+    if (__any(bad) && (threadIdx.x & 63) == 0) *flag = 1;
+}
+
 __global__ void k_convert(const void* in, int in_dtype, void* out, int out_f16, long long n) {
     for (long long i = blockIdx.x * (long long)blockDim.x + threadIdx.x; i < n;
          i += (long long)gridDim.x * blockDim.x) {
-        float v;
-        switch (in_dtype) {
-            case 0: v = (float)static_cast<const unsigned char*>(in)[i]; break;
-            case 1: v = (float)static_cast<const short*>(in)[i]; break;
-            case 2: v = __half2float(static_cast<const __half*>(in)[i]); break;
-            default: v = static_cast<const float*>(in)[i]; break;
-        }
+        const float v = raw_value(in, in_dtype, i);
         if (out_f16) static_cast<__half*>(out)[i] = __float2half_rn(v);
         else static_cast<float*>(out)[i] = v;
     }
 }
-
-// The dynamic LDS layout of k_fused2d: nc FP64 products planes (7 for a moving
-// high-resolution image, 9 plus an integer count plane for a moving ultrasound), the
-// reduction scratch and the warped tile.
-constexpr size_t lds_bytes_2d(int r, bool movi) {
-    const size_t nc = movi ? 7 : 9;
-    const size_t PX = kTile2X + 2 * r, PY = kTile2Y + 2 * r, IXE = PX + 2, IYE = PY + 2;
-    const size_t PS = lds_stride_2d((int)PX);
-    const size_t NI = movi ? (32 + PX / 2) * IYE : PX * PY;
-    return sizeof(double) * (nc * PY * PS + 8) + sizeof(float) * NI +
-           (movi ? 0 : sizeof(int) * PY * PS);
-}
-static_assert(lds_bytes_2d(kMaxR2, false) <= 160 * 1024, "2D fused kernel exceeds the 160 KiB of LDS");
 
 // The launch helpers below either launch (occ == nullptr) or report, in *occ, how many
 // work-groups of the kernel they would launch fit on one CU at once.
@@ -1391,51 +1123,6 @@ hipError_t launch3d(const FusedArgs& a, bool movi, dim3 grid, hipStream_t st, in
                      : launch3r<float, false>(a, movi, grid, st, occ);
 }
 
-template <bool MOVI, bool SRC3D, typename T, int RMAX, bool P2>
-hipError_t launch2r(const FusedArgs& a, dim3 grid, hipStream_t st, int* occ) {
-    const size_t lds = lds_bytes_2d(a.r, MOVI);
-    // allow this variant's largest radius, once per process (client threads and a serving
-    // worker may get here at the same time)
-    static std::once_flag once;
-    static hipError_t set_err = hipSuccess;
-    std::call_once(once, [] {
-        set_err = hipFuncSetAttribute(reinterpret_cast<const void*>(&k_fused2d<MOVI, SRC3D, T, RMAX, P2>),
-                                      hipFuncAttributeMaxDynamicSharedMemorySize,
-                                      (int)lds_bytes_2d(RMAX, MOVI));
-    });
-    if (set_err != hipSuccess) return set_err;
-    if (occ) return hipOccupancyMaxActiveBlocksPerMultiprocessor(occ, k_fused2d<MOVI, SRC3D, T, RMAX, P2>,
-                                                                  kThreads, lds);
-    hipLaunchKernelGGL((k_fused2d<MOVI, SRC3D, T, RMAX, P2>), grid, dim3(kThreads), lds, st, a);
-    return hipGetLastError();
-}
-
-// Radius classes of the 2D kernel: fewer registers for the common small patches.
-template <bool MOVI, bool SRC3D, typename T, bool P2>
-hipError_t launch2(const FusedArgs& a, dim3 grid, hipStream_t st, int* occ) {
-    if (a.r <= 3) return launch2r<MOVI, SRC3D, T, 3, P2>(a, grid, st, occ);
-    if (a.r <= 6) return launch2r<MOVI, SRC3D, T, 6, P2>(a, grid, st, occ);
-    return launch2r<MOVI, SRC3D, T, kMaxR2, P2>(a, grid, st, occ);
-}
-
-template <typename T, bool P2>
-hipError_t launch2t(const FusedArgs& a, bool movi, int src_ndim, dim3 grid, hipStream_t st, int* occ) {
-    if (movi)
-        return src_ndim == 3 ? launch2<true, true, T, P2>(a, grid, st, occ)
-                             : launch2<true, false, T, P2>(a, grid, st, occ);
-    return src_ndim == 3 ? launch2<false, true, T, P2>(a, grid, st, occ)
-                         : launch2<false, false, T, P2>(a, grid, st, occ);
-}
-
-hipError_t launch2d(const FusedArgs& a, bool movi, int src_ndim, dim3 grid, hipStream_t st,
-                    int* occ) {
-    if (a.s.pow2)
-        return a.src_f16 ? launch2t<__half, true>(a, movi, src_ndim, grid, st, occ)
-                         : launch2t<float, true>(a, movi, src_ndim, grid, st, occ);
-    return a.src_f16 ? launch2t<__half, false>(a, movi, src_ndim, grid, st, occ)
-                     : launch2t<float, false>(a, movi, src_ndim, grid, st, occ);
-}
-
 }  // namespace
 
 int fused_blocks_3d(const VGeom& v, int r, int zchunk, int* ntx, int* nty, int* nzc) {
@@ -1453,47 +1140,19 @@ int fused_partials_3d(const VGeom& v, int r) {
     return ntx * nty * nzc * (kTile3X * kTile3Y / 64);  // one per wave
 }
 
-int fused_blocks_2d(const VGeom& v, int r, int* ntx, int* nty) {
-    const int ex = v.X - 2 * r, ey = v.Y - 2 * r;
-    if (ex <= 0 || ey <= 0) { *ntx = *nty = 0; return 0; }
-    *ntx = (ex + kTile2X - 1) / kTile2X;
-    *nty = (ey + kTile2Y - 1) / kTile2Y;
-    return *ntx * *nty * v.Z;
-}
-
-int pose_run(const VGeom& v, int grid_ndim, int src_ndim, int mats_per_pose, int tiles,
-             int n_poses) {
-    // runs of poses per work-group while at least about two work-groups per CU slot remain
-    constexpr int kMaxPoseRun = 8;
-    constexpr long long kPoseRunWGs = 2048;
-    if (grid_ndim != 2 || src_ndim != 2 || v.Z != 1 || mats_per_pose != 1) return 1;
-    const long long tiles8 = (tiles + kXcds - 1) / kXcds * (long long)kXcds;
-    return (int)std::max(1LL, std::min<long long>(kMaxPoseRun, tiles8 * n_poses / kPoseRunWGs));
-}
-
-hipError_t launch_fused(const FusedArgs& a, int grid_ndim, int src_ndim, int movi, int n_poses,
-                        hipStream_t st) {
+hipError_t launch_fused(const FusedArgs& a, int movi, int n_poses, hipStream_t st) {
     if (a.tiles == 0 || n_poses <= 0) return hipSuccess;
-    if (grid_ndim == 3 && (a.zchunk <= 0 || a.zchunk % kZBlock != 0)) return hipErrorInvalidValue;
-    if (grid_ndim == 2 && a.zchunk <= 0) return hipErrorInvalidValue;
+    if (a.zchunk <= 0 || a.zchunk % kZBlock != 0) return hipErrorInvalidValue;
     FusedArgs b = a;
     b.npose = n_poses;
     const long long tiles8 = (a.tiles + kXcds - 1) / kXcds * (long long)kXcds;
-    b.prun = pose_run(a.v, grid_ndim, src_ndim, a.mats_per_pose, a.tiles, n_poses);
-    const long long runs = (n_poses + b.prun - 1) / b.prun;
-    if (tiles8 * runs > 0x7fffffffLL) return hipErrorInvalidValue;
-    const dim3 grid((unsigned)(tiles8 * runs));
-    if (grid_ndim == 3) return launch3d(b, movi, grid, st, nullptr);
-    if (b.r < 1 || b.r > kMaxR2) return hipErrorInvalidValue;
-    return launch2d(b, movi, src_ndim, grid, st, nullptr);
+    if (tiles8 * n_poses > 0x7fffffffLL) return hipErrorInvalidValue;
+    return launch3d(b, movi, dim3((unsigned)(tiles8 * n_poses)), st, nullptr);
 }
 
-hipError_t fused_resident_per_cu(const FusedArgs& a, int grid_ndim, int src_ndim, int movi,
-                                 int* per_cu) {
+hipError_t fused_resident_per_cu(const FusedArgs& a, int movi, int* per_cu) {
     *per_cu = 0;
-    if (grid_ndim == 3) return launch3d(a, movi, dim3(1), nullptr, per_cu);
-    if (a.r < 1 || a.r > kMaxR2) return hipErrorInvalidValue;
-    return launch2d(a, movi, src_ndim, dim3(1), nullptr, per_cu);
+    return launch3d(a, movi, dim3(1), nullptr, per_cu);
 }
 
 static dim3 grid_for(long long n) {
@@ -1553,6 +1212,40 @@ hipError_t launch_sep(const FusedArgs& a, int grid_ndim, int src_ndim, int movi,
     }
     (void)V;
     return hipSuccess;
+}
+
+hipError_t launch_warp_grid(const FusedArgs& a, int grid_ndim, int src_ndim, int movi, int n, hipStream_t st) {
+    return grid_ndim == 3 ? launch_warp3(a, movi, n, st) : launch_warp2(a, src_ndim, n, st);
+}
+
+hipError_t launch_moments(const FusedArgs& a, int grid_ndim, int role, int n, hipStream_t st) {
+    if (a.tiles == 0 || n <= 0) return hipSuccess;
+    FusedArgs b = a;
+    b.npose = n;
+    return grid_ndim == 3 ? moments3(b, role, n, st, nullptr) : moments2(b, role, n, st, nullptr);
+}
+
+void moments_tiling(FusedArgs* a, int grid_ndim, int role) {
+    const VGeom& v = a->v;
+    if (grid_ndim == 3) {
+        int tx, ty, blocks;
+        a->tiles = fused_blocks_3d(v, a->r, a->zchunk, &a->ntx, &a->nty, &a->nzc);
+        (void)fused_blocks_3d(v, a->r, kZBlock, &tx, &ty, &blocks);
+        a->blocks_per_pose = tx * ty * blocks * moments3_waves(a->r, role);
+        return;
+    }
+    // k_moments2d: a strip of columns and 32 rows per work-group, fixed runs of kFrameRun frames
+    const int ex = v.X - 2 * a->r, ey = v.Y - 2 * a->r, w = strip_width_2d(a->r, role);
+    a->zchunk = v.Z < kFrameRun ? v.Z : kFrameRun;
+    a->ntx = ex > 0 && ey > 0 ? (ex + w - 1) / w : 0;
+    a->nty = ex > 0 && ey > 0 ? (ey + 31) / 32 : 0;
+    a->nzc = (v.Z + a->zchunk - 1) / a->zchunk;
+    a->tiles = a->blocks_per_pose = a->ntx * a->nty * a->nzc;
+}
+
+hipError_t moments_resident_per_cu(const FusedArgs& a, int grid_ndim, int role, int* per_cu) {
+    *per_cu = 0;
+    return grid_ndim == 3 ? moments3(a, role, 1, nullptr, per_cu) : moments2(a, role, 1, nullptr, per_cu);
 }
 
 hipError_t launch_reduce(const double* partials, int blocks_per_pose, int n_poses, double* out,
@@ -1678,6 +1371,13 @@ hipError_t scratch_address(int device, void** out) {
     addr[device] = ptr;
     *out = ptr;
     return hipSuccess;
+}
+
+hipError_t launch_check(const void* d_in, int in_dtype, long long n, float lim, int* flag, hipStream_t st) {
+    if (in_dtype == 0) return hipSuccess;  // bytes are always in range
+    const long long blocks = std::min<long long>((n / 4 + 255) / 256 + 1, 2048);
+    hipLaunchKernelGGL(k_check, dim3((unsigned)blocks), dim3(256), 0, st, d_in, in_dtype, n, lim, flag);
+    return hipGetLastError();
 }
 
 hipError_t launch_convert(const void* d_in, int in_dtype, void* d_out, int out_f16, long long n,

@@ -8,9 +8,6 @@
 
 namespace lc2e {
 
-constexpr int kTile2X = 16;    // output tile of the 2D fused kernel: kTile2X x kTile2Y,
-constexpr int kTile2Y = 16;    // one thread per output
-constexpr int kThreads = kTile2X * kTile2Y;  // work-group size of the 2D fused kernel
 constexpr int kTile3X = 16;    // output tile of the 3D fused kernel: 16 x 16 columns,
 constexpr int kTile3Y = 16;    // one work-group of 256 threads (two per CU), one column each
 // Resident volumes carry this many zeroed elements past their last voxel: the pipelined
@@ -21,7 +18,8 @@ constexpr long long volume_pad_elems(long long X, long long Y) { return X * Y + 
 constexpr int kMaxR3 = 4;      // largest patch radius of the 3D fused kernel
 constexpr int kZBlock = 8;     // 3D partial sums per block of 8 output planes; z-chunks are multiples
 constexpr int kXcds = 8;       // MI355X: 8 XCDs, each with its own L2, 32 CUs each
-constexpr int kMaxR2 = 10;     // largest patch radius of the 2D fused kernel
+constexpr int kMaxRFused2 = 3; // largest patch radius of the 2D fused kernel
+constexpr int kMaxR2 = 10;     // largest patch radius of the 2D moments kernel
 constexpr int kMaxRSep = 64;   // largest patch radius of the separable path (larger radii)
 constexpr int kFrameRun = 16;  // frames per 2D work-group (frame stacks)
 // The fused kernels' samplers form voxel offsets with 24-bit multiplies: a 3D source whose
@@ -62,6 +60,8 @@ struct FusedArgs {
     const double* ustat_mean;  // static ultrasound: patch mean per voxel
     const double* ustat_cyy;   // static ultrasound: centred patch energy, < 0 where w = 0
     const float* mats;       // [pose][mats_per_pose][12] VirtualToMoving, 3x4 row-major
+    float m0[12];            // the only matrix of the launch, if inline_mat (mats holds it too)
+    int inline_mat;
     double* partials;        // [pose][blocks_per_pose][2] (sum measure, sum w); 3D: the
                              // blocks are [z block of kZBlock planes][tile column][wave]
     double* wmap;            // optional per-voxel w (single pose), may be null
@@ -74,14 +74,26 @@ struct FusedArgs {
     int mats_per_pose;
     int src_f16;             // moving image stored as half
     int npose;               // poses in this launch (set by launch_fused)
-    int prun;                // 2D single images: poses per work-group (0 or 1: one)
+    int prun;                // 2D fused kernel, single images: poses per work-group (0 or 1: one)
     // separable path (patch radii beyond the fused kernels): the moving image and its
     // |Sobel| on the grid (V floats each) and two [channels][V] f64 box-sum buffers
     float* sep_img;
     float* sep_grad;
     double* sep_a;
     double* sep_b;
-    float2* warp2;  // two-kernel path: (I, |Sobel I|) of the moving image per pose and voxel
+    // two-kernel path: the moving image on the grid per pose and voxel, as (I, |Sobel I|) or as
+    // the ultrasound alone (NaN where it is not above the weight's threshold)
+    float2* warp2;
+    float* warp1;
+    // statistics of a static high-resolution image, kImageStats planes of istat_stride doubles
+    // (store_image_stats); *_out: where the statistics roles write
+    const double* istat;
+    double* istat_out;
+    long long istat_stride;
+    double* ustat_mean_out;
+    double* ustat_cyy_out;
+    int in_place;  // 2D moments: warp the moving image in the kernel, without warp2 / warp1
+    int src3;      // the moving image is a volume (in_place)
 };
 
 // Number of work-groups one pose needs (0 if the grid has no valid patch centre).
@@ -89,29 +101,43 @@ int fused_blocks_3d(const VGeom& v, int r, int zchunk, int* ntx, int* nty, int* 
 // Partial sums per pose of the 3D kernel (tile columns x blocks of kZBlock planes x the
 // 4 waves of a work-group).
 int fused_partials_3d(const VGeom& v, int r);
-int fused_blocks_2d(const VGeom& v, int r, int* ntx, int* nty);
 
-hipError_t launch_fused(const FusedArgs& a, int grid_ndim, int src_ndim, int high_res_is_moving,
-                        int n_poses, hipStream_t st);
-// Poses per work-group of the 2D kernel on a single image of a 2D source (1 otherwise):
-// launch_fused runs several poses of one tile in one work-group while the launch keeps
-// enough work-groups.
-int pose_run(const VGeom& v, int grid_ndim, int src_ndim, int mats_per_pose, int tiles,
-             int n_poses);
+hipError_t launch_fused(const FusedArgs& a, int high_res_is_moving, int n_poses, hipStream_t st);
 // Work-groups of the fused kernel a launch with these arguments would use that fit on one
 // CU at once (hipOccupancyMaxActiveBlocksPerMultiprocessor).
-hipError_t fused_resident_per_cu(const FusedArgs& a, int grid_ndim, int src_ndim, int movi,
-                                 int* per_cu);
-// Two-kernel 3D path (moving high-resolution image, r <= kMaxR3): k_warp_grad3 writes the
-// warped image and its |Sobel| into FusedArgs::warp2 (n poses), k_moments3d forms the patch
-// sums and the partials from it, bit for bit as the fused kernel.
-hipError_t launch_warp_grad3(const FusedArgs& a, int n_poses, hipStream_t st);
-hipError_t launch_moments3(const FusedArgs& a, int n_poses, hipStream_t st);
-int moments_partials_3d(const VGeom& v, int r);  // partial sums per pose
-hipError_t moments_resident_per_cu(const FusedArgs& a, int* per_cu);
+hipError_t fused_resident_per_cu(const FusedArgs& a, int movi, int* per_cu);
+// The 2D fused kernel (moving high-resolution image, r <= kMaxRFused2): number of tiles per
+// frame, launch, and poses per work-group on a single image of a 2D source (1 otherwise):
+// launch_fused2 runs several poses of one tile in one work-group while the launch keeps
+// enough work-groups.
+int fused_blocks_2d(const VGeom& v, int r, int* ntx, int* nty);
+hipError_t launch_fused2(const FusedArgs& a, int src_ndim, int n_poses, hipStream_t st);
+int pose_run(const VGeom& v, int src_ndim, int mats_per_pose, int tiles, int n_poses);
+hipError_t fused2_resident_per_cu(const FusedArgs& a, int src_ndim, int* per_cu);
+// Two-kernel path: launch_warp_grid writes the warped moving image of n poses into
+// FusedArgs::warp2 / warp1, launch_moments forms the patch sums of a role from the grids: the
+// partials of n poses (the first two roles), or the statistics of a static image on the grid
+// (n = 1). kRoleStaticImageFull is kRoleStaticImage without the image's statistics in memory
+// (2D, in place). Radii up to kMaxRMom3 (3D) and kMaxR2 (2D).
+enum { kRoleMovingImage, kRoleStaticImage, kRoleImageStats, kRoleUsStats, kRoleStaticImageFull };
+constexpr int kImageStats = 5;  // doubles per voxel
+constexpr int kMaxRMom3 = 6;
+hipError_t launch_warp_grid(const FusedArgs& a, int grid_ndim, int src_ndim, int movi, int n_poses, hipStream_t st);
+hipError_t launch_moments(const FusedArgs& a, int grid_ndim, int role, int n_poses, hipStream_t st);
+// Fills ntx, nty, nzc, tiles, zchunk (2D), blocks_per_pose of a launch; a.v, a.r and, in 3D,
+// a.zchunk must be set.
+void moments_tiling(FusedArgs* a, int grid_ndim, int role);
+hipError_t moments_resident_per_cu(const FusedArgs& a, int grid_ndim, int role, int* per_cu);
+// grid_ndim 3 and 2 of the above
+hipError_t launch_warp3(const FusedArgs& a, int movi, int n_poses, hipStream_t st);
+hipError_t launch_warp2(const FusedArgs& a, int src_ndim, int n_poses, hipStream_t st);
+hipError_t moments3(const FusedArgs& a, int role, int n_poses, hipStream_t st, int* occ);
+hipError_t moments2(const FusedArgs& a, int role, int n_poses, hipStream_t st, int* occ);
+int strip_width_2d(int r, int role);  // output columns of a wave of the 2D moments kernel
+int moments3_waves(int r, int role);  // combining waves: partial sums per tile column and block
 hipError_t launch_reduce(const double* partials, int blocks_per_pose, int n_poses, double* out,
                          hipStream_t st);
-// Separable path for radii beyond the fused kernels (3D r > kMaxR3, 2D r > kMaxR2): per
+// Separable path for radii beyond the other kernels (3D r > kMaxRMom3, 2D r > kMaxR2): per
 // pose, warp (+ |Sobel|), box sums along each axis through sep_a / sep_b, combine; one
 // partial per 256 output voxels (sep_blocks per pose, fixed positions).
 int sep_blocks(const VGeom& v, int r, int grid_ndim);
@@ -145,6 +171,8 @@ constexpr int kMiMaxBins = 256;
 hipError_t launch_mi(const FusedArgs& a, int grid_ndim, int src_ndim, int high_res_is_moving,
                      int n_poses, int bins_u, int bins_i, const float* stat, int* ext_stat,
                      int stat_ready, int* ext_mov, unsigned* hist, double* out, hipStream_t st);
+// Sets *flag if a voxel of d_in exceeds lim in magnitude or is not a number.
+hipError_t launch_check(const void* d_in, int in_dtype, long long n, float lim, int* flag, hipStream_t st);
 // Host bytes -> resident storage (u8/i16/f16/f32 -> f16/f32).
 hipError_t launch_convert(const void* d_in, int in_dtype, void* d_out, int out_f16, long long n,
                           hipStream_t st);

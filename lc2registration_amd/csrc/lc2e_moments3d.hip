@@ -38,9 +38,7 @@ __global__ __launch_bounds__(256) void k_warp_grad3(FusedArgs a, int ntx, int nt
     const T* __restrict__ src = static_cast<const T*>(a.src);
     float m[12];
     {
-        const float* mp = a.mats + (size_t)pose * 12;
-#pragma unroll
-        for (int k = 0; k < 12; ++k) m[k] = mp[k];
+        load_matrix(a, pose, m);
     }
     const int wbase = __builtin_amdgcn_readfirstlane(tid & ~63);
     float cxy[SPT][3];
@@ -126,12 +124,37 @@ __global__ __launch_bounds__(256) void k_warp_grad3(FusedArgs a, int ntx, int nt
     }
 }
 
-// A uniform base plus a 32-bit byte offset per lane (one saddr + voffset access). The empty
-// asm keeps the sum out of the loop optimiser's sight: it would carry a 64-bit pointer per
-// lane for every unrolled step (46 spilled VGPRs at R = 3).
-__device__ __forceinline__ const char* at_bytes(const void* base, unsigned ofs) {
-    asm volatile("" : "+v"(ofs));
-    return static_cast<const char*>(base) + ofs;
+// The moving ultrasound at every grid voxel of a pose, NaN where it is not above the weight's
+// threshold: every sum that holds such a voxel is NaN then, and its patch has no weight (no
+// count of the voxels above the threshold is needed). A thread marches along z with the next
+// plane's gathers in flight.
+template <typename T, bool P2>
+__global__ __launch_bounds__(256) void k_warp_us3(FusedArgs a, int ntx, int nty, int zc, int tiles, int npose) {
+    int tile, pose;
+    if (!map_block(tiles, npose, tile, pose)) return;
+    const int tcol = tile % (ntx * nty), zci = tile / (ntx * nty);
+    const int gx = (tcol % ntx) * 64 + (threadIdx.x & 63), gy = (tcol / ntx) * 4 + (threadIdx.x >> 6);
+    const int X = a.v.X, Y = a.v.Y, Z = a.v.Z;
+    if (gx >= X || gy >= Y) return;
+    const int z0 = zci * zc, z1 = min(z0 + zc, Z);
+    const T* __restrict__ src = static_cast<const T*>(a.src);
+    float m[12];
+    load_matrix(a, pose, m);
+    const float Lx = fmaf((float)gx, a.v.sx, a.v.ox), Ly = fmaf((float)gy, a.v.sy, a.v.oy);
+    const float c[3] = {fmaf(m[1], Ly, m[0] * Lx), fmaf(m[5], Ly, m[4] * Lx), fmaf(m[9], Ly, m[8] * Lx)};
+    float* out = a.warp1 + (size_t)pose * X * Y * Z + (size_t)gy * X + gx;
+    Pending3<T> p[2];
+    auto issue = [&](int z, Pending3<T>& q) { issue3c<P2>(src, a.s, m, c, fmaf((float)z, a.v.sz, a.v.oz), true, q); };
+    issue(z0, p[0]);
+    issue(min(z0 + 1, z1 - 1), p[1]);
+    for (int z = z0; z < z1; z += 2) {
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+            const float v = finish3(p[e]);
+            if (z + e < z1) out[(size_t)(z + e) * X * Y] = (double)v > kZeroThreshold ? v : NAN;
+            issue(min(z + e + 2, z1 - 1), p[e]);
+        }
+    }
 }
 
 // ---------------------------------------------------------------------------
@@ -153,8 +176,9 @@ __device__ __forceinline__ const char* at_bytes(const void* base, unsigned ofs) 
 // Raised priorities for the x or the y waves: 1 to 8% slower.
 // ---------------------------------------------------------------------------
 // Planes a pipeline step carries: two where three buffers of them fit the LDS.
-template <int R, int NC>
+template <int R, int ROLE>
 struct Mom {
+    static constexpr int NC = Role<ROLE>::NC;
     static constexpr int W = 2 * R + 1, PX = kTile3X + 2 * R, PY = kTile3Y + 2 * R, NP = PX * PY;
     static constexpr int PS = lds_stride(PX), PL = PY * PS;  // LDS row stride, plane size
     static constexpr int KP = 3 * 2 * NC * PL * 8 <= 160 * 1024 ? 2 : 1;
@@ -177,10 +201,11 @@ __device__ __forceinline__ void window2(const double (&in)[W + 1], double& o0, d
     o1 = mid + in[W];
 }
 
-template <int R>
-__global__ __launch_bounds__((Mom<R, 7>::NTHR)) void k_moments3d(FusedArgs a) {
-    constexpr int NC = 7;
-    using M = Mom<R, NC>;
+template <int R, int ROLE>
+__global__ __launch_bounds__((Mom<R, ROLE>::NTHR)) void k_moments3d(FusedArgs a) {
+    using M = Mom<R, ROLE>;
+    using Ro = Role<ROLE>;
+    constexpr int NC = M::NC;
     constexpr int TX = kTile3X, TY = kTile3Y, W = M::W, PX = M::PX, PY = M::PY, NP = M::NP, PS = M::PS,
                   PL = M::PL, KP = M::KP, BUF = M::BUF, N3 = W * W * W;
     extern __shared__ __align__(16) double s_buf[];
@@ -211,15 +236,26 @@ __global__ __launch_bounds__((Mom<R, 7>::NTHR)) void k_moments3d(FusedArgs a) {
             g_ofs[e] = (unsigned)(min(y0 - R + ly, Y - 1) * X + min(x0 - R + lx, X - 1)) * 4u;
         }
         const float2* __restrict__ ig = a.warp2 + (size_t)pose * Z * XY;
-        float2 vi[K][ZP];
-        float vu[K][ZP];
+        const float* __restrict__ wu = a.warp1 + (size_t)pose * Z * XY;
+        float vi[K][ZP], vg[K][ZP], vu[K][ZP];  // the inputs the role has
         auto load = [&](auto slot_c, int z) {
             constexpr int k = decltype(slot_c)::value;
             const size_t zo = (size_t)min(z, Z - 1) * XY;
 #pragma unroll
             for (int e = 0; e < ZP; ++e) {
-                __builtin_memcpy(&vi[k][e], at_bytes(ig + zo, g_ofs[e] * 2u), 8);
-                __builtin_memcpy(&vu[k][e], at_bytes(a.stat_img + zo, g_ofs[e]), 4);
+                if constexpr (ROLE == kRoleMovingImage) {
+                    const float2 v = load_at(ig + zo, g_ofs[e] * 2u);
+                    vi[k][e] = v.x;
+                    vg[k][e] = v.y;
+                    vu[k][e] = load_at(a.stat_img + zo, g_ofs[e]);
+                } else {
+                    if constexpr (Ro::HAS_I) {
+                        vi[k][e] = load_at(a.stat_img + zo, g_ofs[e]);
+                        vg[k][e] = load_at(a.stat_grad + zo, g_ofs[e]);
+                    }
+                    if constexpr (ROLE == kRoleStaticImage) vu[k][e] = load_at(wu + zo, g_ofs[e]);
+                    if constexpr (ROLE == kRoleUsStats) vu[k][e] = load_at(a.stat_img + zo, g_ofs[e]);
+                }
             }
         };
         Unroll<0, K>::run([&](auto kc) { load(kc, z0 - R + decltype(kc)::value); });
@@ -233,28 +269,24 @@ __global__ __launch_bounds__((Mom<R, 7>::NTHR)) void k_moments3d(FusedArgs a) {
 #pragma unroll
                 for (int e = 0; e < ZP; ++e) {
                     auto add = [&](double (&t)[NC], int j) {
-                        const double I = vi[(2 * k + j) % K][e].x, G = vi[(2 * k + j) % K][e].y,
-                                     U = vu[(2 * k + j) % K][e];
-                        t[0] += I;
-                        t[1] += G;
-                        t[2] = fma(I, I, t[2]);  // products of two floats are exact in FP64
-                        t[3] = fma(G, G, t[3]);
-                        t[4] = fma(I, G, t[4]);
-                        t[5] = fma(U, I, t[5]);
-                        t[6] = fma(U, G, t[6]);
+                        const int i = (2 * k + j) % K;
+                        float I = 0.f, G = 0.f, U = 0.f;
+                        if constexpr (Ro::HAS_I) I = vi[i][e], G = vg[i][e];
+                        if constexpr (Ro::HAS_U) U = vu[i][e];
+                        if constexpr (ROLE == kRoleUsStats) U = (double)U > kZeroThreshold ? U : NAN;
+                        Ro::add(t, I, G, U);
                     };
                     // the ring stays in floats: without this the compiler keeps each plane's
                     // FP64 values from step to step as well, and spills
 #pragma unroll
-                    for (int j = 0; j < K; ++j) asm volatile("" : "+v"(vi[j][e].x), "+v"(vi[j][e].y), "+v"(vu[j][e]));
-                    {
-                        const double I = vi[(2 * k + 1) % K][e].x, G = vi[(2 * k + 1) % K][e].y,
-                                     U = vu[(2 * k + 1) % K][e];
-                        s[e][0] = I; s[e][1] = G; s[e][2] = I * I; s[e][3] = G * G; s[e][4] = I * G;
-                        s[e][5] = U * I; s[e][6] = U * G;
+                    for (int j = 0; j < K; ++j) {
+                        if constexpr (Ro::HAS_I) asm volatile("" : "+v"(vi[j][e]), "+v"(vg[j][e]));
+                        if constexpr (Ro::HAS_U) asm volatile("" : "+v"(vu[j][e]));
                     }
 #pragma unroll
-                    for (int j = 2; j < W; ++j) add(s[e], j);
+                    for (int c = 0; c < NC; ++c) s[e][c] = 0.0;
+#pragma unroll
+                    for (int j = 1; j < W; ++j) add(s[e], j);
                     double t[NC];
 #pragma unroll
                     for (int c = 0; c < NC; ++c) t[c] = s[e][c];
@@ -310,16 +342,26 @@ __global__ __launch_bounds__((Mom<R, 7>::NTHR)) void k_moments3d(FusedArgs a) {
     const unsigned vo0 = ok0 ? (unsigned)((y0 + oy) * X + (x0 + ox)) * 8u : 0u;
     const unsigned vo1 = ok1 ? vo0 + (unsigned)X * 8u : 0u;
     double mu[2], cyy[2];
+    ImageStats ist[2];
     auto stats = [&](int zo) {
         const size_t zp = (size_t)min(zo, zend - 1) * XY;
-        __builtin_memcpy(&mu[0], at_bytes(a.ustat_mean + zp, vo0), 8);
-        __builtin_memcpy(&cyy[0], at_bytes(a.ustat_cyy + zp, vo0), 8);
-        __builtin_memcpy(&mu[1], at_bytes(a.ustat_mean + zp, vo1), 8);
-        __builtin_memcpy(&cyy[1], at_bytes(a.ustat_cyy + zp, vo1), 8);
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+            const unsigned vo = j ? vo1 : vo0;
+            if constexpr (ROLE == kRoleMovingImage) {
+                mu[j] = load_at(a.ustat_mean + zp, vo);
+                cyy[j] = load_at(a.ustat_cyy + zp, vo);
+            }
+            if constexpr (ROLE == kRoleStaticImage) {
+                const double* st = a.istat + zp;
+                ist[j] = {load_at(st, vo), load_at(st + a.istat_stride, vo), load_at(st + 2 * a.istat_stride, vo),
+                          load_at(st + 3 * a.istat_stride, vo), load_at(st + 4 * a.istat_stride, vo)};
+            }
+        }
     };
     double acc_m = 0.0, acc_w = 0.0;
     __syncthreads();
-    stats(z0 + plane);
+    if constexpr (Ro::SUMS) stats(z0 + plane);
     __syncthreads();
     int buf = 0;
     for (int s = 0; s < n; ++s) {
@@ -345,25 +387,42 @@ __global__ __launch_bounds__((Mom<R, 7>::NTHR)) void k_moments3d(FusedArgs a) {
             asm volatile("" : "+v"(S[0][c]), "+v"(S[1][c]));
             if (c % 2 == 1) __builtin_amdgcn_sched_barrier(0);
         }
-        const double m0[2] = {mu[0], mu[1]}, c0[2] = {ok0 && zok ? cyy[0] : -1.0, ok1 && zok ? cyy[1] : -1.0};
-        stats(zo + KP);
+        double m0[2], c0[2];
+        ImageStats i0[2];
 #pragma unroll
         for (int j = 0; j < 2; ++j) {
-            double w, meas;
-            const bool ok = c0[j] >= 0.0;
-            combine_static_u_any(S[j], m0[j], ok ? c0[j] : 1.0, N3, w, meas);
-            acc_m += ok ? meas : 0.0;
-            acc_w += ok ? w : 0.0;
-            if (a.wmap && ok) {
-                const size_t vo = (size_t)zo * XY + (size_t)(y0 + oy + j) * X + (x0 + ox);
-                a.wmap[vo] = w;
-                a.mmap[vo] = meas;
+            if constexpr (ROLE == kRoleMovingImage) m0[j] = mu[j], c0[j] = cyy[j];
+            if constexpr (ROLE == kRoleStaticImage) i0[j] = ist[j];
+        }
+        if constexpr (Ro::SUMS) stats(zo + KP);
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+            const bool in = (j ? ok1 : ok0) && zok;
+            const size_t vo = (size_t)zo * XY + (size_t)(y0 + oy + j) * X + (x0 + ox);
+            if constexpr (Ro::SUMS) {
+                double w, meas;
+                bool ok;
+                if constexpr (ROLE == kRoleMovingImage) {
+                    ok = in && c0[j] >= 0.0;
+                    combine_static_u_any(S[j], m0[j], ok ? c0[j] : 1.0, N3, w, meas);
+                } else {
+                    ok = combine_static_image(S[j], i0[j], N3, w, meas) && in;
+                }
+                acc_m += ok ? meas : 0.0;
+                acc_w += ok ? w : 0.0;
+                if (a.wmap && ok) {
+                    a.wmap[vo] = w;
+                    a.mmap[vo] = meas;
+                }
+            } else if (in) {
+                if constexpr (ROLE == kRoleImageStats) store_image_stats(S[j], N3, a.istat_out + vo, a.istat_stride);
+                else store_us_stats(S[j], N3, a.ustat_mean_out + vo, a.ustat_cyy_out + vo);
             }
         }
         // partials per block of kZBlock output planes, tile column and combining wave, at
         // fixed positions in z
         const int ze = z0 + (s + 1) * KP;
-        if ((ze - R) % kZBlock == 0 || ze >= zend) {
+        if (Ro::SUMS && ((ze - R) % kZBlock == 0 || ze >= zend)) {
             wave_reduce_store(acc_m, acc_w,
                               a.partials + (((size_t)pose * a.blocks_per_pose +
                                              ((size_t)((ze - 1 - R) / kZBlock) * cols + tcol) * M::YW + rank) * 2));
@@ -382,72 +441,79 @@ void warp_grad3(const FusedArgs& a, int ntx, int nty, int zc, int tiles, int n, 
                        zc, tiles, n);
 }
 
-template <int R>
-hipError_t moments3(const FusedArgs& a, dim3 grid, hipStream_t st, int* occ) {
-    using M = Mom<R, 7>;
+template <typename T, bool P2>
+void warp_us3(const FusedArgs& a, int ntx, int nty, int zc, int tiles, int n, hipStream_t st) {
+    const int tiles8 = (tiles + kXcds - 1) / kXcds * kXcds;
+    hipLaunchKernelGGL((k_warp_us3<T, P2>), dim3((unsigned)tiles8 * n), dim3(256), 0, st, a, ntx, nty, zc, tiles, n);
+}
+
+template <int R, int ROLE>
+hipError_t moments3k(const FusedArgs& a, dim3 grid, hipStream_t st, int* occ) {
+    using M = Mom<R, ROLE>;
     static std::once_flag once;
     static hipError_t err = hipSuccess;
     std::call_once(once, [] {
-        err = hipFuncSetAttribute(reinterpret_cast<const void*>(&k_moments3d<R>),
+        err = hipFuncSetAttribute(reinterpret_cast<const void*>(&k_moments3d<R, ROLE>),
                                   hipFuncAttributeMaxDynamicSharedMemorySize, (int)M::lds);
     });
     if (err != hipSuccess) return err;
-    if (occ) return hipOccupancyMaxActiveBlocksPerMultiprocessor(occ, k_moments3d<R>, M::NTHR, M::lds);
-    hipLaunchKernelGGL((k_moments3d<R>), grid, dim3(M::NTHR), M::lds, st, a);
+    if (occ) return hipOccupancyMaxActiveBlocksPerMultiprocessor(occ, k_moments3d<R, ROLE>, M::NTHR, M::lds);
+    hipLaunchKernelGGL((k_moments3d<R, ROLE>), grid, dim3(M::NTHR), M::lds, st, a);
     return hipGetLastError();
 }
 
+template <int ROLE, int R = 1>
 hipError_t moments3r(const FusedArgs& a, dim3 grid, hipStream_t st, int* occ) {
-    switch (a.r) {
-        case 1: return moments3<1>(a, grid, st, occ);
-        case 2: return moments3<2>(a, grid, st, occ);
-        case 3: return moments3<3>(a, grid, st, occ);
-        case 4: return moments3<4>(a, grid, st, occ);
-        case 5: return moments3<5>(a, grid, st, occ);
-        case 6: return moments3<6>(a, grid, st, occ);
-        default: return hipErrorInvalidValue;
-    }
+    if (a.r == R) return moments3k<R, ROLE>(a, grid, st, occ);
+    if constexpr (R < kMaxRMom3) return moments3r<ROLE, R + 1>(a, grid, st, occ);
+    return hipErrorInvalidValue;
+}
+template <int ROLE, int R = 1>
+int waves3r(int r) {
+    if (r == R) return Mom<R, ROLE>::YW;
+    if constexpr (R < kMaxRMom3) return waves3r<ROLE, R + 1>(r);
+    return 0;
 }
 
 }  // namespace
 
-hipError_t launch_warp_grad3(const FusedArgs& a, int n, hipStream_t st) {
-    const int ntx = (a.v.X + kGradX - 1) / kGradX, nty = (a.v.Y + kGradY - 1) / kGradY;
+hipError_t launch_warp3(const FusedArgs& a, int movi, int n, hipStream_t st) {
+    const int tx = movi ? kGradX : 64, ty = movi ? kGradY : 4;
+    const int ntx = (a.v.X + tx - 1) / tx, nty = (a.v.Y + ty - 1) / ty;
     // z-chunks: about 2048 work-groups (the CUs hold about that many), at least 8 planes each
-    // (two more are warped per chunk)
+    // (with the Sobel, two more are warped per chunk)
     const int want = (int)std::max(1LL, 2048LL / ((long long)ntx * nty * n));
     const int zc = std::max(8, (a.v.Z + want - 1) / want);
     const int tiles = ntx * nty * ((a.v.Z + zc - 1) / zc);
-    if (a.s.pow2) {
-        if (a.src_f16) warp_grad3<__half, true>(a, ntx, nty, zc, tiles, n, st);
-        else warp_grad3<float, true>(a, ntx, nty, zc, tiles, n, st);
-    } else {
-        if (a.src_f16) warp_grad3<__half, false>(a, ntx, nty, zc, tiles, n, st);
-        else warp_grad3<float, false>(a, ntx, nty, zc, tiles, n, st);
+    const int form = (movi ? 4 : 0) + (a.s.pow2 ? 2 : 0) + (a.src_f16 ? 1 : 0);
+    switch (form) {
+        case 7: warp_grad3<__half, true>(a, ntx, nty, zc, tiles, n, st); break;
+        case 6: warp_grad3<float, true>(a, ntx, nty, zc, tiles, n, st); break;
+        case 5: warp_grad3<__half, false>(a, ntx, nty, zc, tiles, n, st); break;
+        case 4: warp_grad3<float, false>(a, ntx, nty, zc, tiles, n, st); break;
+        case 3: warp_us3<__half, true>(a, ntx, nty, zc, tiles, n, st); break;
+        case 2: warp_us3<float, true>(a, ntx, nty, zc, tiles, n, st); break;
+        case 1: warp_us3<__half, false>(a, ntx, nty, zc, tiles, n, st); break;
+        default: warp_us3<float, false>(a, ntx, nty, zc, tiles, n, st); break;
     }
     return hipGetLastError();
 }
 
-int moments_partials_3d(const VGeom& v, int r) {
-    int ntx, nty, nzc;
-    if (fused_blocks_3d(v, r, kZBlock, &ntx, &nty, &nzc) <= 0) return 0;
-    const int yw = r == 1 ? Mom<1, 7>::YW : r == 2 ? Mom<2, 7>::YW : r == 3 ? Mom<3, 7>::YW : 2;
-    return ntx * nty * nzc * yw;
-}
-
-hipError_t launch_moments3(const FusedArgs& a, int n, hipStream_t st) {
-    if (a.tiles == 0 || n <= 0) return hipSuccess;
-    if (a.zchunk <= 0 || a.zchunk % kZBlock != 0) return hipErrorInvalidValue;
-    FusedArgs b = a;
-    b.npose = n;
+hipError_t moments3(const FusedArgs& a, int role, int n, hipStream_t st, int* occ) {
+    if (!occ && (a.zchunk <= 0 || a.zchunk % kZBlock != 0)) return hipErrorInvalidValue;
     const long long tiles8 = (a.tiles + kXcds - 1) / kXcds * (long long)kXcds;
     if (tiles8 * n > 0x7fffffffLL) return hipErrorInvalidValue;
-    return moments3r(b, dim3((unsigned)(tiles8 * n)), st, nullptr);
+    const dim3 grid((unsigned)(tiles8 * n));
+    switch (role) {
+        case kRoleMovingImage: return moments3r<kRoleMovingImage>(a, grid, st, occ);
+        case kRoleStaticImage: return moments3r<kRoleStaticImage>(a, grid, st, occ);
+        case kRoleImageStats: return moments3r<kRoleImageStats>(a, grid, st, occ);
+        default: return moments3r<kRoleUsStats>(a, grid, st, occ);
+    }
 }
 
-hipError_t moments_resident_per_cu(const FusedArgs& a, int* per_cu) {
-    *per_cu = 0;
-    return moments3r(a, dim3(1), nullptr, per_cu);
+int moments3_waves(int r, int role) {
+    return role == kRoleMovingImage ? waves3r<kRoleMovingImage>(r) : waves3r<kRoleStaticImage>(r);
 }
 
 }  // namespace lc2e

@@ -605,3 +605,114 @@ def test_3d_two_kernel_path_equals_fused_and_oracle(engine, r, dims):
     assert np.allclose(got[0].lc2, got[1].lc2, rtol=1e-10, atol=0)
     assert np.allclose(got[0].sum_w, got[1].sum_w, rtol=1e-10, atol=0)
     budgeted.close()
+
+
+def _random_pair(fixed_dims, moving_dims, r, high_res_is_moving, ndim, seed, spacing=0.9):
+    """Two noisy images (speckled uint8 ultrasound with an empty corner, float32 image)."""
+    rng = np.random.default_rng(seed)
+
+    def image(dims, us):
+        a = rng.random(tuple(reversed(dims))) + np.linspace(0, 1, dims[0])
+        if us:
+            a[..., :2, :3] = 0.0
+            return np.clip(a * 100, 0, 255).astype(np.uint8)
+        return a.astype(np.float32)
+
+    n = len(fixed_dims)
+    f = synth.Image(image(fixed_dims, high_res_is_moving), fixed_dims, (1.0,) * n, (0.0,) * n)
+    m = synth.Image(image(moving_dims, not high_res_is_moving), moving_dims, (spacing,) * n, (-3.0,) * n)
+    pose = np.r_[0.4, -0.6, 1.5, 1.01, 0.99, 0.0] if ndim == 2 else \
+        np.r_[0.4, -0.6, 0.3, 1.0, -1.5, 0.7, 1.01, 0.99, 1.0, 0.0, 0.01, 0.0]
+    return synth.Workload("random", f, m, (1.0,) * n, r, high_res_is_moving, False, ndim, pose)
+
+
+@pytest.mark.parametrize("movi,r,dims", [
+    (False, 1, (3, 3)), (False, 1, (64, 34)), (False, 2, (65, 13)), (False, 3, (65, 39)),
+    (False, 4, (121, 16)), (False, 7, (63, 47)), (False, 9, (64, 27)), (False, 10, (66, 21)),
+    (True, 4, (9, 9)), (True, 4, (63, 40)), (True, 5, (115, 18)), (True, 6, (64, 45)),
+    (True, 8, (62, 49)), (True, 10, (85, 29))])
+def test_2d_strips_equal_oracle_batch_and_budget(engine, movi, r, dims):
+    """The 2D moments kernel at the edges of its strips (64 - 2r columns, 62 - 2r with the moving
+    image as the high-resolution one) and row groups (8 and 32 rows): the oracle's LC2 and maps;
+    a batch large enough to go through the warped grid and one under a budget (warped in place,
+    image statistics formed in the kernel) give single evaluations bit for bit."""
+    print(f"2D strips: movi {movi}, r {r}, grid {dims}", flush=True)
+    w = _random_pair(dims, (dims[0] + 12, dims[1] + 9), r, movi, 2, r)
+    rng = np.random.default_rng(r)
+    p = _pair_for(engine, w, r=r)
+    n = 1 + 2048 // (4 * ((dims[0] - 2 * r) // 60 + 1) * ((dims[1] - 2 * r) // 32 + 1))
+    mats = np.stack([p.pose_to_matrix(w.true_pose)] +
+                    [p.pose_to_matrix(synth.perturb(w.true_pose, rng, 2)) for _ in range(n)])
+    batch = p.eval_batch(mats)
+    few = [0, 1, n]
+    for k in few:
+        res, _, _, _, wm, mm = _oracle_eval(w, mats[k], r=r, maps=True)
+        assert abs(batch.lc2[k] - res.lc2) < LC2_TOL, k
+        assert p.eval(mats[k]) == batch.lc2[k]
+        gw = p.debug_fetch(E.STAGE_W, mats[k])[0]
+        assert np.array_equal(gw > 0, wm > 0)
+        assert np.allclose(gw, wm, rtol=1e-9, atol=1e-12)
+        assert np.allclose(p.debug_fetch(E.STAGE_MEASURE, mats[k])[0], mm, rtol=1e-7, atol=1e-9)
+    p.close()
+    budgeted = E.Engine(0, hbm_budget=64 << 20)
+    p = _pair_for(budgeted, w, r=r)
+    b = p.eval_batch(mats[few])
+    assert np.array_equal(b.lc2, batch.lc2[few]) and np.array_equal(b.sum_w, batch.sum_w[few])
+    p.close()
+    budgeted.close()
+
+
+@pytest.mark.parametrize("movi,r,dims", [
+    (False, 1, (18, 19, 5)), (False, 2, (37, 20, 12)), (False, 3, (39, 23, 18)), (False, 4, (25, 41, 10)),
+    (False, 5, (27, 28, 12)), (False, 6, (29, 45, 14)), (True, 5, (28, 27, 11)), (True, 6, (46, 29, 21))])
+def test_3d_moments_roles_equal_oracle(engine, movi, r, dims):
+    """The 3D moments kernel with the static image as the high-resolution one, and at radii 5 and
+    6 in both roles, on ragged grids: the oracle's LC2 and maps, the same bits in a batch, with
+    short z-chunks and in single calls, and the fused kernel's value to rounding (radius up to 4;
+    an engine with a budget)."""
+    print(f"3D moments: movi {movi}, r {r}, grid {dims}", flush=True)
+    w = _random_pair(dims, tuple(d + 9 for d in dims), r, movi, 3, r, 0.8)
+    rng = np.random.default_rng(r)
+    p = _pair_for(engine, w, r=r)
+    mats = np.stack([p.pose_to_matrix(w.true_pose)] +
+                    [p.pose_to_matrix(synth.perturb(w.true_pose, rng, 3)) for _ in range(3)])
+    batch = p.eval_batch(mats)
+    res, _, _, _, wm, mm = _oracle_eval(w, mats[0], r=r, maps=True)
+    assert abs(batch.lc2[0] - res.lc2) < LC2_TOL
+    gw = p.debug_fetch(E.STAGE_W, mats[0])
+    assert np.array_equal(gw > 0, wm > 0)
+    assert np.allclose(gw, wm, rtol=1e-9, atol=1e-12)
+    assert np.allclose(p.debug_fetch(E.STAGE_MEASURE, mats[0]), mm, rtol=1e-7, atol=1e-9)
+    for k in range(len(mats)):
+        assert p.eval(mats[k]) == batch.lc2[k]
+    p.set_tuning(8)
+    assert np.array_equal(p.eval_batch(mats).lc2, batch.lc2)
+    assert np.array_equal(p.eval_batch_noalloc(mats).lc2, batch.lc2)
+    p.close()
+    budgeted = E.Engine(0, hbm_budget=256 << 20)
+    p = _pair_for(budgeted, w, r=r)
+    assert np.allclose(p.eval_batch(mats).lc2, batch.lc2, rtol=1e-10, atol=0)
+    p.close()
+    budgeted.close()
+
+
+@pytest.mark.parametrize("n,at", [(1, 0), (7, 6), (4096, 0), (100003, 100002), (100003, 99999)])
+def test_upload_finds_the_voxel_out_of_range(engine, n, at):
+    """The range check on the device: a NaN, an infinity or a value past half storage's range, at
+    either end and past the last whole vector, is refused with its index; int16 data leave half
+    storage exactly where a value exceeds 2048."""
+    geom = dict(spacing=(1.0, 1.0, 1.0), origin=(0.0, 0.0, 0.0))
+    for dtype, bad, storage in ((np.float32, np.nan, E.STORE_AUTO), (np.float32, -np.inf, E.F32),
+                                (np.float32, 65520.0, E.F16), (np.float16, np.inf, E.F16)):
+        a = np.ones((1, 1, n), dtype)
+        a[0, 0, at] = bad
+        with pytest.raises(E.LC2Error) as ei:
+            engine.upload(a, storage=storage, **geom)
+        assert ei.value.code == -1 and f" at {at} " in str(ei.value)
+    for value, size in ((2048, 2), (-2049, 4)):
+        used = engine.memory()[0]
+        a = np.zeros((1, 1, n), np.int16)
+        a[0, 0, at] = value
+        v = engine.upload(a, **geom)
+        assert (engine.memory()[0] - used) == (n + n + n + 64) * size
+        v.close()
