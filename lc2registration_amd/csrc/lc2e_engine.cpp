@@ -233,6 +233,8 @@ struct lc2e_pair {
     int* mi_ext = nullptr;
     unsigned* mi_hist = nullptr;
     double* mi_out = nullptr;
+    float* mi_warp = nullptr;  // warped images of mi_warp_poses poses
+    int mi_warp_poses = 0;
     // two-kernel path: the warped moving image of ws_poses poses (ws_bytes each) and, if the
     // static image is the high-resolution one, its statistics; kept with the pair (see
     // make_two_kernel)
@@ -466,6 +468,12 @@ void free_batch(lc2e_pair* p) {
     p->part_bpp = 0;
 }
 
+void free_mi_warp(lc2e_pair* p) {
+    if (p->mi_warp) p->e->raw_free(p->mi_warp, (size_t)p->mi_warp_poses * p->voxels() * sizeof(float));
+    p->mi_warp = nullptr;
+    p->mi_warp_poses = 0;
+}
+
 void free_mi(lc2e_pair* p) {
     lc2e_engine* e = p->e;
     if (p->mi_ext) e->release(p->mi_ext, (size_t)p->mi_cap * 2 * sizeof(int));
@@ -494,6 +502,7 @@ void two_free(lc2e_pair* p, void* d, size_t bytes) {
 // The workspace for n poses, up to kWorkspaceBytes (at least one pose); larger launches go
 // through it in parts. Only an engine without an HBM budget grows it past one pose.
 constexpr size_t kWorkspaceBytes = size_t(1) << 30;
+constexpr size_t kMiWarpBytes = size_t(1) << 28;  // warped images of the mutual information
 int grow_workspace(lc2e_pair* p, int n) {
     if (p->e->budget) {
         if (!p->two_charged) return LC2E_OK;
@@ -563,9 +572,8 @@ int make_two_kernel(lc2e_pair* p, bool required) {
 }
 
 // Batch buffers for n poses whose launches use up to bpp work-groups per pose.
-int ensure_capacity(lc2e_pair* p, int n, int bpp) {
+int ensure_batch(lc2e_pair* p, int n, int bpp) {
     if (bpp < 1) bpp = 1;
-    if (p->ws) (void)grow_workspace(p, n);
     if (n <= p->cap && bpp <= p->part_bpp) return LC2E_OK;
     int cap = p->cap > 1 ? p->cap : 1;
     while (cap < n) cap *= 2;
@@ -614,6 +622,12 @@ int ensure_capacity(lc2e_pair* p, int n, int bpp) {
                     hipGetErrorString(he));
     }
     return LC2E_OK;
+}
+
+// The same, and the workspace.
+int ensure_capacity(lc2e_pair* p, int n, int bpp) {
+    if (p->ws) (void)grow_workspace(p, n);
+    return ensure_batch(p, n, bpp);
 }
 
 lc2e::FusedArgs make_args(lc2e_pair* p, const float* d_mats, double* d_partials, const Tiling& t) {
@@ -1075,6 +1089,7 @@ void lc2e_pair_destroy(lc2e_pair* p) {
     (void)hipStreamSynchronize(p->e->stream);
     free_batch(p);
     free_mi(p);
+    free_mi_warp(p);
     if (p->mi_ext_stat) p->e->release(p->mi_ext_stat, 2 * sizeof(int));
     if (p->ev0) (void)hipEventDestroy(p->ev0);
     if (p->ev1) (void)hipEventDestroy(p->ev1);
@@ -1223,17 +1238,32 @@ int lc2e_eval_mi_batch(lc2e_pair* p, int n, const float* mats, int bins_us, int 
     lc2e_engine* e = p->e;
     hipStream_t st = e->stream;
     const int mpp = p->mats_per_pose();
-    const size_t nb = (size_t)bins_us * bins_hr;
+    const size_t nb = (size_t)lc2e::mi_hist_size(bins_us, bins_hr);
     int rc;
     if (!p->mi_ext_stat) {
         if ((rc = e->alloc((void**)&p->mi_ext_stat, 2 * sizeof(int))) < 0) return rc;
         p->mi_stat_ready = false;
     }
     const int chunk_max = 64;
-    for (int base = 0; base < n; base += chunk_max) {
-        const int m = (n - base) < chunk_max ? (n - base) : chunk_max;
-        const Tiling t = tiling_for(p, m);
-        if ((rc = ensure_capacity(p, m, t.bpp)) < 0) return rc;
+    const Tiling t = tiling_for(p, 1);
+    // Without a budget the warped image is kept between the two passes over it (3D), a float per
+    // voxel and pose; what does not fit goes in parts. A buffer of its own: evaluations on a
+    // caller's stream may be using the pair's workspace.
+    // (Sources of large slices are beyond the pipelined sampler's offsets: warped twice.)
+    int step = std::min(n, chunk_max);
+    if (!e->budget && p->info.grid_ndim == 3 && (long long)p->sg.X * p->sg.Y < lc2e::kMaxFusedSlice) {
+        const size_t per = p->voxels() * sizeof(float);
+        const int want = (int)std::min<size_t>((size_t)step, std::max<size_t>(1, kMiWarpBytes / per));
+        if (want > p->mi_warp_poses) {
+            free_mi_warp(p);
+            if (e->raw_alloc((void**)&p->mi_warp, (size_t)want * per) == hipSuccess) p->mi_warp_poses = want;
+            else (void)hipGetLastError(), p->mi_warp = nullptr;
+        }
+        if (p->mi_warp) step = std::min(step, p->mi_warp_poses);
+    }
+    for (int base = 0; base < n; base += step) {
+        const int m = (n - base) < step ? (n - base) : step;
+        if ((rc = ensure_batch(p, m, t.bpp)) < 0) return rc;
         if (m > p->mi_cap || nb != p->mi_bins) {
             free_mi(p);
             const int cap = m > 8 ? chunk_max : 8;
@@ -1250,6 +1280,7 @@ int lc2e_eval_mi_batch(lc2e_pair* p, int n, const float* mats, int bins_us, int 
         HIP_TRY(hipMemcpyAsync(p->d_mats, p->h_mats, (size_t)m * mpp * 12 * sizeof(float),
                                hipMemcpyHostToDevice, st));
         lc2e::FusedArgs a = make_args(p, p->d_mats, p->d_partials, t);
+        a.warp1 = p->mi_warp;
         // the static image is U when the moving image is the high-resolution one
         const int us_static = p->info.high_res_is_moving;
         HIP_TRY(lc2e::launch_mi(a, p->info.grid_ndim, p->info.src_ndim, us_static, m, bins_us,

@@ -165,9 +165,13 @@ hipError_t launch_sobel(const float* img, const VGeom& v, int grid_ndim, float* 
                         hipStream_t st);
 // Normalized mutual information per pose over the virtual grid (the patchSize 0 metric):
 // extremes (the static image's once, stat_ready = 0 computes them into ext_stat), the
-// joint histogram [pose][bins_i][bins_u] and FP64 entropies into out[pose].
-// ext_mov: 2 ints per pose; hist: n_poses * bins_u * bins_i counters.
+// joint histogram [pose][bins_i][bins_u] and FP64 entropies into out[pose]. a.warp1: room for
+// the warped image of the poses (3D grids), or null: it is warped twice then, with the same
+// values. ext_mov: 2 ints per pose; hist: n_poses * mi_hist_size() counters.
 constexpr int kMiMaxBins = 256;
+inline int mi_hist_size(int bins_u, int bins_i) {  // with room for a group of bins of I, see k_mi_entropy_part
+    return bins_u * bins_i > 8 ? bins_u * bins_i : 8;
+}
 hipError_t launch_mi(const FusedArgs& a, int grid_ndim, int src_ndim, int high_res_is_moving,
                      int n_poses, int bins_u, int bins_i, const float* stat, int* ext_stat,
                      int stat_ready, int* ext_mov, unsigned* hist, double* out, hipStream_t st);

@@ -81,3 +81,33 @@ def test_mi_yaml_registration_maximises_nmi(tmp_path):
     assert abs(out["Outputs"]["LastSimilarity"] - nmi) < 1e-12
     log = open(tmp_path / "RegistrationInfo.log").read().splitlines()
     assert len(log) == nev + 2
+
+
+@pytest.mark.parametrize("dims,dt,bins", [((48, 45, 19), np.uint8, (2, 2)), ((67, 33, 70), np.float32, (7, 255)),
+                                          ((64, 64, 64), np.uint8, (256, 3)), ((130, 70, 41), np.float32, (256, 256))])
+def test_mi_kept_warp_equals_oracle_and_budget(engine, dims, dt, bins):
+    """Odd grids, bin counts at the edges of the entropies' groups and both storages: the
+    oracle's value to 1e-12 and, with the warped image not kept (an engine with a budget),
+    the same bits."""
+    rng = np.random.default_rng(sum(dims))
+    imgs = [rng.integers(0, 256, dims[::-1]).astype(dt) for _ in range(2)]
+    got = []
+    small = E.Engine(0, 1 << 30)
+    for e in (engine, small):
+        fv, mv = [e.upload(d, (1.0, 1.0, 1.0), (0.0, 0.0, 0.0)) for d in imgs]
+        p = e.pair(fv, mv, (1.1, 1.0, 1.0), True, False, 2, 3)
+        poses = np.zeros((3, 6)) + np.arange(3)[:, None] * 0.7
+        mats = np.stack([p.pose_to_matrix(q) for q in poses])
+        got.append(p.eval_mi(mats, *bins))
+        p.close()
+        fv.close()
+        mv.close()
+    small.close()
+    assert np.array_equal(got[0], got[1])
+    g = O.geom(dims, (1.0, 1.0, 1.0), (0.0, 0.0, 0.0))
+    vg = O.geom(O.virtual_dims(g, (1.1, 1.0, 1.0), 3), (1.1, 1.0, 1.0), (0.0, 0.0, 0.0))
+    f32 = [d.astype(np.float32) for d in imgs]
+    U = O.warp_3d(f32[0], g, vg, [1, 0, 0, 0, 0, 1, 0, 0, 0, 0, 1, 0])
+    for k in range(3):
+        I = O.warp_3d(f32[1], g, vg, np.asarray(mats[k]).ravel()[:12])
+        assert abs(got[0][k] - O.nmi(U, I, bins[0], bins[1], fp32=False)) < 1e-12
