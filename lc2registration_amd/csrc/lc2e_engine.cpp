@@ -1063,6 +1063,7 @@ int lc2e_pair_create(lc2e_engine* e, lc2e_volume* fixed, lc2e_volume* moving,
         }
         err = moments ? launch_stats(p, lc2e::kRoleUsStats, e->stream)
                     : lc2e::launch_ustats(p->stat_img, p->v, dim, patch_radius, p->ustat, p->ustat + V,
+                                          p->sep_sums, p->sep ? p->sep_sums + (size_t)lc2e::kSepChannels(true) * V : nullptr,
                                           e->stream);
     }
     if (err == hipSuccess && !high_res_is_moving) {

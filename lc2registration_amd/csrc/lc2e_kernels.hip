@@ -540,151 +540,180 @@ __global__ __launch_bounds__(TX * TY, 1) void k_fused3d(FusedArgs a) {
 // the reference switches to a global-memory kernel there (cu_lc2_3d.cu:769-827, chosen at
 // :1133-1177). Here, per pose: the moving image is warped (and, if it is the high-resolution
 // one, its |Sobel| taken) into two f32 grids, then the patch sums of every moment channel are
-// box sums along x, y (and z) through two f64 buffers, each a van Herk / Gil-Werman pass
+// box sums along z (3D) and y through two f64 buffers, each a van Herk / Gil-Werman pass
 // (exact in the sense of the fused kernels: no partial sum holds a value from outside its
-// window), and a last kernel combines them per voxel and reduces per work-group.
+// window), and a last kernel sums along x, combines per voxel and reduces per work-group.
 // Channels: moving high-resolution image (7): I, G, II, GG, IG, UI, UG; moving ultrasound
-// (10): I, G, U, II, GG, IG, UU, UI, UG and the count of U > 1e-6 (exact as a double).
+// (10): I, G, U, II, GG, IG, UU, UI, UG and the count of U > 1e-6 (exact as a double); static
+// ultrasound's statistics (3): U, UU, count.
 // ---------------------------------------------------------------------------
-template <bool MOVI>
-__device__ __forceinline__ double sep_product(int c, float I, float G, float U) {
-    const double di = I, dg = G, du = U;
-    if (MOVI) {
-        switch (c) {
-            case 0: return di;
-            case 1: return dg;
-            case 2: return di * di;
-            case 3: return dg * dg;
-            case 4: return di * dg;
-            case 5: return du * di;
-            default: return du * dg;
-        }
-    }
-    switch (c) {
-        case 0: return di;
-        case 1: return dg;
-        case 2: return du;
-        case 3: return di * di;
-        case 4: return dg * dg;
-        case 5: return di * dg;
-        case 6: return du * du;
-        case 7: return du * di;
-        case 8: return du * dg;
-        default: return (du > kZeroThreshold) ? 1.0 : 0.0;
-    }
-}
+enum { kSepMovingImage, kSepMovingUs, kSepUsStats };
+template <int KIND>
+constexpr int kSepNC = KIND == kSepMovingImage ? 7 : KIND == kSepMovingUs ? 10 : 3;
 
-// Window sums of width W along one line of n inputs: out(s) = in(s) + ... + in(s + W - 1)
-// for s < n - W + 1, van Herk form with the output itself holding the block suffix sums
-// between the two passes (no per-thread storage of W values).
-template <class In, class Out>
-__device__ __forceinline__ void vh_line(int n, int W, In in, Out out) {
-    const int nw = n - W + 1;
-    for (int b = 0; b < nw; b += W) {  // suffix sums of each block, from its end
+// One box pass: window sums of width W along lines of n elements, `stride` apart, to `dst` at
+// the index of the window start; buffers are [channel][V]. Line l of a channel starts at
+// (l / X) * outer + l % X, a lane per line, so loads and stores are whole rows. KIND >= 0: the
+// inputs are the products of the I, G, U grids; -1: `src`. A work-group (one wave) takes the
+// outputs [s, s + seg) of its lines, seg a multiple of W. A block's inputs lie in LDS, where they
+// become its suffix sums; the sum of output j is suffix j plus the running prefix of the next
+// block, so each input is read and each output written once. Channels of the same lines run on one
+// XCD one after the other (they read the same grids). Bound by memory: a pose of 161x150x131, r = 7,
+// 7 channels: z 53 us, y 110, then 76 for the last kernel; 2D, 260x260, r = 16, 10 channels: 22 and 15.
+// With the suffix sums in `dst` and a pass along x with a lane per line (strided loads) the
+// three passes took 240 to 1500 us each, the 2D ones 160 and over 360.
+template <int KIND>
+__global__ __launch_bounds__(64) void k_sep_pass(const float* __restrict__ I, const float* __restrict__ G,
+                                                 const float* __restrict__ U, const double* __restrict__ src,
+                                                 double* __restrict__ dst, long long V, int X, long long lines,
+                                                 long long outer, int stride, int n, int W, int seg, int nc) {
+    extern __shared__ double s_sep[];
+    double* suf = s_sep + threadIdx.x;
+    const int xcd = blockIdx.x % kXcds, k = blockIdx.x / kXcds;
+    const int c = k % nc;
+    const long long l = ((long long)(k / nc) * kXcds + xcd) * 64 + threadIdx.x;
+    if (l >= lines) return;  // (no barriers: a lane only touches its own LDS column)
+    const long long base = (l / X) * outer + l % X;
+    const int s0 = blockIdx.y * seg, s1 = min(s0 + seg, n - W + 1);
+    double* o = dst + (size_t)c * V + base;
+    // channel c is p * q of the grids, p alone, or the count
+    const float *p = nullptr, *q = nullptr;
+    bool count = false;
+    if constexpr (KIND == kSepMovingImage) {
+        p = c == 0 || c == 2 || c == 4 ? I : c == 1 || c == 3 ? G : U;
+        q = c < 2 ? nullptr : c == 2 || c == 5 ? I : G;
+    } else if constexpr (KIND == kSepMovingUs) {
+        p = c == 0 || c == 3 || c == 5 ? I : c == 1 || c == 4 ? G : U;
+        q = c < 3 || c == 9 ? nullptr : c == 3 || c == 7 ? I : c == 6 ? U : G;
+        count = c == 9;
+    } else if constexpr (KIND == kSepUsStats) {
+        p = U;
+        q = c == 1 ? U : nullptr;
+        count = c == 2;
+    }
+    constexpr int B = 8;  // inputs in flight
+    // inputs i .. i + B - 1, none past `last`
+    auto load = [&](int i, int last, double (&x)[B]) {
+        if constexpr (KIND >= 0) {
+            float f[B], g[B];
+#pragma unroll
+            for (int e = 0; e < B; ++e) f[e] = p[base + (long long)min(i + e, last) * stride];
+            if (q) {
+#pragma unroll
+                for (int e = 0; e < B; ++e) g[e] = q[base + (long long)min(i + e, last) * stride];
+            }
+#pragma unroll
+            for (int e = 0; e < B; ++e) {
+                x[e] = q ? (double)f[e] * (double)g[e] : (double)f[e];
+                if (count) x[e] = x[e] > kZeroThreshold ? 1.0 : 0.0;
+            }
+        } else {
+            const double* in = src + (size_t)c * V + base;
+#pragma unroll
+            for (int e = 0; e < B; ++e) x[e] = in[(long long)min(i + e, last) * stride];
+        }
+    };
+    for (int j0 = 0; j0 < W; j0 += B) {
+        double x[B];
+        load(s0 + j0, s0 + W - 1, x);
+#pragma unroll
+        for (int e = 0; e < B; ++e)
+            if (j0 + e < W) suf[(j0 + e) * 64] = x[e];
+    }
+    for (int b = s0;; b += W) {
         double acc = 0.0;
-        for (int i = min(b + W, n) - 1; i >= b; --i) {
-            acc += in(i);
-            if (i < nw) out(i) = acc;
+#pragma unroll 8
+        for (int j = W - 1; j >= 0; --j) {
+            acc += suf[j * 64];
+            suf[j * 64] = acc;
         }
-    }
-    for (int b = 0; b < nw; b += W) {  // plus the prefix of the next block
+        o[(long long)b * stride] = acc;
+        const bool more = b + W < s1;
+        const int m = min(W, s1 - b);           // outputs of this block
+        const int cnt = more ? W : m - 1;       // inputs of the next one that are needed
         double pre = 0.0;
-        for (int j = 0; j < W && b + j < nw; ++j) {
-            if (j > 0) out(b + j) = out(b + j) + pre;
-            if (b + W + j < n) pre += in(b + W + j);
+        for (int j0 = 0; j0 < cnt; j0 += B) {
+            double x[B];
+            load(b + W + j0, b + W + cnt - 1, x);
+#pragma unroll
+            for (int e = 0; e < B; ++e) {
+                const int j = j0 + e;
+                if (j < cnt) {
+                    pre += x[e];
+                    if (j + 1 < m) o[(long long)(b + j + 1) * stride] = suf[(j + 1) * 64] + pre;
+                    suf[j * 64] = x[e];
+                }
+            }
         }
+        if (!more) return;
     }
 }
 
-// One box pass. axis 0 reads the products of the I, G, U grids (U: ultrasound on the grid,
-// I: high-resolution image, G: its |Sobel|); axes 1 and 2 read `src`. Window sums of lines
-// along `axis` go to `dst` at the index of the window start. Buffers are [channel][V].
-template <bool MOVI>
-__global__ __launch_bounds__(256) void k_sep_pass(const float* __restrict__ I,
-                                                  const float* __restrict__ G,
-                                                  const float* __restrict__ U,
-                                                  const double* __restrict__ src,
-                                                  double* __restrict__ dst, VGeom v, int W,
-                                                  int axis) {
-    constexpr int NC = MOVI ? 7 : 10;
-    const long long V = (long long)v.X * v.Y * v.Z;
-    const int nX = axis == 0 ? 1 : v.X - W + 1;  // x positions of the lines (window starts)
-    const int nY = axis == 2 ? v.Y - W + 1 : (axis == 1 ? 1 : v.Y);
-    const long long lines = axis == 0 ? (long long)v.Y * v.Z
-                          : axis == 1 ? (long long)nX * v.Z
-                                      : (long long)nX * nY;
-    const long long tasks = lines * NC;
-    for (long long t = blockIdx.x * 256LL + threadIdx.x; t < tasks; t += (long long)gridDim.x * 256) {
-        const int c = (int)(t / lines);
-        const long long l = t % lines;
-        long long base;  // index of the line's first element
-        long long stride;
-        int n;
-        if (axis == 0) {
-            base = l * v.X;
-            stride = 1;
-            n = v.X;
-        } else if (axis == 1) {
-            const int x = (int)(l % nX), z = (int)(l / nX);
-            base = (long long)z * v.X * v.Y + x;
-            stride = v.X;
-            n = v.Y;
-        } else {
-            const int x = (int)(l % nX), y = (int)(l / nX);
-            base = (long long)y * v.X + x;
-            stride = (long long)v.X * v.Y;
-            n = v.Z;
-        }
-        double* o = dst + (long long)c * V + base;
-        if (axis == 0) {
-            vh_line(n, W, [&](int i) { return sep_product<MOVI>(c, I[base + i], G[base + i], U[base + i]); },
-                    [&](int s) -> double& { return o[s]; });
-        } else {
-            const double* in = src + (long long)c * V + base;
-            vh_line(n, W, [&](int i) { return in[i * stride]; },
-                    [&](int s) -> double& { return o[s * stride]; });
-        }
-    }
+// Orders a wave's LDS writes and reads across its lanes (the hardware keeps them in order).
+__device__ __forceinline__ void wave_lds_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
 }
 
-// Per output voxel: the patch sums (at the window-start index of `S`), weight and measure;
-// per work-group sums into the pose's partials (fixed positions, fixed order).
-template <bool MOVI>
-__global__ __launch_bounds__(256) void k_sep_combine(const double* __restrict__ S,
-                                                     const double* __restrict__ ustat_mean,
-                                                     const double* __restrict__ ustat_cyy,
-                                                     VGeom v, int r, int grid3, double* partials,
-                                                     double* wmap, double* mmap) {
+// Sums along x and combine: a wave takes 64 outputs of a row, with the row's 64 + 2r sums of every
+// channel in its part of the LDS; wave i of the grid takes the strips i, i + waves, ... Per
+// output voxel: weight and measure; per work-group sums into the pose's partials (fixed
+// positions, fixed order). kSepUsStats writes the statistics instead.
+template <int KIND>
+__global__ __launch_bounds__(256) void k_sep_combine(const double* __restrict__ S, double* __restrict__ ustat_mean,
+                                                     double* __restrict__ ustat_cyy, VGeom v, int r, int grid3,
+                                                     double* partials, double* wmap, double* mmap) {
+    extern __shared__ double s_rows[];
     __shared__ double s_red[8];
-    constexpr int NC = MOVI ? 7 : 10;
+    constexpr int NC = kSepNC<KIND>;
     const long long V = (long long)v.X * v.Y * v.Z;
-    const int W = 2 * r + 1;
+    const int W = 2 * r + 1, L = 64 + 2 * r;
     const int ex = v.X - 2 * r, ey = v.Y - 2 * r, ez = grid3 ? v.Z - 2 * r : v.Z;
     const int N = grid3 ? W * W * W : W * W;
-    const long long nout = (long long)ex * ey * ez;
-    const long long o = blockIdx.x * 256LL + threadIdx.x;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    double* row = s_rows + (size_t)wave * NC * L;
+    const int per_row = (ex + 63) / 64;
+    const long long strips = (long long)per_row * ey * ez;
     double am = 0.0, aw = 0.0;
-    if (o < nout) {
-        const int sx = (int)(o % ex), sy = (int)((o / ex) % ey), sz = (int)(o / ((long long)ex * ey));
-        const long long si = ((long long)sz * v.Y + sy) * v.X + sx;           // window start
-        const long long vo = ((long long)(sz + (grid3 ? r : 0)) * v.Y + (sy + r)) * v.X + (sx + r);
-        double Sc[NC];
+    for (long long s = (long long)blockIdx.x * 4 + wave; s < strips; s += (long long)gridDim.x * 4) {
+        const int x0 = (int)(s % per_row) * 64;
+        const long long yz = s / per_row;
+        const int sy = (int)(yz % ey), sz = (int)(yz / ey);
+        const long long line = ((long long)sz * v.Y + sy) * v.X;
+        for (int i = lane; i < L; i += 64)
 #pragma unroll
-        for (int c = 0; c < NC; ++c) Sc[c] = S[(long long)c * V + si];
-        double w, meas;
-        bool ok;
-        if (MOVI) ok = combine_static_u(Sc, ustat_mean[vo], ustat_cyy[vo], N, w, meas);
-        else ok = combine(Sc, (int)Sc[9], N, w, meas);
-        if (ok) {
-            am = meas;
-            aw = w;
-            if (wmap) {
-                wmap[vo] = w;
-                mmap[vo] = meas;
+            for (int c = 0; c < NC; ++c) row[c * L + i] = x0 + i < v.X ? S[(size_t)c * V + line + x0 + i] : 0.0;
+        wave_lds_sync();
+        double Sc[NC] = {};
+#pragma unroll 2
+        for (int j = 0; j < W; ++j)
+#pragma unroll
+            for (int c = 0; c < NC; ++c) Sc[c] += row[c * L + lane + j];
+        wave_lds_sync();
+        if (x0 + lane < ex) {
+            const long long vo = ((long long)(sz + (grid3 ? r : 0)) * v.Y + (sy + r)) * v.X + (x0 + lane + r);
+            if constexpr (KIND == kSepUsStats) {
+                const double cc = Sc[1] - Sc[0] * Sc[0] * (1.0 / (double)N);
+                const bool ok = Sc[2] == (double)N && cc * (1.0 / (double)(N - 1)) > kZeroThreshold;
+                ustat_mean[vo] = ok ? Sc[0] * (1.0 / (double)N) : 0.0;
+                ustat_cyy[vo] = ok ? cc : -1.0;
+            } else {
+                double w, meas;
+                bool ok;
+                if constexpr (KIND == kSepMovingImage) ok = combine_static_u(Sc, ustat_mean[vo], ustat_cyy[vo], N, w, meas);
+                else ok = combine(Sc, (int)Sc[9], N, w, meas);
+                if (ok) {
+                    am += meas;
+                    aw += w;
+                    if (wmap) {
+                        wmap[vo] = w;
+                        mmap[vo] = meas;
+                    }
+                }
             }
         }
     }
-    block_reduce_store<256>(am, aw, s_red, partials + (size_t)blockIdx.x * 2);
+    if constexpr (KIND != kSepUsStats) block_reduce_store<256>(am, aw, s_red, partials + (size_t)blockIdx.x * 2);
 }
 
 // Per-pose fixed-order reduction of the work-group partials -> (sum m, sum w, LC2)
@@ -766,7 +795,8 @@ __global__ void k_warp_moving(FusedArgs a, int grid3, int src3, float* out) {
 
 // Static ultrasound patch statistics (weight half of cu_lc2_3d.cu:181-287 /
 // cu_lc2_2d.cu:88-180) per voxel in FP64: count of U > 1e-6, sum, sum of squares in a
-// fixed x-fastest order; mean and centred energy, or -1 where w = 0.
+// fixed x-fastest order; mean and centred energy, or -1 where w = 0. For grids of large planes
+// only: the others have the moments kernels' or the box passes' statistics.
 __global__ void k_ustats(const float* img, VGeom v, int grid3, int r, double* mean, double* cyy) {
     const long long n = (long long)v.X * v.Y * v.Z;
     const int w = 2 * r + 1;
@@ -801,6 +831,13 @@ __global__ void k_ustats(const float* img, VGeom v, int grid3, int r, double* me
         }
         mean[i] = m;
         cyy[i] = c;
+    }
+}
+
+__global__ void k_ustats_none(long long n, double* mean, double* cyy) {
+    for (long long i = blockIdx.x * (long long)blockDim.x + threadIdx.x; i < n; i += (long long)gridDim.x * blockDim.x) {
+        mean[i] = 0.0;
+        cyy[i] = -1.0;
     }
 }
 
@@ -984,14 +1021,68 @@ int sep_blocks(const VGeom& v, int r, int grid_ndim) {
     return (int)((ex * ey * ez + 255) / 256);
 }
 
+namespace {
+
+// The box passes over the grids, and the last kernel on nb work-groups.
+template <int KIND>
+hipError_t sep_sums(const float* I, const float* G, const float* U, double* sum_a, double* sum_b, const VGeom& v,
+                    int r, int grid_ndim, int nb, double* mean, double* cyy, double* partials, double* wmap,
+                    double* mmap, hipStream_t st) {
+    constexpr int NC = kSepNC<KIND>;
+    const long long V = (long long)v.X * v.Y * v.Z;
+    const int W = 2 * r + 1;
+    static std::once_flag once;
+    static hipError_t set_err = hipSuccess;
+    std::call_once(once, [] {  // 66 KB at the largest radius, 61 KB for the rows
+        for (const void* f : {reinterpret_cast<const void*>(&k_sep_pass<KIND>), reinterpret_cast<const void*>(&k_sep_pass<-1>)})
+            if (set_err == hipSuccess)
+                set_err = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                              (2 * kMaxRSep + 1) * 64 * sizeof(double));
+        if (set_err == hipSuccess)
+            set_err = hipFuncSetAttribute(reinterpret_cast<const void*>(&k_sep_combine<KIND>),
+                                          hipFuncAttributeMaxDynamicSharedMemorySize,
+                                          4 * NC * (64 + 2 * kMaxRSep) * sizeof(double));
+    });
+    if (set_err != hipSuccess) return set_err;
+    bool first = true;
+    auto pass = [&](long long lines, long long outer, int stride, int n, const double* src, double* dst) {
+        const long long tiles8 = ((lines + 63) / 64 + kXcds - 1) / kXcds * kXcds;
+        // 16 waves per CU where that leaves each at least two blocks (the first one's inputs
+        // are read twice)
+        const int blocks = (n - W + 1 + W - 1) / W;
+        const int segs = (int)std::max(1LL, std::min<long long>(4096 / (tiles8 * NC), blocks / 2));
+        const int seg = (blocks + segs - 1) / segs * W;
+        const dim3 grid((unsigned)(tiles8 * NC), (unsigned)((n - W + seg) / seg));
+        const size_t lds = (size_t)W * 64 * sizeof(double);
+        if (first)
+            hipLaunchKernelGGL(k_sep_pass<KIND>, grid, dim3(64), lds, st, I, G, U, src, dst, V, v.X, lines, outer,
+                               stride, n, W, seg, NC);
+        else
+            hipLaunchKernelGGL(k_sep_pass<-1>, grid, dim3(64), lds, st, I, G, U, src, dst, V, v.X, lines, outer,
+                               stride, n, W, seg, NC);
+        first = false;
+    };
+    const int XY = v.X * v.Y;
+    const double* S = sum_a;
+    if (grid_ndim == 3) {
+        pass(XY, v.X, XY, v.Z, nullptr, sum_a);
+        pass((long long)v.X * (v.Z - W + 1), XY, v.X, v.Y, sum_a, sum_b);
+        S = sum_b;
+    } else {
+        pass((long long)v.X * v.Z, XY, v.X, v.Y, nullptr, sum_a);
+    }
+    hipLaunchKernelGGL(k_sep_combine<KIND>, dim3(nb), dim3(256), 4 * NC * (size_t)(64 + 2 * r) * sizeof(double), st, S,
+                       mean, cyy, v, r, grid_ndim == 3 ? 1 : 0, partials, wmap, mmap);
+    return hipGetLastError();
+}
+
+}  // namespace
+
 hipError_t launch_sep(const FusedArgs& a, int grid_ndim, int src_ndim, int movi, int n_poses,
                       hipStream_t st) {
     const VGeom& v = a.v;
-    const int W = 2 * a.r + 1;
     const int nb = sep_blocks(v, a.r, grid_ndim);
     if (nb == 0 || n_poses <= 0) return hipSuccess;
-    const long long V = (long long)v.X * v.Y * v.Z;
-    const int nc = movi ? 7 : 10;
     for (int pose = 0; pose < n_poses; ++pose) {
         FusedArgs b = a;
         b.mats = a.mats + (size_t)pose * a.mats_per_pose * 12;
@@ -999,34 +1090,14 @@ hipError_t launch_sep(const FusedArgs& a, int grid_ndim, int src_ndim, int movi,
         hipError_t e = launch_warp_moving(b, grid_ndim, src_ndim, a.sep_img, st);
         if (e != hipSuccess) return e;
         if (movi && (e = launch_sobel(a.sep_img, v, grid_ndim, a.sep_grad, st)) != hipSuccess) return e;
-        const float* I = movi ? a.sep_img : a.stat_img;
-        const float* G = movi ? a.sep_grad : a.stat_grad;
-        const float* U = movi ? a.stat_img : a.sep_img;
-        const int passes = grid_ndim == 3 ? 3 : 2;
-        for (int axis = 0; axis < passes; ++axis) {
-            const long long lines = axis == 0 ? (long long)v.Y * v.Z
-                                  : axis == 1 ? (long long)(v.X - W + 1) * v.Z
-                                              : (long long)(v.X - W + 1) * (v.Y - W + 1);
-            const dim3 grid = grid_for(lines * nc);
-            const double* src = axis == 1 ? a.sep_a : a.sep_b;
-            double* dst = axis == 1 ? a.sep_b : a.sep_a;
-            if (movi)
-                hipLaunchKernelGGL(k_sep_pass<true>, grid, dim3(256), 0, st, I, G, U, src, dst, v, W, axis);
-            else
-                hipLaunchKernelGGL(k_sep_pass<false>, grid, dim3(256), 0, st, I, G, U, src, dst, v, W, axis);
-            if ((e = hipGetLastError()) != hipSuccess) return e;
-        }
-        const double* S = passes == 3 ? a.sep_a : a.sep_b;
         double* part = a.partials + (size_t)pose * a.blocks_per_pose * 2;
-        if (movi)
-            hipLaunchKernelGGL(k_sep_combine<true>, dim3(nb), dim3(256), 0, st, S, a.ustat_mean,
-                               a.ustat_cyy, v, a.r, grid_ndim == 3 ? 1 : 0, part, a.wmap, a.mmap);
-        else
-            hipLaunchKernelGGL(k_sep_combine<false>, dim3(nb), dim3(256), 0, st, S, a.ustat_mean,
-                               a.ustat_cyy, v, a.r, grid_ndim == 3 ? 1 : 0, part, a.wmap, a.mmap);
-        if ((e = hipGetLastError()) != hipSuccess) return e;
+        double *mean = const_cast<double*>(a.ustat_mean), *cyy = const_cast<double*>(a.ustat_cyy);  // read only
+        e = movi ? sep_sums<kSepMovingImage>(a.sep_img, a.sep_grad, a.stat_img, a.sep_a, a.sep_b, v, a.r, grid_ndim,
+                                             nb, mean, cyy, part, a.wmap, a.mmap, st)
+                 : sep_sums<kSepMovingUs>(a.stat_img, a.stat_grad, a.sep_img, a.sep_a, a.sep_b, v, a.r, grid_ndim,
+                                          nb, mean, cyy, part, a.wmap, a.mmap, st);
+        if (e != hipSuccess) return e;
     }
-    (void)V;
     return hipSuccess;
 }
 
@@ -1100,10 +1171,17 @@ hipError_t launch_warp_moving(const FusedArgs& a, int grid_ndim, int src_ndim, f
 }
 
 hipError_t launch_ustats(const float* img, const VGeom& v, int grid_ndim, int r, double* mean,
-                         double* cyy, hipStream_t st) {
+                         double* cyy, double* sum_a, double* sum_b, hipStream_t st) {
     const long long n = (long long)v.X * v.Y * v.Z;
-    hipLaunchKernelGGL(k_ustats, grid_for(n), dim3(256), 0, st, img, v, grid_ndim == 3 ? 1 : 0, r,
-                       mean, cyy);
+    const int nb = sep_blocks(v, r, grid_ndim);
+    if (sum_a) {
+        hipLaunchKernelGGL(k_ustats_none, grid_for(n), dim3(256), 0, st, n, mean, cyy);
+        if (nb > 0)
+            return sep_sums<kSepUsStats>(nullptr, nullptr, img, sum_a, sum_b, v, r, grid_ndim, nb, mean, cyy, nullptr,
+                                         nullptr, nullptr, st);
+    } else {
+        hipLaunchKernelGGL(k_ustats, grid_for(n), dim3(256), 0, st, img, v, grid_ndim == 3 ? 1 : 0, r, mean, cyy);
+    }
     return hipGetLastError();
 }
 

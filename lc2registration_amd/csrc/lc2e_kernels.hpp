@@ -138,8 +138,8 @@ int moments3_waves(int r, int role);  // combining waves: partial sums per tile 
 hipError_t launch_reduce(const double* partials, int blocks_per_pose, int n_poses, double* out,
                          hipStream_t st);
 // Separable path for radii beyond the other kernels (3D r > kMaxRMom3, 2D r > kMaxR2): per
-// pose, warp (+ |Sobel|), box sums along each axis through sep_a / sep_b, combine; one
-// partial per 256 output voxels (sep_blocks per pose, fixed positions).
+// pose, warp (+ |Sobel|), box sums along z and y through sep_a / sep_b, sums along x and
+// combine; a work-group and a partial per 256 output voxels (sep_blocks per pose, fixed positions).
 int sep_blocks(const VGeom& v, int r, int grid_ndim);
 hipError_t launch_sep(const FusedArgs& a, int grid_ndim, int src_ndim, int movi, int n_poses,
                       hipStream_t st);
@@ -157,9 +157,10 @@ hipError_t launch_warp_static(const void* fixed, int fixed_f16, const SGeom& fg,
 hipError_t launch_warp_moving(const FusedArgs& a, int grid_ndim, int src_ndim, float* out,
                               hipStream_t st);
 // Patch statistics of a static ultrasound grid: mean and centred energy per voxel
-// (negative where the reference's weight is 0), FP64, fixed summation order.
+// (negative where the reference's weight is 0), FP64, fixed summation order. sum_a, sum_b: room for
+// the box passes' 3 channels, or null: one pass over every patch.
 hipError_t launch_ustats(const float* img, const VGeom& v, int grid_ndim, int r, double* mean,
-                         double* cyy, hipStream_t st);
+                         double* cyy, double* sum_a, double* sum_b, hipStream_t st);
 // |Sobel| of a virtual-grid image (3D, or per frame for 2D grids), separable order.
 hipError_t launch_sobel(const float* img, const VGeom& v, int grid_ndim, float* out,
                         hipStream_t st);

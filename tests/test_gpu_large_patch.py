@@ -152,3 +152,30 @@ def test_radius_limits(engine):
     p.close()
     fv.close()
     mv.close()
+
+
+@pytest.mark.parametrize("dims,r,moving_high_res", [
+    ((83, 31, 70), 7, True), ((40, 37, 33), 9, False), ((16, 64, 15), 7, True),   # several blocks, remainders, one
+    ((201, 145), 11, True), ((130, 139), 64, False), ((66, 400), 16, True)])      # row; the largest window; segments
+def test_box_passes_equal_oracle(engine, dims, r, moving_high_res):
+    """Lines of less than a wave, strips with a remainder, lines split over several work-groups
+    and the largest radius: every voxel's weight and measure, to rounding of the sums."""
+    rng = np.random.default_rng(r)
+    dim = len(dims)
+    a, b = [rng.uniform(1.0, 200.0, dims[::-1]).astype(np.float32) for _ in range(2)]
+    one, zero = (1.0,) * dim, (0.0,) * dim
+    w = synth.Workload("box", synth.Image(a, dims, one, zero), synth.Image(b, dims, one, zero), one, r,
+                       moving_high_res, False, dim, np.zeros(6))
+    print(f"box passes {dims} r={r}", flush=True)
+    p, vols = _pair(engine, w, r, dim)
+    M = np.eye(3, 4, dtype=np.float32)
+    res, wm, mm = _oracle(w, M, r, dim, dim, maps=True)
+    assert res.n_valid > 0
+    assert abs(p.eval(M) - res.lc2) < LC2_TOL
+    gw, gm = [p.debug_fetch(s, M).reshape(wm.shape) for s in (E.STAGE_W, E.STAGE_MEASURE)]
+    assert np.array_equal(gw > 0, wm > 0)
+    assert np.allclose(gw, wm, rtol=1e-9, atol=1e-12)
+    assert np.allclose(gm, mm, rtol=1e-7, atol=1e-9)
+    p.close()
+    for v in vols:
+        v.close()
