@@ -29,7 +29,7 @@ ALG_BYTES_PER_VOXEL = 1.0 + 0.5
 ALG_F32_PER_VOXEL = 116.0   # warp 40, Sobel 27, products 5, window sums 42, reduction 2
 ALG_F64_PER_VOXEL = 45.0    # centred moments, 2x2 solve, variance/measure, thresholds
 ALG_F32_SWEEP = 89.0        # 2D frames from 3D: warp 40, Sobel 14, products 5, sums 28, reduction 2
-PROFILE_TRAFFIC = os.path.join(ROOT, "profiles", "k_fused3d_r3_affine3d_us192_traffic.json")
+PROFILE_TRAFFIC = os.path.join(ROOT, "profiles", "lc2_3d_r3_affine3d_us192_traffic.json")
 SIMDS, CLOCK_HZ = 256 * 4, 2.4e9  # MI355X: 256 CUs of 4 SIMDs, peak engine clock
 
 
@@ -870,7 +870,7 @@ def main():
     roofline = {"bound": "valu", "achieved": _f32_equiv(P * V) / avg_kernel_s / 1e12,
                 "peak": FP32_PEAK / 1e12, "unit": "TFLOP/s", "frac": t_valu / avg_kernel_s,
                 "traffic": traffic,
-                "kernel": "k_fused3d<R=3, moving high-res>",
+                "kernel": "k_warp_grad3 + k_moments3d<R=3, moving high-res>",
                 "kernel_ms_per_launch": avg_kernel_s * 1e3, "launches": launches,
                 "algorithmic_flops_per_launch": {"f32": P * V * ALG_F32_PER_VOXEL,
                                                  "f64": P * V * ALG_F64_PER_VOXEL},
