@@ -636,11 +636,12 @@ __device__ __forceinline__ V load_at(const V* base, unsigned ofs) {
     return v;
 }
 
-// Matrix i of the launch: from memory, or a single matrix from the kernel's arguments.
+// Matrix i of the launch: from memory, or from the kernel's arguments, which spares small
+// launches a round trip to the host's memory.
 __device__ __forceinline__ void load_matrix(const FusedArgs& a, size_t i, float (&m)[12]) {
     if (a.inline_mat) {
 #pragma unroll
-        for (int k = 0; k < 12; ++k) m[k] = a.m0[k];
+        for (int k = 0; k < 12; ++k) m[k] = a.m0[i * 12 + k];
     } else {
         const float* mp = a.mats + i * 12;
 #pragma unroll

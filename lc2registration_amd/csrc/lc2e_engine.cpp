@@ -314,6 +314,7 @@ hipError_t launch_eval(lc2e_pair* p, const lc2e::FusedArgs& a, int n, hipStream_
             const int m = std::min(step, n - b);
             lc2e::FusedArgs s = a;
             s.mats = a.mats + (size_t)b * a.mats_per_pose * 12;
+            if (b) s.inline_mat = 0;
             s.partials = a.partials + (size_t)b * a.blocks_per_pose * 2;
             hipError_t err = lc2e::launch_warp_grid(s, p->info.grid_ndim, p->info.src_ndim,
                                                     p->info.high_res_is_moving, m, st);
@@ -677,7 +678,8 @@ lc2e::FusedArgs make_args(lc2e_pair* p, const float* d_mats, double* d_partials,
 // per batch instead of four. Where a launch is not captured, a single matrix goes with the
 // kernel's arguments (a read from pinned memory takes 1.2 us at a kernel's start), and few
 // partials go straight to pinned memory for the host to add up (*host_sum; a launch less:
-// 2D 256x256 single pose 30.7 -> 24.5 us with both).
+// 2D 256x256 single pose 30.7 -> 24.5 us with both). Such launches carry their matrices in the
+// kernels' arguments: 4 poses 194x248, r = 5, 33.4 -> 31.6 us, 6 poses 145x114, r = 3, 29.1 -> 27.0.
 int enqueue_batch(lc2e_pair* p, int n, const Tiling& t, hipStream_t st, bool captured, bool* host_sum) {
     const int mpp = p->mats_per_pose();
     const bool direct = !p->sep && mpp == 1 && n <= kDirectPoses &&
@@ -689,9 +691,9 @@ int enqueue_batch(lc2e_pair* p, int n, const Tiling& t, hipStream_t st, bool cap
                                hipMemcpyHostToDevice, st));
     if (t.tiles > 0) {
         lc2e::FusedArgs a = make_args(p, direct ? p->h_mats_dev : p->d_mats, host ? p->h_part_dev : p->d_partials, t);
-        if (direct && n == 1 && !captured) {
+        if (direct && n <= lc2e::kInlineMats && !captured) {
             a.inline_mat = 1;
-            std::memcpy(a.m0, p->h_mats, sizeof(a.m0));
+            std::memcpy(a.m0, p->h_mats, (size_t)n * 12 * sizeof(float));
         }
         // timed launches are eager (run_batch), the events bracket the fused kernel
         const bool timed = p->profile;
@@ -707,16 +709,19 @@ int enqueue_batch(lc2e_pair* p, int n, const Tiling& t, hipStream_t st, bool cap
 }
 
 // The sums of k_reduce from the partials in h_part, added in its order: 256 running sums of
-// every 256th partial, then halves (here at most one partial each).
+// every 256th partial, then halves (here at most one partial each; halvings that would only add
+// the zeros past the last partial are left out).
 void sum_partials(lc2e_pair* p, int n, int bpp) {
     double m[kHostPose], w[kHostPose];
+    int top = 1;
+    while (top < bpp) top *= 2;
     for (int i = 0; i < n; ++i) {
         const double* s = p->h_part + (size_t)i * bpp * 2;
-        for (int k = 0; k < kHostPose; ++k) {
+        for (int k = 0; k < top; ++k) {
             m[k] = k < bpp ? 0.0 + s[2 * k] : 0.0;
             w[k] = k < bpp ? 0.0 + s[2 * k + 1] : 0.0;
         }
-        for (int h = kHostPose / 2; h > 0; h >>= 1)
+        for (int h = top / 2; h > 0; h >>= 1)
             for (int k = 0; k < h; ++k) {
                 m[k] += m[k + h];
                 w[k] += w[k + h];

@@ -1086,6 +1086,7 @@ hipError_t launch_sep(const FusedArgs& a, int grid_ndim, int src_ndim, int movi,
     for (int pose = 0; pose < n_poses; ++pose) {
         FusedArgs b = a;
         b.mats = a.mats + (size_t)pose * a.mats_per_pose * 12;
+        b.inline_mat = 0;
         // the moving image on the grid; its |Sobel| when it is the high-resolution image
         hipError_t e = launch_warp_moving(b, grid_ndim, src_ndim, a.sep_img, st);
         if (e != hipSuccess) return e;

@@ -21,6 +21,7 @@ constexpr int kXcds = 8;       // MI355X: 8 XCDs, each with its own L2, 32 CUs e
 constexpr int kMaxRFused2 = 3; // largest patch radius of the 2D fused kernel
 constexpr int kMaxR2 = 10;     // largest patch radius of the 2D moments kernel
 constexpr int kMaxRSep = 64;   // largest patch radius of the separable path (larger radii)
+constexpr int kInlineMats = 8; // matrices a launch carries in its arguments
 constexpr int kFrameRun = 16;  // frames per 2D work-group (frame stacks)
 // The fused kernels' samplers form voxel offsets with 24-bit multiplies: a 3D source whose
 // slices hold this many voxels or more is evaluated by the separable path instead.
@@ -60,7 +61,7 @@ struct FusedArgs {
     const double* ustat_mean;  // static ultrasound: patch mean per voxel
     const double* ustat_cyy;   // static ultrasound: centred patch energy, < 0 where w = 0
     const float* mats;       // [pose][mats_per_pose][12] VirtualToMoving, 3x4 row-major
-    float m0[12];            // the only matrix of the launch, if inline_mat (mats holds it too)
+    float m0[kInlineMats * 12];  // the launch's matrices, if inline_mat (mats holds them too)
     int inline_mat;
     double* partials;        // [pose][blocks_per_pose][2] (sum measure, sum w); 3D: the
                              // blocks are [z block of kZBlock planes][tile column][wave]

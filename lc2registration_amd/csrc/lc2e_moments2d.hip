@@ -109,6 +109,8 @@ __global__ __launch_bounds__(256) void k_warp2(FusedArgs a, int ntx, int nty, in
 // VGPRs); bound by the latency of the three LDS trips per channel and of the FP64 chains (VALU a
 // quarter busy). Measured, static image: 256x256, R = 3, 64 poses 104 -> 42 us; 261x261, R = 9,
 // 13 poses 100 -> 30 us; moving image: 336x205 slice in a CT, R = 9, 13 poses 60 -> 38 us.
+// In place the four waves share the warped rows (32 + 2R for 32, where each warped 8 + 2R of its
+// own): per call 256x256, R = 3, 64 poses 62 -> 55 us, one pose 27.7 -> 26.9; R = 9, 13 poses 45 -> 40.
 // ---------------------------------------------------------------------------
 // LDS column x of a wave's row: 2 doubles of padding after every 8, and rows 80 doubles apart,
 // spread the 16-byte reads of the x pass (8 runs of 8 columns, 8 rows) over all banks.
@@ -124,23 +126,25 @@ __device__ __forceinline__ void wave_fence() {
 // lanes only feed the Sobel of the variant that warps in place.
 constexpr int strip2(int r, int role) { return (role == kRoleMovingImage ? 62 : 64) - 2 * r; }
 
-// Rows of the warped image a wave keeps in LDS when it warps in place, 64 floats each.
+// Rows of the warped image a work-group keeps in LDS when it warps in place, 64 floats each: its 32
+// output rows' with their halo, each warped once for the four waves.
 template <int R, int ROLE>
 struct InPlace {
     static constexpr int H = ROLE == kRoleMovingImage ? 1 : 0;  // halo of the Sobel
-    static constexpr int ROWS = 2 * R + 8 + 2 * H, FLOATS = ROWS * 64 * (1 + H);
+    static constexpr int ROWS = 32 + 2 * R + 2 * H, FLOATS = ROWS * 64 * (1 + H);
 };
 
 // The moving image at column gx (this lane's) of rows gy0 .. gy0 + rows - 1 of frame's matrix m,
-// 0 outside the grid, into dst (rows 64 floats apart); four rows of gathers in flight.
+// 0 outside the grid, into dst (rows 64 floats apart): this wave's share of the work-group's, every
+// fourth group of four rows, whose gathers are in flight at once.
 template <bool P2, bool SRC3D, typename T>
 __device__ __forceinline__ void warp_rows(const FusedArgs& a, const float* m, int gx, int gy0, int rows,
-                                          float* dst) {
+                                          float* dst, int wave) {
     const T* __restrict__ src = static_cast<const T*>(a.src);
     using Pend = typename std::conditional<SRC3D, Pending3<T>, Pending2<T>>::type;
     const float lx = fmaf((float)gx, a.v.sx, a.v.ox);
     const bool inx = gx >= 0 && gx < a.v.X;
-    for (int j0 = 0; j0 < rows; j0 += 4) {
+    for (int j0 = 4 * wave; j0 < rows; j0 += 16) {
         Pend p[4];
 #pragma unroll
         for (int k = 0; k < 4; ++k) {
@@ -156,17 +160,17 @@ __device__ __forceinline__ void warp_rows(const FusedArgs& a, const float* m, in
     }
 }
 __device__ __forceinline__ void warp_rows_any(const FusedArgs& a, int src3, const float* m, int gx, int gy0,
-                                              int rows, float* dst) {
+                                              int rows, float* dst, int wave) {
     const int form = (src3 ? 4 : 0) + (a.s.pow2 ? 2 : 0) + (a.src_f16 ? 1 : 0);  // uniform
     switch (form) {
-        case 7: return warp_rows<true, true, __half>(a, m, gx, gy0, rows, dst);
-        case 6: return warp_rows<true, true, float>(a, m, gx, gy0, rows, dst);
-        case 5: return warp_rows<false, true, __half>(a, m, gx, gy0, rows, dst);
-        case 4: return warp_rows<false, true, float>(a, m, gx, gy0, rows, dst);
-        case 3: return warp_rows<true, false, __half>(a, m, gx, gy0, rows, dst);
-        case 2: return warp_rows<true, false, float>(a, m, gx, gy0, rows, dst);
-        case 1: return warp_rows<false, false, __half>(a, m, gx, gy0, rows, dst);
-        default: return warp_rows<false, false, float>(a, m, gx, gy0, rows, dst);
+        case 7: return warp_rows<true, true, __half>(a, m, gx, gy0, rows, dst, wave);
+        case 6: return warp_rows<true, true, float>(a, m, gx, gy0, rows, dst, wave);
+        case 5: return warp_rows<false, true, __half>(a, m, gx, gy0, rows, dst, wave);
+        case 4: return warp_rows<false, true, float>(a, m, gx, gy0, rows, dst, wave);
+        case 3: return warp_rows<true, false, __half>(a, m, gx, gy0, rows, dst, wave);
+        case 2: return warp_rows<true, false, float>(a, m, gx, gy0, rows, dst, wave);
+        case 1: return warp_rows<false, false, __half>(a, m, gx, gy0, rows, dst, wave);
+        default: return warp_rows<false, false, float>(a, m, gx, gy0, rows, dst, wave);
     }
 }
 
@@ -180,7 +184,7 @@ void k_moments2d(FusedArgs a) {
     constexpr int H = INPLACE ? IP::H : 0;  // lane of the first column
     __shared__ __align__(16) double s_all[4 * kWaveS];
     __shared__ double s_red[8];
-    extern __shared__ float s_rows[];  // INPLACE: IP::FLOATS per wave
+    extern __shared__ float s_rows[];  // INPLACE: IP::FLOATS
 
     int tile, pose;
     if (!map_block(a.tiles, a.npose, tile, pose)) return;  // whole work-group
@@ -190,10 +194,11 @@ void k_moments2d(FusedArgs a) {
     const int X = a.v.X, Y = a.v.Y, Z = a.v.Z, XY = X * Y;
     const int x0 = R + (tcol % a.ntx) * TX, y0 = R + (tcol / a.ntx) * 32 + wave * 8;
     const int col = lane - H;  // column of the strip
-    const int f0 = run * a.zchunk, f1 = min(f0 + a.zchunk, Z);
+    const bool has_rows = y0 < Y - R;  // the wave has output rows
+    const int f0 = run * a.zchunk, f1 = INPLACE || has_rows ? min(f0 + a.zchunk, Z) : f0;
     double acc_m = 0.0, acc_w = 0.0;
 
-    if (y0 < Y - R) {  // the wave has output rows
+    {
         double* const s = s_all + wave * kWaveS;
         // this lane's column; rows and columns past the grid repeat its edge and only reach
         // outputs that are not valid
@@ -202,7 +207,7 @@ void k_moments2d(FusedArgs a) {
         const bool okx = col >= 0 && col < TX && ox < X - R;
         const int s_col = lds_col(min(max(col, 0), 63));
         const bool has_col = col >= 0;
-        float* const rows = s_rows + (INPLACE ? wave * IP::FLOATS + lane : 0);
+        float* const rows = s_rows + (INPLACE ? wave * 8 * 64 + lane : 0);
         const int run_x = lane % 8, run_y = lane / 8;
         double* const xp = s + run_y * kRowS + run_x * 10;
         for (int f = f0; f < f1; ++f) {
@@ -210,27 +215,37 @@ void k_moments2d(FusedArgs a) {
             if constexpr (INPLACE) {
                 float m[12];
                 load_matrix(a, (size_t)pose * a.mats_per_pose + (a.mats_per_pose > 1 ? f : 0), m);
-                warp_rows_any(a, a.src3, m, x0 - R + col, y0 - R - H, IP::ROWS, rows);
+                const int top = y0 - wave * 8 - R - H;  // grid row of the first one
+                const int nrows = min(IP::ROWS, Y + H - top);  // none past the grid's but the Sobel's
+                if (f > f0) __syncthreads();  // the last frame's are read
+                warp_rows_any(a, a.src3, m, x0 - R + col, top, nrows, s_rows + lane, wave);
+                __syncthreads();
                 if constexpr (ROLE == kRoleMovingImage) {
-                    wave_fence();
-                    // |Sobel| of rows y0 - R .., the outermost lanes' is not used
-                    float* const g = rows + IP::ROWS * 64;
+                    // |Sobel| of the rows between, a quarter per wave; the outermost lanes' is not used
+                    constexpr int Q = (IP::ROWS - 2 + 3) / 4;
+                    const float* const in = s_rows + lane;
+                    float* const g = s_rows + IP::ROWS * 64 + lane;
                     const int left = lane > 0 ? -1 : 0, right = lane < 63 ? 1 : 0;
+                    const int j0 = wave * Q, j1 = min(j0 + Q + 2, nrows);
                     float sm[3], df[3];
                     auto line = [&](int j, int k) {
-                        const float l = rows[j * 64 + left], c = rows[j * 64], r = rows[j * 64 + right];
+                        const float l = in[j * 64 + left], c = in[j * 64], r = in[j * 64 + right];
                         sm[k] = fmaf(2.0f, c, l) + r;
                         df[k] = r - l;
                     };
-                    line(0, 0);
-                    line(1, 1);
-                    for (int j = 2; j < IP::ROWS; ++j) {
+                    if (j0 + 2 < j1) {
+                        line(j0, 0);
+                        line(j0 + 1, 1);
+                    }
+                    for (int j = j0 + 2; j < j1; ++j) {
                         line(j, 2);
                         const float gxv = fmaf(2.0f, df[1], df[0]) + df[2], gyv = sm[2] - sm[0];
                         g[(j - 1) * 64] = sqrtf(fmaf(gyv, gyv, gxv * gxv));
                         sm[0] = sm[1], sm[1] = sm[2], df[0] = df[1], df[1] = df[2];
                     }
+                    __syncthreads();
                 }
+                if (!has_rows) continue;
             }
             auto input = [&](int j, double& I, double& G, double& U) {
                 const size_t row = (size_t)min(y0 - R + j, Y - 1) * X;  // wave-uniform
@@ -465,7 +480,7 @@ void warp2t(const FusedArgs& a, int n, hipStream_t st) {
 
 template <int R, int ROLE, bool INPLACE>
 hipError_t moments2k(const FusedArgs& a, dim3 grid, hipStream_t st, int* occ) {
-    const size_t lds = INPLACE ? 4 * InPlace<R, ROLE>::FLOATS * sizeof(float) : 0;
+    const size_t lds = INPLACE ? InPlace<R, ROLE>::FLOATS * sizeof(float) : 0;
     if constexpr (INPLACE) {
         static std::once_flag once;
         static hipError_t err = hipSuccess;
