@@ -197,6 +197,23 @@ struct Pending3<__half> {
     unsigned a, b, c, d;  // half2: x0 in the low half, x0 + 1 in the high half
     float rx, ry, rz;
 };
+// Half sources of even X: each pair within the two aligned words that hold it (a load at an odd
+// element takes longer than one of 8 aligned bytes), shifted into place when it is used. All four
+// pairs of a sample are at offsets of the same parity then. The last word read is 2 elements past
+// what the zeroed tail must hold, of its 64 to spare.
+struct Pending3W {
+    uint2 a, b, c, d;
+    unsigned sh;  // bits, in the low 5
+    float rx, ry, rz;
+};
+template <typename T, bool WORDS>
+struct PendSel {
+    using type = Pending3<T>;
+};
+template <>
+struct PendSel<__half, true> {
+    using type = Pending3W;
+};
 
 
 template <typename T>
@@ -217,9 +234,9 @@ __device__ __forceinline__ void ld2_off(const T* __restrict__ base, unsigned idx
     }
 }
 
-template <bool P2, typename T>
+template <bool P2, typename T, typename PEND>
 __device__ __forceinline__ void issue3v(const T* __restrict__ src, const SGeom& s, float px,
-                                        float py, float pz, bool inside, Pending3<T>& p);
+                                        float py, float pz, bool inside, PEND& p);
 
 template <bool P2, typename T>
 __device__ __forceinline__ void issue3(const T* __restrict__ src, const SGeom& s, const float* m,
@@ -256,9 +273,9 @@ __device__ __forceinline__ void corners_off(const T* __restrict__ src, const SGe
 }
 
 // issue3 from the source position (px, py, pz) in mm.
-template <bool P2, typename T>
+template <bool P2, typename T, typename PEND>
 __device__ __forceinline__ void issue3v(const T* __restrict__ src, const SGeom& s, float px,
-                                        float py, float pz, bool inside, Pending3<T>& p) {
+                                        float py, float pz, bool inside, PEND& p) {
     float vx, vy, vz;
     to_voxel<P2>(s, px, py, pz, vx, vy, vz);
     const float xm = (float)(s.X - 1), ym = (float)(s.Y - 1), zm = (float)(s.Z - 1);
@@ -284,7 +301,14 @@ __device__ __forceinline__ void issue3v(const T* __restrict__ src, const SGeom& 
     unsigned o0, o1;
     const char *b0, *b1;
     corners_off(src, s, e0, sxy, o0, o1, b0, b1);
-    if constexpr (sizeof(T) == 2) {
+    if constexpr (std::is_same<PEND, Pending3W>::value) {
+        p.sh = o0 << 3;
+        const unsigned q0 = o0 & ~3u, q1 = o1 & ~3u;
+        __builtin_memcpy(&p.a, __builtin_assume_aligned(b0 + q0, 4), 8);
+        __builtin_memcpy(&p.b, __builtin_assume_aligned(b0 + q1, 4), 8);
+        __builtin_memcpy(&p.c, __builtin_assume_aligned(b1 + q0, 4), 8);
+        __builtin_memcpy(&p.d, __builtin_assume_aligned(b1 + q1, 4), 8);
+    } else if constexpr (sizeof(T) == 2) {
         __builtin_memcpy(&p.a, b0 + o0, 4);  // (y0, z0)
         __builtin_memcpy(&p.b, b0 + o1, 4);  // (y0, z0 + 1)
         __builtin_memcpy(&p.c, b1 + o0, 4);  // (y0 + 1, z0)
@@ -304,9 +328,9 @@ __device__ __forceinline__ void issue3v(const T* __restrict__ src, const SGeom& 
 
 // issue3 with the in-plane part of the source coordinates given: c = m*(lx, ly, 0) as
 // issue3 forms it, so px = fmaf(m[2], lz, c[0]) + m[3] is issue3's px bit for bit.
-template <bool P2, typename T>
+template <bool P2, typename T, typename PEND>
 __device__ __forceinline__ void issue3c(const T* __restrict__ src, const SGeom& s, const float* m,
-                                        const float* c, float lz, bool inside, Pending3<T>& p) {
+                                        const float* c, float lz, bool inside, PEND& p) {
     const float px = fmaf(m[2], lz, c[0]) + m[3];
     const float py = fmaf(m[6], lz, c[1]) + m[7];
     const float pz = fmaf(m[10], lz, c[2]) + m[11];
@@ -330,6 +354,17 @@ __device__ __forceinline__ float finish3(const Pending3<T>& p) {
     const float yl = fmaf(p.ry, lb - lu, lu);
     const float yr = fmaf(p.ry, rb - ru, ru);
     return fmaf(p.rx, yr - yl, yl);
+}
+__device__ __forceinline__ float finish3(const Pending3W& p) {
+    Pending3<__half> q;
+    q.a = __builtin_amdgcn_alignbit(p.a.y, p.a.x, p.sh);
+    q.b = __builtin_amdgcn_alignbit(p.b.y, p.b.x, p.sh);
+    q.c = __builtin_amdgcn_alignbit(p.c.y, p.c.x, p.sh);
+    q.d = __builtin_amdgcn_alignbit(p.d.y, p.d.x, p.sh);
+    q.rx = p.rx;
+    q.ry = p.ry;
+    q.rz = p.rz;
+    return finish3(q);
 }
 
 // Interpolate_2Dkernel sample (interpolator.cu:186-230): bilinear, y then x. The 2x3

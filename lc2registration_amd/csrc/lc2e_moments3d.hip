@@ -22,7 +22,7 @@ constexpr int kGradX = 32, kGradY = 16;  // output tile of k_warp_grad3
 // column; the gathers of the next plane are in flight during the Sobel of this one, and the
 // two LDS planes take one barrier per step. Bound by VALU issue (102 instructions per voxel,
 // 73% of the issue slots): 365 us for 16 poses of 192x192x160, 2 TB/s written.
-template <typename T, bool P2>
+template <typename T, bool P2, bool WORDS>
 __global__ __launch_bounds__(256) void k_warp_grad3(FusedArgs a, int ntx, int nty, int zc, int tiles,
                                                     int npose) {
     constexpr int IXE = kGradX + 2, IYE = kGradY + 2, NI = IXE * IYE;
@@ -54,7 +54,7 @@ __global__ __launch_bounds__(256) void k_warp_grad3(FusedArgs a, int ntx, int nt
         cxy[j][1] = fmaf(m[5], Ly, m[4] * Lx);
         cxy[j][2] = fmaf(m[9], Ly, m[8] * Lx);
     }
-    Pending3<T> pend[SPT];
+    typename PendSel<T, WORDS>::type pend[SPT];
     auto has = [&](int j) { return (j + 1) * 256 <= NI || j * 256 + wbase < NI; };
     auto issue = [&](int z) {
         const bool zin = z >= 0 && z < Z;
@@ -434,10 +434,10 @@ __global__ __launch_bounds__((Mom<R, ROLE>::NTHR)) void k_moments3d(FusedArgs a)
     }
 }
 
-template <typename T, bool P2>
+template <typename T, bool P2, bool WORDS = false>
 void warp_grad3(const FusedArgs& a, int ntx, int nty, int zc, int tiles, int n, hipStream_t st) {
     const int tiles8 = (tiles + kXcds - 1) / kXcds * kXcds;
-    hipLaunchKernelGGL((k_warp_grad3<T, P2>), dim3((unsigned)tiles8 * n), dim3(256), 0, st, a, ntx, nty,
+    hipLaunchKernelGGL((k_warp_grad3<T, P2, WORDS>), dim3((unsigned)tiles8 * n), dim3(256), 0, st, a, ntx, nty,
                        zc, tiles, n);
 }
 
@@ -486,6 +486,13 @@ hipError_t launch_warp3(const FusedArgs& a, int movi, int n, hipStream_t st) {
     const int zc = std::max(8, (a.v.Z + want - 1) / want);
     const int tiles = ntx * nty * ((a.v.Z + zc - 1) / zc);
     const int form = (movi ? 4 : 0) + (a.s.pow2 ? 2 : 0) + (a.src_f16 ? 1 : 0);
+    // half sources of even X in aligned words: 8 poses of the CT 660 -> 610 us
+    const bool words = movi && a.src_f16 && a.s.X % 2 == 0;
+    if (words) {
+        if (a.s.pow2) warp_grad3<__half, true, true>(a, ntx, nty, zc, tiles, n, st);
+        else warp_grad3<__half, false, true>(a, ntx, nty, zc, tiles, n, st);
+        return hipGetLastError();
+    }
     switch (form) {
         case 7: warp_grad3<__half, true>(a, ntx, nty, zc, tiles, n, st); break;
         case 6: warp_grad3<float, true>(a, ntx, nty, zc, tiles, n, st); break;

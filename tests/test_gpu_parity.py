@@ -716,3 +716,25 @@ def test_upload_finds_the_voxel_out_of_range(engine, n, at):
         v = engine.upload(a, **geom)
         assert (engine.memory()[0] - used) == (n + n + n + 64) * size
         v.close()
+
+
+@pytest.mark.parametrize("mx", [40, 41])
+@pytest.mark.parametrize("spacing", [1.0, 0.8])
+def test_3d_half_source_of_even_and_odd_rows_equals_single_precision(engine, mx, spacing):
+    """Half storage of whole numbers, read in aligned words (even rows) or pair by pair: the bits
+    of the same volume in single precision, at poses that leave it on every side."""
+    rng = np.random.default_rng(mx)
+    mov = rng.integers(-1000, 1000, (23, 31, mx)).astype(np.int16)
+    us = rng.integers(1, 256, (30, 28, 37)).astype(np.uint8)
+    fv = engine.upload(us, (0.9, 0.9, 0.9), (0.0, 0.0, 0.0))
+    got = []
+    for data, store in ((mov, E.STORE_AUTO), (mov.astype(np.float32), E.F16), (mov.astype(np.float32), E.F32)):
+        mv = engine.upload(data, (spacing,) * 3, (0.0, 0.0, 0.0), store)
+        p = engine.pair(fv, mv, (0.9, 0.9, 0.9), True, False, 2, 3)
+        poses = [[0.1 * k, -0.05 * k, 0.07 * k, 4.0 * (k - 2), 3.0 - k, 2.0 * k] for k in range(5)]
+        got.append(p.eval_batch(np.stack([p.pose_to_matrix(np.array(q)) for q in poses])).lc2)
+        p.close()
+        mv.close()
+    fv.close()
+    assert np.all(got[2] > 0.0)
+    assert np.array_equal(got[0], got[2]) and np.array_equal(got[1], got[2])
