@@ -562,6 +562,7 @@ __device__ __forceinline__ bool combine_static_u(const double* S, double mu, dou
 // The part of the fit that a static high-resolution image decides, from its channels I, G, II,
 // GG, IG: patch means and the coefficients of e = A p^2 + B p q + C q^2, the explained part of
 // an ultrasound with the centred products p = C_UI, q = C_UG (explained_var with its rank rule).
+// A is 0 exactly where the column I is dropped, C where G is.
 __device__ __forceinline__ void store_image_stats(const double* S, int N, double* out, long long stride) {
     const double inv_n = 1.0 / (double)N;
     const double si = S[0], sg = S[1], mi = si * inv_n, mg = sg * inv_n;
@@ -608,7 +609,9 @@ __device__ __forceinline__ bool combine_static_image(const double* S, const Imag
     const double su = S[0], my = su * inv_n;
     const double cyy = fma(-my, su, S[1]);
     const bool ok = cyy * inv_n1 > kZeroThreshold;
-    const double p = fma(-t.mi, su, S[2]), q = fma(-t.mg, su, S[3]);
+    // a column left out of the fit may hold infinities (|Sobel| past single precision's range),
+    // which its zero coefficient would turn into NaN
+    const double p = t.A == 0.0 ? 0.0 : fma(-t.mi, su, S[2]), q = t.C == 0.0 ? 0.0 : fma(-t.mg, su, S[3]);
     const double e = fma(fma(t.B, q, t.A * p), p, (t.C * q) * q);
     weight_measure(ok ? cyy : 1.0, e, inv_n1, w_out, m_out);
     return ok;
