@@ -181,6 +181,7 @@ struct lc2e_volume {
     void* d = nullptr;
     size_t bytes = 0;
     int f16 = 0;
+    bool large = false;  // a voxel exceeds kHalfRange
     lc2e_geom g{};
 };
 
@@ -870,8 +871,8 @@ int lc2e_volume_upload(lc2e_engine* e, const void* host, lc2e_dtype dtype, const
     if (storage != LC2E_STORE_AUTO && storage != LC2E_F16 && storage != LC2E_F32)
         return fail(LC2E_ERR_INVALID, "storage must be F16, F32 or AUTO");
     HIP_TRY(hipSetDevice(e->device));
-    // The raw voxels on the device (also its conversion's input) and a word that the kernels
-    // set where a voxel is out of range: the device reads them at the memory's rate, where a
+    // The raw voxels on the device (also its conversion's input) and two words that the kernels
+    // set where a voxel is out of range (launch_check): the device reads them at the memory's rate, where a
     // scan on the host took half of an upload.
     struct Scope {
         lc2e_engine* e;
@@ -880,13 +881,13 @@ int lc2e_volume_upload(lc2e_engine* e, const void* host, lc2e_dtype dtype, const
         int* flag = nullptr;
         ~Scope() {
             e->raw_free(staging, bytes);
-            e->host_free(flag, sizeof(int));
+            e->host_free(flag, 2 * sizeof(int));
         }
     } tmp{e};
-    HIP_TRY(e->host_alloc((void**)&tmp.flag, sizeof(int)));
+    HIP_TRY(e->host_alloc((void**)&tmp.flag, 2 * sizeof(int)));
     void* flag_dev = nullptr;
     HIP_TRY(hipHostGetDevicePointer(&flag_dev, tmp.flag, 0));
-    *tmp.flag = 0;
+    tmp.flag[0] = tmp.flag[1] = 0;
     auto stage = [&]() {
         tmp.bytes = (size_t)n * dsz;
         hipError_t err = e->raw_alloc(&tmp.staging, tmp.bytes);
@@ -970,6 +971,7 @@ int lc2e_volume_upload(lc2e_engine* e, const void* host, lc2e_dtype dtype, const
         if (err == hipSuccess && (rc = bad_voxel()) < 0) return rc;
         return fail(LC2E_ERR_HIP, "volume upload failed: %s", hipGetErrorString(err));
     }
+    v->large = tmp.flag[1] != 0;
     *out = v;
     return LC2E_OK;
 }
@@ -1008,9 +1010,11 @@ int lc2e_pair_create(lc2e_engine* e, lc2e_volume* fixed, lc2e_volume* moving,
     const long long V = (long long)pg.virt.dims[0] * pg.virt.dims[1] * pg.virt.dims[2];
     if (V >= (1LL << 31)) return fail(LC2E_ERR_UNSUPPORTED, "virtual grid exceeds 2^31 voxels");
 
-    // (the 3D moments kernel addresses a plane of the grid with 32-bit byte offsets)
+    // (the 3D moments kernel addresses a plane of the grid with 32-bit byte offsets; where two
+    // voxels may differ by more than single precision holds, the separable path's sampler, which
+    // reads only the neighbours a sample needs, keeps the radii beyond the fused kernels)
     const bool big_plane = dim == 3 && (long long)pg.virt.dims[0] * pg.virt.dims[1] >= (1LL << 28);
-    const bool moments = patch_radius <= two_max && !big_plane;
+    const bool moments = patch_radius <= two_max && !big_plane && (small_r || !moving->large);
     const bool sep = big_slices || (!small_r && !moments);
     auto* p = new lc2e_pair();
     p->gen = g_generation.fetch_add(1);
@@ -1255,9 +1259,10 @@ int lc2e_eval_mi_batch(lc2e_pair* p, int n, const float* mats, int bins_us, int 
     // Without a budget the warped image is kept between the two passes over it (3D), a float per
     // voxel and pose; what does not fit goes in parts. A buffer of its own: evaluations on a
     // caller's stream may be using the pair's workspace.
-    // (Sources of large slices are beyond the pipelined sampler's offsets: warped twice.)
+    // (Sources of large slices are beyond the pipelined sampler's offsets, those of large voxels
+    // beyond its range: warped twice.)
     int step = std::min(n, chunk_max);
-    if (!e->budget && p->info.grid_ndim == 3 && (long long)p->sg.X * p->sg.Y < lc2e::kMaxFusedSlice) {
+    if (!e->budget && p->info.grid_ndim == 3 && !p->moving->large && (long long)p->sg.X * p->sg.Y < lc2e::kMaxFusedSlice) {
         const size_t per = p->voxels() * sizeof(float);
         const int want = (int)std::min<size_t>((size_t)step, std::max<size_t>(1, kMiWarpBytes / per));
         if (want > p->mi_warp_poses) {

@@ -904,7 +904,7 @@ __device__ __forceinline__ void for_vectors(long long n, int per, F&& f) {
 }
 
 __global__ __launch_bounds__(256) void k_check(const void* in, int in_dtype, long long n, float lim, int* flag) {
-    bool bad = false;
+    bool bad = false, large = false;
     const int per = in_dtype == 3 ? 4 : 8;
     for_vectors(n, per, [&](long long i0, long long m) {
         if (m == per) {
@@ -913,7 +913,10 @@ __global__ __launch_bounds__(256) void k_check(const void* in, int in_dtype, lon
                 float x[4];
                 __builtin_memcpy(x, &w, 16);
 #pragma unroll
-                for (int k = 0; k < 4; ++k) bad |= !(fabsf(x[k]) <= lim);
+                for (int k = 0; k < 4; ++k) {
+                    bad |= !(fabsf(x[k]) <= lim);
+                    large |= fabsf(x[k]) > kHalfRange;
+                }
             } else {
                 short x[8];
                 __builtin_memcpy(x, &w, 16);
@@ -925,10 +928,15 @@ __global__ __launch_bounds__(256) void k_check(const void* in, int in_dtype, lon
                 }
             }
         } else {
-            for (long long i = i0; i < i0 + m; ++i) bad |= !(fabsf(raw_value(in, in_dtype, i)) <= lim);
+            for (long long i = i0; i < i0 + m; ++i) {
+                const float x = fabsf(raw_value(in, in_dtype, i));
+                bad |= !(x <= lim);
+                large |= x > kHalfRange;
+            }
         }
     });
-    if (__any(bad) && (threadIdx.x & 63) == 0) *flag = 1;
+    if (__any(bad) && (threadIdx.x & 63) == 0) flag[0] = 1;
+    if (__any(large) && (threadIdx.x & 63) == 0) flag[1] = 1;
 }
 
 __global__ void k_convert(const void* in, int in_dtype, void* out, int out_f16, long long n) {

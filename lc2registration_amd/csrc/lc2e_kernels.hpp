@@ -177,7 +177,10 @@ inline int mi_hist_size(int bins_u, int bins_i) {  // with room for a group of b
 hipError_t launch_mi(const FusedArgs& a, int grid_ndim, int src_ndim, int high_res_is_moving,
                      int n_poses, int bins_u, int bins_i, const float* stat, int* ext_stat,
                      int stat_ready, int* ext_mov, unsigned* hist, double* out, hipStream_t st);
-// Sets *flag if a voxel of d_in exceeds lim in magnitude or is not a number.
+// Sets flag[0] if a voxel of d_in exceeds lim in magnitude or is not a number, flag[1] if one
+// exceeds kHalfRange: two such voxels may differ by more than single precision holds, and the
+// pipelined samplers, which weigh a neighbour the sample does not need by 0, give NaN there.
+constexpr float kHalfRange = 1.7014117e38f;
 hipError_t launch_check(const void* d_in, int in_dtype, long long n, float lim, int* flag, hipStream_t st);
 // Host bytes -> resident storage (u8/i16/f16/f32 -> f16/f32).
 hipError_t launch_convert(const void* d_in, int in_dtype, void* d_out, int out_f16, long long n,
