@@ -147,8 +147,11 @@ int lc2e_eval_batch(lc2e_pair* p, int n, const float* mats, double* lc2, double*
  * cannot allocate device memory (code under HIP graph capture, tight serving loops, harnesses
  * that forbid hipMalloc). The launch's matrices, partial sums and results live in a fixed
  * device array of the library (16 MiB per device, held until the process ends) instead of
- * the pair's batch buffers; the call uses no hipMalloc/hipFree and no allocating library
- * routine. Same kernels, so the results are bit-identical to lc2e_eval_batch. A call needs
+ * the pair's batch buffers, and the warped images that the two-kernel path writes in a workspace of
+ * the engine that is made with the pair, not in the pair's own: the call may run beside a
+ * launch of the same pair on a caller's stream (except on the separable path, and at 3D radii 5
+ * and 6 under a budget, whose buffers every launch of a pair shares). The call uses no
+ * hipMalloc/hipFree and no allocating library routine. Same kernels, so the results are bit-identical to lc2e_eval_batch. A call needs
  * n*(24 + 48*mats_per_pose) + n*16*(partial sums per pose) bytes (each part rounded up to
  * 256); a larger call fails with LC2E_ERR_INVALID. Every call on a device shares that
  * device's array: concurrent calls would race on it, so the library serialises them per
@@ -158,8 +161,8 @@ int lc2e_eval_batch_noalloc(lc2e_pair* p, int n, const float* mats, double* lc2,
 
 /* Stream-ordered form for serving loops: d_mats and d_out are DEVICE pointers,
  * d_out receives 3 doubles per pose (sum_measure, sum_w, lc2). `stream` is a hipStream_t
- * (NULL = the engine's stream). Nothing is synchronised. The pair's partial-sum buffer is
- * shared by its launches: two launches of ONE pair must not overlap (enqueue them on one
+ * (NULL = the engine's stream). Nothing is synchronised. The pair's partial-sum buffer and
+ * workspace are shared by its launches: two launches of ONE pair must not overlap (enqueue them on one
  * stream, or wait for the first); launches of different pairs may run concurrently. A
  * batch larger than any before it on this pair grows that buffer first (hipFree and
  * hipMalloc, which wait for the device). */

@@ -60,6 +60,11 @@ struct lc2e_engine {
     // then scratch_error says why)
     void* scratch = nullptr;
     std::string scratch_error;
+    // workspace of lc2e_eval_batch_noalloc for the pairs that need one (na_pairs of them); its
+    // calls on a device run one at a time, so one serves them all (guarded by noalloc_lock)
+    void* na = nullptr;
+    size_t na_bytes = 0;
+    int na_pairs = 0;
     size_t budget = 0;  // 0 = unlimited
     size_t used = 0;
     std::mutex mu;      // guards `used`: a serving loop allocates from its own thread
@@ -244,6 +249,7 @@ struct lc2e_pair {
     void* ws = nullptr;
     size_t ws_bytes = 0;
     int ws_poses = 0;
+    bool na = false;  // counted in the engine's na_pairs
     double* istat = nullptr;
     int resident_per_cu = 0;  // fused work-groups one CU holds at once (0: not queried yet)
     // separable path (radius beyond the fused kernels): grids and box-sum buffers, made at
@@ -296,24 +302,30 @@ lc2e::FusedArgs make_args(lc2e_pair* p, const float* d_mats, double* d_partials,
 // in place, 58 us through the grid; moving, 128 frames 512x384, r = 6, 3 poses: 1.99 ms in
 // place, 1.59 ms through the grid). The same values either way, bit for bit.
 constexpr long long kInPlaceWaves = 2048;
-bool in_place(const lc2e_pair* p, int tiles, int n) {
-    return p->info.grid_ndim == 2 && (!p->ws || (long long)tiles * 4 * n < kInPlaceWaves);
+struct Workspace {
+    void* d;
+    int poses;
+};
+bool in_place(const lc2e_pair* p, const Workspace& w, int tiles, int n) {
+    return p->info.grid_ndim == 2 && (!w.d || (long long)tiles * 4 * n < kInPlaceWaves);
 }
 
 // The pair's evaluation kernels for n poses: the fused kernel, or the separable path for
 // radii beyond it.
-hipError_t launch_eval(lc2e_pair* p, const lc2e::FusedArgs& a, int n, hipStream_t st) {
-    if (p->two && in_place(p, a.tiles, n)) {
+hipError_t launch_eval(lc2e_pair* p, const lc2e::FusedArgs& a, int n, hipStream_t st, const Workspace& w) {
+    if (p->two && in_place(p, w, a.tiles, n)) {
         lc2e::FusedArgs s = a;
         s.in_place = 1;
         return lc2e::launch_moments(s, p->info.grid_ndim, p->role(), n, st);
     }
     if (p->two) {
         // as many poses at a time as the workspace holds, in equal parts
-        const int parts = (n + p->ws_poses - 1) / p->ws_poses, step = (n + parts - 1) / parts;
+        const int parts = (n + w.poses - 1) / w.poses, step = (n + parts - 1) / parts;
         for (int b = 0; b < n; b += step) {
             const int m = std::min(step, n - b);
             lc2e::FusedArgs s = a;
+            s.warp2 = static_cast<float2*>(w.d);
+            s.warp1 = static_cast<float*>(w.d);
             s.mats = a.mats + (size_t)b * a.mats_per_pose * 12;
             if (b) s.inline_mat = 0;
             s.partials = a.partials + (size_t)b * a.blocks_per_pose * 2;
@@ -527,7 +539,51 @@ int grow_workspace(lc2e_pair* p, int n) {
     return LC2E_OK;
 }
 
+std::mutex& noalloc_lock(int device) {
+    static std::mutex locks[64];
+    return locks[device & 63];
+}
+
+// Room in the engine's workspace of the allocation-free entry point for one pose of the pair.
+// Its calls do not touch the pair's own workspace, which launches on a caller's stream may be
+// using at the same time.
+int reserve_noalloc(lc2e_pair* p) {
+    lc2e_engine* e = p->e;
+    std::lock_guard<std::mutex> lk(noalloc_lock(e->device));
+    if (e->na_bytes < p->ws_bytes) {
+        void* d = nullptr;
+        if (e->raw_alloc(&d, p->ws_bytes) != hipSuccess) {
+            (void)hipGetLastError();
+            return fail(LC2E_ERR_HIP, "workspace of %zu bytes", p->ws_bytes);
+        }
+        e->raw_free(e->na, e->na_bytes);
+        e->na = d;
+        e->na_bytes = p->ws_bytes;
+    }
+    p->na = true;
+    ++e->na_pairs;
+    return LC2E_OK;
+}
+void release_noalloc(lc2e_pair* p) {
+    if (!p->na) return;
+    lc2e_engine* e = p->e;
+    std::lock_guard<std::mutex> lk(noalloc_lock(e->device));
+    p->na = false;
+    if (--e->na_pairs) return;
+    e->raw_free(e->na, e->na_bytes);
+    e->na = nullptr;
+    e->na_bytes = 0;
+}
+// Under noalloc_lock. Without a reservation: 2D launches warp in place; the others share the
+// pair's workspace, as radii beyond the fused kernels share their box-sum buffers.
+Workspace noalloc_workspace(const lc2e_pair* p) {
+    if (p->na) return {p->e->na, 1};
+    if (p->info.grid_ndim == 2) return {nullptr, 0};
+    return {p->ws, p->ws_poses};
+}
+
 void free_two(lc2e_pair* p) {
+    release_noalloc(p);
     two_free(p, p->ws, (size_t)p->ws_poses * p->ws_bytes);
     two_free(p, p->istat, lc2e::kImageStats * p->voxels() * sizeof(double));
     p->ws = nullptr;
@@ -564,6 +620,7 @@ int make_two_kernel(lc2e_pair* p, bool required) {
     p->two = true;
     const bool grid = !two_d || p->info.high_res_is_moving;  // else warped in place
     int rc = grid ? grow_workspace(p, 1) : LC2E_OK;
+    if (rc >= 0 && p->ws && !p->two_charged && reserve_noalloc(p) < 0 && !two_d && !required) rc = LC2E_ERR_HIP;
     if (rc >= 0 && !p->info.high_res_is_moving)
         rc = two_alloc(p, (void**)&p->istat, lc2e::kImageStats * p->voxels() * sizeof(double));
     if (rc < 0) {
@@ -655,8 +712,6 @@ lc2e::FusedArgs make_args(lc2e_pair* p, const float* d_mats, double* d_partials,
     a.blocks_per_pose = t.bpp;
     a.tiles = t.tiles;
     a.mats_per_pose = p->mats_per_pose();
-    a.warp2 = static_cast<float2*>(p->ws);
-    a.warp1 = static_cast<float*>(p->ws);
     a.istat = p->istat;
     a.src3 = p->info.src_ndim == 3 ? 1 : 0;
     a.in_place = p->two && !p->ws && p->info.grid_ndim == 2 ? 1 : 0;
@@ -699,7 +754,7 @@ int enqueue_batch(lc2e_pair* p, int n, const Tiling& t, hipStream_t st, bool cap
         // timed launches are eager (run_batch), the events bracket the fused kernel
         const bool timed = p->profile;
         if (timed) HIP_TRY(hipEventRecord(p->ev0, st));
-        HIP_TRY(launch_eval(p, a, n, st));
+        HIP_TRY(launch_eval(p, a, n, st, {p->ws, p->ws_poses}));
         if (timed) HIP_TRY(hipEventRecord(p->ev1, st));
         if (!host) HIP_TRY(lc2e::launch_reduce(p->d_partials, t.bpp, n, p->h_out_dev, st));
     } else {
@@ -842,6 +897,7 @@ void lc2e_destroy(lc2e_engine* e) {
     (void)hipSetDevice(e->device);
     (void)hipStreamSynchronize(e->stream);
     (void)hipStreamDestroy(e->stream);
+    e->raw_free(e->na, e->na_bytes);
     e->give_back();
     delete e;
 }
@@ -1174,8 +1230,7 @@ int lc2e_eval_batch_noalloc(lc2e_pair* p, int n, const float* mats, double* lc2,
         return fail(LC2E_ERR_HIP, "device scratch unavailable: %s", e->scratch_error.c_str());
     // One device array serves every call on the device: calls are serialised here, so a
     // call that overlaps another one on the same device waits for it.
-    static std::mutex device_locks[64];
-    std::lock_guard<std::mutex> lk(device_locks[e->device & 63]);
+    std::lock_guard<std::mutex> lk(noalloc_lock(e->device));
     HIP_TRY(hipSetDevice(e->device));
     hipStream_t st = e->stream;
     const int mpp = p->mats_per_pose();
@@ -1200,7 +1255,7 @@ int lc2e_eval_batch_noalloc(lc2e_pair* p, int n, const float* mats, double* lc2,
         // every partial slot is written by the fused kernel before k_reduce reads it, so the
         // previous call's contents need no clearing
         const lc2e::FusedArgs a = make_args(p, d_mats, d_part, t);
-        HIP_TRY(launch_eval(p, a, n, st));
+        HIP_TRY(launch_eval(p, a, n, st, noalloc_workspace(p)));
     }
     HIP_TRY(lc2e::launch_reduce(d_part, t.tiles > 0 ? t.bpp : 0, n, d_out, st));
     // results back through a fixed host buffer, a chunk of poses at a time
@@ -1232,7 +1287,7 @@ int lc2e_eval_batch_async(lc2e_pair* p, int n, const float* d_mats, double* d_ou
     if (rc < 0) return rc;
     if (t.tiles > 0) {
         lc2e::FusedArgs a = make_args(p, d_mats, p->d_partials, t);
-        HIP_TRY(launch_eval(p, a, n, st));
+        HIP_TRY(launch_eval(p, a, n, st, {p->ws, p->ws_poses}));
     }
     HIP_TRY(lc2e::launch_reduce(p->d_partials, t.tiles > 0 ? t.bpp : 0, n, d_out, st));
     return LC2E_OK;
@@ -1359,7 +1414,7 @@ int lc2e_debug_fetch(lc2e_pair* p, lc2e_stage stage, const float* m12, void* hos
     a.wmap = maps;
     a.mmap = maps + V;
     if (err == hipSuccess && t.tiles > 0)
-        err = launch_eval(p, a, 1, st);
+        err = launch_eval(p, a, 1, st, {p->ws, p->ws_poses});
     if (err == hipSuccess)
         err = hipMemcpyAsync(host, stage == LC2E_STAGE_W ? a.wmap : a.mmap, V * sizeof(double),
                              hipMemcpyDeviceToHost, st);
@@ -1425,9 +1480,9 @@ int lc2e_pair_autotune(lc2e_pair* p, int n, const float* mats, int iters, int* b
         HIP_TRY(hipMemcpy(p->d_mats, mats, (size_t)n * p->mats_per_pose() * 12 * sizeof(float),
                           hipMemcpyHostToDevice));
         lc2e::FusedArgs a = make_args(p, p->d_mats, p->d_partials, t);
-        HIP_TRY(launch_eval(p, a, n, st));
+        HIP_TRY(launch_eval(p, a, n, st, {p->ws, p->ws_poses}));
         HIP_TRY(hipEventRecord(e0, st));
-        for (int it = 0; it < iters; ++it) HIP_TRY(launch_eval(p, a, n, st));
+        for (int it = 0; it < iters; ++it) HIP_TRY(launch_eval(p, a, n, st, {p->ws, p->ws_poses}));
         HIP_TRY(hipEventRecord(e1, st));
         HIP_TRY(hipEventSynchronize(e1));
         float ms = 0.0f;

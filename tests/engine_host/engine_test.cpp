@@ -1,0 +1,140 @@
+// Scenarios of the engine's host code (lc2e_engine.cpp and the kernels' launchers) on the fake
+// runtime; the name of one is the argument.
+#include <cstdio>
+#include <cstdlib>
+#include <cstring>
+#include <functional>
+#include <map>
+#include <string>
+#include <vector>
+
+#include "fake_hip.hpp"
+#include "lc2e.h"
+
+namespace {
+
+#define CHECK(x)                                                                  \
+    do {                                                                          \
+        if (!(x)) {                                                               \
+            std::printf("%s:%d: %s (%s)\n", __FILE__, __LINE__, #x, lc2e_last_error()); \
+            std::exit(1);                                                         \
+        }                                                                         \
+    } while (0)
+
+constexpr size_t GB = size_t(1) << 30, MB = size_t(1) << 20;
+
+lc2e_engine* engine(size_t budget = 0, int device = 0) {
+    lc2e_engine* e = nullptr;
+    CHECK(lc2e_create(device, budget, &e) == LC2E_OK);
+    return e;
+}
+
+// A pair on a grid of the given size: the images are as small as they can be, the grid's
+// spacing does the rest.
+struct Pair {
+    lc2e_volume *f = nullptr, *m = nullptr;
+    lc2e_pair* p = nullptr;
+    int frames = 1;
+
+    Pair(lc2e_engine* e, int dim, int x, int y, int z, int movi, int r, bool src3, bool tracked = false) {
+        CHECK(make(e, dim, x, y, z, movi, r, src3, tracked) >= 0);
+    }
+    Pair() = default;
+    int make(lc2e_engine* e, int dim, int x, int y, int z, int movi, int r, bool src3, bool tracked = false) {
+        const bool stack = dim == 2 && z > 1;
+        std::vector<float> img(size_t(stack ? z : 1) * 64 + 4096, 1.0f);
+        lc2e_geom g{};
+        const int d[3] = {4, 4, dim == 3 ? 4 : z};
+        const int n[3] = {x, y, z};
+        float rs[3] = {1, 1, 1};
+        for (int a = 0; a < 3; ++a) {
+            g.dims[a] = d[a];
+            g.spacing[a] = 1.0f;
+            if (a < dim) rs[a] = (float)d[a] / ((float)n[a] - 0.5f);  // the grid's size is rounded up
+        }
+        int rc = lc2e_volume_upload(e, img.data(), LC2E_F32, &g, LC2E_STORE_AUTO, &f);
+        if (rc < 0) return rc;
+        lc2e_geom h{};
+        for (int a = 0; a < 3; ++a) {
+            h.dims[a] = a < 2 || src3 ? 8 : 1;
+            h.spacing[a] = 1.0f;
+        }
+        if ((rc = lc2e_volume_upload(e, img.data(), LC2E_F32, &h, LC2E_STORE_AUTO, &m)) < 0) return rc;
+        if ((rc = lc2e_pair_create(e, f, m, rs, movi, 0, r, dim, &p)) < 0) return rc;
+        lc2e_pair_info info{};
+        CHECK(lc2e_pair_get_info(p, &info) == LC2E_OK);
+        for (int a = 0; a < 3; ++a) CHECK(info.virt.dims[a] == n[a]);
+        if (tracked) CHECK(lc2e_pair_set_per_frame(p, 1) == LC2E_OK);
+        frames = tracked ? z : 1;
+        return LC2E_OK;
+    }
+    std::vector<float> mats(int n) const { return std::vector<float>(size_t(n) * frames * 12, 0.0f); }
+    int batch(int n) { return lc2e_eval_batch(p, n, mats(n).data(), nullptr, nullptr, nullptr); }
+    int noalloc(int n) { return lc2e_eval_batch_noalloc(p, n, mats(n).data(), nullptr, nullptr, nullptr); }
+    int async(int n, hipStream_t st) {
+        static float d_mats[64 * 12];
+        static double d_out[64 * 3];
+        return lc2e_eval_batch_async(p, n, d_mats, d_out, st);
+    }
+    int mi(int n) {
+        std::vector<double> out(n);
+        return lc2e_eval_mi_batch(p, n, mats(n).data(), 256, 256, out.data());
+    }
+    ~Pair() {
+        if (p) lc2e_pair_destroy(p);
+        if (m) lc2e_volume_destroy(m);
+        if (f) lc2e_volume_destroy(f);
+    }
+};
+
+// The allocation-free entry point may run while a launch of the same pair is in flight on a
+// caller's stream: they must not write the same warped image.
+void noalloc_has_its_own_workspace() {
+    lc2e_engine* e = engine();
+    hipStream_t st = nullptr;
+    CHECK(hipStreamCreateWithFlags(&st, 0) == hipSuccess);
+    struct {
+        int dim, x, y, z, movi, r;
+        bool src3;
+    } cases[] = {{3, 64, 64, 64, 1, 3, true}, {3, 64, 64, 64, 0, 2, true}, {3, 48, 48, 48, 1, 5, true},
+                 {2, 512, 512, 1, 1, 5, false}, {2, 256, 200, 40, 1, 9, true}};
+    for (const auto& c : cases) {
+        Pair p(e, c.dim, c.x, c.y, c.z, c.movi, c.r, c.src3);
+        const size_t bytes = size_t(c.x) * c.y * c.z * (c.movi ? 8 : 4);
+        fake::launches().clear();
+        CHECK(p.async(20, st) >= 0);
+        CHECK(p.noalloc(20) >= 0);
+        int own = 0, callers = 0;
+        for (const auto& a : fake::launches()) {
+            if (!a.is("k_moments") || !a.a.warp1 || a.a.in_place) continue;
+            (a.stream == st ? callers : own)++;
+            for (const auto& b : fake::launches())
+                if (b.is("k_warp") && (a.stream == st) != (b.stream == st)) {
+                    const char *u = (const char*)a.a.warp1, *v = (const char*)b.a.warp1;
+                    CHECK(u + bytes <= v || v + bytes <= u);
+                }
+        }
+        CHECK(callers > 0 && own > 0);
+    }
+    hipStreamDestroy(st);
+    lc2e_destroy(e);
+    CHECK(fake::used(0) == 0);
+}
+
+//@SCENARIOS
+
+const std::map<std::string, std::function<void()>> kScenarios = {
+    {"noalloc_has_its_own_workspace", noalloc_has_its_own_workspace},
+//@TABLE
+};
+
+}  // namespace
+
+int main(int argc, char** argv) {
+    const auto it = kScenarios.find(argc > 1 ? argv[1] : "");
+    if (it == kScenarios.end()) return std::printf("no such scenario\n"), 2;
+    fake::reset(64 * GB);
+    it->second();
+    std::printf("%s passed\n", argv[1]);
+    return 0;
+}

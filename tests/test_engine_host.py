@@ -1,0 +1,40 @@
+"""The engine's host code on a fake HIP runtime (tests/engine_host): the built library is linked
+behind it, so the decisions of lc2e_engine.cpp and of the kernels' launchers -- which memory a
+launch uses, how a batch is split, what happens where memory runs out -- are the real ones, and
+no GPU is needed."""
+import os
+import shutil
+import subprocess
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+HERE = os.path.join(ROOT, "tests", "engine_host")
+LIB = os.path.join(ROOT, "lc2registration_amd", "_lib")
+
+
+@pytest.fixture(scope="module")
+def engine_test(tmp_path_factory):
+    cxx = shutil.which("g++")
+    if cxx is None or not os.path.isdir("/opt/rocm/include/hip"):
+        pytest.skip("a host C++ compiler and the HIP headers are needed")
+    if not os.path.exists(os.path.join(LIB, "liblc2e.so")):
+        from lc2registration_amd import build
+        build.build()
+    exe = str(tmp_path_factory.mktemp("engine_host") / "engine_test")
+    subprocess.run([cxx, "-std=c++17", "-O1", "-Wall", "-Wextra", "-Wno-unused-parameter",
+                    "-Wno-unused-result", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include",
+                    "-I" + os.path.join(ROOT, "include"),
+                    "-I" + os.path.join(ROOT, "lc2registration_amd", "csrc"),
+                    os.path.join(HERE, "fake_hip.cpp"), os.path.join(HERE, "engine_test.cpp"),
+                    "-o", exe, "-rdynamic", "-pthread", "-L" + LIB, "-llc2e", "-Wl,-rpath," + LIB,
+                    "-Wl,--allow-shlib-undefined"], check=True, timeout=240)
+    return exe
+
+
+@pytest.mark.parametrize("scenario", [
+    "noalloc_has_its_own_workspace",
+])
+def test_engine_host(engine_test, scenario):
+    r = subprocess.run([engine_test, scenario], capture_output=True, text=True, timeout=120)
+    assert r.returncode == 0 and f"{scenario} passed" in r.stdout, r.stdout + r.stderr
