@@ -306,8 +306,14 @@ struct Workspace {
     void* d;
     int poses;
 };
+// Launches of more poses than the workspace holds go through it in equal parts; `part` is their
+// size, and what decides on a launch's shape.
+int part(const Workspace& w, int n) {
+    const int parts = w.poses > 0 ? (n + w.poses - 1) / w.poses : 1;
+    return (n + parts - 1) / parts;
+}
 bool in_place(const lc2e_pair* p, const Workspace& w, int tiles, int n) {
-    return p->info.grid_ndim == 2 && (!w.d || (long long)tiles * 4 * n < kInPlaceWaves);
+    return p->info.grid_ndim == 2 && (!w.d || (long long)tiles * 4 * part(w, n) < kInPlaceWaves);
 }
 
 // The pair's evaluation kernels for n poses: the fused kernel, or the separable path for
@@ -319,8 +325,7 @@ hipError_t launch_eval(lc2e_pair* p, const lc2e::FusedArgs& a, int n, hipStream_
         return lc2e::launch_moments(s, p->info.grid_ndim, p->role(), n, st);
     }
     if (p->two) {
-        // as many poses at a time as the workspace holds, in equal parts
-        const int parts = (n + w.poses - 1) / w.poses, step = (n + parts - 1) / parts;
+        const int step = part(w, n);
         for (int b = 0; b < n; b += step) {
             const int m = std::min(step, n - b);
             lc2e::FusedArgs s = a;
@@ -418,7 +423,9 @@ int model_zchunk(lc2e_pair* p, int n) {
     return best;
 }
 
-Tiling tiling_for(lc2e_pair* p, int n) {
+// `poses`: what the launch's workspace holds (0: it has none). The partial sums do not depend on
+// n or poses.
+Tiling tiling_for(lc2e_pair* p, int n, int poses) {
     Tiling t;
     const int r = p->info.patch_radius;
     if (p->sep) {  // one partial per 256 output voxels
@@ -428,7 +435,8 @@ Tiling tiling_for(lc2e_pair* p, int n) {
     if (p->info.grid_ndim == 3) {
         auto it = p->tuned.find(n);
         t.zchunk = round_zchunk(p->zchunk_forced > 0 ? p->zchunk_forced
-                                : it != p->tuned.end() ? it->second : model_zchunk(p, n));
+                                : it != p->tuned.end() ? it->second
+                                : model_zchunk(p, p->two ? part({nullptr, poses}, n) : n));
         t.tiles = lc2e::fused_blocks_3d(p->v, r, t.zchunk, &t.ntx, &t.nty, &t.nzc);
         t.bpp = lc2e::fused_partials_3d(p->v, r);
         p->last_zchunk = t.zchunk;
@@ -517,6 +525,12 @@ void two_free(lc2e_pair* p, void* d, size_t bytes) {
 // through it in parts. Only an engine without an HBM budget grows it past one pose.
 constexpr size_t kWorkspaceBytes = size_t(1) << 30;
 constexpr size_t kMiWarpBytes = size_t(1) << 28;  // warped images of the mutual information
+// The allocation-free entry point's workspace is made with the pair, so its size cannot follow the
+// batches: 64 poses within 512 MiB, at least one. A fresh pair's first call, 32 poses: 64^3, R = 3
+// 1820 -> 166 us against parts of one pose (148 in a batch); 192x192x160 4.45 -> 3.10 ms (3.19 with
+// 256 MiB, 2.78 in a batch).
+constexpr size_t kNoallocBytes = size_t(1) << 29;
+constexpr int kNoallocPoses = 64;
 int grow_workspace(lc2e_pair* p, int n) {
     if (p->e->budget) {
         if (!p->two_charged) return LC2E_OK;
@@ -535,7 +549,6 @@ int grow_workspace(lc2e_pair* p, int n) {
     p->ws = d;
     p->ws_bytes = per;
     p->ws_poses = want;
-    p->model_cache.clear();
     return LC2E_OK;
 }
 
@@ -544,22 +557,25 @@ std::mutex& noalloc_lock(int device) {
     return locks[device & 63];
 }
 
-// Room in the engine's workspace of the allocation-free entry point for one pose of the pair.
+// Room in the engine's workspace of the allocation-free entry point for poses of the pair.
 // Its calls do not touch the pair's own workspace, which launches on a caller's stream may be
 // using at the same time.
 int reserve_noalloc(lc2e_pair* p) {
     lc2e_engine* e = p->e;
     std::lock_guard<std::mutex> lk(noalloc_lock(e->device));
-    if (e->na_bytes < p->ws_bytes) {
+    const size_t most = std::max(p->ws_bytes, std::min(kNoallocBytes, kNoallocPoses * p->ws_bytes));
+    for (size_t bytes : {most, p->ws_bytes}) {
+        if (e->na_bytes >= bytes) break;
         void* d = nullptr;
-        if (e->raw_alloc(&d, p->ws_bytes) != hipSuccess) {
+        if (e->raw_alloc(&d, bytes) != hipSuccess) {
             (void)hipGetLastError();
-            return fail(LC2E_ERR_HIP, "workspace of %zu bytes", p->ws_bytes);
+            continue;
         }
         e->raw_free(e->na, e->na_bytes);
         e->na = d;
-        e->na_bytes = p->ws_bytes;
+        e->na_bytes = bytes;
     }
+    if (e->na_bytes < p->ws_bytes) return fail(LC2E_ERR_HIP, "workspace of %zu bytes", p->ws_bytes);
     p->na = true;
     ++e->na_pairs;
     return LC2E_OK;
@@ -577,7 +593,7 @@ void release_noalloc(lc2e_pair* p) {
 // Under noalloc_lock. Without a reservation: 2D launches warp in place; the others share the
 // pair's workspace, as radii beyond the fused kernels share their box-sum buffers.
 Workspace noalloc_workspace(const lc2e_pair* p) {
-    if (p->na) return {p->e->na, 1};
+    if (p->na) return {p->e->na, (int)std::min<size_t>(p->e->na_bytes / p->ws_bytes, 1 << 20)};
     if (p->info.grid_ndim == 2) return {nullptr, 0};
     return {p->ws, p->ws_poses};
 }
@@ -683,10 +699,10 @@ int ensure_batch(lc2e_pair* p, int n, int bpp) {
     return LC2E_OK;
 }
 
-// The same, and the workspace.
-int ensure_capacity(lc2e_pair* p, int n, int bpp) {
+// The same for launches of the pair's kernels, and the workspace.
+int ensure_capacity(lc2e_pair* p, int n) {
     if (p->ws) (void)grow_workspace(p, n);
-    return ensure_batch(p, n, bpp);
+    return ensure_batch(p, n, tiling_for(p, n, p->ws_poses).bpp);
 }
 
 lc2e::FusedArgs make_args(lc2e_pair* p, const float* d_mats, double* d_partials, const Tiling& t) {
@@ -844,12 +860,9 @@ int engine_device(lc2e_engine* e) { return e->device; }
 unsigned long long pair_generation(lc2e_pair* p) { return p->gen; }
 // Make the pair's batch buffers fit n poses now, so that a following
 // lc2e_eval_batch_async of n poses allocates nothing (e.g. under stream capture).
-int pair_prepare(lc2e_pair* p, int n) {
-    const Tiling t = tiling_for(p, n);
-    return ensure_capacity(p, n, t.bpp);
-}
+int pair_prepare(lc2e_pair* p, int n) { return ensure_capacity(p, n); }
 double launch_share(lc2e_pair* p, int n) {
-    const Tiling t = tiling_for(p, n);
+    const Tiling t = tiling_for(p, n, p->ws_poses);
     if (t.tiles <= 0 || n <= 0) return 0.0;
     const int per_cu = resident_per_cu(p);
     const bool fused2 = p->info.grid_ndim == 2 && !p->two && !p->sep;
@@ -1200,9 +1213,9 @@ int lc2e_eval_batch(lc2e_pair* p, int n, const float* mats, double* lc2, double*
     int status = LC2E_OK;
     for (int base = 0; base < n; base += chunk_max) {
         const int m = (n - base) < chunk_max ? (n - base) : chunk_max;
-        const Tiling t = tiling_for(p, m);
-        int rc = ensure_capacity(p, m, t.bpp);
+        int rc = ensure_capacity(p, m);
         if (rc < 0) return rc;
+        const Tiling t = tiling_for(p, m, p->ws_poses);
         std::memcpy(p->h_mats, mats + (size_t)base * mpp * 12, (size_t)m * mpp * 12 * sizeof(float));
         rc = run_batch(p, m, t);
         if (rc < 0) return rc;
@@ -1234,7 +1247,8 @@ int lc2e_eval_batch_noalloc(lc2e_pair* p, int n, const float* mats, double* lc2,
     HIP_TRY(hipSetDevice(e->device));
     hipStream_t st = e->stream;
     const int mpp = p->mats_per_pose();
-    const Tiling t = tiling_for(p, n);
+    const Workspace ws = noalloc_workspace(p);
+    const Tiling t = tiling_for(p, n, ws.poses);
     // scratch layout: results [n][3] f64, matrices [n][mpp][12] f32, partials [n][bpp][2] f64
     auto up256 = [](size_t b) { return (b + 255) / 256 * 256; };
     const size_t out_b = up256((size_t)n * 3 * sizeof(double));
@@ -1255,7 +1269,7 @@ int lc2e_eval_batch_noalloc(lc2e_pair* p, int n, const float* mats, double* lc2,
         // every partial slot is written by the fused kernel before k_reduce reads it, so the
         // previous call's contents need no clearing
         const lc2e::FusedArgs a = make_args(p, d_mats, d_part, t);
-        HIP_TRY(launch_eval(p, a, n, st, noalloc_workspace(p)));
+        HIP_TRY(launch_eval(p, a, n, st, ws));
     }
     HIP_TRY(lc2e::launch_reduce(d_part, t.tiles > 0 ? t.bpp : 0, n, d_out, st));
     // results back through a fixed host buffer, a chunk of poses at a time
@@ -1282,9 +1296,9 @@ int lc2e_eval_batch_async(lc2e_pair* p, int n, const float* d_mats, double* d_ou
     if (!p || !d_mats || !d_out || n <= 0) return fail(LC2E_ERR_INVALID, "invalid argument");
     hipStream_t st = stream ? static_cast<hipStream_t>(stream) : p->e->stream;
     // partials are per pair; size them for n
-    const Tiling t = tiling_for(p, n);
-    int rc = ensure_capacity(p, n, t.bpp);
+    int rc = ensure_capacity(p, n);
     if (rc < 0) return rc;
+    const Tiling t = tiling_for(p, n, p->ws_poses);
     if (t.tiles > 0) {
         lc2e::FusedArgs a = make_args(p, d_mats, p->d_partials, t);
         HIP_TRY(launch_eval(p, a, n, st, {p->ws, p->ws_poses}));
@@ -1310,7 +1324,7 @@ int lc2e_eval_mi_batch(lc2e_pair* p, int n, const float* mats, int bins_us, int 
         p->mi_stat_ready = false;
     }
     const int chunk_max = 64;
-    const Tiling t = tiling_for(p, 1);
+    const Tiling t = tiling_for(p, 1, 0);
     // Without a budget the warped image is kept between the two passes over it (3D), a float per
     // voxel and pose; what does not fit goes in parts. A buffer of its own: evaluations on a
     // caller's stream may be using the pair's workspace.
@@ -1375,9 +1389,9 @@ int lc2e_debug_fetch(lc2e_pair* p, lc2e_stage stage, const float* m12, void* hos
     hipStream_t st = p->e->stream;
     const long long V = (long long)p->v.X * p->v.Y * p->v.Z;
     const int mpp = p->mats_per_pose();
-    const Tiling t = tiling_for(p, 1);
-    int rc = ensure_capacity(p, 1, t.bpp);
+    int rc = ensure_capacity(p, 1);
     if (rc < 0) return rc;
+    const Tiling t = tiling_for(p, 1, p->ws_poses);
     HIP_TRY(hipMemcpy(p->d_mats, m12, (size_t)mpp * 12 * sizeof(float), hipMemcpyHostToDevice));
     lc2e::FusedArgs a = make_args(p, p->d_mats, p->d_partials, t);
     const bool movi = p->info.high_res_is_moving != 0;
@@ -1472,11 +1486,11 @@ int lc2e_pair_autotune(lc2e_pair* p, int n, const float* mats, int iters, int* b
     drop_graphs(p);
     const int forced = p->zchunk_forced;
     for (int zc : cand) {
-        p->zchunk_forced = zc;
-        const Tiling t = tiling_for(p, n);
-        p->zchunk_forced = forced;
-        int rc = ensure_capacity(p, n, t.bpp);
+        int rc = ensure_capacity(p, n);
         if (rc < 0) return rc;
+        p->zchunk_forced = zc;
+        const Tiling t = tiling_for(p, n, p->ws_poses);
+        p->zchunk_forced = forced;
         HIP_TRY(hipMemcpy(p->d_mats, mats, (size_t)n * p->mats_per_pose() * 12 * sizeof(float),
                           hipMemcpyHostToDevice));
         lc2e::FusedArgs a = make_args(p, p->d_mats, p->d_partials, t);

@@ -121,10 +121,53 @@ void noalloc_has_its_own_workspace() {
     CHECK(fake::used(0) == 0);
 }
 
+// A fresh pair's allocation-free call: as few launches as the reserve allows, 2D launches through
+// the grid only in parts that fill the device, and chunks chosen for the parts.
+void noalloc_runs_in_large_parts() {
+    lc2e_engine* e = engine();
+    {
+        Pair p(e, 3, 64, 64, 64, 1, 3, true);  // 2 MiB a pose
+        fake::launches().clear();
+        CHECK(p.noalloc(32) >= 0);
+        CHECK(fake::count("k_warp_grad3") == 1 && fake::count("k_moments3d") == 1);
+        CHECK(fake::launches()[0].a.npose == 32 || fake::launches()[1].a.npose == 32);
+    }
+    {
+        Pair p(e, 3, 192, 192, 160, 1, 3, true);  // 45 MiB a pose: 11 in the reserve
+        fake::launches().clear();
+        CHECK(p.noalloc(32) >= 0);
+        CHECK(fake::count("k_moments3d") == 3);
+        const int chunk = fake::launches()[1].a.zchunk;
+        fake::launches().clear();
+        CHECK(p.noalloc(11) >= 0);  // one part of the same size
+        CHECK(fake::count("k_moments3d") == 1 && fake::launches()[1].a.zchunk == chunk);
+    }
+    {
+        // 93 MiB a pose, five in the reserve: a batch of 8 goes through the grid, and so do its
+        // parts of four poses, of 2048 waves and more
+        Pair p(e, 2, 300, 200, 204, 1, 5, true);
+        fake::launches().clear();
+        CHECK(p.noalloc(8) >= 0);
+        CHECK(fake::count("k_warp2") == 2 && fake::count("k_moments2d") == 2);
+    }
+    {
+        // where there was no memory for more than one pose, whose launch would not fill the
+        // device: warped in place, all poses in one launch
+        fake::reset(24 * MB);
+        Pair p(e, 2, 256, 256, 1, 1, 5, false);
+        fake::launches().clear();
+        CHECK(p.noalloc(64) >= 0);
+        CHECK(fake::count("k_warp2") == 0 && fake::count("k_moments2d") == 1);
+    }
+    lc2e_destroy(e);
+    CHECK(fake::used(0) == 0);
+}
+
 //@SCENARIOS
 
 const std::map<std::string, std::function<void()>> kScenarios = {
     {"noalloc_has_its_own_workspace", noalloc_has_its_own_workspace},
+    {"noalloc_runs_in_large_parts", noalloc_runs_in_large_parts},
 //@TABLE
 };
 
