@@ -249,6 +249,7 @@ struct lc2e_pair {
     void* ws = nullptr;
     size_t ws_bytes = 0;
     int ws_poses = 0;
+    bool pinned = false;  // a caller's graph holds launches that use the workspace
     bool na = false;  // counted in the engine's na_pairs
     double* istat = nullptr;
     int resident_per_cu = 0;  // fused work-groups one CU holds at once (0: not queried yet)
@@ -488,6 +489,7 @@ void free_batch(lc2e_pair* p) {
     p->h_out_dev = nullptr;
     p->cap = 0;
     p->part_bpp = 0;
+    p->pinned = false;  // captured launches hold these buffers too
 }
 
 void free_mi_warp(lc2e_pair* p) {
@@ -538,7 +540,7 @@ int grow_workspace(lc2e_pair* p, int n) {
     }
     const size_t per = p->voxels() * (p->info.high_res_is_moving ? sizeof(float2) : sizeof(float));
     const int want = (int)std::min<size_t>((size_t)std::max(n, 1), std::max<size_t>(1, kWorkspaceBytes / per));
-    if (want <= p->ws_poses) return LC2E_OK;
+    if (want <= p->ws_poses || p->pinned) return LC2E_OK;
     void* d = nullptr;
     const int rc = two_alloc(p, &d, (size_t)want * per);
     if (rc < 0) return p->ws ? LC2E_OK : rc;  // what is there still serves
@@ -699,10 +701,14 @@ int ensure_batch(lc2e_pair* p, int n, int bpp) {
     return LC2E_OK;
 }
 
-// The same for launches of the pair's kernels, and the workspace.
-int ensure_capacity(lc2e_pair* p, int n) {
-    if (p->ws) (void)grow_workspace(p, n);
-    return ensure_batch(p, n, tiling_for(p, n, p->ws_poses).bpp);
+// The same for launches of the pair's kernels, and the workspace. A launch that a caller captures
+// takes the workspace as it is (nothing may be allocated then), and keeps it where it is.
+int ensure_capacity(lc2e_pair* p, int n, bool captured = false) {
+    const int rc = ensure_batch(p, n, tiling_for(p, n, p->ws_poses).bpp);
+    if (rc < 0 || !p->ws) return rc;
+    if (captured) p->pinned = true;
+    else (void)grow_workspace(p, n);
+    return rc;
 }
 
 lc2e::FusedArgs make_args(lc2e_pair* p, const float* d_mats, double* d_partials, const Tiling& t) {
@@ -860,7 +866,11 @@ int engine_device(lc2e_engine* e) { return e->device; }
 unsigned long long pair_generation(lc2e_pair* p) { return p->gen; }
 // Make the pair's batch buffers fit n poses now, so that a following
 // lc2e_eval_batch_async of n poses allocates nothing (e.g. under stream capture).
-int pair_prepare(lc2e_pair* p, int n) { return ensure_capacity(p, n); }
+int pair_prepare(lc2e_pair* p, int n) {
+    const int rc = ensure_capacity(p, n);
+    if (rc >= 0 && p->ws) (void)grow_workspace(p, p->cap);  // once captured it stays as it is
+    return rc;
+}
 double launch_share(lc2e_pair* p, int n) {
     const Tiling t = tiling_for(p, n, p->ws_poses);
     if (t.tiles <= 0 || n <= 0) return 0.0;
@@ -1296,7 +1306,9 @@ int lc2e_eval_batch_async(lc2e_pair* p, int n, const float* d_mats, double* d_ou
     if (!p || !d_mats || !d_out || n <= 0) return fail(LC2E_ERR_INVALID, "invalid argument");
     hipStream_t st = stream ? static_cast<hipStream_t>(stream) : p->e->stream;
     // partials are per pair; size them for n
-    int rc = ensure_capacity(p, n);
+    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+    HIP_TRY(hipStreamIsCapturing(st, &capture));
+    int rc = ensure_capacity(p, n, capture != hipStreamCaptureStatusNone);
     if (rc < 0) return rc;
     const Tiling t = tiling_for(p, n, p->ws_poses);
     if (t.tiles > 0) {

@@ -163,11 +163,40 @@ void noalloc_runs_in_large_parts() {
     CHECK(fake::used(0) == 0);
 }
 
+// A launch captured by the caller allocates and frees nothing where the pair's batch buffers
+// fit, and what it uses stays in place for its replays until a larger batch replaces those.
+void captured_launches_keep_their_workspace() {
+    lc2e_engine* e = engine();
+    hipStream_t st = nullptr;
+    hipGraph_t graph = nullptr;
+    CHECK(hipStreamCreateWithFlags(&st, 0) == hipSuccess);
+    {
+        Pair p(e, 3, 64, 64, 64, 1, 3, true);
+        CHECK(p.mi(4) >= 0);  // sizes the batch buffers alone
+        CHECK(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal) == hipSuccess);
+        fake::launches().clear();
+        CHECK(p.async(4, st) >= 0);
+        CHECK(hipStreamEndCapture(st, &graph) == hipSuccess);
+        CHECK(fake::in_capture() == 0);
+        const float* ws = fake::launches()[0].a.warp1;
+        fake::launches().clear();
+        CHECK(p.batch(4) >= 0);
+        CHECK(fake::launches()[0].is("k_warp") && fake::launches()[0].a.warp1 == ws);
+        CHECK(p.batch(32) >= 0);  // replaces the batch buffers, as documented
+        fake::launches().clear();
+        CHECK(p.batch(32) >= 0 && fake::count("k_warp") == 1);
+    }
+    CHECK(hipGraphDestroy(graph) == hipSuccess);
+    CHECK(hipStreamDestroy(st) == hipSuccess);
+    lc2e_destroy(e);
+}
+
 //@SCENARIOS
 
 const std::map<std::string, std::function<void()>> kScenarios = {
     {"noalloc_has_its_own_workspace", noalloc_has_its_own_workspace},
     {"noalloc_runs_in_large_parts", noalloc_runs_in_large_parts},
+    {"captured_launches_keep_their_workspace", captured_launches_keep_their_workspace},
 //@TABLE
 };
 

@@ -29,7 +29,7 @@ struct State {
     std::map<std::pair<const void*, int>, void*> var_addr;  // (variable, device) -> address
     std::set<hipStream_t> capturing;
     int in_capture = 0;
-    long long mallocs = 0;
+    long long mallocs = 0, attempts = 0;
 };
 State& g() {
     static State* s = new State();
@@ -60,12 +60,13 @@ void reset(size_t device_bytes) {
     g().limit = device_bytes;
     g().launches.clear();
     g().in_capture = 0;
-    g().mallocs = 0;
+    g().mallocs = g().attempts = 0;
 }
 std::vector<Launch>& launches() { return g().launches; }
 int in_capture() { return g().in_capture; }
 size_t used(int device) { return g().used[device]; }
 long long mallocs() { return g().mallocs; }
+long long attempts() { return g().attempts; }
 bool live(const void* p) {
     std::lock_guard<std::recursive_mutex> lk(g().mu);
     for (const auto& b : g().blocks)
@@ -94,6 +95,7 @@ hipError_t hipGetLastError() { return hipSuccess; }
 hipError_t hipMalloc(void** p, size_t n) {
     LOCK;
     note_capture();
+    ++g().attempts;
     if (g().used[t_device] + n > g().limit) return *p = nullptr, hipErrorOutOfMemory;
     if (!(*p = map_bytes(n))) return hipErrorOutOfMemory;
     g().blocks[*p] = {n, t_device};
