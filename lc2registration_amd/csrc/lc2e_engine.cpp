@@ -249,6 +249,7 @@ struct lc2e_pair {
     void* ws = nullptr;
     size_t ws_bytes = 0;
     int ws_poses = 0;
+    int ws_refused = 0;   // > 0: memory for that many poses was not to be had
     bool pinned = false;  // a caller's graph holds launches that use the workspace
     bool na = false;  // counted in the engine's na_pairs
     double* istat = nullptr;
@@ -540,10 +541,13 @@ int grow_workspace(lc2e_pair* p, int n) {
     }
     const size_t per = p->voxels() * (p->info.high_res_is_moving ? sizeof(float2) : sizeof(float));
     const int want = (int)std::min<size_t>((size_t)std::max(n, 1), std::max<size_t>(1, kWorkspaceBytes / per));
-    if (want <= p->ws_poses || p->pinned) return LC2E_OK;
+    if (want <= p->ws_poses || p->pinned || (p->ws_refused && want >= p->ws_refused)) return LC2E_OK;
     void* d = nullptr;
     const int rc = two_alloc(p, &d, (size_t)want * per);
-    if (rc < 0) return p->ws ? LC2E_OK : rc;  // what is there still serves
+    if (rc < 0) {
+        p->ws_refused = want;  // not tried again on every call
+        return p->ws ? LC2E_OK : rc;  // what is there still serves
+    }
     if (p->ws) {
         drop_graphs(p);
         two_free(p, p->ws, (size_t)p->ws_poses * p->ws_bytes);

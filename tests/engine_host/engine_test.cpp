@@ -191,12 +191,30 @@ void captured_launches_keep_their_workspace() {
     lc2e_destroy(e);
 }
 
+// Where a larger workspace is not to be had, calls go on with the one there is and do not ask
+// for memory each time.
+void a_refused_workspace_is_not_asked_for_again() {
+    lc2e_engine* e = engine();
+    {
+        fake::reset(300 * MB);  // 192x192x160: 45 MiB a pose
+        Pair p(e, 3, 192, 192, 160, 1, 3, true);
+        CHECK(p.batch(8) >= 0);
+        const long long asked = fake::attempts();
+        fake::launches().clear();
+        CHECK(p.batch(8) >= 0 && p.batch(8) >= 0);
+        CHECK(fake::attempts() == asked);
+        CHECK(fake::count("k_moments3d") > 2);
+    }
+    lc2e_destroy(e);
+}
+
 //@SCENARIOS
 
 const std::map<std::string, std::function<void()>> kScenarios = {
     {"noalloc_has_its_own_workspace", noalloc_has_its_own_workspace},
     {"noalloc_runs_in_large_parts", noalloc_runs_in_large_parts},
     {"captured_launches_keep_their_workspace", captured_launches_keep_their_workspace},
+    {"a_refused_workspace_is_not_asked_for_again", a_refused_workspace_is_not_asked_for_again},
 //@TABLE
 };
 
