@@ -83,11 +83,15 @@ int lc2e_create(int device, size_t hbm_budget_bytes, lc2e_engine** out);
 void lc2e_destroy(lc2e_engine* e);
 /* Bytes currently charged to the engine's budget, and the budget. An engine without a budget
  * also keeps, and does not count here: with a pair, its statistics of a static high-resolution
- * image (40 bytes per grid voxel) or a workspace for the warped moving image (4 or 8 bytes per
- * grid voxel and pose of its largest batch, at most 1 GiB or one pose); and up to 1 GiB of
- * freed blocks for the next allocations of their size, given back with the engine. Under a
- * budget a pair does without them, so what a budget admits does not depend on them: 2D values
- * are the same bits, 3D values up to radius 4 come from another kernel and agree to rounding. */
+ * image (40 bytes per grid voxel), a workspace for the warped moving image (4 or 8 bytes per grid
+ * voxel and pose of its largest batch, at most 1 GiB or one pose) and one for the mutual
+ * information (4 bytes, at most 256 MiB or one pose); a workspace for the allocation-free entry
+ * point (64 poses of the largest pair, at most 512 MiB or one pose); and up to 1 GiB of freed blocks
+ * for the next allocations of their size. All of it goes back where an allocation of any engine
+ * on the device would fail: a pair that is in no call then, and in no graph of a caller, loses it.
+ * Under a budget a pair does without, so what a budget admits does not depend on it. Without:
+ * 2D values are the same bits, 3D values up to radius 4 come from another kernel and agree to
+ * rounding. */
 int lc2e_memory(lc2e_engine* e, size_t* used, size_t* budget);
 
 /* Upload a resident fixed or moving image. Replaces Interpolator*'s thrust copies of the

@@ -11,6 +11,7 @@
 #include <functional>
 #include <map>
 #include <mutex>
+#include <set>
 #include <string>
 #include <vector>
 
@@ -49,6 +50,10 @@ int dtype_size(int dt) {
         default: return 0;
     }
 }
+
+// Gives memory of the device back that its owners can do without, a piece at a time; false if
+// there is no more (defined below).
+bool reclaim(int device);
 
 }  // namespace
 
@@ -111,7 +116,7 @@ struct lc2e_engine {
         return true;
     }
     std::map<void*, size_t> sizes;  // reused blocks in use that are larger than asked for
-    void give_back() {
+    bool give_back() {
         std::vector<Block> d, h;
         {
             std::lock_guard<std::mutex> lk(mu);
@@ -120,9 +125,11 @@ struct lc2e_engine {
         }
         for (const Block& b : d) (void)hipFree(b.p);
         for (const Block& b : h) (void)hipHostFree(b.p);
+        return !d.empty();
     }
-    // Device memory without a charge to the budget.
-    hipError_t raw_alloc(void** p, size_t bytes) {
+    // Device memory without a charge to the budget; `must`: the call fails without it, so what
+    // pairs and engines only keep to be faster makes room.
+    hipError_t raw_alloc(void** p, size_t bytes, bool must) {
         if (!bytes) bytes = 1;
         if ((*p = take(kept_device, bytes))) return hipSuccess;
         hipError_t err = hipSetDevice(device);
@@ -130,6 +137,10 @@ struct lc2e_engine {
         if (err != hipSuccess) {  // again without the kept blocks
             (void)hipGetLastError();
             give_back();
+            err = hipMalloc(p, bytes);
+        }
+        while (err == hipErrorOutOfMemory && must && reclaim(device)) {
+            (void)hipGetLastError();
             err = hipMalloc(p, bytes);
         }
         return err;
@@ -143,7 +154,13 @@ struct lc2e_engine {
     // Mapped, coherent pinned host memory.
     hipError_t host_alloc(void** p, size_t bytes) {
         if ((*p = take(kept_host, bytes))) return hipSuccess;
-        return hipHostMalloc(p, bytes, hipHostMallocMapped | hipHostMallocCoherent);
+        hipError_t err = hipHostMalloc(p, bytes, hipHostMallocMapped | hipHostMallocCoherent);
+        if (err != hipSuccess) {
+            (void)hipGetLastError();
+            give_back();
+            err = hipHostMalloc(p, bytes, hipHostMallocMapped | hipHostMallocCoherent);
+        }
+        return err;
     }
     void host_free(void* p, size_t bytes) {
         if (p && !keep(kept_host, kKeepHost, p, bytes)) {
@@ -164,7 +181,7 @@ struct lc2e_engine {
                             used, bytes, budget);
             used += bytes;  // reserved before the allocation, returned if it fails
         }
-        const hipError_t err = raw_alloc(p, bytes);
+        const hipError_t err = raw_alloc(p, bytes, true);
         if (err != hipSuccess) {
             std::lock_guard<std::mutex> lk(mu);
             used -= bytes;
@@ -229,7 +246,7 @@ struct lc2e_pair {
     // changes whenever captured launches of this pair go stale (buffers or decomposition
     // changed); unique across pairs, so a graph cached by address is never reused for
     // another pair
-    unsigned long long gen = 0;
+    std::atomic<unsigned long long> gen = 0;
     // mutual information (patchSize 0): extremes of the static image, per-pose extremes,
     // joint histograms and results, sized for mi_cap poses of mi_bins counters
     int* mi_ext_stat = nullptr;
@@ -241,14 +258,17 @@ struct lc2e_pair {
     double* mi_out = nullptr;
     float* mi_warp = nullptr;  // warped images of mi_warp_poses poses
     int mi_warp_poses = 0;
+    int mi_refused = 0;  // > 0: memory for that many was not to be had
     // two-kernel path: the warped moving image of ws_poses poses (ws_bytes each) and, if the
     // static image is the high-resolution one, its statistics; kept with the pair (see
     // make_two_kernel)
     bool two = false;
     bool two_charged = false;  // the memory below counts against the engine's budget
+    bool two_required = false;  // no other path evaluates the pair
     void* ws = nullptr;
     size_t ws_bytes = 0;
     int ws_poses = 0;
+    int users = 0;        // calls in progress (guarded by g_registry_mu)
     int ws_refused = 0;   // > 0: memory for that many poses was not to be had
     bool pinned = false;  // a caller's graph holds launches that use the workspace
     bool na = false;  // counted in the engine's na_pairs
@@ -277,6 +297,23 @@ struct lc2e_pair {
 namespace {
 
 std::atomic<unsigned long long> g_generation{1};
+
+// The pairs and engines that hold memory they can do without, for reclaim(). A pair in a call
+// (users > 0) keeps its own.
+std::mutex g_registry_mu;
+std::set<lc2e_pair*> g_pairs;
+std::set<lc2e_engine*> g_engines;
+struct Use {
+    lc2e_pair* p;
+    explicit Use(lc2e_pair* pair) : p(pair) {
+        std::lock_guard<std::mutex> lk(g_registry_mu);
+        ++p->users;
+    }
+    ~Use() {
+        std::lock_guard<std::mutex> lk(g_registry_mu);
+        --p->users;
+    }
+};
 
 void drop_graphs(lc2e_pair* p) {
     for (auto& kv : p->graphs) {
@@ -514,7 +551,7 @@ void free_mi(lc2e_pair* p) {
 // Memory of the two-kernel path beside the budgeted buffers.
 int two_alloc(lc2e_pair* p, void** d, size_t bytes) {
     if (p->two_charged) return p->e->alloc(d, bytes);
-    if (p->e->raw_alloc(d, bytes) == hipSuccess) return LC2E_OK;
+    if (p->e->raw_alloc(d, bytes, p->two_required) == hipSuccess) return LC2E_OK;
     (void)hipGetLastError();
     return fail(LC2E_ERR_HIP, "workspace of %zu bytes", bytes);
 }
@@ -573,7 +610,7 @@ int reserve_noalloc(lc2e_pair* p) {
     for (size_t bytes : {most, p->ws_bytes}) {
         if (e->na_bytes >= bytes) break;
         void* d = nullptr;
-        if (e->raw_alloc(&d, bytes) != hipSuccess) {
+        if (e->raw_alloc(&d, bytes, false) != hipSuccess) {
             (void)hipGetLastError();
             continue;
         }
@@ -599,7 +636,8 @@ void release_noalloc(lc2e_pair* p) {
 // Under noalloc_lock. Without a reservation: 2D launches warp in place; the others share the
 // pair's workspace, as radii beyond the fused kernels share their box-sum buffers.
 Workspace noalloc_workspace(const lc2e_pair* p) {
-    if (p->na) return {p->e->na, (int)std::min<size_t>(p->e->na_bytes / p->ws_bytes, 1 << 20)};
+    const size_t poses = p->na ? p->e->na_bytes / p->ws_bytes : 0;
+    if (poses) return {p->e->na, (int)std::min<size_t>(poses, 1 << 20)};
     if (p->info.grid_ndim == 2) return {nullptr, 0};
     return {p->ws, p->ws_poses};
 }
@@ -612,6 +650,69 @@ void free_two(lc2e_pair* p) {
     p->istat = nullptr;
     p->ws_poses = 0;
     p->two = false;
+}
+
+// Gives back memory of an idle pair (under g_registry_mu): the mutual information's warped images
+// and the workspace beyond one pose, whose absence changes no value; with `all` the rest of the
+// two-kernel path's, after which 2D pairs warp in place (the same bits) and 3D pairs run the fused
+// kernel (the same to rounding). False if there was nothing.
+bool shrink(lc2e_pair* p, bool all) {
+    if (p->mi_warp) {
+        free_mi_warp(p);
+        p->mi_refused = 1;
+        return true;
+    }
+    if (p->two_charged || p->pinned) return false;
+    if (!all && p->ws_poses > 1) {
+        drop_graphs(p);
+        two_free(p, p->ws, (size_t)p->ws_poses * p->ws_bytes);
+        p->e->give_back();
+        p->ws = nullptr;
+        p->ws_poses = 0;
+        p->ws_refused = 2;
+        if (hipMalloc(&p->ws, p->ws_bytes) == hipSuccess) {
+            p->ws_poses = 1;
+        } else {
+            (void)hipGetLastError();
+            p->ws = nullptr;
+            free_two(p);
+            p->two = p->info.grid_ndim == 2;
+        }
+        return true;
+    }
+    if (!all || p->two_required || (!p->ws && !p->istat)) return false;
+    drop_graphs(p);
+    free_two(p);
+    p->two = p->info.grid_ndim == 2;
+    p->resident_per_cu = 0;
+    p->model_cache.clear();
+    return true;
+}
+
+// The allocation-free entry point's workspace down to one pose of the pairs that use it.
+bool shrink_noalloc(lc2e_engine* e) {
+    size_t one = 0;
+    for (const lc2e_pair* p : g_pairs)
+        if (p->e == e && p->na) one = std::max(one, p->ws_bytes);
+    std::lock_guard<std::mutex> lk(noalloc_lock(e->device));
+    if (!one || e->na_bytes <= one) return false;
+    e->raw_free(e->na, e->na_bytes);
+    e->give_back();
+    e->na = nullptr;
+    e->na_bytes = 0;
+    if (hipMalloc(&e->na, one) == hipSuccess) e->na_bytes = one;
+    else (void)hipGetLastError(), e->na = nullptr;
+    return true;
+}
+
+bool reclaim(int device) {
+    std::lock_guard<std::mutex> lk(g_registry_mu);
+    for (lc2e_engine* e : g_engines)
+        if (e->device == device && (e->give_back() || shrink_noalloc(e))) return true;
+    for (bool all : {false, true})
+        for (lc2e_pair* p : g_pairs)
+            if (p->e->device == device && !p->users && shrink(p, all)) return true;
+    return false;
 }
 
 lc2e::FusedArgs make_args(lc2e_pair* p, const float* d_mats, double* d_partials, const Tiling& t);
@@ -637,6 +738,7 @@ int make_two_kernel(lc2e_pair* p, bool required) {
     const bool two_d = p->info.grid_ndim == 2;
     if (two_d && p->info.high_res_is_moving && p->info.patch_radius <= lc2e::kMaxRFused2) return LC2E_OK;
     p->two_charged = required && p->e->budget;
+    p->two_required = required;
     p->two = two_d;
     if (!required && p->e->budget) return LC2E_OK;
     p->two = true;
@@ -871,11 +973,16 @@ unsigned long long pair_generation(lc2e_pair* p) { return p->gen; }
 // Make the pair's batch buffers fit n poses now, so that a following
 // lc2e_eval_batch_async of n poses allocates nothing (e.g. under stream capture).
 int pair_prepare(lc2e_pair* p, int n) {
+    Use use(p);
     const int rc = ensure_capacity(p, n);
-    if (rc >= 0 && p->ws) (void)grow_workspace(p, p->cap);  // once captured it stays as it is
+    if (rc >= 0 && p->ws) {  // once captured it stays as it is
+        (void)grow_workspace(p, p->cap);
+        p->pinned = true;
+    }
     return rc;
 }
 double launch_share(lc2e_pair* p, int n) {
+    Use use(p);
     const Tiling t = tiling_for(p, n, p->ws_poses);
     if (t.tiles <= 0 || n <= 0) return 0.0;
     const int per_cu = resident_per_cu(p);
@@ -915,12 +1022,20 @@ int lc2e_create(int device, size_t hbm_budget_bytes, lc2e_engine** out) {
         e->scratch = nullptr;
         e->scratch_error = hipGetErrorString(se);
     }
+    {
+        std::lock_guard<std::mutex> lk(g_registry_mu);
+        g_engines.insert(e);
+    }
     *out = e;
     return LC2E_OK;
 }
 
 void lc2e_destroy(lc2e_engine* e) {
     if (!e) return;
+    {
+        std::lock_guard<std::mutex> lk(g_registry_mu);
+        g_engines.erase(e);
+    }
     (void)hipSetDevice(e->device);
     (void)hipStreamSynchronize(e->stream);
     (void)hipStreamDestroy(e->stream);
@@ -973,7 +1088,7 @@ int lc2e_volume_upload(lc2e_engine* e, const void* host, lc2e_dtype dtype, const
     tmp.flag[0] = tmp.flag[1] = 0;
     auto stage = [&]() {
         tmp.bytes = (size_t)n * dsz;
-        hipError_t err = e->raw_alloc(&tmp.staging, tmp.bytes);
+        hipError_t err = e->raw_alloc(&tmp.staging, tmp.bytes, true);
         if (err == hipSuccess)
             err = hipMemcpyAsync(tmp.staging, host, tmp.bytes, hipMemcpyHostToDevice, e->stream);
         return err;
@@ -1173,12 +1288,20 @@ int lc2e_pair_create(lc2e_engine* e, lc2e_volume* fixed, lc2e_volume* moving,
         lc2e_pair_destroy(p);
         return fail(LC2E_ERR_HIP, "pair set-up failed: %s", hipGetErrorString(err));
     }
+    {
+        std::lock_guard<std::mutex> lk(g_registry_mu);
+        g_pairs.insert(p);
+    }
     *out = p;
     return LC2E_OK;
 }
 
 void lc2e_pair_destroy(lc2e_pair* p) {
     if (!p) return;
+    {
+        std::lock_guard<std::mutex> lk(g_registry_mu);
+        g_pairs.erase(p);
+    }
     (void)hipStreamSynchronize(p->e->stream);
     free_batch(p);
     free_mi(p);
@@ -1205,6 +1328,7 @@ int lc2e_pair_set_per_frame(lc2e_pair* p, int per_frame) {
     if (!p) return fail(LC2E_ERR_INVALID, "null pair");
     if (p->info.grid_ndim != 2 && per_frame)
         return fail(LC2E_ERR_INVALID, "per-frame matrices need a 2D frame stack");
+    Use use(p);
     free_batch(p);
     p->info.per_frame_matrices = per_frame ? 1 : 0;
     return LC2E_OK;
@@ -1221,6 +1345,7 @@ int lc2e_eval_batch(lc2e_pair* p, int n, const float* mats, double* lc2, double*
                     double* sum_w) {
     if (!p || !mats || n < 0) return fail(LC2E_ERR_INVALID, "invalid argument");
     if (n == 0) return LC2E_OK;
+    Use use(p);
     HIP_TRY(hipSetDevice(p->e->device));
     const int mpp = p->mats_per_pose();
     const int chunk_max = 65535;
@@ -1252,6 +1377,7 @@ int lc2e_eval_batch_noalloc(lc2e_pair* p, int n, const float* mats, double* lc2,
                             double* sum_measure, double* sum_w) {
     if (!p || !mats || n < 0) return fail(LC2E_ERR_INVALID, "invalid argument");
     if (n == 0) return LC2E_OK;
+    Use use(p);
     lc2e_engine* e = p->e;
     if (!e->scratch)
         return fail(LC2E_ERR_HIP, "device scratch unavailable: %s", e->scratch_error.c_str());
@@ -1308,6 +1434,7 @@ int lc2e_eval_batch_noalloc(lc2e_pair* p, int n, const float* mats, double* lc2,
 
 int lc2e_eval_batch_async(lc2e_pair* p, int n, const float* d_mats, double* d_out, void* stream) {
     if (!p || !d_mats || !d_out || n <= 0) return fail(LC2E_ERR_INVALID, "invalid argument");
+    Use use(p);
     hipStream_t st = stream ? static_cast<hipStream_t>(stream) : p->e->stream;
     // partials are per pair; size them for n
     hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
@@ -1329,6 +1456,7 @@ int lc2e_eval_mi_batch(lc2e_pair* p, int n, const float* mats, int bins_us, int 
     if (n == 0) return LC2E_OK;
     if (bins_us < 2 || bins_hr < 2 || bins_us > lc2e::kMiMaxBins || bins_hr > lc2e::kMiMaxBins)
         return fail(LC2E_ERR_INVALID, "histogram bins must lie in [2, %d]", lc2e::kMiMaxBins);
+    Use use(p);
     HIP_TRY(hipSetDevice(p->e->device));
     lc2e_engine* e = p->e;
     hipStream_t st = e->stream;
@@ -1350,10 +1478,16 @@ int lc2e_eval_mi_batch(lc2e_pair* p, int n, const float* mats, int bins_us, int 
     if (!e->budget && p->info.grid_ndim == 3 && !p->moving->large && (long long)p->sg.X * p->sg.Y < lc2e::kMaxFusedSlice) {
         const size_t per = p->voxels() * sizeof(float);
         const int want = (int)std::min<size_t>((size_t)step, std::max<size_t>(1, kMiWarpBytes / per));
-        if (want > p->mi_warp_poses) {
-            free_mi_warp(p);
-            if (e->raw_alloc((void**)&p->mi_warp, (size_t)want * per) == hipSuccess) p->mi_warp_poses = want;
-            else (void)hipGetLastError(), p->mi_warp = nullptr;
+        if (want > p->mi_warp_poses && (!p->mi_refused || want < p->mi_refused)) {
+            void* d = nullptr;
+            if (e->raw_alloc(&d, (size_t)want * per, false) == hipSuccess) {
+                free_mi_warp(p);
+                p->mi_warp = static_cast<float*>(d);
+                p->mi_warp_poses = want;
+            } else {
+                (void)hipGetLastError();
+                p->mi_refused = want;
+            }
         }
         if (p->mi_warp) step = std::min(step, p->mi_warp_poses);
     }
@@ -1401,6 +1535,7 @@ int lc2e_sync(lc2e_engine* e) {
 
 int lc2e_debug_fetch(lc2e_pair* p, lc2e_stage stage, const float* m12, void* host) {
     if (!p || !host || !m12) return fail(LC2E_ERR_INVALID, "null argument");
+    Use use(p);
     HIP_TRY(hipSetDevice(p->e->device));
     hipStream_t st = p->e->stream;
     const long long V = (long long)p->v.X * p->v.Y * p->v.Z;
@@ -1415,7 +1550,8 @@ int lc2e_debug_fetch(lc2e_pair* p, lc2e_stage stage, const float* m12, void* hos
         const bool want_moving = (stage == LC2E_STAGE_WARP_I) == movi || (stage == LC2E_STAGE_GRAD && movi);
         float* buf = nullptr;
         float* buf2 = nullptr;
-        HIP_TRY(hipMalloc(&buf, V * sizeof(float)));
+        lc2e_engine* e = p->e;
+        HIP_TRY(e->raw_alloc((void**)&buf, V * sizeof(float), true));
         hipError_t err = hipSuccess;
         const float* src = p->stat_img;
         if (stage == LC2E_STAGE_GRAD && !movi) {
@@ -1424,22 +1560,22 @@ int lc2e_debug_fetch(lc2e_pair* p, lc2e_stage stage, const float* m12, void* hos
             err = lc2e::launch_warp_moving(a, p->info.grid_ndim, p->info.src_ndim, buf, st);
             src = buf;
             if (err == hipSuccess && stage == LC2E_STAGE_GRAD) {
-                err = hipMalloc(&buf2, V * sizeof(float));
+                err = e->raw_alloc((void**)&buf2, V * sizeof(float), true);
                 if (err == hipSuccess) err = lc2e::launch_sobel(buf, p->v, p->info.grid_ndim, buf2, st);
                 src = buf2;
             }
         }
         if (err == hipSuccess) err = hipMemcpyAsync(host, src, V * sizeof(float), hipMemcpyDeviceToHost, st);
         if (err == hipSuccess) err = hipStreamSynchronize(st);
-        (void)hipFree(buf);
-        if (buf2) (void)hipFree(buf2);
+        e->raw_free(buf, V * sizeof(float));
+        e->raw_free(buf2, V * sizeof(float));
         if (err != hipSuccess) return fail(LC2E_ERR_HIP, "debug fetch failed: %s", hipGetErrorString(err));
         return LC2E_OK;
     }
     if (stage != LC2E_STAGE_W && stage != LC2E_STAGE_MEASURE)
         return fail(LC2E_ERR_INVALID, "unknown stage %d", (int)stage);
     double* maps = nullptr;
-    HIP_TRY(hipMalloc(&maps, 2 * V * sizeof(double)));
+    HIP_TRY(p->e->raw_alloc((void**)&maps, 2 * V * sizeof(double), true));
     hipError_t err = hipMemsetAsync(maps, 0, 2 * V * sizeof(double), st);
     a.wmap = maps;
     a.mmap = maps + V;
@@ -1449,13 +1585,14 @@ int lc2e_debug_fetch(lc2e_pair* p, lc2e_stage stage, const float* m12, void* hos
         err = hipMemcpyAsync(host, stage == LC2E_STAGE_W ? a.wmap : a.mmap, V * sizeof(double),
                              hipMemcpyDeviceToHost, st);
     if (err == hipSuccess) err = hipStreamSynchronize(st);
-    (void)hipFree(maps);
+    p->e->raw_free(maps, 2 * V * sizeof(double));
     if (err != hipSuccess) return fail(LC2E_ERR_HIP, "debug fetch failed: %s", hipGetErrorString(err));
     return LC2E_OK;
 }
 
 int lc2e_pair_set_tuning(lc2e_pair* p, int zchunk) {
     if (!p || zchunk < 0) return fail(LC2E_ERR_INVALID, "invalid argument");
+    Use use(p);
     (void)hipStreamSynchronize(p->e->stream);
     drop_graphs(p);  // captured launches carry the old decomposition
     p->zchunk_forced = zchunk > 0 ? round_zchunk(zchunk) : 0;
@@ -1464,6 +1601,7 @@ int lc2e_pair_set_tuning(lc2e_pair* p, int zchunk) {
 
 int lc2e_pair_set_tuning_n(lc2e_pair* p, int n, int zchunk) {
     if (!p || n <= 0 || zchunk < 0) return fail(LC2E_ERR_INVALID, "invalid argument");
+    Use use(p);
     (void)hipStreamSynchronize(p->e->stream);
     drop_graphs(p);
     if (zchunk == 0) p->tuned.erase(n);
@@ -1474,6 +1612,7 @@ int lc2e_pair_set_tuning_n(lc2e_pair* p, int n, int zchunk) {
 int lc2e_pair_autotune(lc2e_pair* p, int n, const float* mats, int iters, int* best_zchunk,
                        double* best_ms) {
     if (!p || !mats || n <= 0 || iters <= 0) return fail(LC2E_ERR_INVALID, "invalid argument");
+    Use use(p);
     HIP_TRY(hipSetDevice(p->e->device));
     if (p->info.grid_ndim != 3 || p->sep) {
         if (best_zchunk) *best_zchunk = 1;
@@ -1559,6 +1698,7 @@ int lc2e_pair_profile_read(lc2e_pair* p, double* kernel_ms, long long* launches)
 
 int lc2e_pair_use_graph(lc2e_pair* p, int enable) {
     if (!p) return fail(LC2E_ERR_INVALID, "null pair");
+    Use use(p);
     if (!enable) drop_graphs(p);
     p->use_graph = enable != 0;
     return LC2E_OK;

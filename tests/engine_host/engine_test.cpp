@@ -40,6 +40,7 @@ struct Pair {
         CHECK(make(e, dim, x, y, z, movi, r, src3, tracked) >= 0);
     }
     Pair() = default;
+    Pair(const Pair&) = delete;
     int make(lc2e_engine* e, int dim, int x, int y, int z, int movi, int r, bool src3, bool tracked = false) {
         const bool stack = dim == 2 && z > 1;
         std::vector<float> img(size_t(stack ? z : 1) * 64 + 4096, 1.0f);
@@ -208,6 +209,44 @@ void a_refused_workspace_is_not_asked_for_again() {
     lc2e_destroy(e);
 }
 
+// Memory that pairs and engines keep only to be faster never makes a call fail: with 200 MiB,
+// pairs of a 64^3 grid (4 MiB each without it, 15 with it, and more for batches and mutual
+// information) fit as if there were none, on this engine and on another, and all of them
+// evaluate; a pair that a caller's graph uses is left alone.
+void kept_memory_makes_room() {
+    fake::reset(200 * MB);
+    lc2e_engine *e = engine(), *other = engine();
+    hipStream_t st = nullptr;
+    hipGraph_t graph = nullptr;
+    CHECK(hipStreamCreateWithFlags(&st, 0) == hipSuccess);
+    std::vector<Pair> pairs(44);
+    Pair held(e, 3, 64, 64, 64, 1, 3, true);
+    CHECK(held.batch(2) >= 0);
+    CHECK(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal) == hipSuccess);
+    fake::launches().clear();
+    CHECK(held.async(2, st) >= 0);
+    CHECK(hipStreamEndCapture(st, &graph) == hipSuccess);
+    const float* ws = fake::launches()[0].a.warp1;
+    for (size_t i = 0; i < pairs.size(); ++i) {
+        CHECK(pairs[i].make(i % 2 ? other : e, 3, 64, 64, 64, 0, i % 3 ? 3 : 4, true) >= 0);
+        CHECK(pairs[i].batch(4) >= 0);
+        CHECK(pairs[i].mi(2) >= 0);
+    }
+    for (Pair& p : pairs) CHECK(p.batch(4) >= 0 && p.noalloc(3) >= 0 && p.mi(2) >= 0);
+    fake::launches().clear();
+    CHECK(held.batch(2) >= 0 && fake::launches()[0].a.warp1 == ws);
+    // and the other way round: a volume that needs what they keep
+    lc2e_volume* v = nullptr;
+    lc2e_geom g{};
+    for (int a = 0; a < 3; ++a) g.dims[a] = a < 2 ? 160 : 100, g.spacing[a] = 1.0f;
+    std::vector<unsigned char> img(size_t(160) * 160 * 100);
+    CHECK(lc2e_volume_upload(e, img.data(), LC2E_U8, &g, LC2E_STORE_AUTO, &v) == LC2E_OK);
+    lc2e_volume_destroy(v);
+    pairs.clear();
+    CHECK(hipGraphDestroy(graph) == hipSuccess);
+    CHECK(hipStreamDestroy(st) == hipSuccess);
+}
+
 //@SCENARIOS
 
 const std::map<std::string, std::function<void()>> kScenarios = {
@@ -215,6 +254,7 @@ const std::map<std::string, std::function<void()>> kScenarios = {
     {"noalloc_runs_in_large_parts", noalloc_runs_in_large_parts},
     {"captured_launches_keep_their_workspace", captured_launches_keep_their_workspace},
     {"a_refused_workspace_is_not_asked_for_again", a_refused_workspace_is_not_asked_for_again},
+    {"kept_memory_makes_room", kept_memory_makes_room},
 //@TABLE
 };
 

@@ -37,6 +37,7 @@ def engine_test(tmp_path_factory):
     "noalloc_runs_in_large_parts",
     "captured_launches_keep_their_workspace",
     "a_refused_workspace_is_not_asked_for_again",
+    "kept_memory_makes_room",
 ])
 def test_engine_host(engine_test, scenario):
     r = subprocess.run([engine_test, scenario], capture_output=True, text=True, timeout=120)
