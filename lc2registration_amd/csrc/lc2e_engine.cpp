@@ -102,7 +102,11 @@ struct lc2e_engine {
     // true if the block is kept
     bool keep(std::vector<Block>& kept, size_t limit, void* p, size_t bytes) {
         if (budget || bytes > limit / 2) return false;
-        if (hipSetDevice(device) != hipSuccess || hipDeviceSynchronize() != hipSuccess) return false;
+        int current = device;  // the caller's device stays current, as it does in hipFree
+        bool idle = hipGetDevice(&current) == hipSuccess && hipSetDevice(device) == hipSuccess &&
+                    hipDeviceSynchronize() == hipSuccess;
+        if (current != device) idle = hipSetDevice(current) == hipSuccess && idle;
+        if (!idle) return false;
         std::lock_guard<std::mutex> lk(mu);
         auto it = sizes.find(p);
         if (it != sizes.end()) {

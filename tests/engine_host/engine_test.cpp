@@ -247,6 +247,20 @@ void kept_memory_makes_room() {
     CHECK(hipStreamDestroy(st) == hipSuccess);
 }
 
+// Giving memory back does not change the calling thread's device, as hipFree does not.
+void releases_leave_the_current_device() {
+    lc2e_engine* e = engine(0, 0);
+    int device = 0;
+    {
+        Pair p(e, 3, 64, 64, 64, 1, 3, true);
+        CHECK(p.batch(4) >= 0);
+        CHECK(hipSetDevice(1) == hipSuccess);
+    }
+    CHECK(hipGetDevice(&device) == hipSuccess && device == 1);
+    lc2e_destroy(e);
+    CHECK(fake::used(0) == 0);
+}
+
 //@SCENARIOS
 
 const std::map<std::string, std::function<void()>> kScenarios = {
@@ -255,6 +269,7 @@ const std::map<std::string, std::function<void()>> kScenarios = {
     {"captured_launches_keep_their_workspace", captured_launches_keep_their_workspace},
     {"a_refused_workspace_is_not_asked_for_again", a_refused_workspace_is_not_asked_for_again},
     {"kept_memory_makes_room", kept_memory_makes_room},
+    {"releases_leave_the_current_device", releases_leave_the_current_device},
 //@TABLE
 };
 
