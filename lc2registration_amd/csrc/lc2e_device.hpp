@@ -6,6 +6,8 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <atomic>
+#include <initializer_list>
 #include <type_traits>
 
 #include "lc2e_kernels.hpp"
@@ -700,6 +702,23 @@ __device__ __forceinline__ bool map_block(int tiles, int npose, int& tile, int& 
     tile = (slot / npose) * kXcds + xcd;
     return tile < tiles;
 }
+
+// Raises the dynamic LDS limit of a kernel, once per device: the attribute belongs to the function
+// on the current device.
+struct LdsLimit {
+    std::atomic<unsigned long long> done{0};  // bit d: device d
+    hipError_t raise(std::initializer_list<const void*> kernels, size_t bytes) {
+        int d = 0;
+        hipError_t err = hipGetDevice(&d);
+        const unsigned long long bit = 1ULL << (d & 63);
+        if (err != hipSuccess || (done.load() & bit)) return err;
+        for (const void* k : kernels)
+            if ((err = hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes)) != hipSuccess)
+                return err;
+        done |= bit;
+        return hipSuccess;
+    }
+};
 
 template <int NTHR>
 __device__ __forceinline__ void block_reduce_store(double am, double aw, double* s_red,

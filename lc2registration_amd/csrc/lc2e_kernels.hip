@@ -1039,19 +1039,15 @@ hipError_t sep_sums(const float* I, const float* G, const float* U, double* sum_
     constexpr int NC = kSepNC<KIND>;
     const long long V = (long long)v.X * v.Y * v.Z;
     const int W = 2 * r + 1;
-    static std::once_flag once;
-    static hipError_t set_err = hipSuccess;
-    std::call_once(once, [] {  // 66 KB at the largest radius, 61 KB for the rows
-        for (const void* f : {reinterpret_cast<const void*>(&k_sep_pass<KIND>), reinterpret_cast<const void*>(&k_sep_pass<-1>)})
-            if (set_err == hipSuccess)
-                set_err = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                              (2 * kMaxRSep + 1) * 64 * sizeof(double));
-        if (set_err == hipSuccess)
-            set_err = hipFuncSetAttribute(reinterpret_cast<const void*>(&k_sep_combine<KIND>),
-                                          hipFuncAttributeMaxDynamicSharedMemorySize,
-                                          4 * NC * (64 + 2 * kMaxRSep) * sizeof(double));
-    });
-    if (set_err != hipSuccess) return set_err;
+    // 66 KB at the largest radius, 61 KB for the rows
+    static LdsLimit pass_limit, rows_limit;
+    hipError_t err = pass_limit.raise({reinterpret_cast<const void*>(&k_sep_pass<KIND>),
+                                       reinterpret_cast<const void*>(&k_sep_pass<-1>)},
+                                      (2 * kMaxRSep + 1) * 64 * sizeof(double));
+    if (err == hipSuccess)
+        err = rows_limit.raise({reinterpret_cast<const void*>(&k_sep_combine<KIND>)},
+                               4 * NC * (64 + 2 * kMaxRSep) * sizeof(double));
+    if (err != hipSuccess) return err;
     bool first = true;
     auto pass = [&](long long lines, long long outer, int stride, int n, const double* src, double* dst) {
         const long long tiles8 = ((lines + 63) / 64 + kXcds - 1) / kXcds * kXcds;

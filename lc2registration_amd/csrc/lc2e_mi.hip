@@ -1,6 +1,5 @@
 // Normalized mutual information (the patchSize 0 metric).
 #include <algorithm>
-#include <mutex>
 
 #include "lc2e_device.hpp"
 
@@ -379,17 +378,10 @@ hipError_t launch_mi(const FusedArgs& a, int grid_ndim, int src_ndim, int movi, 
     const long long chunk = (n + per_pose - 1) / per_pose;
     const dim3 gj((unsigned)((n + chunk - 1) / chunk), (unsigned)n_poses);
     const size_t lds = (size_t)((nb + 1) / 2) * sizeof(unsigned);
-    static std::once_flag once;
-    static hipError_t set_err = hipSuccess;
-    std::call_once(once, [] {
-        for (const void* f : {reinterpret_cast<const void*>(&k_mi_joint<float>),
-                              reinterpret_cast<const void*>(&k_mi_joint<__half>)}) {
-            set_err = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                          (int)((kMiMaxBins * kMiMaxBins / 2) * sizeof(unsigned)));
-            if (set_err != hipSuccess) return;
-        }
-    });
-    if (set_err != hipSuccess) return set_err;
+    static LdsLimit limit;
+    e = limit.raise({reinterpret_cast<const void*>(&k_mi_joint<float>), reinterpret_cast<const void*>(&k_mi_joint<__half>)},
+                    (kMiMaxBins * kMiMaxBins / 2) * sizeof(unsigned));
+    if (e != hipSuccess) return e;
     const int stat_is_u = movi ? 1 : 0;
     if (a.src_f16)
         hipLaunchKernelGGL(k_mi_joint<__half>, gj, dim3(1024), lds, st, a, g3, s3, stat, stat_is_u,

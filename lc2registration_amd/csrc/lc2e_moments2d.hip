@@ -2,8 +2,6 @@
 // moments of strips of columns and combines them. It warps the moving image in place, or, where
 // that is the high-resolution one and the launch is large, reads it and its |Sobel| from the
 // grid, written by k_warp2.
-#include <mutex>
-
 #include "lc2e_device.hpp"
 
 namespace lc2e {
@@ -482,12 +480,9 @@ template <int R, int ROLE, bool INPLACE>
 hipError_t moments2k(const FusedArgs& a, dim3 grid, hipStream_t st, int* occ) {
     const size_t lds = INPLACE ? InPlace<R, ROLE>::FLOATS * sizeof(float) : 0;
     if constexpr (INPLACE) {
-        static std::once_flag once;
-        static hipError_t err = hipSuccess;
-        std::call_once(once, [&] {
-            err = hipFuncSetAttribute(reinterpret_cast<const void*>(&k_moments2d<R, ROLE, INPLACE>),
-                                      hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-        });
+        static LdsLimit limit;
+        const hipError_t err =
+            limit.raise({reinterpret_cast<const void*>(&k_moments2d<R, ROLE, INPLACE>)}, lds);
         if (err != hipSuccess) return err;
     }
     if (occ) return hipOccupancyMaxActiveBlocksPerMultiprocessor(occ, k_moments2d<R, ROLE, INPLACE>, 256, lds);

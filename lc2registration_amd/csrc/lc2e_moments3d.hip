@@ -7,8 +7,6 @@
 // the first kernel's tile has 1.2 warped positions per voxel, and the second needs 84 VGPRs.
 // The grids cost 8 bytes written and about 10 read per voxel and pose, at 1 TB/s far from the
 // memory's rate. 192x192x160 grid, 7^3 patch, 32 poses: 3.40 -> 2.80 ms.
-#include <mutex>
-
 #include "lc2e_device.hpp"
 
 namespace lc2e {
@@ -450,12 +448,8 @@ void warp_us3(const FusedArgs& a, int ntx, int nty, int zc, int tiles, int n, hi
 template <int R, int ROLE>
 hipError_t moments3k(const FusedArgs& a, dim3 grid, hipStream_t st, int* occ) {
     using M = Mom<R, ROLE>;
-    static std::once_flag once;
-    static hipError_t err = hipSuccess;
-    std::call_once(once, [] {
-        err = hipFuncSetAttribute(reinterpret_cast<const void*>(&k_moments3d<R, ROLE>),
-                                  hipFuncAttributeMaxDynamicSharedMemorySize, (int)M::lds);
-    });
+    static LdsLimit limit;
+    const hipError_t err = limit.raise({reinterpret_cast<const void*>(&k_moments3d<R, ROLE>)}, M::lds);
     if (err != hipSuccess) return err;
     if (occ) return hipOccupancyMaxActiveBlocksPerMultiprocessor(occ, k_moments3d<R, ROLE>, M::NTHR, M::lds);
     hipLaunchKernelGGL((k_moments3d<R, ROLE>), grid, dim3(M::NTHR), M::lds, st, a);

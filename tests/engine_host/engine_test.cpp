@@ -261,6 +261,20 @@ void releases_leave_the_current_device() {
     CHECK(fake::used(0) == 0);
 }
 
+// Kernels of more than 64 KB of LDS need their limit raised on each device they run on.
+void every_device_gets_its_lds_limit() {
+    for (int device : {0, 1}) {
+        lc2e_engine* e = engine(0, device);
+        for (int r : {1, 3, 4, 6, 12}) {
+            Pair p(e, 3, 48, 48, 48, r % 2, r, true);
+            CHECK(p.batch(2) >= 0);
+            CHECK(p.mi(1) >= 0);
+        }
+        CHECK(Pair(e, 2, 256, 256, 1, 0, 64, false).batch(1) >= 0);
+        lc2e_destroy(e);
+    }
+}
+
 //@SCENARIOS
 
 const std::map<std::string, std::function<void()>> kScenarios = {
@@ -270,6 +284,7 @@ const std::map<std::string, std::function<void()>> kScenarios = {
     {"a_refused_workspace_is_not_asked_for_again", a_refused_workspace_is_not_asked_for_again},
     {"kept_memory_makes_room", kept_memory_makes_room},
     {"releases_leave_the_current_device", releases_leave_the_current_device},
+    {"every_device_gets_its_lds_limit", every_device_gets_its_lds_limit},
 //@TABLE
 };
 

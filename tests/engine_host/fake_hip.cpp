@@ -12,6 +12,7 @@
 namespace {
 
 thread_local int t_device = 0;
+thread_local hipError_t t_error = hipSuccess;  // a refused launch's
 struct Block {
     size_t bytes;
     int device;
@@ -90,7 +91,11 @@ hipError_t hipGetDevice(int* d) { return *d = t_device, hipSuccess; }
 hipError_t hipSetDevice(int d) { return d < 0 || d > 1 ? hipErrorInvalidDevice : (t_device = d, hipSuccess); }
 hipError_t hipDeviceGetAttribute(int* v, hipDeviceAttribute_t, int) { return *v = 256, hipSuccess; }
 const char* hipGetErrorString(hipError_t e) { return e == hipErrorOutOfMemory ? "out of memory" : "error"; }
-hipError_t hipGetLastError() { return hipSuccess; }
+hipError_t hipGetLastError() {
+    const hipError_t e = t_error;
+    t_error = hipSuccess;
+    return e;
+}
 
 hipError_t hipMalloc(void** p, size_t n) {
     LOCK;
@@ -204,9 +209,9 @@ hipError_t hipLaunchKernel(const void* fn, dim3 grid, dim3 block, void** args, s
     l.device = t_device;
     l.stream = st;
     l.captured = g().capturing.count(st) != 0;
-    if ((unsigned long long)grid.x * block.x >= (1ULL << 32)) return hipErrorInvalidConfiguration;
+    if ((unsigned long long)grid.x * block.x >= (1ULL << 32)) return t_error = hipErrorInvalidConfiguration;
     const auto it = g().lds.find({fn, t_device});
-    if (lds > 65536 && (it == g().lds.end() || (size_t)it->second < lds)) return hipErrorInvalidValue;
+    if (lds > 65536 && (it == g().lds.end() || (size_t)it->second < lds)) return t_error = hipErrorInvalidValue;
     for (const char* k : {"k_moments", "k_warp_grad3", "k_warp_us3", "k_warp2", "k_fused", "k_mi_warp3", "k_mi_joint"})
         if (l.is(k)) std::memcpy(&l.a, args[0], sizeof(l.a));
     g().launches.push_back(l);

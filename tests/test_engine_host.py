@@ -39,6 +39,7 @@ def engine_test(tmp_path_factory):
     "a_refused_workspace_is_not_asked_for_again",
     "kept_memory_makes_room",
     "releases_leave_the_current_device",
+    "every_device_gets_its_lds_limit",
 ])
 def test_engine_host(engine_test, scenario):
     r = subprocess.run([engine_test, scenario], capture_output=True, text=True, timeout=120)
