@@ -368,7 +368,11 @@ hipError_t launch_eval(lc2e_pair* p, const lc2e::FusedArgs& a, int n, hipStream_
         return lc2e::launch_moments(s, p->info.grid_ndim, p->role(), n, st);
     }
     if (p->two) {
-        const int step = part(w, n);
+        // (a launch has less than 2^32 work-items, of which the moments kernels take up to 1024
+        // per tile and pose)
+        const long long tiles8 = (a.tiles + lc2e::kXcds - 1) / lc2e::kXcds * (long long)lc2e::kXcds;
+        const int most = (int)std::max(1LL, std::min<long long>(1 << 30, ((1LL << 22) - 1) / std::max(1LL, tiles8)));
+        const int step = std::min(part(w, n), most);
         for (int b = 0; b < n; b += step) {
             const int m = std::min(step, n - b);
             lc2e::FusedArgs s = a;

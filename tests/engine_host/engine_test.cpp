@@ -275,6 +275,17 @@ void every_device_gets_its_lds_limit() {
     }
 }
 
+// Many poses of a tiny grid: no launch of 2^32 work-items or more.
+void launches_stay_below_the_runtime_limit() {
+    lc2e_engine* e = engine();
+    {
+        Pair p(e, 3, 3, 3, 3, 1, 1, true), q(e, 2, 9, 9, 1, 1, 4, false);
+        CHECK(p.async(800000, nullptr) >= 0);
+        CHECK(q.async(800000, nullptr) >= 0);
+    }
+    lc2e_destroy(e);
+}
+
 //@SCENARIOS
 
 const std::map<std::string, std::function<void()>> kScenarios = {
@@ -285,6 +296,7 @@ const std::map<std::string, std::function<void()>> kScenarios = {
     {"kept_memory_makes_room", kept_memory_makes_room},
     {"releases_leave_the_current_device", releases_leave_the_current_device},
     {"every_device_gets_its_lds_limit", every_device_gets_its_lds_limit},
+    {"launches_stay_below_the_runtime_limit", launches_stay_below_the_runtime_limit},
 //@TABLE
 };
 

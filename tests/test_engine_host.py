@@ -40,6 +40,7 @@ def engine_test(tmp_path_factory):
     "kept_memory_makes_room",
     "releases_leave_the_current_device",
     "every_device_gets_its_lds_limit",
+    "launches_stay_below_the_runtime_limit",
 ])
 def test_engine_host(engine_test, scenario):
     r = subprocess.run([engine_test, scenario], capture_output=True, text=True, timeout=120)
