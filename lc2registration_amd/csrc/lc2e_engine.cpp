@@ -511,6 +511,18 @@ Tiling tiling_for(lc2e_pair* p, int n, int poses) {
     return t;
 }
 
+// Partial sums per pose by which the allocation-free entry point admits a call, of the kernels it
+// was specified with: one per 16x16 tile and 16 frames (2D), per wave of a 16x16 tile and 8 planes
+// (3D), or per 256 outputs (radii beyond both). What is admitted does not depend on the kernel.
+size_t admitted_partials(const lc2e_pair* p) {
+    const int r = p->info.patch_radius;
+    if (p->sep || (p->info.grid_ndim == 3 && r > lc2e::kMaxR3)) return lc2e::sep_blocks(p->v, r, p->info.grid_ndim);
+    if (p->info.grid_ndim == 3) return lc2e::fused_partials_3d(p->v, r);
+    int ntx, nty;
+    lc2e::fused_blocks_2d(p->v, r, &ntx, &nty);
+    return (size_t)ntx * nty * ((p->v.Z + lc2e::kFrameRun - 1) / lc2e::kFrameRun);
+}
+
 // Launches of up to kDirectPoses poses with at most kHostPose partials each add them up on the
 // host (enqueue_batch).
 constexpr int kDirectPoses = 8;
@@ -1396,45 +1408,56 @@ int lc2e_eval_batch_noalloc(lc2e_pair* p, int n, const float* mats, double* lc2,
     hipStream_t st = e->stream;
     const int mpp = p->mats_per_pose();
     const Workspace ws = noalloc_workspace(p);
-    const Tiling t = tiling_for(p, n, ws.poses);
-    // scratch layout: results [n][3] f64, matrices [n][mpp][12] f32, partials [n][bpp][2] f64
+    // scratch layout: results [m][3] f64, matrices [m][mpp][12] f32, partials [m][bpp][2] f64
     auto up256 = [](size_t b) { return (b + 255) / 256 * 256; };
-    const size_t out_b = up256((size_t)n * 3 * sizeof(double));
-    const size_t mat_b = up256((size_t)n * mpp * 12 * sizeof(float));
-    const size_t part_b = (size_t)n * (t.tiles > 0 ? t.bpp : 0) * 2 * sizeof(double);
-    if (out_b + mat_b + part_b > lc2e::kScratchBytes)
+    auto bytes = [&](size_t m, size_t bpp) {
+        return up256(m * 3 * sizeof(double)) + up256(m * mpp * 12 * sizeof(float)) + m * bpp * 2 * sizeof(double);
+    };
+    const Tiling one = tiling_for(p, 1, ws.poses);
+    const size_t bpp = one.tiles > 0 ? one.bpp : 0;
+    const size_t need = bytes(n, admitted_partials(p));
+    if (need > lc2e::kScratchBytes || bytes(1, bpp) > lc2e::kScratchBytes)
         return fail(LC2E_ERR_INVALID,
                     "%d poses need %zu bytes of device scratch; the allocation-free entry point "
                     "has %zu (use lc2e_eval_batch or fewer poses per call)",
-                    n, out_b + mat_b + part_b, lc2e::kScratchBytes);
+                    n, need, lc2e::kScratchBytes);
+    // an admitted call whose partial sums take more than the scratch holds runs in parts
+    int most = n;
+    while (bytes(most, bpp) > lc2e::kScratchBytes) most = (most + 1) / 2;
     char* base = static_cast<char*>(e->scratch);
-    double* d_out = reinterpret_cast<double*>(base);
-    float* d_mats = reinterpret_cast<float*>(base + out_b);
-    double* d_part = reinterpret_cast<double*>(base + out_b + mat_b);
-    HIP_TRY(hipMemcpyAsync(d_mats, mats, (size_t)n * mpp * 12 * sizeof(float),
-                           hipMemcpyHostToDevice, st));
-    if (t.tiles > 0) {
-        // every partial slot is written by the fused kernel before k_reduce reads it, so the
-        // previous call's contents need no clearing
-        const lc2e::FusedArgs a = make_args(p, d_mats, d_part, t);
-        HIP_TRY(launch_eval(p, a, n, st, ws));
-    }
-    HIP_TRY(lc2e::launch_reduce(d_part, t.tiles > 0 ? t.bpp : 0, n, d_out, st));
-    // results back through a fixed host buffer, a chunk of poses at a time
     int status = LC2E_OK;
-    constexpr int kChunk = 128;
-    double h[kChunk * 3];
-    for (int b = 0; b < n; b += kChunk) {
-        const int m = n - b < kChunk ? n - b : kChunk;
-        HIP_TRY(hipMemcpyAsync(h, d_out + (size_t)b * 3, (size_t)m * 3 * sizeof(double),
-                               hipMemcpyDeviceToHost, st));
-        HIP_TRY(hipStreamSynchronize(st));
-        for (int i = 0; i < m; ++i) {
-            const double sm = h[3 * i], sw = h[3 * i + 1], l = h[3 * i + 2];
-            if (lc2) lc2[b + i] = l;
-            if (sum_measure) sum_measure[b + i] = sm;
-            if (sum_w) sum_w[b + i] = sw;
-            if (!(sw > 0.0) || !std::isfinite(sm / sw)) status = LC2E_OK_DEGENERATE;
+    for (int b0 = 0; b0 < n; b0 += most) {
+        const int nb = std::min(most, n - b0);
+        double* d_out = reinterpret_cast<double*>(base);
+        float* d_mats = reinterpret_cast<float*>(base + up256((size_t)nb * 3 * sizeof(double)));
+        double* d_part = reinterpret_cast<double*>(reinterpret_cast<char*>(d_mats) +
+                                                   up256((size_t)nb * mpp * 12 * sizeof(float)));
+        HIP_TRY(hipMemcpyAsync(d_mats, mats + (size_t)b0 * mpp * 12, (size_t)nb * mpp * 12 * sizeof(float),
+                               hipMemcpyHostToDevice, st));
+        const Tiling t = tiling_for(p, nb, ws.poses);
+        if (t.tiles > 0) {
+            // every partial slot is written by the kernels before k_reduce reads it, so the
+            // previous call's contents need no clearing
+            const lc2e::FusedArgs a = make_args(p, d_mats, d_part, t);
+            HIP_TRY(launch_eval(p, a, nb, st, ws));
+        }
+        HIP_TRY(lc2e::launch_reduce(d_part, (int)bpp, nb, d_out, st));
+        // results back through a fixed host buffer, a chunk of poses at a time
+        constexpr int kChunk = 128;
+        double h[kChunk * 3];
+        for (int b = 0; b < nb; b += kChunk) {
+            const int m = nb - b < kChunk ? nb - b : kChunk;
+            HIP_TRY(hipMemcpyAsync(h, d_out + (size_t)b * 3, (size_t)m * 3 * sizeof(double),
+                                   hipMemcpyDeviceToHost, st));
+            HIP_TRY(hipStreamSynchronize(st));
+            for (int i = 0; i < m; ++i) {
+                const double sm = h[3 * i], sw = h[3 * i + 1], l = h[3 * i + 2];
+                const int k = b0 + b + i;
+                if (lc2) lc2[k] = l;
+                if (sum_measure) sum_measure[k] = sm;
+                if (sum_w) sum_w[k] = sw;
+                if (!(sw > 0.0) || !std::isfinite(sm / sw)) status = LC2E_OK_DEGENERATE;
+            }
         }
     }
     return status;

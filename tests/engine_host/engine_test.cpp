@@ -286,6 +286,25 @@ void launches_stay_below_the_runtime_limit() {
     lc2e_destroy(e);
 }
 
+// The allocation-free entry point admits by the sizes it was specified with, whatever the kernels'
+// own partial sums take.
+void noalloc_admits_what_it_did() {
+    lc2e_engine* e = engine();
+    {
+        // one output voxel per plane: 100 / 256 -> 1 sum per pose, where the kernel writes more
+        Pair p(e, 3, 11, 11, 110, 1, 5, true);
+        fake::launches().clear();
+        CHECK(p.noalloc(100000) >= 0);
+        CHECK(fake::count("k_reduce") >= 1);
+        CHECK(p.noalloc(200000) == LC2E_ERR_INVALID);
+        // 256 tiles of 16x16 outputs per pose, which the kernel covers with fewer
+        Pair q(e, 2, 262, 262, 1, 0, 3, false);
+        CHECK(q.noalloc(4000) >= 0);
+        CHECK(q.noalloc(4100) == LC2E_ERR_INVALID);
+    }
+    lc2e_destroy(e);
+}
+
 //@SCENARIOS
 
 const std::map<std::string, std::function<void()>> kScenarios = {
@@ -297,6 +316,7 @@ const std::map<std::string, std::function<void()>> kScenarios = {
     {"releases_leave_the_current_device", releases_leave_the_current_device},
     {"every_device_gets_its_lds_limit", every_device_gets_its_lds_limit},
     {"launches_stay_below_the_runtime_limit", launches_stay_below_the_runtime_limit},
+    {"noalloc_admits_what_it_did", noalloc_admits_what_it_did},
 //@TABLE
 };
 

@@ -41,6 +41,7 @@ def engine_test(tmp_path_factory):
     "releases_leave_the_current_device",
     "every_device_gets_its_lds_limit",
     "launches_stay_below_the_runtime_limit",
+    "noalloc_admits_what_it_did",
 ])
 def test_engine_host(engine_test, scenario):
     r = subprocess.run([engine_test, scenario], capture_output=True, text=True, timeout=120)
