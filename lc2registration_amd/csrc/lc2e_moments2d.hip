@@ -399,6 +399,8 @@ void k_moments2d(FusedArgs a) {
                             for (int j = 1; j < W; ++j) out[o] += in[o + j];
                         }
                     }
+                    // other lanes read what is overwritten now: no store before the last read
+                    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
                     double* p = static_cast<double*>(__builtin_assume_aligned(xp, 16));
 #pragma unroll
                     for (int o = 0; o < 8; ++o) p[o] = out[o];
