@@ -133,16 +133,16 @@ struct InPlace {
 };
 
 // The moving image at column gx (this lane's) of rows gy0 .. gy0 + rows - 1 of frame's matrix m,
-// 0 outside the grid, into dst (rows 64 floats apart): this wave's share of the work-group's, every
-// fourth group of four rows, whose gathers are in flight at once.
-template <bool P2, bool SRC3D, typename T>
+// 0 outside the grid, into dst (rows 64 floats apart): this wave's share of the work-group's NW
+// waves', every NWth group of four rows, whose gathers are in flight at once.
+template <int NW, bool P2, bool SRC3D, typename T>
 __device__ __forceinline__ void warp_rows(const FusedArgs& a, const float* m, int gx, int gy0, int rows,
                                           float* dst, int wave) {
     const T* __restrict__ src = static_cast<const T*>(a.src);
     using Pend = typename std::conditional<SRC3D, Pending3<T>, Pending2<T>>::type;
     const float lx = fmaf((float)gx, a.v.sx, a.v.ox);
     const bool inx = gx >= 0 && gx < a.v.X;
-    for (int j0 = 4 * wave; j0 < rows; j0 += 16) {
+    for (int j0 = 4 * wave; j0 < rows; j0 += 4 * NW) {
         Pend p[4];
 #pragma unroll
         for (int k = 0; k < 4; ++k) {
@@ -157,44 +157,62 @@ __device__ __forceinline__ void warp_rows(const FusedArgs& a, const float* m, in
         }
     }
 }
+template <int NW>
 __device__ __forceinline__ void warp_rows_any(const FusedArgs& a, int src3, const float* m, int gx, int gy0,
                                               int rows, float* dst, int wave) {
     const int form = (src3 ? 4 : 0) + (a.s.pow2 ? 2 : 0) + (a.src_f16 ? 1 : 0);  // uniform
     switch (form) {
-        case 7: return warp_rows<true, true, __half>(a, m, gx, gy0, rows, dst, wave);
-        case 6: return warp_rows<true, true, float>(a, m, gx, gy0, rows, dst, wave);
-        case 5: return warp_rows<false, true, __half>(a, m, gx, gy0, rows, dst, wave);
-        case 4: return warp_rows<false, true, float>(a, m, gx, gy0, rows, dst, wave);
-        case 3: return warp_rows<true, false, __half>(a, m, gx, gy0, rows, dst, wave);
-        case 2: return warp_rows<true, false, float>(a, m, gx, gy0, rows, dst, wave);
-        case 1: return warp_rows<false, false, __half>(a, m, gx, gy0, rows, dst, wave);
-        default: return warp_rows<false, false, float>(a, m, gx, gy0, rows, dst, wave);
+        case 7: return warp_rows<NW, true, true, __half>(a, m, gx, gy0, rows, dst, wave);
+        case 6: return warp_rows<NW, true, true, float>(a, m, gx, gy0, rows, dst, wave);
+        case 5: return warp_rows<NW, false, true, __half>(a, m, gx, gy0, rows, dst, wave);
+        case 4: return warp_rows<NW, false, true, float>(a, m, gx, gy0, rows, dst, wave);
+        case 3: return warp_rows<NW, true, false, __half>(a, m, gx, gy0, rows, dst, wave);
+        case 2: return warp_rows<NW, true, false, float>(a, m, gx, gy0, rows, dst, wave);
+        case 1: return warp_rows<NW, false, false, __half>(a, m, gx, gy0, rows, dst, wave);
+        default: return warp_rows<NW, false, false, float>(a, m, gx, gy0, rows, dst, wave);
     }
 }
 
-template <int R, int ROLE, bool INPLACE>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(
+// OUT = 8: as above. OUT = 4, for launches that leave the chip idle: two waves share a block of eight
+// rows and take four outputs each, summed over the same suffixes and prefixes, so every pixel's
+// sums keep their bits; the x pass takes two channels at a time (all lanes busy, half the trips), and
+// a wave's chain is about half as long. Measures and weights are added up per lane over the four
+// rows of a half block, over its lanes, and then half block by half block, in either form.
+template <int R, int ROLE, bool INPLACE, int OUT>
+__global__ __launch_bounds__(64 * 32 / OUT) __attribute__((amdgpu_waves_per_eu(
     ROLE == kRoleStaticImage || ROLE == kRoleUsStats ? 3 : 2)))
 void k_moments2d(FusedArgs a) {
     using Ro = Role<ROLE>;
     using IP = InPlace<R, ROLE>;
     constexpr int NC = Ro::NC, W = 2 * R + 1, TX = strip2(R, ROLE), N = W * W;
     constexpr int H = INPLACE ? IP::H : 0;  // lane of the first column
-    __shared__ __align__(16) double s_all[4 * kWaveS];
-    __shared__ double s_red[8];
+    constexpr int NW = 32 / OUT, CP = 8 / OUT;  // waves; channels per trip of the x pass
+    __shared__ __align__(16) double s_all[NW * kWaveS];
+    __shared__ double s_red[16];
     extern __shared__ float s_rows[];  // INPLACE: IP::FLOATS
 
     int tile, pose;
-    if (!map_block(a.tiles, a.npose, tile, pose)) return;  // whole work-group
+    if constexpr (OUT == 4) {
+        // A part of a small launch's time is its reads of the arguments, which lie in the host's
+        // memory: one request for every line of them, where the compiler would read and wait seven
+        // times (1.9 -> 1.4 us), and a pose that does not depend on them.
+        asm volatile("" ::"s"(a.v.X), "s"(a.s.oz), "s"(a.src), "s"(a.stat_img), "s"(a.stat_grad), "s"(a.mats),
+                     "s"(a.inline_mat), "s"(a.ntx), "s"(a.tiles), "s"(a.istat), "s"(a.src3));
+        tile = blockIdx.x;
+        pose = blockIdx.y;
+        if (tile >= a.tiles) return;
+    } else {
+        if (!map_block(a.tiles, a.npose, tile, pose)) return;  // whole work-group
+    }
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     const int cols = a.ntx * a.nty;
     const int tcol = tile % cols, run = tile / cols;
     const int X = a.v.X, Y = a.v.Y, Z = a.v.Z, XY = X * Y;
-    const int x0 = R + (tcol % a.ntx) * TX, y0 = R + (tcol / a.ntx) * 32 + wave * 8;
+    const int x0 = R + (tcol % a.ntx) * TX, y0 = R + (tcol / a.ntx) * 32 + wave * OUT;
     const int col = lane - H;  // column of the strip
     const bool has_rows = y0 < Y - R;  // the wave has output rows
     const int f0 = run * a.zchunk, f1 = INPLACE || has_rows ? min(f0 + a.zchunk, Z) : f0;
-    double acc_m = 0.0, acc_w = 0.0;
+    double acc_m[OUT / 4] = {}, acc_w[OUT / 4] = {};
 
     {
         double* const s = s_all + wave * kWaveS;
@@ -205,7 +223,7 @@ void k_moments2d(FusedArgs a) {
         const bool okx = col >= 0 && col < TX && ox < X - R;
         const int s_col = lds_col(min(max(col, 0), 63));
         const bool has_col = col >= 0;
-        float* const rows = s_rows + (INPLACE ? wave * 8 * 64 + lane : 0);
+        float* const rows = s_rows + (INPLACE ? wave * OUT * 64 + lane : 0);
         const int run_x = lane % 8, run_y = lane / 8;
         double* const xp = s + run_y * kRowS + run_x * 10;
         for (int f = f0; f < f1; ++f) {
@@ -213,14 +231,14 @@ void k_moments2d(FusedArgs a) {
             if constexpr (INPLACE) {
                 float m[12];
                 load_matrix(a, (size_t)pose * a.mats_per_pose + (a.mats_per_pose > 1 ? f : 0), m);
-                const int top = y0 - wave * 8 - R - H;  // grid row of the first one
+                const int top = y0 - wave * OUT - R - H;  // grid row of the first one
                 const int nrows = min(IP::ROWS, Y + H - top);  // none past the grid's but the Sobel's
                 if (f > f0) __syncthreads();  // the last frame's are read
-                warp_rows_any(a, a.src3, m, x0 - R + col, top, nrows, s_rows + lane, wave);
+                warp_rows_any<NW>(a, a.src3, m, x0 - R + col, top, nrows, s_rows + lane, wave);
                 __syncthreads();
                 if constexpr (ROLE == kRoleMovingImage) {
-                    // |Sobel| of the rows between, a quarter per wave; the outermost lanes' is not used
-                    constexpr int Q = (IP::ROWS - 2 + 3) / 4;
+                    // |Sobel| of the rows between, a part per wave; the outermost lanes' is not used
+                    constexpr int Q = (IP::ROWS - 2 + NW - 1) / NW;
                     const float* const in = s_rows + lane;
                     float* const g = s_rows + IP::ROWS * 64 + lane;
                     const int left = lane > 0 ? -1 : 0, right = lane < 63 ? 1 : 0;
@@ -231,20 +249,24 @@ void k_moments2d(FusedArgs a) {
                         sm[k] = fmaf(2.0f, c, l) + r;
                         df[k] = r - l;
                     };
+                    auto store = [&](int j, int k) {  // of lines k, k + 1, k + 2
+                        const float gxv = fmaf(2.0f, df[k + 1], df[k]) + df[k + 2], gyv = sm[k + 2] - sm[k];
+                        g[(j + 1) * 64] = sqrtf(fmaf(gyv, gyv, gxv * gxv));
+                    };
                     if (j0 + 2 < j1) {
                         line(j0, 0);
                         line(j0 + 1, 1);
                     }
                     for (int j = j0 + 2; j < j1; ++j) {
                         line(j, 2);
-                        const float gxv = fmaf(2.0f, df[1], df[0]) + df[2], gyv = sm[2] - sm[0];
-                        g[(j - 1) * 64] = sqrtf(fmaf(gyv, gyv, gxv * gxv));
+                        store(j - 2, 0);
                         sm[0] = sm[1], sm[1] = sm[2], df[0] = df[1], df[1] = df[2];
                     }
                     __syncthreads();
                 }
                 if (!has_rows) continue;
             }
+            // row y0 - R + j at this lane's column
             auto input = [&](int j, double& I, double& G, double& U) {
                 const size_t row = (size_t)min(y0 - R + j, Y - 1) * X;  // wave-uniform
                 I = G = U = 0.0;
@@ -272,20 +294,23 @@ void k_moments2d(FusedArgs a) {
                     }
                 }
             };
-            // 1. y window sums of rows y0 .. y0 + 7: the rows all eight windows share, the
-            // suffixes before them and the prefixes after them
-            double S[8][NC];
-            if constexpr (W >= 7) {
+            // 1. y window sums of the wave's rows. Of a block of eight: the rows all eight windows
+            // share, the suffixes before them and the prefixes after them; A: the wave's first row
+            // of its block
+            double S[OUT][NC];
+            auto y_sums = [&](auto first) {
+                constexpr int A = decltype(first)::value, B = A + OUT;
                 double t[NC];
 #pragma unroll
                 for (int c = 0; c < NC; ++c) t[c] = 0.0;
 #pragma unroll
-                for (int j = 6; j >= 0; --j) {
+                for (int j = 6; j >= A; --j) {
                     double I, G, U;
-                    input(j, I, G, U);
+                    input(j - A, I, G, U);
                     Ro::add(t, I, G, U);
+                    if (j < B)
 #pragma unroll
-                    for (int c = 0; c < NC; ++c) S[j][c] = t[c];
+                        for (int c = 0; c < NC; ++c) S[j - A][c] = t[c];
                 }
                 __builtin_amdgcn_sched_barrier(0);  // bounds the loads in flight
 #pragma unroll
@@ -293,53 +318,61 @@ void k_moments2d(FusedArgs a) {
 #pragma unroll
                 for (int j = 7; j < W; ++j) {
                     double I, G, U;
-                    input(j, I, G, U);
+                    input(j - A, I, G, U);
                     Ro::add(t, I, G, U);
                     if (j % 8 == 7) __builtin_amdgcn_sched_barrier(0);
                 }
                 if constexpr (W > 7)
 #pragma unroll
-                    for (int o = 0; o < 7; ++o)
+                    for (int o = A; o < B && o < 7; ++o)
 #pragma unroll
-                        for (int c = 0; c < NC; ++c) S[o][c] += t[c];
+                        for (int c = 0; c < NC; ++c) S[o - A][c] += t[c];
 #pragma unroll
-                for (int c = 0; c < NC; ++c) S[7][c] = t[c], t[c] = 0.0;
-#pragma unroll
-                for (int o = 1; o < 8; ++o) {
-                    double I, G, U;
-                    input(W - 1 + o, I, G, U);
-                    Ro::add(t, I, G, U);
-#pragma unroll
-                    for (int c = 0; c < NC; ++c) S[o][c] += t[c];
+                for (int c = 0; c < NC; ++c) {
+                    if (B == 8) S[OUT - 1][c] = t[c];
+                    t[c] = 0.0;
                 }
+#pragma unroll
+                for (int o = 1; o < B; ++o) {
+                    double I, G, U;
+                    input(W - 1 + o - A, I, G, U);
+                    Ro::add(t, I, G, U);
+                    if (o >= A)
+#pragma unroll
+                        for (int c = 0; c < NC; ++c) S[o - A][c] += t[c];
+                }
+            };
+            if constexpr (W >= 7) {
+                if (OUT == 8 || wave % 2 == 0) y_sums(std::integral_constant<int, 0>{});
+                else if constexpr (OUT == 4) y_sums(std::integral_constant<int, 4>{});
             } else {
 #pragma unroll
-                for (int o = 0; o < 8; ++o)
+                for (int o = 0; o < OUT; ++o)
 #pragma unroll
                     for (int c = 0; c < NC; ++c) S[o][c] = 0.0;
 #pragma unroll
-                for (int j = 0; j < W + 7; ++j) {
+                for (int j = 0; j < W + OUT - 1; ++j) {
                     double I, G, U;
                     input(j, I, G, U);
 #pragma unroll
-                    for (int o = 0; o < 8; ++o)
+                    for (int o = 0; o < OUT; ++o)
                         if (j >= o && j < o + W) Ro::add(S[o], I, G, U);
                 }
             }
-            // 2. x window sums, channel by channel (the pins and scheduling barriers keep the
+            // 2. x window sums, CP channels at a time (the pins and scheduling barriers keep the
             // compiler from running phases into each other, which costs a wave per SIMD)
             auto pin = [&]() {
 #pragma unroll
-                for (int o = 0; o < 8; ++o)
+                for (int o = 0; o < OUT; ++o)
 #pragma unroll
                     for (int c = 0; c < NC; ++c) asm volatile("" : "+v"(S[o][c]));
                 __builtin_amdgcn_sched_barrier(0);
             };
             pin();
-            // the pixels' statistics, requested before the last channel's LDS work
+            // the pixels' statistics, requested before the last channels' LDS work
             const unsigned vx = (unsigned)(okx ? ox : R) * 8u;
-            double mu[8], cyy[8];
-            ImageStats ist[8];
+            double mu[OUT], cyy[OUT];
+            ImageStats ist[OUT];
             auto stats = [&](int o0, int o1) {
 #pragma unroll
                 for (int o = o0; o < o1; ++o) {
@@ -356,12 +389,15 @@ void k_moments2d(FusedArgs a) {
                     }
                 }
             };
+            constexpr bool EARLY = ROLE == kRoleMovingImage || (ROLE == kRoleStaticImage && OUT == 4);
 #pragma unroll
-            for (int c = 0; c < NC; ++c) {
-                if (ROLE == kRoleMovingImage && c == NC - 1) stats(0, 8);
+            for (int c = 0; c < NC; c += CP) {
+                if (EARLY && c + CP >= NC) stats(0, OUT);
 #pragma unroll
-                for (int o = 0; o < 8; ++o)
-                    if (has_col) s[o * kRowS + s_col] = S[o][c];
+                for (int k = 0; k < CP && c + k < NC; ++k)
+#pragma unroll
+                    for (int o = 0; o < OUT; ++o)
+                        if (has_col) s[(k * OUT + o) * kRowS + s_col] = S[o][c + k];
                 wave_fence();
                 if (run_x * 8 < TX) {
                     double in[W + 8], out[8];
@@ -407,24 +443,26 @@ void k_moments2d(FusedArgs a) {
                 }
                 wave_fence();
 #pragma unroll
-                for (int o = 0; o < 8; ++o) {
-                    S[o][c] = s[o * kRowS + s_col];
-                    asm volatile("" : "+v"(S[o][c]));
-                }
+                for (int k = 0; k < CP && c + k < NC; ++k)
+#pragma unroll
+                    for (int o = 0; o < OUT; ++o) {
+                        S[o][c + k] = s[(k * OUT + o) * kRowS + s_col];
+                        asm volatile("" : "+v"(S[o][c + k]));
+                    }
                 wave_fence();
                 __builtin_amdgcn_sched_barrier(0);
             }
             pin();
             // 3. combine
 #pragma unroll
-            for (int o = 0; o < 8; ++o) {
+            for (int o = 0; o < OUT; ++o) {
                 const int oy = y0 + o;
                 if (o % 2 == 0) __builtin_amdgcn_sched_barrier(0);
                 const bool ok_row = oy < Y - R;  // wave-uniform
                 const size_t vz = plane + (size_t)min(oy, Y - R - 1) * X + (okx ? ox : R);
                 double w = 0.0, meas = 0.0;
                 bool ok = okx && ok_row;
-                if (ROLE == kRoleStaticImage && o % 2 == 0) stats(o, o + 2);
+                if (ROLE == kRoleStaticImage && !EARLY && o % 2 == 0) stats(o, o + 2);
                 if constexpr (ROLE == kRoleMovingImage) {
                     ok = ok && cyy[o] >= 0.0;
                     combine_static_u_any(S[o], mu[o], ok ? cyy[o] : 1.0, N, w, meas);
@@ -440,8 +478,8 @@ void k_moments2d(FusedArgs a) {
                     if (ok) store_us_stats(S[o], N, a.ustat_mean_out + vz, a.ustat_cyy_out + vz);
                 }
                 if constexpr (Ro::SUMS) {
-                    acc_m += ok ? meas : 0.0;
-                    acc_w += ok ? w : 0.0;
+                    acc_m[o / 4] += ok ? meas : 0.0;
+                    acc_w[o / 4] += ok ? w : 0.0;
                     if (a.wmap && ok) {
                         a.wmap[vz] = w;
                         a.mmap[vz] = meas;
@@ -450,9 +488,20 @@ void k_moments2d(FusedArgs a) {
             }
         }
     }
-    if constexpr (Ro::SUMS)
-        block_reduce_store<256>(acc_m, acc_w, s_red,
-                                a.partials + ((size_t)pose * a.blocks_per_pose + tile) * 2);
+    if constexpr (Ro::SUMS) {
+#pragma unroll
+        for (int h = 0; h < OUT / 4; ++h) {
+            wave_reduce_store(acc_m[h], acc_w[h], s_red + 2 * (wave * (OUT / 4) + h));
+        }
+        __syncthreads();
+        if (threadIdx.x == 0) {
+            double m = 0.0, w = 0.0;
+            for (int h = 0; h < 8; ++h) m += s_red[2 * h], w += s_red[2 * h + 1];
+            double* dst = a.partials + ((size_t)pose * a.blocks_per_pose + tile) * 2;
+            dst[0] = m;
+            dst[1] = w;
+        }
+    }
 }
 
 template <bool SRC3D, typename T, bool P2>
@@ -478,24 +527,35 @@ void warp2t(const FusedArgs& a, int n, hipStream_t st) {
     }
 }
 
-template <int R, int ROLE, bool INPLACE>
+template <int R, int ROLE, bool INPLACE, int OUT>
 hipError_t moments2k(const FusedArgs& a, dim3 grid, hipStream_t st, int* occ) {
     const size_t lds = INPLACE ? InPlace<R, ROLE>::FLOATS * sizeof(float) : 0;
+    constexpr int NT = 64 * 32 / OUT;
     if constexpr (INPLACE) {
         static LdsLimit limit;
         const hipError_t err =
-            limit.raise({reinterpret_cast<const void*>(&k_moments2d<R, ROLE, INPLACE>)}, lds);
+            limit.raise({reinterpret_cast<const void*>(&k_moments2d<R, ROLE, INPLACE, OUT>)}, lds);
         if (err != hipSuccess) return err;
     }
-    if (occ) return hipOccupancyMaxActiveBlocksPerMultiprocessor(occ, k_moments2d<R, ROLE, INPLACE>, 256, lds);
-    hipLaunchKernelGGL((k_moments2d<R, ROLE, INPLACE>), grid, dim3(256), lds, st, a);
+    if (occ) return hipOccupancyMaxActiveBlocksPerMultiprocessor(occ, k_moments2d<R, ROLE, INPLACE, OUT>, NT, lds);
+    hipLaunchKernelGGL((k_moments2d<R, ROLE, INPLACE, OUT>), grid, dim3(NT), lds, st, a);
     return hipGetLastError();
 }
-template <int ROLE, bool INPLACE, int R = ROLE == kRoleMovingImage ? kMaxRFused2 + 1 : 1>
+template <int ROLE, bool INPLACE, int OUT, int R = ROLE == kRoleMovingImage ? kMaxRFused2 + 1 : 1>
 hipError_t moments2r(const FusedArgs& a, dim3 grid, hipStream_t st, int* occ) {
-    if (a.r == R) return moments2k<R, ROLE, INPLACE>(a, grid, st, occ);
-    if constexpr (R < kMaxR2) return moments2r<ROLE, INPLACE, R + 1>(a, grid, st, occ);
+    if (a.r == R) return moments2k<R, ROLE, INPLACE, OUT>(a, grid, st, occ);
+    if constexpr (R < kMaxR2) return moments2r<ROLE, INPLACE, OUT, R + 1>(a, grid, st, occ);
     return hipErrorInvalidValue;
+}
+// In place: four rows per wave up to one work-group per CU. Kernel, 256x256, four rows and eight:
+// moving, R = 4, 40 to 160 work-groups 12.2 and 16.2 us, 320 20.9 and 19.8; R = 9, 192 14.9 and 18.4,
+// 384 25.0 and 22.2; static, R = 3, 40 10.2 and 12.8, 640 18.6 and 18.6; R = 9, 192 12.4 and 15.2,
+// 384 20.5 and 17.7 (with events; radii up to 3 of a static image would gain up to 600).
+constexpr long long kSplitGroups = 256;
+template <int ROLE>
+hipError_t moments2i(const FusedArgs& a, dim3 grid, hipStream_t st, int* occ) {
+    if (!occ && (long long)a.tiles * a.npose <= kSplitGroups) return moments2r<ROLE, true, 4>(a, dim3((unsigned)((a.tiles + kXcds - 1) / kXcds * kXcds), (unsigned)a.npose), st, occ);
+    return moments2r<ROLE, true, 8>(a, grid, st, occ);
 }
 
 }  // namespace
@@ -514,12 +574,12 @@ hipError_t moments2(const FusedArgs& a, int role, int n, hipStream_t st, int* oc
     const dim3 grid((unsigned)(tiles8 * n));
     switch (role) {
         case kRoleMovingImage:
-            return a.in_place ? moments2r<kRoleMovingImage, true>(a, grid, st, occ)
-                              : moments2r<kRoleMovingImage, false>(a, grid, st, occ);
-        case kRoleStaticImage: return moments2r<kRoleStaticImage, true>(a, grid, st, occ);
-        case kRoleStaticImageFull: return moments2r<kRoleStaticImageFull, true>(a, grid, st, occ);
-        case kRoleImageStats: return moments2r<kRoleImageStats, false>(a, grid, st, occ);
-        default: return moments2r<kRoleUsStats, false>(a, grid, st, occ);
+            return a.in_place ? moments2i<kRoleMovingImage>(a, grid, st, occ)
+                              : moments2r<kRoleMovingImage, false, 8>(a, grid, st, occ);
+        case kRoleStaticImage: return moments2i<kRoleStaticImage>(a, grid, st, occ);
+        case kRoleStaticImageFull: return moments2i<kRoleStaticImageFull>(a, grid, st, occ);
+        case kRoleImageStats: return moments2r<kRoleImageStats, false, 8>(a, grid, st, occ);
+        default: return moments2r<kRoleUsStats, false, 8>(a, grid, st, occ);
     }
 }
 

@@ -305,6 +305,24 @@ void noalloc_admits_what_it_did() {
     lc2e_destroy(e);
 }
 
+// A 2D launch that leaves the chip idle runs in twice the waves of half the chain each; one of
+// more than a work-group per CU does not.
+void small_2d_launches_have_short_waves() {
+    lc2e_engine *e = engine(), *b = engine(GB);
+    for (lc2e_engine* x : {e, b})
+        for (int movi : {0, 1}) {
+            Pair p(x, 2, 256, 256, 1, movi, 5, false);
+            fake::launches().clear();
+            CHECK(p.batch(1) >= 0 && p.batch(64) >= 0);
+            std::vector<unsigned> threads;
+            for (const auto& l : fake::launches())
+                if (l.is("k_moments2d")) threads.push_back(l.threads);
+            CHECK(threads.size() == 2 && threads[0] == 512 && threads[1] == 256);
+        }
+    lc2e_destroy(b);
+    lc2e_destroy(e);
+}
+
 //@SCENARIOS
 
 const std::map<std::string, std::function<void()>> kScenarios = {
@@ -317,6 +335,7 @@ const std::map<std::string, std::function<void()>> kScenarios = {
     {"every_device_gets_its_lds_limit", every_device_gets_its_lds_limit},
     {"launches_stay_below_the_runtime_limit", launches_stay_below_the_runtime_limit},
     {"noalloc_admits_what_it_did", noalloc_admits_what_it_did},
+    {"small_2d_launches_have_short_waves", small_2d_launches_have_short_waves},
 //@TABLE
 };
 

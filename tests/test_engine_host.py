@@ -42,6 +42,7 @@ def engine_test(tmp_path_factory):
     "every_device_gets_its_lds_limit",
     "launches_stay_below_the_runtime_limit",
     "noalloc_admits_what_it_did",
+    "small_2d_launches_have_short_waves",
 ])
 def test_engine_host(engine_test, scenario):
     r = subprocess.run([engine_test, scenario], capture_output=True, text=True, timeout=120)
