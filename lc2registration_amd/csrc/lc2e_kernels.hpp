@@ -22,7 +22,7 @@ constexpr int kMaxRFused2 = 3; // largest patch radius of the 2D fused kernel
 constexpr int kMaxR2 = 10;     // largest patch radius of the 2D moments kernel
 constexpr int kMaxRSep = 64;   // largest patch radius of the separable path (larger radii)
 constexpr int kInlineMats = 8; // matrices a launch carries in its arguments
-constexpr int kFrameRun = 16;  // frames per 2D work-group (frame stacks)
+constexpr int kFrameRun = 16;  // most frames per 2D work-group (frame stacks)
 // The fused kernels' samplers form voxel offsets with 24-bit multiplies: a 3D source whose
 // slices hold this many voxels or more is evaluated by the separable path instead.
 constexpr long long kMaxFusedSlice = 1LL << 24;

@@ -323,6 +323,32 @@ void small_2d_launches_have_short_waves() {
     lc2e_destroy(e);
 }
 
+// One pose of a stack spreads over the chip, with no more partial sums than 16x16 tiles over 16
+// frames each had (by which memory and the allocation-free entry point are sized).
+void one_pose_of_a_stack_fills_the_device() {
+    lc2e_engine *e = engine(), *b = engine(8 * GB);
+    struct {
+        int x, y, z, r, groups;
+    } cases[] = {{256, 200, 40, 4, 400}, {256, 200, 40, 9, 400}, {512, 384, 128, 5, 1024}, {90, 70, 100, 10, 64}, {21, 22, 50, 10, 4}};
+    for (lc2e_engine* x : {e, b})
+        for (const auto& c : cases)
+            for (int movi : {0, 1}) {
+                Pair p(x, 2, c.x, c.y, c.z, movi, c.r, true, true);
+                fake::launches().clear();
+                CHECK(p.batch(1) >= 0);
+                const int ex = c.x - 2 * c.r, ey = c.y - 2 * c.r;
+                const int most = (ex + 15) / 16 * ((ey + 15) / 16) * ((c.z + 15) / 16);
+                for (const auto& l : fake::launches())
+                    if (l.is("k_moments2d")) {
+                        CHECK(l.a.tiles >= c.groups);
+                        CHECK(l.a.blocks_per_pose <= most);
+                    }
+                CHECK(fake::count("k_moments2d") == 1);
+            }
+    lc2e_destroy(b);
+    lc2e_destroy(e);
+}
+
 //@SCENARIOS
 
 const std::map<std::string, std::function<void()>> kScenarios = {
@@ -336,6 +362,7 @@ const std::map<std::string, std::function<void()>> kScenarios = {
     {"launches_stay_below_the_runtime_limit", launches_stay_below_the_runtime_limit},
     {"noalloc_admits_what_it_did", noalloc_admits_what_it_did},
     {"small_2d_launches_have_short_waves", small_2d_launches_have_short_waves},
+    {"one_pose_of_a_stack_fills_the_device", one_pose_of_a_stack_fills_the_device},
 //@TABLE
 };
 

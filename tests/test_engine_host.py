@@ -43,6 +43,7 @@ def engine_test(tmp_path_factory):
     "launches_stay_below_the_runtime_limit",
     "noalloc_admits_what_it_did",
     "small_2d_launches_have_short_waves",
+    "one_pose_of_a_stack_fills_the_device",
 ])
 def test_engine_host(engine_test, scenario):
     r = subprocess.run([engine_test, scenario], capture_output=True, text=True, timeout=120)

@@ -1,0 +1,80 @@
+"""Frame stacks with a matrix per frame on the 2D moments path (radii 4 to 10 of a moving
+high-resolution volume, every radius of a fixed one) against the oracle, frame by frame; and the
+same bits whichever way a call goes: warped in place, through the grid, through it in parts."""
+import numpy as np
+import pytest
+
+from lc2registration_amd import engine as E
+from oracle import oracle as O
+
+pytestmark = pytest.mark.gpu
+
+
+def _stack(movi, dims, seed):
+    rng = np.random.default_rng(seed)
+    x, y, z = dims
+    ramp = np.linspace(0, 1, x)
+    fixed = rng.random((z, y, x)) + ramp
+    volume = rng.random((20, y + 6, x + 8)) + np.linspace(0, 1, x + 8)
+
+    def us(a):
+        a = np.clip(a * 100, 1, 255)
+        a[..., :2, :3] = 0
+        return a.astype(np.uint8)
+
+    return (us(fixed), volume.astype(np.float32)) if movi else (fixed.astype(np.float32), us(volume))
+
+
+def _mats(n, frames, seed):
+    rng = np.random.default_rng(seed)
+    out = np.zeros((n, frames, 3, 4), np.float32)
+    for k in range(n):
+        for f in range(frames):
+            a, b = 0.03 * rng.standard_normal(2)
+            out[k, f] = [[np.cos(a), -np.sin(a), 0.1 * b, 3 + rng.uniform(-1, 1)],
+                         [np.sin(a), np.cos(a), -0.2 * b, 2 + rng.uniform(-1, 1)],
+                         [0.05 * b, 0.1 * a, 1, 1.0 + 17.0 * f / frames]]
+    return out
+
+
+@pytest.mark.parametrize("movi,r,dims", [
+    (True, 4, (70, 53, 18)), (True, 9, (61, 47, 19)), (True, 10, (95, 29, 33)),
+    (False, 1, (66, 35, 17)), (False, 3, (61, 41, 18)), (False, 9, (64, 59, 35))])
+def test_tracked_stacks_equal_oracle_however_they_run(movi, r, dims):
+    fixed, volume = _stack(movi, dims, r)
+    x, y, z = dims
+    n = 1 + 2048 // (4 * z)  # more waves than a launch that warps in place has
+    mats = _mats(n, z, r)
+    print(f"tracked stack: movi {movi}, r {r}, {dims}, {n} poses", flush=True)
+    got = {}
+    for name, budget in (("engine", 0), ("budget", 1 << 30)):
+        e = E.Engine(0, budget)
+        fv = e.upload(fixed, (1.0, 1.0, 1.0), (0.0, 0.0, 0.0))
+        mv = e.upload(volume, (1.0, 1.0, 1.0), (0.0, 0.0, 0.0))
+        p = e.pair(fv, mv, (1.0, 1.0), movi, False, r, 2)
+        p.set_per_frame(True)
+        got[name + " noalloc"] = p.eval_batch_noalloc(mats)
+        got[name + " batch"] = p.eval_batch(mats)
+        for k in (0, n - 1):
+            one = p.eval_batch(mats[k][None])
+            assert one.lc2[0] == got[name + " batch"].lc2[k] and one.sum_w[0] == got[name + " batch"].sum_w[k]
+        p.close()
+        fv.close()
+        mv.close()
+        e.close()
+    b = got["engine batch"]
+    for name, g in got.items():
+        assert np.array_equal(g.sum_measure, b.sum_measure) and np.array_equal(g.sum_w, b.sum_w), name
+    mg = O.geom(volume.shape[::-1], (1.0,) * 3, (0.0,) * 3)
+    vg = O.geom((x, y, 1), (1.0,) * 3, (0.0,) * 3)
+    for k in (0, n - 1):
+        sm = sw = 0.0
+        for f in range(z):
+            warped = O.warp_3d(volume.astype(np.float32), mg, vg, mats[k, f].ravel())[0]
+            U, I = (fixed[f].astype(np.float32), warped) if movi else (warped, fixed[f])
+            res = O.lc2_exact(U, I, O.sobel(I, "sep"), r)
+            sm += res.sum_measure
+            sw += res.sum_w
+        assert sw > 0
+        assert abs(b.sum_w[k] - sw) < 1e-9 * sw
+        assert abs(b.sum_measure[k] - sm) < 1e-8 * sm
