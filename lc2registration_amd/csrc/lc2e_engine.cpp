@@ -523,11 +523,11 @@ size_t admitted_partials(const lc2e_pair* p) {
     return (size_t)ntx * nty * ((p->v.Z + lc2e::kFrameRun - 1) / lc2e::kFrameRun);
 }
 
-// Launches of up to kDirectPoses poses with at most kHostPose partials each add them up on the
-// host (enqueue_batch).
+// Launches of at most kHostPartials partials, kHostPose per pose, add them up on the host
+// (enqueue_batch).
 constexpr int kDirectPoses = 8;
 constexpr int kHostPose = 256;
-constexpr size_t kHostPartials = (size_t)kDirectPoses * kHostPose;
+constexpr size_t kHostPartials = 2048;
 
 void free_batch(lc2e_pair* p) {
     drop_graphs(p);
@@ -879,23 +879,24 @@ lc2e::FusedArgs make_args(lc2e_pair* p, const float* d_mats, double* d_partials,
 // (up to kDirectPoses poses of one matrix each, on a single volume or image: each
 // work-group reads its pose's 12 floats once) read the pinned matrices in place instead of
 // copying them, and the reduction always writes the results in place: one or two commands
-// per batch instead of four. Where a launch is not captured, a single matrix goes with the
-// kernel's arguments (a read from pinned memory takes 1.2 us at a kernel's start), and few
-// partials go straight to pinned memory for the host to add up (*host_sum; a launch less:
-// 2D 256x256 single pose 30.7 -> 24.5 us with both). Such launches carry their matrices in the
-// kernels' arguments: 4 poses 194x248, r = 5, 33.4 -> 31.6 us, 6 poses 145x114, r = 3, 29.1 -> 27.0.
+// per batch instead of four. Where a launch is not captured, up to kInlineMats such matrices go
+// with the arguments of the kernels that read them there (all but the 2D fused kernel; a read from
+// pinned memory takes 1.2 us at a kernel's start: 4 poses 194x248, r = 5, 33.4 -> 31.6 us), and few
+// partials go straight to pinned memory for the host to add up (*host_sum), a launch less: 13 poses
+// 96x96, r = 9, 34.0 -> 30.9 us, 256x256, r = 3, static image, 37.8 -> 34.6; sums of 512 to 4096
+// partials took the same.
 int enqueue_batch(lc2e_pair* p, int n, const Tiling& t, hipStream_t st, bool captured, bool* host_sum) {
     const int mpp = p->mats_per_pose();
     const bool direct = !p->sep && mpp == 1 && n <= kDirectPoses &&
                         (p->info.grid_ndim == 3 || p->v.Z == 1);
-    const bool host = !captured && n <= kDirectPoses && t.tiles > 0 && t.bpp <= kHostPose;
+    const bool host = !captured && t.tiles > 0 && t.bpp <= kHostPose && (size_t)n * t.bpp <= kHostPartials;
     *host_sum = host;
     if (!direct)
         HIP_TRY(hipMemcpyAsync(p->d_mats, p->h_mats, (size_t)n * mpp * 12 * sizeof(float),
                                hipMemcpyHostToDevice, st));
     if (t.tiles > 0) {
         lc2e::FusedArgs a = make_args(p, direct ? p->h_mats_dev : p->d_mats, host ? p->h_part_dev : p->d_partials, t);
-        if (direct && n <= lc2e::kInlineMats && !captured) {
+        if (direct && n <= lc2e::kInlineMats && !captured && (p->two || p->info.grid_ndim == 3)) {
             a.inline_mat = 1;
             std::memcpy(a.m0, p->h_mats, (size_t)n * 12 * sizeof(float));
         }
@@ -912,15 +913,15 @@ int enqueue_batch(lc2e_pair* p, int n, const Tiling& t, hipStream_t st, bool cap
     return LC2E_OK;
 }
 
-// The sums of k_reduce from the partials in h_part, added in its order: 256 running sums of
+// The sums of k_reduce from the partials of n poses on the host, added in its order: 256 running sums of
 // every 256th partial, then halves (here at most one partial each; halvings that would only add
 // the zeros past the last partial are left out).
-void sum_partials(lc2e_pair* p, int n, int bpp) {
+void sum_partials(const double* partials, int n, int bpp, double* out) {
     double m[kHostPose], w[kHostPose];
     int top = 1;
     while (top < bpp) top *= 2;
     for (int i = 0; i < n; ++i) {
-        const double* s = p->h_part + (size_t)i * bpp * 2;
+        const double* s = partials + (size_t)i * bpp * 2;
         for (int k = 0; k < top; ++k) {
             m[k] = k < bpp ? 0.0 + s[2 * k] : 0.0;
             w[k] = k < bpp ? 0.0 + s[2 * k + 1] : 0.0;
@@ -932,9 +933,9 @@ void sum_partials(lc2e_pair* p, int n, int bpp) {
             }
         double l = m[0] / w[0];
         if (!std::isfinite(l)) l = 0.0;
-        p->h_out[3 * i] = m[0];
-        p->h_out[3 * i + 1] = w[0];
-        p->h_out[3 * i + 2] = l;
+        out[3 * i] = m[0];
+        out[3 * i + 1] = w[0];
+        out[3 * i + 2] = l;
     }
 }
 
@@ -965,7 +966,7 @@ int run_batch(lc2e_pair* p, int n, const Tiling& t) {
         if (rc < 0) return rc;
     }
     HIP_TRY(hipStreamSynchronize(st));
-    if (host_sum) sum_partials(p, n, t.bpp);
+    if (host_sum) sum_partials(p->h_part, n, t.bpp, p->h_out);
     if (p->profile && t.tiles > 0) {
         float ms = 0.0f;
         HIP_TRY(hipEventElapsedTime(&ms, p->ev0, p->ev1));
@@ -1432,24 +1433,38 @@ int lc2e_eval_batch_noalloc(lc2e_pair* p, int n, const float* mats, double* lc2,
         float* d_mats = reinterpret_cast<float*>(base + up256((size_t)nb * 3 * sizeof(double)));
         double* d_part = reinterpret_cast<double*>(reinterpret_cast<char*>(d_mats) +
                                                    up256((size_t)nb * mpp * 12 * sizeof(float)));
-        HIP_TRY(hipMemcpyAsync(d_mats, mats + (size_t)b0 * mpp * 12, (size_t)nb * mpp * 12 * sizeof(float),
-                               hipMemcpyHostToDevice, st));
         const Tiling t = tiling_for(p, nb, ws.poses);
+        // few matrices go with the kernels' arguments, where one launch takes all poses
+        const bool inline_mats = p->two && mpp == 1 && nb <= lc2e::kInlineMats &&
+                                 (p->info.grid_ndim == 3 || p->v.Z == 1) &&
+                                 (in_place(p, ws, t.tiles, nb) || part(ws, nb) == nb);
+        if (!inline_mats)
+            HIP_TRY(hipMemcpyAsync(d_mats, mats + (size_t)b0 * mpp * 12, (size_t)nb * mpp * 12 * sizeof(float),
+                                   hipMemcpyHostToDevice, st));
         if (t.tiles > 0) {
             // every partial slot is written by the kernels before k_reduce reads it, so the
             // previous call's contents need no clearing
-            const lc2e::FusedArgs a = make_args(p, d_mats, d_part, t);
+            lc2e::FusedArgs a = make_args(p, d_mats, d_part, t);
+            if (inline_mats) {
+                a.inline_mat = 1;
+                std::memcpy(a.m0, mats + (size_t)b0 * 12, (size_t)nb * 12 * sizeof(float));
+            }
             HIP_TRY(launch_eval(p, a, nb, st, ws));
         }
-        HIP_TRY(lc2e::launch_reduce(d_part, (int)bpp, nb, d_out, st));
-        // results back through a fixed host buffer, a chunk of poses at a time
+        // results back through a fixed host buffer, a chunk of poses at a time; few partials come
+        // back themselves and are added up here, a launch less
         constexpr int kChunk = 128;
-        double h[kChunk * 3];
+        constexpr size_t kFew = 256;
+        double h[kChunk * 3], few[kFew * 2];
+        const bool host = t.tiles > 0 && bpp <= kHostPose && nb <= kChunk && nb * bpp <= kFew;
+        if (!host) HIP_TRY(lc2e::launch_reduce(d_part, (int)bpp, nb, d_out, st));
         for (int b = 0; b < nb; b += kChunk) {
             const int m = nb - b < kChunk ? nb - b : kChunk;
-            HIP_TRY(hipMemcpyAsync(h, d_out + (size_t)b * 3, (size_t)m * 3 * sizeof(double),
-                                   hipMemcpyDeviceToHost, st));
+            HIP_TRY(host ? hipMemcpyAsync(few, d_part, nb * bpp * 2 * sizeof(double), hipMemcpyDeviceToHost, st)
+                         : hipMemcpyAsync(h, d_out + (size_t)b * 3, (size_t)m * 3 * sizeof(double),
+                                          hipMemcpyDeviceToHost, st));
             HIP_TRY(hipStreamSynchronize(st));
+            if (host) sum_partials(few, nb, (int)bpp, h);
             for (int i = 0; i < m; ++i) {
                 const double sm = h[3 * i], sw = h[3 * i + 1], l = h[3 * i + 2];
                 const int k = b0 + b + i;

@@ -349,6 +349,26 @@ void one_pose_of_a_stack_fills_the_device() {
     lc2e_destroy(e);
 }
 
+// Small calls: no reduction launch where the host adds up few partial sums, and matrices in the
+// arguments of the kernels that read them there, without allocation too.
+void small_calls_have_few_commands() {
+    lc2e_engine* e = engine();
+    {
+        Pair p(e, 2, 96, 96, 1, 1, 9, false), f(e, 2, 96, 96, 1, 1, 3, false), v(e, 3, 64, 64, 64, 1, 3, true);
+        fake::launches().clear();
+        CHECK(p.batch(13) >= 0 && f.batch(13) >= 0 && fake::count("k_reduce") == 0);
+        fake::launches().clear();
+        CHECK(p.noalloc(8) >= 0 && v.noalloc(8) >= 0);
+        for (const auto& l : fake::launches())
+            if (l.is("k_moments") || l.is("k_warp")) CHECK(l.a.inline_mat == 1);
+        fake::launches().clear();
+        CHECK(p.noalloc(9) >= 0 && v.noalloc(9) >= 0 && f.noalloc(2) >= 0 && f.batch(2) >= 0);
+        for (const auto& l : fake::launches())
+            if (l.is("k_moments") || l.is("k_warp") || l.is("k_fused")) CHECK(l.a.inline_mat == 0);
+    }
+    lc2e_destroy(e);
+}
+
 //@SCENARIOS
 
 const std::map<std::string, std::function<void()>> kScenarios = {
@@ -363,6 +383,7 @@ const std::map<std::string, std::function<void()>> kScenarios = {
     {"noalloc_admits_what_it_did", noalloc_admits_what_it_did},
     {"small_2d_launches_have_short_waves", small_2d_launches_have_short_waves},
     {"one_pose_of_a_stack_fills_the_device", one_pose_of_a_stack_fills_the_device},
+    {"small_calls_have_few_commands", small_calls_have_few_commands},
 //@TABLE
 };
 
