@@ -525,7 +525,7 @@ size_t admitted_partials(const lc2e_pair* p) {
 
 // Launches of at most kHostPartials partials, kHostPose per pose, add them up on the host
 // (enqueue_batch).
-constexpr int kDirectPoses = 8;
+constexpr int kDirectPoses = 32;
 constexpr int kHostPose = 256;
 constexpr size_t kHostPartials = 2048;
 
@@ -878,7 +878,7 @@ lc2e::FusedArgs make_args(lc2e_pair* p, const float* d_mats, double* d_partials,
 // pinned result buffer. Each launch command costs several microseconds, so small launches
 // (up to kDirectPoses poses of one matrix each, on a single volume or image: each
 // work-group reads its pose's 12 floats once) read the pinned matrices in place instead of
-// copying them, and the reduction always writes the results in place: one or two commands
+// copying them (13 poses 1.5 us less, 32 poses 2 us), and the reduction always writes the results in place: one or two commands
 // per batch instead of four. Where a launch is not captured, up to kInlineMats such matrices go
 // with the arguments of the kernels that read them there (all but the 2D fused kernel; a read from
 // pinned memory takes 1.2 us at a kernel's start: 4 poses 194x248, r = 5, 33.4 -> 31.6 us), and few

@@ -369,6 +369,23 @@ void small_calls_have_few_commands() {
     lc2e_destroy(e);
 }
 
+// A small 3D launch is cut into short chunks, and calls of up to 32 poses copy no matrices.
+void small_3d_launches_are_spread_out() {
+    lc2e_engine* e = engine();
+    {
+        Pair p(e, 3, 64, 64, 64, 1, 1, true);
+        CHECK(p.batch(32) >= 0);
+        fake::launches().clear();
+        const long long copies = fake::copies();
+        CHECK(p.batch(4) >= 0);
+        for (const auto& l : fake::launches())
+            if (l.is("k_warp_grad3")) CHECK(l.groups >= 512);  // 2 x 4 columns, 4 poses, 16 chunks
+        CHECK(p.batch(13) >= 0 && p.batch(32) >= 0);
+        CHECK(fake::copies() == copies);
+    }
+    lc2e_destroy(e);
+}
+
 //@SCENARIOS
 
 const std::map<std::string, std::function<void()>> kScenarios = {
@@ -384,6 +401,7 @@ const std::map<std::string, std::function<void()>> kScenarios = {
     {"small_2d_launches_have_short_waves", small_2d_launches_have_short_waves},
     {"one_pose_of_a_stack_fills_the_device", one_pose_of_a_stack_fills_the_device},
     {"small_calls_have_few_commands", small_calls_have_few_commands},
+    {"small_3d_launches_are_spread_out", small_3d_launches_are_spread_out},
 //@TABLE
 };
 

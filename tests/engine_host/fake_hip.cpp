@@ -30,7 +30,7 @@ struct State {
     std::map<std::pair<const void*, int>, void*> var_addr;  // (variable, device) -> address
     std::set<hipStream_t> capturing;
     int in_capture = 0;
-    long long mallocs = 0, attempts = 0;
+    long long mallocs = 0, attempts = 0, copies = 0;
 };
 State& g() {
     static State* s = new State();
@@ -61,13 +61,14 @@ void reset(size_t device_bytes) {
     g().limit = device_bytes;
     g().launches.clear();
     g().in_capture = 0;
-    g().mallocs = g().attempts = 0;
+    g().mallocs = g().attempts = g().copies = 0;
 }
 std::vector<Launch>& launches() { return g().launches; }
 int in_capture() { return g().in_capture; }
 size_t used(int device) { return g().used[device]; }
 long long mallocs() { return g().mallocs; }
 long long attempts() { return g().attempts; }
+long long copies() { return g().copies; }
 bool live(const void* p) {
     std::lock_guard<std::recursive_mutex> lk(g().mu);
     for (const auto& b : g().blocks)
@@ -123,7 +124,11 @@ hipError_t hipHostMalloc(void** p, size_t n, unsigned) { return (*p = std::callo
 hipError_t hipHostFree(void* p) { return std::free(p), hipSuccess; }
 hipError_t hipHostGetDevicePointer(void** d, void* h, unsigned) { return *d = h, hipSuccess; }
 hipError_t hipMemcpy(void* d, const void* s, size_t n, hipMemcpyKind) { return std::memcpy(d, s, n), hipSuccess; }
-hipError_t hipMemcpyAsync(void* d, const void* s, size_t n, hipMemcpyKind, hipStream_t) { return std::memcpy(d, s, n), hipSuccess; }
+hipError_t hipMemcpyAsync(void* d, const void* s, size_t n, hipMemcpyKind, hipStream_t) {
+    LOCK;
+    ++g().copies;
+    return std::memcpy(d, s, n), hipSuccess;
+}
 hipError_t hipMemsetAsync(void* d, int v, size_t n, hipStream_t) { return std::memset(d, v, n), hipSuccess; }
 
 hipError_t hipStreamCreateWithFlags(hipStream_t* s, unsigned) { return *s = reinterpret_cast<hipStream_t>(std::malloc(1)), hipSuccess; }
@@ -188,7 +193,7 @@ hipError_t hipFuncSetAttribute(const void* fn, hipFuncAttribute, int v) {
     g().lds[{fn, t_device}] = v;
     return hipSuccess;
 }
-hipError_t hipOccupancyMaxActiveBlocksPerMultiprocessor(int* n, const void*, int, size_t) { return *n = 2, hipSuccess; }
+hipError_t hipOccupancyMaxActiveBlocksPerMultiprocessor(int* n, const void*, int, size_t lds) { return *n = lds > 80 * 1024 ? 1 : 2, hipSuccess; }
 hipError_t __hipPushCallConfiguration(dim3 grid, dim3 block, size_t lds, hipStream_t st) {
     t_configs.push_back({grid, block, lds, st});
     return hipSuccess;

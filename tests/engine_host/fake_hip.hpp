@@ -35,6 +35,7 @@ size_t used(int device);            // device bytes allocated
 bool live(const void* p);           // p lies in an allocation of device memory
 long long mallocs();                // hipMalloc calls that succeeded
 long long attempts();               // all
+long long copies();                 // asynchronous ones
 int count(const char* kernel_part);  // launches whose kernel's name holds the text
 
 }  // namespace fake

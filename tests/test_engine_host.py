@@ -45,6 +45,7 @@ def engine_test(tmp_path_factory):
     "small_2d_launches_have_short_waves",
     "one_pose_of_a_stack_fills_the_device",
     "small_calls_have_few_commands",
+    "small_3d_launches_are_spread_out",
 ])
 def test_engine_host(engine_test, scenario):
     r = subprocess.run([engine_test, scenario], capture_output=True, text=True, timeout=120)
