@@ -412,16 +412,16 @@ int resident_per_cu(lc2e_pair* p) {
     return p->resident_per_cu;
 }
 
-// z-chunk for n poses when nothing is tuned. A work-group of chunk c marches
-// min(c, planes left) + 2R + 2 plane steps. Work-groups go to the XCDs round-robin by id
+// z-chunk for a launch of n poses when nothing is tuned. A work-group of chunk c marches
+// min(c, planes left) + 2R + 4 plane steps (fused kernel), or as many planes and its pipeline's fill
+// (two-kernel path: 4 planes' worth with a moving high-resolution image, 8 with a static one; against
+// every chunk at 588 launches of 7 grids, radii 1 to 6, 1 to 32 poses the choice is 0.5% off the
+// fastest on average and 7% and 13% at worst, 8 planes for both 1.1% and 21%). Work-groups go to the XCDs round-robin by id
 // and, within an XCD, to the first free slot in id order (map_block: tile-major, the poses
 // of a tile consecutive; tiles ordered by z-chunk), each CU holding resident_per_cu of them.
 // The model replays that dispatch with a min-heap of slot finishing times per XCD and takes
 // the latest finish; launches of more than 32 rounds fall back to rounds x steps. Minimise
-// over the chunk lengths (multiples of kZBlock; ties: longer chunks). Against exhaustive
-// timing on MI355X (3D affine grid 192x192x160 and CT grid 256^3, 1 to 32 poses) it picks
-// within 4% of the fastest chunk in all but one case (3.5%); a rounds-only model lost up to
-// 16%. Cached per batch size.
+// over the chunk lengths (multiples of kZBlock; ties: longer chunks). Cached per launch size.
 int model_zchunk(lc2e_pair* p, int n) {
     auto hit = p->model_cache.find(n);
     if (hit != p->model_cache.end()) return hit->second;
@@ -433,8 +433,7 @@ int model_zchunk(lc2e_pair* p, int n) {
     const int cus = p->e->cus > 0 ? p->e->cus : 256;
     const int per_xcd = std::max(1, cus / lc2e::kXcds * resident_per_cu(p));
     const int cmax = round_zchunk(ez);
-    // per work-group, in plane steps (fitted): the two-kernel path only fills its pipeline
-    const double extra = p->two ? 8.0 : 2 * r + 2 + 2.0;
+    const double extra = !p->two ? 2 * r + 4.0 : p->info.high_res_is_moving ? 4.0 : 8.0;
     int best = cmax;
     double best_cost = -1.0;
     std::vector<double> heap;

@@ -386,6 +386,24 @@ void small_3d_launches_are_spread_out() {
     lc2e_destroy(e);
 }
 
+// The chunk model's overhead per work-group is that of the kernels that run: one plane per step at
+// radii from 4 with a moving high-resolution image, whose short chunks cost little.
+void chunks_fit_the_kernel_that_runs() {
+    lc2e_engine* e = engine();
+    {
+        struct {
+            int x, y, z, r, n, most;
+        } cases[] = {{48, 48, 48, 4, 13, 16}, {64, 64, 64, 6, 17, 32}, {64, 64, 64, 5, 9, 24}};
+        for (const auto& c : cases) {
+            Pair p(e, 3, c.x, c.y, c.z, 1, c.r, true);
+            CHECK(p.batch(c.n) >= 0);
+            int zchunk = 0;
+            CHECK(lc2e_pair_get_tuning(p.p, &zchunk) == LC2E_OK && zchunk <= c.most);
+        }
+    }
+    lc2e_destroy(e);
+}
+
 //@SCENARIOS
 
 const std::map<std::string, std::function<void()>> kScenarios = {
@@ -402,6 +420,7 @@ const std::map<std::string, std::function<void()>> kScenarios = {
     {"one_pose_of_a_stack_fills_the_device", one_pose_of_a_stack_fills_the_device},
     {"small_calls_have_few_commands", small_calls_have_few_commands},
     {"small_3d_launches_are_spread_out", small_3d_launches_are_spread_out},
+    {"chunks_fit_the_kernel_that_runs", chunks_fit_the_kernel_that_runs},
 //@TABLE
 };
 

@@ -46,6 +46,7 @@ def engine_test(tmp_path_factory):
     "one_pose_of_a_stack_fills_the_device",
     "small_calls_have_few_commands",
     "small_3d_launches_are_spread_out",
+    "chunks_fit_the_kernel_that_runs",
 ])
 def test_engine_host(engine_test, scenario):
     r = subprocess.run([engine_test, scenario], capture_output=True, text=True, timeout=120)
