@@ -522,6 +522,22 @@ size_t admitted_partials(const lc2e_pair* p) {
     return (size_t)ntx * nty * ((p->v.Z + lc2e::kFrameRun - 1) / lc2e::kFrameRun);
 }
 
+// The partial sums per pose of every launch of the pair (tiling_for without a choice of chunks; 0:
+// no patch centre fits).
+int partials_per_pose(lc2e_pair* p) {
+    if (p->sep || p->info.grid_ndim == 2) {
+        const Tiling t = tiling_for(p, 1, 0);
+        return t.tiles > 0 ? t.bpp : 0;
+    }
+    if (!p->two) return lc2e::fused_partials_3d(p->v, p->info.patch_radius);
+    lc2e::FusedArgs a{};
+    a.v = p->v;
+    a.r = p->info.patch_radius;
+    a.zchunk = lc2e::kZBlock;
+    lc2e::moments_tiling(&a, 3, p->role());
+    return a.tiles > 0 ? a.blocks_per_pose : 0;
+}
+
 // Launches of at most kHostPartials partials, kHostPose per pose, add them up on the host
 // (enqueue_batch).
 constexpr int kDirectPoses = 32;
@@ -647,7 +663,7 @@ void release_noalloc(lc2e_pair* p) {
     lc2e_engine* e = p->e;
     std::lock_guard<std::mutex> lk(noalloc_lock(e->device));
     p->na = false;
-    if (--e->na_pairs) return;
+    if (--e->na_pairs || e->na_bytes <= kNoallocBytes) return;  // kept for the next pair
     e->raw_free(e->na, e->na_bytes);
     e->na = nullptr;
     e->na_bytes = 0;
@@ -714,11 +730,12 @@ bool shrink_noalloc(lc2e_engine* e) {
     for (const lc2e_pair* p : g_pairs)
         if (p->e == e && p->na) one = std::max(one, p->ws_bytes);
     std::lock_guard<std::mutex> lk(noalloc_lock(e->device));
-    if (!one || e->na_bytes <= one) return false;
+    if (e->na_bytes <= one) return false;
     e->raw_free(e->na, e->na_bytes);
     e->give_back();
     e->na = nullptr;
     e->na_bytes = 0;
+    if (!one) return true;
     if (hipMalloc(&e->na, one) == hipSuccess) e->na_bytes = one;
     else (void)hipGetLastError(), e->na = nullptr;
     return true;
@@ -829,7 +846,7 @@ int ensure_batch(lc2e_pair* p, int n, int bpp) {
 // The same for launches of the pair's kernels, and the workspace. A launch that a caller captures
 // takes the workspace as it is (nothing may be allocated then), and keeps it where it is.
 int ensure_capacity(lc2e_pair* p, int n, bool captured = false) {
-    const int rc = ensure_batch(p, n, tiling_for(p, n, p->ws_poses).bpp);
+    const int rc = ensure_batch(p, n, partials_per_pose(p));
     if (rc < 0 || !p->ws) return rc;
     if (captured) p->pinned = true;
     else (void)grow_workspace(p, n);
@@ -1413,8 +1430,7 @@ int lc2e_eval_batch_noalloc(lc2e_pair* p, int n, const float* mats, double* lc2,
     auto bytes = [&](size_t m, size_t bpp) {
         return up256(m * 3 * sizeof(double)) + up256(m * mpp * 12 * sizeof(float)) + m * bpp * 2 * sizeof(double);
     };
-    const Tiling one = tiling_for(p, 1, ws.poses);
-    const size_t bpp = one.tiles > 0 ? one.bpp : 0;
+    const size_t bpp = partials_per_pose(p);
     const size_t need = bytes(n, admitted_partials(p));
     if (need > lc2e::kScratchBytes || bytes(1, bpp) > lc2e::kScratchBytes)
         return fail(LC2E_ERR_INVALID,

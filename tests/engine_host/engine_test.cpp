@@ -393,7 +393,7 @@ void chunks_fit_the_kernel_that_runs() {
     {
         struct {
             int x, y, z, r, n, most;
-        } cases[] = {{48, 48, 48, 4, 13, 16}, {64, 64, 64, 6, 17, 32}, {64, 64, 64, 5, 9, 24}};
+        } cases[] = {{48, 48, 48, 4, 13, 32}, {64, 64, 64, 6, 17, 32}, {64, 64, 64, 5, 9, 24}};
         for (const auto& c : cases) {
             Pair p(e, 3, c.x, c.y, c.z, 1, c.r, true);
             CHECK(p.batch(c.n) >= 0);
