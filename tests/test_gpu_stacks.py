@@ -43,7 +43,7 @@ def _mats(n, frames, seed):
 def test_tracked_stacks_equal_oracle_however_they_run(movi, r, dims):
     fixed, volume = _stack(movi, dims, r)
     x, y, z = dims
-    n = 1 + 2048 // (4 * z)  # more waves than a launch that warps in place has
+    n = 1 + 2048 // z  # more waves than a launch that warps in place has
     mats = _mats(n, z, r)
     print(f"tracked stack: movi {movi}, r {r}, {dims}, {n} poses", flush=True)
     got = {}

@@ -70,3 +70,23 @@ def test_noalloc_rejects_calls_beyond_the_scratch(engine):
     p.close()
     for v in vols:
         v.close()
+
+
+@pytest.mark.parametrize("ndim,r,n", [(3, 7, 3), (2, 12, 5), (3, 3, 70), (3, 6, 70), (2, 5, 150)])
+def test_noalloc_equals_batch_on_the_separable_path_and_in_parts(engine, ndim, r, n):
+    """The box passes (3D radius 7, 2D radius 12), and calls of more poses than the reserved
+    workspace holds, on a fresh pair: the bits of a batch."""
+    w = synth.small3d() if ndim == 3 else synth.config0(n=96)
+    w.patch_radius = r
+    if ndim == 2:
+        w.high_res_is_moving = True
+    p, vols = _pair(engine, w)
+    mats = _mats(p, w, n, r)
+    print(f"no-alloc {ndim}D r {r}, {n} poses: virtual grid {p.virt_dims}", flush=True)
+    a = p.eval_batch_noalloc(mats)
+    b = p.eval_batch(mats)
+    assert np.array_equal(a.lc2, b.lc2) and np.array_equal(a.sum_w, b.sum_w)
+    assert np.array_equal(a.sum_measure, b.sum_measure) and (b.sum_w > 0).any()
+    p.close()
+    for v in vols:
+        v.close()
