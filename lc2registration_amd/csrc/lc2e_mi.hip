@@ -167,10 +167,12 @@ struct MiBin {
 // Bound by the LDS atomics and VALU issue (a voxel took 20 FP64 operations; its 2 loads take 80 us
 // of 8 poses of 192x192x160 at the copy rate). Measured there: 699 us while it warped each
 // voxel again, 190 with chunks of 65535 voxels and FP64 bins, now 129.
-constexpr int kMiVox = 4096;            // voxels per step: 4 per thread, the next step's in flight
+// U: voxels per thread and step, the next step's in flight. WAVES: per SIMD.
+constexpr int kMiVox = 4096;  // of four voxels per thread
 constexpr int kMiSweep = 7 * kMiVox;  // + 32767 < 65536
-template <typename T>
-__global__ __launch_bounds__(1024) void k_mi_joint(FusedArgs a, int grid3, int src3, const float* stat,
+template <typename T, int U, int WAVES>
+__global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(WAVES)))
+void k_mi_joint(FusedArgs a, int grid3, int src3, const float* stat,
                                                    int stat_is_u, const int* ext_mov, const int* ext_stat,
                                                    int bins_u, int bins_i, long long chunk, int stride,
                                                    unsigned* hist) {
@@ -189,7 +191,7 @@ __global__ __launch_bounds__(1024) void k_mi_joint(FusedArgs a, int grid3, int s
     const long long len = min(chunk, n - i0);
     const float* wm = a.warp1 ? a.warp1 + (size_t)pose * n + i0 : nullptr;
     const float* ws = stat + i0;
-    constexpr int U = kMiVox / 1024;
+    constexpr int VOX = U * 1024;  // per step
     float vm[U], vs[U];
     auto load = [&](long long k0) {
 #pragma unroll
@@ -201,11 +203,11 @@ __global__ __launch_bounds__(1024) void k_mi_joint(FusedArgs a, int grid3, int s
     };
     load(0);
     int since = 0;
-    for (long long k0 = 0; k0 < len; k0 += kMiVox) {
+    for (long long k0 = 0; k0 < len; k0 += VOX) {
         float cm[U], cs[U];
 #pragma unroll
         for (int k = 0; k < U; ++k) cm[k] = vm[k], cs[k] = vs[k];
-        if (k0 + kMiVox < len) load(k0 + kMiVox);
+        if (k0 + VOX < len) load(k0 + VOX);
 #pragma unroll
         for (int k = 0; k < U; ++k) {
             const int bm = bin_m(cm[k]), bs = bin_s(cs[k]);
@@ -218,7 +220,7 @@ __global__ __launch_bounds__(1024) void k_mi_joint(FusedArgs a, int grid3, int s
                 atomicAdd(&s_h[j >> 1], (j & 1) ? 65536u : 1u);
             }
         }
-        since += kMiVox;
+        since += VOX;
         if (since == kMiSweep) {  // work-group uniform
             since = 0;
             __syncthreads();
@@ -351,7 +353,7 @@ hipError_t launch_mi(const FusedArgs& a, int grid_ndim, int src_ndim, int movi, 
     const int nb = bins_u * bins_i, stride = mi_hist_size(bins_u, bins_i);
     hipLaunchKernelGGL(k_mi_init, dim3((n_poses + 1 + 255) / 256), dim3(256), 0, st, ext_mov,
                        n_poses);
-    // 16 work-groups per CU for the extremes: each ends with two atomics on one address
+    // 4 work-groups per CU and pose for the extremes: each ends with two atomics on one address
     const unsigned ge = (unsigned)std::min<long long>((n + 255) / 256, 1024);
     if (!stat_ready) {
         hipLaunchKernelGGL(k_mi_init, dim3(1), dim3(256), 0, st, ext_stat, 1);
@@ -372,23 +374,33 @@ hipError_t launch_mi(const FusedArgs& a, int grid_ndim, int src_ndim, int movi, 
     }
     hipError_t e = hipMemsetAsync(hist, 0, (size_t)n_poses * stride * sizeof(unsigned), st);
     if (e != hipSuccess) return e;
-    // one round of the 256 CUs (one work-group each, by its LDS) for all poses; at least 4096
-    // voxels per work-group, or the final additions dominate
-    const long long per_pose = std::max(1LL, std::min<long long>(std::max(1, 256 / n_poses), n / kMiVox));
+    // One round of the 256 CUs (one work-group each, by its LDS) for all poses; at least 4096
+    // voxels per work-group, or the final additions dominate. Where each voxel is warped again, a
+    // chain of gathers, and the histograms leave room for two work-groups per CU, large launches
+    // take eight rounds of two voxels per thread, twice the wavefronts: 40 poses of 200x180x160, 32
+    // bins, 2.61 -> 2.25 ms; 5 poses of 128^3 (10 million voxels) 254 -> 258 us, 13 poses 508 -> 466.
+    const size_t lds = (size_t)((nb + 1) / 2) * sizeof(unsigned);
+    const bool many = !a.warp1 && lds <= 80 * 1024 && n * n_poses >= 1LL << 24;
+    const long long per_pose = std::max(1LL, std::min<long long>(std::max(1, (many ? 2048 : 256) / n_poses), n / kMiVox));
     const long long chunk = (n + per_pose - 1) / per_pose;
     const dim3 gj((unsigned)((n + chunk - 1) / chunk), (unsigned)n_poses);
-    const size_t lds = (size_t)((nb + 1) / 2) * sizeof(unsigned);
-    static LdsLimit limit;
-    e = limit.raise({reinterpret_cast<const void*>(&k_mi_joint<float>), reinterpret_cast<const void*>(&k_mi_joint<__half>)},
-                    (kMiMaxBins * kMiMaxBins / 2) * sizeof(unsigned));
-    if (e != hipSuccess) return e;
     const int stat_is_u = movi ? 1 : 0;
-    if (a.src_f16)
-        hipLaunchKernelGGL(k_mi_joint<__half>, gj, dim3(1024), lds, st, a, g3, s3, stat, stat_is_u,
-                           ext_mov, ext_stat, bins_u, bins_i, chunk, stride, hist);
-    else
-        hipLaunchKernelGGL(k_mi_joint<float>, gj, dim3(1024), lds, st, a, g3, s3, stat, stat_is_u,
-                           ext_mov, ext_stat, bins_u, bins_i, chunk, stride, hist);
+    auto joint = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, gj, dim3(1024), lds, st, a, g3, s3, stat, stat_is_u, ext_mov, ext_stat, bins_u,
+                           bins_i, chunk, stride, hist);
+    };
+    if (many) {
+        if (a.src_f16) joint(k_mi_joint<__half, 2, 8>);
+        else joint(k_mi_joint<float, 2, 8>);
+    } else {
+        static LdsLimit limit;
+        e = limit.raise({reinterpret_cast<const void*>(&k_mi_joint<float, 4, 4>),
+                         reinterpret_cast<const void*>(&k_mi_joint<__half, 4, 4>)},
+                        (kMiMaxBins * kMiMaxBins / 2) * sizeof(unsigned));
+        if (e != hipSuccess) return e;
+        if (a.src_f16) joint(k_mi_joint<__half, 4, 4>);
+        else joint(k_mi_joint<float, 4, 4>);
+    }
     const int groups = std::max(1, bins_i / kMiRows);
     hipLaunchKernelGGL(k_mi_entropy_part, dim3((unsigned)groups, (unsigned)n_poses), dim3(256), 0, st, hist, stride,
                        bins_u, bins_i, (double)n);

@@ -77,9 +77,9 @@ struct Pair {
         static double d_out[64 * 3];
         return lc2e_eval_batch_async(p, n, d_mats, d_out, st);
     }
-    int mi(int n) {
+    int mi(int n, int bins = 256) {
         std::vector<double> out(n);
-        return lc2e_eval_mi_batch(p, n, mats(n).data(), 256, 256, out.data());
+        return lc2e_eval_mi_batch(p, n, mats(n).data(), bins, bins, out.data());
     }
     ~Pair() {
         if (p) lc2e_pair_destroy(p);
@@ -404,6 +404,29 @@ void chunks_fit_the_kernel_that_runs() {
     lc2e_destroy(e);
 }
 
+// Mutual information without a kept warp gathers every voxel in the joint histogram: a large
+// launch of small histograms has many work-groups, the others one round of the CUs.
+void joint_histograms_that_warp_again_spread_out() {
+    lc2e_engine *e = engine(), *b = engine(8 * GB);
+    {
+        Pair kept(e, 3, 128, 128, 128, 1, 2, true), again(b, 3, 128, 128, 128, 1, 2, true);
+        struct {
+            Pair& p;
+            int n, bins;
+            unsigned long long least, most;
+        } cases[] = {{kept, 30, 32, 200, 256}, {again, 30, 256, 200, 256}, {again, 40, 32, 1024, 2048}, {again, 5, 32, 200, 256}};
+        for (const auto& c : cases) {
+            fake::launches().clear();
+            CHECK(c.p.mi(c.n, c.bins) >= 0);
+            for (const auto& l : fake::launches())
+                if (l.is("k_mi_joint")) CHECK(l.groups >= c.least && l.groups <= c.most);
+            CHECK(fake::count("k_mi_joint") == 1);
+        }
+    }
+    lc2e_destroy(b);
+    lc2e_destroy(e);
+}
+
 //@SCENARIOS
 
 const std::map<std::string, std::function<void()>> kScenarios = {
@@ -421,6 +444,7 @@ const std::map<std::string, std::function<void()>> kScenarios = {
     {"small_calls_have_few_commands", small_calls_have_few_commands},
     {"small_3d_launches_are_spread_out", small_3d_launches_are_spread_out},
     {"chunks_fit_the_kernel_that_runs", chunks_fit_the_kernel_that_runs},
+    {"joint_histograms_that_warp_again_spread_out", joint_histograms_that_warp_again_spread_out},
 //@TABLE
 };
 
