@@ -107,16 +107,23 @@ struct lc2e_engine {
                     hipDeviceSynchronize() == hipSuccess;
         if (current != device) idle = hipSetDevice(current) == hipSuccess && idle;
         if (!idle) return false;
-        std::lock_guard<std::mutex> lk(mu);
-        auto it = sizes.find(p);
-        if (it != sizes.end()) {
-            bytes = it->second;  // the block's own size, if it had been reused
-            sizes.erase(it);
+        std::vector<Block> oldest;  // make room
+        {
+            std::lock_guard<std::mutex> lk(mu);
+            auto it = sizes.find(p);
+            if (it != sizes.end()) {
+                bytes = it->second;  // the block's own size, if it had been reused
+                sizes.erase(it);
+            }
+            size_t total = bytes;
+            for (const Block& b : kept) total += b.bytes;
+            size_t out = 0;
+            while (total > limit && out < kept.size()) total -= kept[out++].bytes;
+            oldest.assign(kept.begin(), kept.begin() + out);
+            kept.erase(kept.begin(), kept.begin() + out);
+            kept.push_back({p, bytes});
         }
-        size_t total = bytes;
-        for (const Block& b : kept) total += b.bytes;
-        if (total > limit) return false;
-        kept.push_back({p, bytes});
+        for (const Block& b : oldest) (void)(&kept == &kept_host ? hipHostFree(b.p) : hipFree(b.p));
         return true;
     }
     std::map<void*, size_t> sizes;  // reused blocks in use that are larger than asked for

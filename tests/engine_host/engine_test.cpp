@@ -427,6 +427,27 @@ void joint_histograms_that_warp_again_spread_out() {
     lc2e_destroy(e);
 }
 
+// Freed blocks are kept up to a limit; past it the oldest go, so what a program frees now is there
+// for its next object of that size whatever it freed before.
+void old_blocks_make_room_for_new_ones() {
+    lc2e_engine* e = engine();
+    for (int side : {400, 440, 480}) {  // 0.26 to 0.44 GB each, in single precision
+        lc2e_volume* v = nullptr;
+        lc2e_geom g{};
+        for (int a = 0; a < 3; ++a) g.dims[a] = side, g.spacing[a] = 1.0f;
+        std::vector<float> img(size_t(side) * side * side);
+        CHECK(lc2e_volume_upload(e, img.data(), LC2E_F32, &g, LC2E_STORE_AUTO, &v) == LC2E_OK);
+        lc2e_volume_destroy(v);
+        CHECK(fake::used(0) <= GB);
+    }
+    { Pair p(e, 3, 128, 128, 128, 0, 3, true); }
+    const long long mallocs = fake::mallocs();
+    { Pair p(e, 3, 128, 128, 128, 0, 3, true); }
+    CHECK(fake::mallocs() == mallocs);
+    lc2e_destroy(e);
+    CHECK(fake::used(0) == 0);
+}
+
 //@SCENARIOS
 
 const std::map<std::string, std::function<void()>> kScenarios = {
@@ -445,6 +466,7 @@ const std::map<std::string, std::function<void()>> kScenarios = {
     {"small_3d_launches_are_spread_out", small_3d_launches_are_spread_out},
     {"chunks_fit_the_kernel_that_runs", chunks_fit_the_kernel_that_runs},
     {"joint_histograms_that_warp_again_spread_out", joint_histograms_that_warp_again_spread_out},
+    {"old_blocks_make_room_for_new_ones", old_blocks_make_room_for_new_ones},
 //@TABLE
 };
 

@@ -48,6 +48,7 @@ def engine_test(tmp_path_factory):
     "small_3d_launches_are_spread_out",
     "chunks_fit_the_kernel_that_runs",
     "joint_histograms_that_warp_again_spread_out",
+    "old_blocks_make_room_for_new_ones",
 ])
 def test_engine_host(engine_test, scenario):
     r = subprocess.run([engine_test, scenario], capture_output=True, text=True, timeout=120)
