@@ -179,6 +179,26 @@ struct lc2e_engine {
             (void)hipHostFree(p);
         }
     }
+    // Words that an upload's checks set (2, pinned, zeroed), kept with the engine whether or not it has
+    // a budget: making them takes longer than a small upload.
+    std::vector<int*> flags;  // free ones, guarded by mu
+    hipError_t take_flags(int** f) {
+        {
+            std::lock_guard<std::mutex> lk(mu);
+            if (!flags.empty()) {
+                *f = flags.back();
+                flags.pop_back();
+            }
+        }
+        const hipError_t err = *f ? hipSuccess : hipHostMalloc((void**)f, 2 * sizeof(int), hipHostMallocMapped | hipHostMallocCoherent);
+        if (err == hipSuccess) (*f)[0] = (*f)[1] = 0;
+        return err;
+    }
+    void give_flags(int* f) {
+        if (!f) return;
+        std::lock_guard<std::mutex> lk(mu);
+        flags.push_back(f);
+    }
     void forget(void* p) {
         std::lock_guard<std::mutex> lk(mu);
         sizes.erase(p);
@@ -1085,6 +1105,7 @@ void lc2e_destroy(lc2e_engine* e) {
     (void)hipStreamDestroy(e->stream);
     e->raw_free(e->na, e->na_bytes);
     e->give_back();
+    for (int* f : e->flags) (void)hipHostFree(f);
     delete e;
 }
 
@@ -1123,13 +1144,14 @@ int lc2e_volume_upload(lc2e_engine* e, const void* host, lc2e_dtype dtype, const
         int* flag = nullptr;
         ~Scope() {
             e->raw_free(staging, bytes);
-            e->host_free(flag, 2 * sizeof(int));
+            if (idle) e->give_flags(flag);  // no kernel of a failed upload may still set it
+            else if (flag && hipDeviceSynchronize() == hipSuccess) e->give_flags(flag);
         }
+        bool idle = false;
     } tmp{e};
-    HIP_TRY(e->host_alloc((void**)&tmp.flag, 2 * sizeof(int)));
+    HIP_TRY(e->take_flags(&tmp.flag));
     void* flag_dev = nullptr;
     HIP_TRY(hipHostGetDevicePointer(&flag_dev, tmp.flag, 0));
-    tmp.flag[0] = tmp.flag[1] = 0;
     auto stage = [&]() {
         tmp.bytes = (size_t)n * dsz;
         hipError_t err = e->raw_alloc(&tmp.staging, tmp.bytes, true);
@@ -1142,14 +1164,22 @@ int lc2e_volume_upload(lc2e_engine* e, const void* host, lc2e_dtype dtype, const
         f16 = (dtype == LC2E_U8 || dtype == LC2E_F16) ? 1 : 0;
         if (dtype == LC2E_I16) {
             // every integer in [-2048, 2048] is exact in half precision (11-bit significand),
-            // which covers CT in Hounsfield units: half storage is then lossless
-            hipError_t err = stage();
-            if (err == hipSuccess)
-                err = lc2e::launch_check(tmp.staging, dtype, n, 2048.0f, (int*)flag_dev, e->stream);
-            if (err == hipSuccess) err = hipStreamSynchronize(e->stream);
-            if (err != hipSuccess) return fail(LC2E_ERR_HIP, "volume upload failed: %s", hipGetErrorString(err));
-            f16 = *tmp.flag ? 0 : 1;
-            *tmp.flag = 0;
+            // which covers CT in Hounsfield units: half storage is then lossless. The first voxels
+            // are looked at here: all of a small volume, and often enough to tell.
+            constexpr long long kFirst = 32768;
+            const short* h = static_cast<const short*>(host);
+            f16 = 1;
+            for (long long i = 0; i < std::min(n, kFirst) && f16; ++i)
+                if (h[i] < -2048 || h[i] > 2048) f16 = 0;
+            if (f16 && n > kFirst) {
+                hipError_t err = stage();
+                if (err == hipSuccess)
+                    err = lc2e::launch_check(tmp.staging, dtype, n, 2048.0f, (int*)flag_dev, e->stream);
+                if (err == hipSuccess) err = hipStreamSynchronize(e->stream);
+                if (err != hipSuccess) return fail(LC2E_ERR_HIP, "volume upload failed: %s", hipGetErrorString(err));
+                f16 = *tmp.flag ? 0 : 1;
+                *tmp.flag = 0;
+            }
         }
     }
     else f16 = storage == LC2E_F16;
@@ -1207,6 +1237,7 @@ int lc2e_volume_upload(lc2e_engine* e, const void* host, lc2e_dtype dtype, const
             err = lc2e::launch_convert(tmp.staging, (int)dtype, v->d, f16, n, e->stream);
     }
     if (err == hipSuccess) err = hipStreamSynchronize(e->stream);
+    tmp.idle = err == hipSuccess;
     if (err != hipSuccess || *tmp.flag) {
         e->release(v->d, v->bytes);
         delete v;

@@ -448,6 +448,34 @@ void old_blocks_make_room_for_new_ones() {
     CHECK(fake::used(0) == 0);
 }
 
+// After the first one an upload makes no pinned memory, with a budget or without, and a small int16
+// volume's storage is settled without the device.
+void small_uploads_make_nothing_pinned() {
+    for (size_t budget : {size_t(0), GB}) {
+        lc2e_engine* e = engine(budget);
+        std::vector<short> img(33 * 32 * 32);
+        long long pinned = 0;
+        for (int k = 0; k < 4; ++k) {
+            lc2e_volume* v = nullptr;
+            lc2e_geom g{};
+            for (int a = 0; a < 3; ++a) g.dims[a] = a ? 32 : k < 2 ? 32 : 33, g.spacing[a] = 1.0f;
+            if (k == 3) img[32 * 32 * 32] = 3000;  // past the voxels that the host looks at
+            fake::launches().clear();
+            size_t used0 = 0, used = 0;
+            CHECK(lc2e_memory(e, &used0, nullptr) == LC2E_OK);
+            CHECK(lc2e_volume_upload(e, img.data(), LC2E_I16, &g, LC2E_STORE_AUTO, &v) == LC2E_OK);
+            CHECK(lc2e_memory(e, &used, nullptr) == LC2E_OK);
+            const size_t n = size_t(g.dims[0]) * 32 * 32, pad = size_t(g.dims[0]) * 33 + 64;
+            CHECK(used - used0 == (n + pad) * 2);  // (kernels do not run here: nothing is flagged)
+            CHECK(fake::count("k_check") == (k < 2 ? 0 : 1));
+            lc2e_volume_destroy(v);
+            if (k == 0) pinned = fake::pinned();
+        }
+        CHECK(fake::pinned() == pinned);
+        lc2e_destroy(e);
+    }
+}
+
 //@SCENARIOS
 
 const std::map<std::string, std::function<void()>> kScenarios = {
@@ -467,6 +495,7 @@ const std::map<std::string, std::function<void()>> kScenarios = {
     {"chunks_fit_the_kernel_that_runs", chunks_fit_the_kernel_that_runs},
     {"joint_histograms_that_warp_again_spread_out", joint_histograms_that_warp_again_spread_out},
     {"old_blocks_make_room_for_new_ones", old_blocks_make_room_for_new_ones},
+    {"small_uploads_make_nothing_pinned", small_uploads_make_nothing_pinned},
 //@TABLE
 };
 

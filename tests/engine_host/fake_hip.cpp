@@ -30,7 +30,7 @@ struct State {
     std::map<std::pair<const void*, int>, void*> var_addr;  // (variable, device) -> address
     std::set<hipStream_t> capturing;
     int in_capture = 0;
-    long long mallocs = 0, attempts = 0, copies = 0;
+    long long mallocs = 0, attempts = 0, copies = 0, pinned = 0;
 };
 State& g() {
     static State* s = new State();
@@ -61,7 +61,7 @@ void reset(size_t device_bytes) {
     g().limit = device_bytes;
     g().launches.clear();
     g().in_capture = 0;
-    g().mallocs = g().attempts = g().copies = 0;
+    g().mallocs = g().attempts = g().copies = g().pinned = 0;
 }
 std::vector<Launch>& launches() { return g().launches; }
 int in_capture() { return g().in_capture; }
@@ -69,6 +69,7 @@ size_t used(int device) { return g().used[device]; }
 long long mallocs() { return g().mallocs; }
 long long attempts() { return g().attempts; }
 long long copies() { return g().copies; }
+long long pinned() { return g().pinned; }
 bool live(const void* p) {
     std::lock_guard<std::recursive_mutex> lk(g().mu);
     for (const auto& b : g().blocks)
@@ -120,7 +121,11 @@ hipError_t hipFree(void* p) {
     g().blocks.erase(it);
     return hipSuccess;
 }
-hipError_t hipHostMalloc(void** p, size_t n, unsigned) { return (*p = std::calloc(1, n ? n : 1)) ? hipSuccess : hipErrorOutOfMemory; }
+hipError_t hipHostMalloc(void** p, size_t n, unsigned) {
+    LOCK;
+    ++g().pinned;
+    return (*p = std::calloc(1, n ? n : 1)) ? hipSuccess : hipErrorOutOfMemory;
+}
 hipError_t hipHostFree(void* p) { return std::free(p), hipSuccess; }
 hipError_t hipHostGetDevicePointer(void** d, void* h, unsigned) { return *d = h, hipSuccess; }
 hipError_t hipMemcpy(void* d, const void* s, size_t n, hipMemcpyKind) { return std::memcpy(d, s, n), hipSuccess; }

@@ -36,6 +36,7 @@ bool live(const void* p);           // p lies in an allocation of device memory
 long long mallocs();                // hipMalloc calls that succeeded
 long long attempts();               // all
 long long copies();                 // asynchronous ones
+long long pinned();                 // hipHostMalloc calls
 int count(const char* kernel_part);  // launches whose kernel's name holds the text
 
 }  // namespace fake

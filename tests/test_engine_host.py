@@ -49,6 +49,7 @@ def engine_test(tmp_path_factory):
     "chunks_fit_the_kernel_that_runs",
     "joint_histograms_that_warp_again_spread_out",
     "old_blocks_make_room_for_new_ones",
+    "small_uploads_make_nothing_pinned",
 ])
 def test_engine_host(engine_test, scenario):
     r = subprocess.run([engine_test, scenario], capture_output=True, text=True, timeout=120)
