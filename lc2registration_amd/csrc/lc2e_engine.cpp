@@ -265,11 +265,12 @@ struct lc2e_pair {
     int part_bpp = 0;  // partial sums per pose the partials buffer holds
     float* d_mats = nullptr;
     double* d_partials = nullptr;
-    float* h_mats = nullptr;   // pinned, mapped and coherent
-    double* h_out = nullptr;   // pinned, mapped and coherent
+    float* h_mats = nullptr;   // pinned, mapped and coherent, in one block of h_bytes
+    double* h_out = nullptr;
+    size_t h_bytes = 0;
     float* h_mats_dev = nullptr;   // their device addresses
     double* h_out_dev = nullptr;
-    double* h_part = nullptr;      // pinned, mapped and coherent: kHostPartials partials
+    double* h_part = nullptr;      // kHostPartials partials
     double* h_part_dev = nullptr;
     size_t cap_bytes = 0;
     bool use_graph = false;
@@ -576,9 +577,7 @@ void free_batch(lc2e_pair* p) {
     lc2e_engine* e = p->e;
     if (p->d_mats) e->release(p->d_mats, (size_t)p->cap * p->mats_per_pose() * 12 * sizeof(float));
     if (p->d_partials) e->release(p->d_partials, (size_t)p->cap * p->part_bpp * 2 * sizeof(double));
-    e->host_free(p->h_mats, (size_t)p->cap * p->mats_per_pose() * 12 * sizeof(float));
-    e->host_free(p->h_out, (size_t)p->cap * 3 * sizeof(double));
-    e->host_free(p->h_part, kHostPartials * 2 * sizeof(double));
+    e->host_free(p->h_mats, p->h_bytes);
     p->h_part = nullptr;
     p->h_part_dev = nullptr;
     p->d_mats = nullptr;
@@ -836,31 +835,25 @@ int ensure_batch(lc2e_pair* p, int n, int bpp) {
     }
     p->cap = cap;  // free_batch returns the device bytes by these sizes
     p->part_bpp = bpp;
-    void* hm = nullptr;
-    void* ho = nullptr;
-    // mapped and coherent: small launches read their matrices from here and every launch's
-    // reduction writes its results here, with no copy command (enqueue_batch)
-    hipError_t he = e->host_alloc(&hm, (size_t)cap * mpp * 12 * sizeof(float));
+    // Mapped and coherent: small launches read their matrices from here and every launch's
+    // reduction writes its results here, with no copy command (enqueue_batch). One block: an
+    // engine with a budget makes and frees it with every pair, 30 us each.
+    auto up256 = [](size_t b) { return (b + 255) / 256 * 256; };
+    const size_t mats_b = up256((size_t)cap * mpp * 12 * sizeof(float)), out_b = up256((size_t)cap * 3 * sizeof(double));
+    void *h = nullptr, *d = nullptr;
+    p->h_bytes = mats_b + out_b + kHostPartials * 2 * sizeof(double);
+    hipError_t he = e->host_alloc(&h, p->h_bytes);
     if (he == hipSuccess) {
-        p->h_mats = (float*)hm;
-        he = e->host_alloc(&ho, (size_t)cap * 3 * sizeof(double));
-        if (he == hipSuccess) p->h_out = (double*)ho;
+        p->h_mats = static_cast<float*>(h);
+        he = hipHostGetDevicePointer(&d, h, 0);
     }
-    void* hp = nullptr;
     if (he == hipSuccess) {
-        he = e->host_alloc(&hp, kHostPartials * 2 * sizeof(double));
-        if (he == hipSuccess) p->h_part = (double*)hp;
-    }
-    void* dm = nullptr;
-    void* dout = nullptr;
-    void* dpart = nullptr;
-    if (he == hipSuccess) he = hipHostGetDevicePointer(&dpart, hp, 0);
-    p->h_part_dev = (double*)dpart;
-    if (he == hipSuccess) he = hipHostGetDevicePointer(&dm, hm, 0);
-    if (he == hipSuccess) he = hipHostGetDevicePointer(&dout, ho, 0);
-    if (he == hipSuccess) {
-        p->h_mats_dev = (float*)dm;
-        p->h_out_dev = (double*)dout;
+        auto at = [](void* base, size_t ofs) { return reinterpret_cast<double*>(static_cast<char*>(base) + ofs); };
+        p->h_out = at(h, mats_b);
+        p->h_part = at(h, mats_b + out_b);
+        p->h_mats_dev = static_cast<float*>(d);
+        p->h_out_dev = at(d, mats_b);
+        p->h_part_dev = at(d, mats_b + out_b);
     }
     if (he != hipSuccess) {
         free_batch(p);  // no half-made buffers: the next call allocates again
