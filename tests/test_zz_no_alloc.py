@@ -90,3 +90,31 @@ def test_noalloc_equals_batch_on_the_separable_path_and_in_parts(engine, ndim, r
     p.close()
     for v in vols:
         v.close()
+
+
+def test_noalloc_beside_a_launch_on_another_stream(engine):
+    """Allocation-free calls while stream-ordered launches of the same pair are in flight: neither
+    sees the other's warped images."""
+    import ctypes as C
+
+    import torch
+
+    w = synth.small3d()
+    p, vols = _pair(engine, w)
+    here, there = _mats(p, w, 24, 3), _mats(p, w, 24, 4)
+    want_here, want_there = p.eval_batch(here), p.eval_batch(there)
+    stream = torch.cuda.Stream()
+    d_mats = torch.from_numpy(np.ascontiguousarray(there)).cuda()
+    outs = [torch.zeros(24, 3, dtype=torch.float64, device="cuda") for _ in range(8)]
+    torch.cuda.synchronize()
+    for out in outs:
+        assert E.lib().lc2e_eval_batch_async(p.h, 24, C.c_void_p(d_mats.data_ptr()),
+                                             C.c_void_p(out.data_ptr()), C.c_void_p(stream.cuda_stream)) >= 0
+        got = p.eval_batch_noalloc(here)
+        assert np.array_equal(got.lc2, want_here.lc2)
+    stream.synchronize()
+    for out in outs:
+        assert np.array_equal(out.cpu().numpy()[:, 2], want_there.lc2)
+    p.close()
+    for v in vols:
+        v.close()
