@@ -265,12 +265,12 @@ struct lc2e_pair {
     int part_bpp = 0;  // partial sums per pose the partials buffer holds
     float* d_mats = nullptr;
     double* d_partials = nullptr;
-    float* h_mats = nullptr;   // pinned, mapped and coherent, in one block of h_bytes
+    float* h_mats = nullptr;   // pinned, mapped and coherent; with h_out a block of h_bytes
     double* h_out = nullptr;
     size_t h_bytes = 0;
     float* h_mats_dev = nullptr;   // their device addresses
     double* h_out_dev = nullptr;
-    double* h_part = nullptr;      // kHostPartials partials
+    double* h_part = nullptr;      // pinned, mapped and coherent: kHostPartials partials
     double* h_part_dev = nullptr;
     size_t cap_bytes = 0;
     bool use_graph = false;
@@ -578,6 +578,7 @@ void free_batch(lc2e_pair* p) {
     if (p->d_mats) e->release(p->d_mats, (size_t)p->cap * p->mats_per_pose() * 12 * sizeof(float));
     if (p->d_partials) e->release(p->d_partials, (size_t)p->cap * p->part_bpp * 2 * sizeof(double));
     e->host_free(p->h_mats, p->h_bytes);
+    e->host_free(p->h_part, kHostPartials * 2 * sizeof(double));
     p->h_part = nullptr;
     p->h_part_dev = nullptr;
     p->d_mats = nullptr;
@@ -836,24 +837,23 @@ int ensure_batch(lc2e_pair* p, int n, int bpp) {
     p->cap = cap;  // free_batch returns the device bytes by these sizes
     p->part_bpp = bpp;
     // Mapped and coherent: small launches read their matrices from here and every launch's
-    // reduction writes its results here, with no copy command (enqueue_batch). One block: an
-    // engine with a budget makes and frees it with every pair, 30 us each.
-    auto up256 = [](size_t b) { return (b + 255) / 256 * 256; };
-    const size_t mats_b = up256((size_t)cap * mpp * 12 * sizeof(float)), out_b = up256((size_t)cap * 3 * sizeof(double));
-    void *h = nullptr, *d = nullptr;
-    p->h_bytes = mats_b + out_b + kHostPartials * 2 * sizeof(double);
+    // reduction writes its results here, with no copy command (enqueue_batch). Two blocks: an
+    // engine with a budget makes and frees them with every pair, 30 us each (with the partial sums
+    // in the first one too, 4 poses 256x256, r = 3, take 0.6 us longer).
+    const size_t mats_b = ((size_t)cap * mpp * 12 * sizeof(float) + 255) / 256 * 256;
+    void *h = nullptr, *d = nullptr, *hp = nullptr, *dp = nullptr;
+    p->h_bytes = mats_b + (size_t)cap * 3 * sizeof(double);
     hipError_t he = e->host_alloc(&h, p->h_bytes);
+    p->h_mats = static_cast<float*>(h);
+    if (he == hipSuccess) he = e->host_alloc(&hp, kHostPartials * 2 * sizeof(double));
+    p->h_part = static_cast<double*>(hp);
+    if (he == hipSuccess) he = hipHostGetDevicePointer(&d, h, 0);
+    if (he == hipSuccess) he = hipHostGetDevicePointer(&dp, hp, 0);
     if (he == hipSuccess) {
-        p->h_mats = static_cast<float*>(h);
-        he = hipHostGetDevicePointer(&d, h, 0);
-    }
-    if (he == hipSuccess) {
-        auto at = [](void* base, size_t ofs) { return reinterpret_cast<double*>(static_cast<char*>(base) + ofs); };
-        p->h_out = at(h, mats_b);
-        p->h_part = at(h, mats_b + out_b);
+        p->h_out = reinterpret_cast<double*>(static_cast<char*>(h) + mats_b);
         p->h_mats_dev = static_cast<float*>(d);
-        p->h_out_dev = at(d, mats_b);
-        p->h_part_dev = at(d, mats_b + out_b);
+        p->h_out_dev = reinterpret_cast<double*>(static_cast<char*>(d) + mats_b);
+        p->h_part_dev = static_cast<double*>(dp);
     }
     if (he != hipSuccess) {
         free_batch(p);  // no half-made buffers: the next call allocates again

@@ -298,9 +298,10 @@ void k_moments2d(FusedArgs a) {
             // share, the suffixes before them and the prefixes after them (A: the wave's first row
             // of its block)
             double S[OUT][NC];
-            if constexpr (W >= 7 && OUT == 8 && ROLE != kRoleMovingImage) {
-                // (as the lambda below, with A = 0, these roles take 2 to 6% longer; the other one
-                // 2 to 5% less: the compiler orders the loads differently)
+            if constexpr (W >= 7 && OUT == 8 && (ROLE != kRoleMovingImage || (!INPLACE && R == 6))) {
+                // (As the lambda below, with A = 0, these take 2 to 11% longer, and the others 2 to 18%
+                // less: the compiler orders the loads differently. 512x400, moving image, 32 poses,
+                // in line and lambda: R = 6 99 and 110 us, R = 7 114 and 110, R = 9 141 and 116.)
                 double t[NC];
 #pragma unroll
                 for (int c = 0; c < NC; ++c) t[c] = 0.0;

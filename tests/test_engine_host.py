@@ -50,7 +50,7 @@ def engine_test(tmp_path_factory):
     "joint_histograms_that_warp_again_spread_out",
     "old_blocks_make_room_for_new_ones",
     "small_uploads_make_nothing_pinned",
-    "a_pair_makes_one_pinned_block",
+    "a_pair_makes_two_pinned_blocks",
 ])
 def test_engine_host(engine_test, scenario):
     r = subprocess.run([engine_test, scenario], capture_output=True, text=True, timeout=120)
