@@ -141,8 +141,9 @@ int lc2e_pose_to_matrix(lc2e_pair* p, const double* params, int n_params, float 
  * per-frame stacks). LC2 NaN/Inf -> 0 with status LC2E_OK_DEGENERATE. */
 int lc2e_eval(lc2e_pair* p, const float* m12, double* lc2);
 
-/* n poses in one fused launch; no counterpart in the reference, whose global __constant__
- * transform allows one pose in flight (interpolator.cuh:27-41). Results are bit-identical
+/* n poses in one call (one launch, or several where a workspace holds fewer poses); no
+ * counterpart in the reference, whose global __constant__ transform allows one pose in flight
+ * (interpolator.cuh:27-41). Results are bit-identical
  * to n single evaluations. Optional outputs (NULL to skip): sum of measures, sum of w. */
 int lc2e_eval_batch(lc2e_pair* p, int n, const float* mats, double* lc2, double* sum_measure,
                     double* sum_w);
@@ -189,17 +190,17 @@ int lc2e_eval_mi_batch(lc2e_pair* p, int n, const float* mats, int bins_us, int 
  * (WARP_I, WARP_US, GRAD) or float64 (W, MEASURE). */
 int lc2e_debug_fetch(lc2e_pair* p, lc2e_stage stage, const float* m12, void* host);
 
-/* Launch configuration of the 3D fused kernel: output planes per work-group (z-chunk).
+/* Launch configuration of the 3D kernels: output planes per work-group (z-chunk).
  * Each launch of n poses uses, in order: the value forced by lc2e_pair_set_tuning
  * (0 = none), the value set or tuned for batches of exactly n poses
  * (lc2e_pair_set_tuning_n, lc2e_pair_autotune; 0 = none), or a model of the launch
- * (work-group rounds over the CUs times the planes each work-group marches).
+ * (the finishing time of its last work-group, from the planes each one marches).
  * get_tuning reports the forced value, else the one the last launch used.
  * No counterpart in the reference (its launch shape is fixed at 8x8x8). */
 int lc2e_pair_set_tuning(lc2e_pair* p, int zchunk);
 int lc2e_pair_set_tuning_n(lc2e_pair* p, int n, int zchunk);
 int lc2e_pair_get_tuning(lc2e_pair* p, int* zchunk);
-/* Autotuner: times the fused kernel over candidate z-chunks (HIP events, `iters` launches
+/* Autotuner: times the evaluation's kernels over candidate z-chunks (HIP events, `iters` launches
  * each after one warm-up) for batches of n poses `mats`, records the fastest for batches
  * of n and returns it. A z-chunk forced with lc2e_pair_set_tuning stays in force (and
  * takes precedence) until it is cleared with 0. 2D pairs have nothing to tune and
@@ -207,10 +208,10 @@ int lc2e_pair_get_tuning(lc2e_pair* p, int* zchunk);
 int lc2e_pair_autotune(lc2e_pair* p, int n, const float* mats, int iters, int* best_zchunk,
                        double* best_ms);
 
-/* Kernel timing with HIP events recorded around every fused-kernel launch on the engine's
+/* Kernel timing with HIP events recorded around the kernels of every launch on the engine's
  * stream. While timing is on, batches are launched eagerly even where graph replay is on
  * (the events bracket the kernel itself); replay resumes when it is turned off. enable = 1
- * resets the counters. read returns the summed fused-kernel time in ms and the number of
+ * resets the counters. read returns the summed kernel time in ms and the number of
  * launches since the reset. */
 int lc2e_pair_profile(lc2e_pair* p, int enable);
 int lc2e_pair_profile_read(lc2e_pair* p, double* kernel_ms, long long* launches);

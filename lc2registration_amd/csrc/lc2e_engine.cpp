@@ -305,7 +305,7 @@ struct lc2e_pair {
     bool pinned = false;  // a caller's graph holds launches that use the workspace
     bool na = false;  // counted in the engine's na_pairs
     double* istat = nullptr;
-    int resident_per_cu = 0;  // fused work-groups one CU holds at once (0: not queried yet)
+    int resident_per_cu = 0;  // work-groups of the evaluation one CU holds at once (0: not queried yet)
     // separable path (radius beyond the fused kernels): grids and box-sum buffers, made at
     // pair creation
     bool sep = false;
@@ -387,8 +387,8 @@ bool in_place(const lc2e_pair* p, const Workspace& w, int tiles, int n) {
     return p->info.grid_ndim == 2 && (!w.d || (long long)tiles * 4 * part(w, n) < kInPlaceWaves);
 }
 
-// The pair's evaluation kernels for n poses: the fused kernel, or the separable path for
-// radii beyond it.
+// The pair's evaluation kernels for n poses: the moments kernels after a warp into the workspace
+// (or in place), the fused kernel, or the separable path.
 hipError_t launch_eval(lc2e_pair* p, const lc2e::FusedArgs& a, int n, hipStream_t st, const Workspace& w) {
     if (p->two && in_place(p, w, a.tiles, n)) {
         lc2e::FusedArgs s = a;
@@ -441,13 +441,13 @@ int resident_per_cu(lc2e_pair* p) {
 }
 
 // z-chunk for a launch of n poses when nothing is tuned. A work-group of chunk c marches
-// min(c, planes left) + 2R + 4 plane steps (fused kernel), or as many planes and its pipeline's fill
-// (two-kernel path: 4 planes' worth with a moving high-resolution image, 8 with a static one; against
-// every chunk at 588 launches of 7 grids, radii 1 to 6, 1 to 32 poses the choice is 0.5% off the
-// fastest on average and 7% and 13% at worst, 8 planes for both 1.1% and 21%). Work-groups go to the XCDs round-robin by id
-// and, within an XCD, to the first free slot in id order (map_block: tile-major, the poses
-// of a tile consecutive; tiles ordered by z-chunk), each CU holding resident_per_cu of them.
-// The model replays that dispatch with a min-heap of slot finishing times per XCD and takes
+// min(c, planes left) + 2R + 4 plane steps (fused kernel), or as many planes and its pipeline's
+// fill (two-kernel path: 4 planes' worth with a moving high-resolution image, 8 with a static
+// one; against every chunk at 588 launches of 7 grids, radii 1 to 6, 1 to 32 poses the choice is
+// 0.5% off the fastest on average and 7% and 13% at worst, 8 planes for both 1.1% and 21%).
+// Work-groups go to the XCDs round-robin by id and, within an XCD, to the first free slot in id
+// order (map_block: tile-major, the poses of a tile consecutive; tiles ordered by z-chunk), each
+// CU holding resident_per_cu of them. The model replays that dispatch with a min-heap of slot finishing times per XCD and takes
 // the latest finish; launches of more than 32 rounds fall back to rounds x steps. Minimise
 // over the chunk lengths (multiples of kZBlock; ties: longer chunks). Cached per launch size.
 int model_zchunk(lc2e_pair* p, int n) {
@@ -910,12 +910,12 @@ lc2e::FusedArgs make_args(lc2e_pair* p, const float* d_mats, double* d_partials,
     return a;
 }
 
-// Enqueue: the staged matrices to the device, the fused kernel, the reduction into the
-// pinned result buffer. Each launch command costs several microseconds, so small launches
-// (up to kDirectPoses poses of one matrix each, on a single volume or image: each
-// work-group reads its pose's 12 floats once) read the pinned matrices in place instead of
-// copying them (13 poses 1.5 us less, 32 poses 2 us), and the reduction always writes the results in place: one or two commands
-// per batch instead of four. Where a launch is not captured, up to kInlineMats such matrices go
+// Enqueue: the staged matrices to the device, the evaluation, the reduction into the pinned
+// result buffer. Each launch command costs several microseconds, so small launches (up to
+// kDirectPoses poses of one matrix each, on a single volume or image: each work-group reads its
+// pose's 12 floats once) read the pinned matrices in place instead of copying them (13 poses
+// 1.5 us less, 32 poses 2 us), and the reduction always writes the results in place: two
+// commands less per batch. Where a launch is not captured, up to kInlineMats such matrices go
 // with the arguments of the kernels that read them there (all but the 2D fused kernel; a read from
 // pinned memory takes 1.2 us at a kernel's start: 4 poses 194x248, r = 5, 33.4 -> 31.6 us), and few
 // partials go straight to pinned memory for the host to add up (*host_sum), a launch less: 13 poses
@@ -936,7 +936,7 @@ int enqueue_batch(lc2e_pair* p, int n, const Tiling& t, hipStream_t st, bool cap
             a.inline_mat = 1;
             std::memcpy(a.m0, p->h_mats, (size_t)n * 12 * sizeof(float));
         }
-        // timed launches are eager (run_batch), the events bracket the fused kernel
+        // timed launches are eager (run_batch), the events bracket the evaluation
         const bool timed = p->profile;
         if (timed) HIP_TRY(hipEventRecord(p->ev0, st));
         HIP_TRY(launch_eval(p, a, n, st, {p->ws, p->ws_poses}));
@@ -1022,7 +1022,7 @@ void set_last_error(const std::string& msg) { g_last_error = msg; }
 int engine_alloc(lc2e_engine* e, void** p, size_t bytes) { return e->alloc(p, bytes); }
 void engine_release(lc2e_engine* e, void* p, size_t bytes) { e->release(p, bytes); }
 int engine_device(lc2e_engine* e) { return e->device; }
-// The share of the device one fused launch of n poses occupies: its work-groups over the
+// The share of the device one launch of n poses occupies: its work-groups over the
 // work-groups all CUs hold at once (>= 1: it fills the GPU by itself). The serving loop
 // runs launches side by side only while their shares add up to at most 1.
 // Generation of the pair's launch state: graphs captured under another generation are stale.
@@ -1128,8 +1128,8 @@ int lc2e_volume_upload(lc2e_engine* e, const void* host, lc2e_dtype dtype, const
         return fail(LC2E_ERR_INVALID, "storage must be F16, F32 or AUTO");
     HIP_TRY(hipSetDevice(e->device));
     // The raw voxels on the device (also its conversion's input) and two words that the kernels
-    // set where a voxel is out of range (launch_check): the device reads them at the memory's rate, where a
-    // scan on the host took half of an upload.
+    // set where a voxel is out of range (launch_check): the device reads them at the memory's rate,
+    // where a scan on the host took half of an upload.
     struct Scope {
         lc2e_engine* e;
         void* staging = nullptr;

@@ -61,9 +61,9 @@ __device__ __forceinline__ void box_xy_inplace_r(int r, double* s_prod, int tid)
 // 2D fused kernel for a moving high-resolution image at small radii (r <= kMaxRFused2; from r = 4
 // on its 16x16 tiles' halos make k_moments2d the faster one: 128 frames 512x384, 3 poses, r = 4
 // 2.02 -> 1.68 ms, r = 6 2.28 -> 1.59 ms; at r = 3 this kernel takes 4.45 ms for 13 poses, that
-// one 6.35): one 16x16 output tile of a run of `zchunk` (kFrameRun) consecutive
-// frames of one pose (a single image is one frame). Dynamic LDS sized for the runtime patch
-// radius. Frame f + 1's gathers (and its static image values and ultrasound statistics)
+// one 4.9 in place and 6.4 through the grid): one 16x16 output tile of a run of `zchunk`
+// (kFrameRun) consecutive frames of one pose (a single image is one frame). Dynamic LDS sized for
+// the runtime patch radius. Frame f + 1's gathers (and its static image values and ultrasound statistics)
 // are issued while frame f's box sums and combine run, as in the 3D kernel's z-steps. Each
 // thread adds its pixel's measure and weight over the run's frames in frame order, and the
 // work-group reduces them once into the partial of (run, tile). The run length does not

@@ -68,7 +68,7 @@ struct FusedArgs {
     double* wmap;            // optional per-voxel w (single pose), may be null
     double* mmap;            // optional per-voxel measure, may be null
     int r;
-    int zchunk;              // 3D: output planes per work-group
+    int zchunk;              // 3D: output planes per work-group; 2D: frames per work-group
     int ntx, nty, nzc;       // tiles along x, y and z chunks (3D) / frames (2D)
     int blocks_per_pose;     // partial sums per pose
     int tiles;               // work-groups per pose

@@ -8,7 +8,7 @@ namespace lc2e {
 
 namespace {
 
-constexpr int kWarpX = 32, kWarpY = 16;  // output tile of k_warp_grad2
+constexpr int kWarpX = 32, kWarpY = 16;  // output tile of k_warp2
 
 template <bool P2, bool SRC3D, typename T, typename Pend>
 __device__ __forceinline__ void issue_any(const T* src, const SGeom& s, const float* m, float lx, float ly,
@@ -95,20 +95,23 @@ __global__ __launch_bounds__(256) void k_warp2(FusedArgs a, int ntx, int nty, in
 }
 
 // ---------------------------------------------------------------------------
-// Patch moments and combine. A wave owns 64 columns (64 - 2R outputs per row) and 8 output rows:
-// each lane forms the y window sums of its column for the 8 rows in registers, then per channel
-// the x window sums through 5 KB of LDS that no other wave uses (no barrier), and combines the 8
-// pixels of its column. Four waves of a work-group take four groups of rows and share one
-// partial sum per run of frames. A tile has no halo along y but the rows' own (2R + 8 for 8) and
+// Patch moments and combine. A wave owns 64 columns (64 - 2R outputs per row; 62 - 2R with the
+// Sobel in place) and 8 output rows: each lane forms the y window sums of its column for the 8
+// rows in registers, then per channel the x window sums through 5 KB of LDS that no other wave uses
+// (wave fences, no barrier), and combines the 8 pixels of its column. Four waves of a work-group take
+// four groups of rows and share one partial sum per run of frames. Warping in place takes barriers
+// around the shared rows: per frame one before and one after the warp, and one after the Sobel.
+// OUT = 4 (below) has eight waves of four rows. A tile has no halo along y but the rows' own (2R + 8 for 8) and
 // a short one along x, where 16x16 tiles form the products of (16 + 2R)^2 positions for 256
 // outputs: 4.5 times each at R = 9.
 // With a static high-resolution image its sums do not depend on the pose (kRoleImageStats, at
 // pair creation): 4 channels instead of 9 and a count. Two to three waves per SIMD (130 to 230
 // VGPRs); bound by the latency of the three LDS trips per channel and of the FP64 chains (VALU a
-// quarter busy). Measured, static image: 256x256, R = 3, 64 poses 104 -> 42 us; 261x261, R = 9,
-// 13 poses 100 -> 30 us; moving image: 336x205 slice in a CT, R = 9, 13 poses 60 -> 38 us.
-// In place the four waves share the warped rows (32 + 2R for 32, where each warped 8 + 2R of its
-// own): per call 256x256, R = 3, 64 poses 62 -> 55 us, one pose 27.7 -> 26.9; R = 9, 13 poses 45 -> 40.
+// quarter busy). Measured, static image: 256x256, R = 3, 64 poses 104 -> 38 us; 261x261, R = 9,
+// 13 poses 100 -> 20 us; moving image: 336x205 slice in a CT, R = 9, 13 poses 60 -> 25 us after
+// 11 us of k_warp2. In place the waves share the warped rows (32 + 2R for 32, where each warped
+// 8 + 2R of its own): per call 256x256, R = 3, 64 poses 62 -> 55 us, one pose 27.7 -> 26.9 (OUT = 4:
+// 25.2); R = 9, 13 poses 45 -> 40 (OUT = 4: 36.5).
 // ---------------------------------------------------------------------------
 // LDS column x of a wave's row: 2 doubles of padding after every 8, and rows 80 doubles apart,
 // spread the 16-byte reads of the x pass (8 runs of 8 columns, 8 rows) over all banks.

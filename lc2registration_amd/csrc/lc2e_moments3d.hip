@@ -1,12 +1,14 @@
-// 3D LC2 with the moving image as the high-resolution one, in two kernels: k_warp_grad3 writes
-// the warped image and its |Sobel| for every voxel of the grid and pose (8 bytes), and
-// k_moments3d forms the patch moments from those grids and combines them.
+// 3D LC2 in two kernels. The first writes the warped moving image of every voxel of the grid and
+// pose: k_warp_grad3 a high-resolution one and its |Sobel| (8 bytes), k_warp_us3 an ultrasound
+// (4 bytes). k_moments3d forms the patch moments from those grids and combines them.
 //
 // The fused kernel (k_fused3d) computes both per 16x16 tile, so it warps 2.25 and takes the
 // Sobel of 1.89 positions per output voxel, and its 238 VGPRs hold two waves per SIMD. Apart,
 // the first kernel's tile has 1.2 warped positions per voxel, and the second needs 84 VGPRs.
 // The grids cost 8 bytes written and about 10 read per voxel and pose, at 1 TB/s far from the
-// memory's rate. 192x192x160 grid, 7^3 patch, 32 poses: 3.40 -> 2.80 ms.
+// memory's rate. Per call, 192x192x160 grid, 7^3 patch, moving image high-resolution, 32 poses:
+// 3.40 -> 2.65 ms; static, 16 poses: the ultrasound's 4 channels, the other sums once per pair
+// (kRoleImageStats), 226 us of warp and 848 of moments.
 #include "lc2e_device.hpp"
 
 namespace lc2e {
@@ -19,7 +21,7 @@ constexpr int kGradX = 32, kGradY = 16;  // output tile of k_warp_grad3
 // float2, bit for bit as k_fused3d forms them. A work-group marches along z over a 32x16
 // column; the gathers of the next plane are in flight during the Sobel of this one, and the
 // two LDS planes take one barrier per step. Bound by VALU issue (102 instructions per voxel,
-// 73% of the issue slots): 365 us for 16 poses of 192x192x160, 2 TB/s written.
+// 73% of the issue slots): 352 us for 16 poses of 192x192x160, 2.1 TB/s written.
 template <typename T, bool P2, bool WORDS>
 __global__ __launch_bounds__(256) void k_warp_grad3(FusedArgs a, int ntx, int nty, int zc, int tiles,
                                                     int npose) {
@@ -168,7 +170,7 @@ __global__ __launch_bounds__(256) void k_warp_us3(FusedArgs a, int ntx, int nty,
 // per wave a ds_write_b64 takes 6.2 cycles, a ds_write_b128 13, a ds_read_b64 2.2, a
 // ds_read_b128 4.1, but a ds_read2_b64 of two rows 8.0 (measured), so the y sums stay in
 // registers up to the combine (no second write) and are read row by row.
-// Measured at 192x192x160, R = 3, 16 poses: 1.03 ms; with every phase on all waves and a
+// Measured at 192x192x160, R = 3, 16 poses: 0.95 ms. Before its last change of layout (1.03 ms): every phase on all waves, a
 // barrier between phases 1.13 ms (512 threads, 80 VGPRs), with the z sums last in a VGPR ring
 // 1.13 ms (256 threads, 158 VGPRs); one plane per step, two work-groups per CU: 1.62 ms.
 // Raised priorities for the x or the y waves: 1 to 8% slower.
