@@ -158,7 +158,8 @@ int lc2e_eval_batch(lc2e_pair* p, int n, const float* mats, double* lc2, double*
  * and 6 under a budget, whose buffers every launch of a pair shares). The call uses no
  * hipMalloc/hipFree and no allocating library routine. Same kernels, so the results are bit-identical to lc2e_eval_batch. A call needs
  * n*(24 + 48*mats_per_pose) + n*16*(partial sums per pose) bytes (each part rounded up to
- * 256); a larger call fails with LC2E_ERR_INVALID. Every call on a device shares that
+ * 256; 2D: a partial sum per 16x16 outputs and 16 frames, 3D: four per 16x16x8, beyond radius
+ * 4 (3D) and 10 (2D): one per 256); a larger call fails with LC2E_ERR_INVALID. Every call on a device shares that
  * device's array: concurrent calls would race on it, so the library serialises them per
  * device (a call waits for the one in progress). */
 int lc2e_eval_batch_noalloc(lc2e_pair* p, int n, const float* mats, double* lc2,
@@ -220,7 +221,7 @@ int lc2e_pair_profile_read(lc2e_pair* p, double* kernel_ms, long long* launches)
  * HIP graph on its second lc2e_eval_batch with n poses and replay it for later calls with
  * the same n (1 = on, 0 = off, the default). Graphs are dropped when the pair's buffers or
  * launch shape change. Results are identical either way. On MI355X with ROCm 7.2 a
- * replayed batch took 5-13 us longer than an eager one at 1 to 64 poses, so nothing in
+ * replayed batch took 4-17 us longer than an eager one at 1 to 64 poses, so nothing in
  * this library turns it on by itself (the facade does with LC2E_GRAPHS=1). */
 int lc2e_pair_use_graph(lc2e_pair* p, int enable);
 
